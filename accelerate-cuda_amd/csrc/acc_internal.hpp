@@ -25,6 +25,9 @@
 
 namespace acc {
 
+// sources and targets up to which a permute whose combination is the new value runs in one workgroup (skel_scatter.h)
+constexpr int SCATTER_SMALL = 4096;
+
 // thread-local message of the last failure; returns `code` so that call
 // sites read `return fail(ACC_ERR_INVALID, "...")`
 int fail(int code, const char *fmt, ...) __attribute__((format(printf, 2, 3)));

@@ -255,65 +255,6 @@ permute_join(ACC_ENV_PARAMS ACC_OUT_PARAMS, const ACC_ELT *__restrict__ dump_val
   acc = acc_wave_reduce(acc, lf);
   if (lane == 0 && acc.ok) ACC_SET(arrOut, j, f(acc.v, ACC_READ(arrOut, j)));
 }
-
-/* ---- permute const: the new value, whatever was there ----------------------
- * Where the combination is spelt as its first operand (the host says so by launching these two instead) nothing has
- * to be read or locked: the scatter of a stream compaction or of a sorting pass over pairs, whose targets are all
- * different.  A scalar of one or two bytes is simply stored (permute_place with winner == NULL).  A tuple's components
- * are arrays of their own, and of several sources on one target one must win whole: permute_claim stores every
- * source's index in its target's word of `winner` -- one of them stays -- and permute_place stores the components of
- * the sources that find their own index there.  (`winner` need not be cleared: what permute_place looks at,
- * permute_claim has written in the same call.)  2^24 pairs of Int32, half of them kept, in order: 277 us under
- * locks; a sorting pass by a 4-bit digit: 771 us. */
-#define ACC_CONST_BATCH 4
-extern "C" __global__ void __launch_bounds__(256)
-permute_claim(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 shIn_0, unsigned int *__restrict__ winner ACC_GUARD_PARAM)
-{
-  ACC_GUARD_CHECK
-  ACC_ENV_ASSUME
-  auto perm = [&](const Int64 ix) -> Int64 { return (Int64)(ACC_PERMUTATION(ix)); };
-  const Int64 n = shIn_0;
-  const Int64 ntarget = (ACC_OUT_SIZE);
-  for (Int64 ix0 = (Int64)blockIdx.x * (256 * ACC_CONST_BATCH) + threadIdx.x; ix0 < n; ix0 += (Int64)gridDim.x * (256 * ACC_CONST_BATCH)) {
-    Int64 j[ACC_CONST_BATCH];
-#pragma unroll
-    for (int k = 0; k < ACC_CONST_BATCH; ++k) j[k] = ix0 + k * 256 < n ? perm(ix0 + k * 256) : -1;
-#pragma unroll
-    for (int k = 0; k < ACC_CONST_BATCH; ++k)
-      if (j[k] >= 0 && j[k] < ntarget) winner[j[k]] = (unsigned int)(ix0 + k * 256);
-  }
-}
-
-extern "C" __global__ void __launch_bounds__(256)
-permute_place(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 shIn_0, const unsigned int *__restrict__ winner ACC_GUARD_PARAM)
-{
-  ACC_GUARD_CHECK
-  typedef ACC_ELT T;
-  ACC_ENV_ASSUME
-  auto get  = [&](const Int64 ix) -> T { return (ACC_GET(ix)); };
-  auto perm = [&](const Int64 ix) -> Int64 { return (Int64)(ACC_PERMUTATION(ix)); };
-  const Int64 n = shIn_0;
-  const Int64 ntarget = (ACC_OUT_SIZE);
-  for (Int64 ix0 = (Int64)blockIdx.x * (256 * ACC_CONST_BATCH) + threadIdx.x; ix0 < n; ix0 += (Int64)gridDim.x * (256 * ACC_CONST_BATCH)) {
-    Int64 j[ACC_CONST_BATCH];
-    bool mine[ACC_CONST_BATCH];
-#pragma unroll
-    for (int k = 0; k < ACC_CONST_BATCH; ++k) {
-      j[k] = ix0 + k * 256 < n ? perm(ix0 + k * 256) : -1;
-      mine[k] = j[k] >= 0 && j[k] < ntarget;
-    }
-    if (winner) {
-      unsigned int w[ACC_CONST_BATCH];
-#pragma unroll
-      for (int k = 0; k < ACC_CONST_BATCH; ++k) w[k] = mine[k] ? winner[j[k]] : 0u;
-#pragma unroll
-      for (int k = 0; k < ACC_CONST_BATCH; ++k) mine[k] = mine[k] && w[k] == (unsigned int)(ix0 + k * 256);
-    }
-#pragma unroll
-    for (int k = 0; k < ACC_CONST_BATCH; ++k)
-      if (mine[k]) ACC_SET(arrOut, j[k], get(ix0 + k * 256));
-  }
-}
 #else /* atomics */
 
 #ifndef ACC_RUNS
@@ -326,11 +267,6 @@ permute_place(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 shIn_0, const unsigned 
 #define ACC_HINT_AND 4
 #define ACC_HINT_OR  5
 #define ACC_HINT_XOR 6
-/* (not a hint of the interface: the generator says so where the combination is spelt `x`, the new value whatever was
- * there -- `permute const`, the scatter of a stream compaction or of a sorting pass, whose targets are all different.
- * A plain store then: nothing is read, and of several sources on one target one wins whole, as under any order of
- * the combinations) */
-#define ACC_HINT_REPLACE 7
 
 /* identity of the hinted operator */
 template <typename T>
@@ -362,13 +298,7 @@ ACC_DEV T acc_hint_identity()
 template <int SCOPE, typename T, typename F>
 ACC_DEV void acc_hint_apply(T *p, const T &x, F combine)
 {
-#if ACC_COMBINE_HINT == ACC_HINT_REPLACE
-  (void)combine;
-  typedef typename acc_bits<sizeof(T)>::type B;
-  B nb;
-  __builtin_memcpy(&nb, &x, sizeof(T));
-  __hip_atomic_store((B *)p, nb, __ATOMIC_RELAXED, SCOPE);
-#elif ACC_ELT_IS_INTEGER && ACC_COMBINE_HINT != ACC_HINT_GENERIC
+#if ACC_ELT_IS_INTEGER && ACC_COMBINE_HINT != ACC_HINT_GENERIC
   (void)combine;
 #if ACC_COMBINE_HINT == ACC_HINT_ADD
   (void)__hip_atomic_fetch_add(p, x, __ATOMIC_RELAXED, SCOPE);
@@ -411,7 +341,7 @@ ACC_DEV void acc_hint_apply(T *p, const T &x, F combine)
  * the wave they stand (neighbouring elements of one lane are taken care of by ACC_RUNS).  To find out, a lane looks
  * at its neighbour's target only: with a hot target some two neighbours share it, and where no two neighbours share
  * a target -- nearly always, for targets that are spread -- all this is five instructions an element.           */
-#define ACC_PERMUTE_CAS (ACC_COMBINE_HINT == ACC_HINT_GENERIC || (!ACC_ELT_IS_INTEGER && ACC_COMBINE_HINT != ACC_HINT_ADD && ACC_COMBINE_HINT != ACC_HINT_REPLACE))
+#define ACC_PERMUTE_CAS (ACC_COMBINE_HINT == ACC_HINT_GENERIC || (!ACC_ELT_IS_INTEGER && ACC_COMBINE_HINT != ACC_HINT_ADD))
 template <typename U, typename T, typename F>
 ACC_DEV void acc_wave_gather(U &t, T &x, F f)
 {

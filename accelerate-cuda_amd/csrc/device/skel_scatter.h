@@ -1,0 +1,178 @@
+/*
+ * skel_scatter.h -- forward permutation whose combination is the new value (`permute const`):
+ *
+ *     out = defaults;   for every source index ix:   j = permutation(ix);
+ *     unless j is `ignore`:   out[j] = get(ix)
+ *
+ * The scatter behind `filter`, behind every pass of a sort and behind any reordering (CodeGen/IndexSpace.hs:160-303
+ * takes a lock per element for it, as for every permute).  Nothing is read from the result and nothing is locked; of
+ * several sources on one target one wins whole, as under any order of the combinations.
+ *
+ * What bounds it: memory.  The source is read once (a lane takes single elements, a wave's worth side by side, so that
+ * the elements of a compaction or of a sorting pass leave a wave as runs of neighbouring targets, which the memory
+ * pipeline sends out as whole cache lines), and the stores are ordinary ones that meet in the L2 of the die: every
+ * store with device scope goes through to memory by itself.
+ *
+ * Kernels:
+ *   permute        a tile of ACC_BLOCK x ACC_BATCH sources per workgroup; `winner` as below, or NULL
+ *   permute_claim  for an element that no single store covers -- a tuple, whose components are arrays of their own, or a
+ *                  scalar wider than 8 bytes: every source's index into its target's word of `winner`, where one of them
+ *                  stays; `permute` then stores the sources that find their own index there.  (`winner` need not be
+ *                  cleared: what is looked at has been written in the same call.)
+ *   permute_fill   the defaults into the result
+ *   permute_small  all of it in one workgroup, for sources and results of at most ACC_SMALL elements
+ *
+ * A launch works on the sources [first, past); indices in `winner` count from `first`.
+ *
+ * The operands that the fragments read at the element's own index (ACC_OWN_*, all of them arrays at least `past` long)
+ * are asked for ahead of everything else, for the whole batch: `filter` reads a place only where the element stays, and a
+ * read behind such a test is waited for on the spot, one element after the other.
+ *
+ * Measured with the operands in HBM, 2^24 Int32 sources, defaults included, before (stores of device scope, a lane four
+ * elements side by side, reads behind tests) and now: half of them kept in order 64 us -> 43, a sorting pass by 4 bits
+ * 146 -> 79, by 8 bits 356 -> 176, a random permutation 392 -> 344, all of them on 10 targets of 2^24 9.7 ms -> 0.05;
+ * the scatter of `filter` (flag, place and value of 2^24 read, half stored) 98 -> 27, at 2^20 9.4 -> 4.0.  A lane takes 8
+ * elements (ACC_BATCH): 32 do the sorting pass by 8 bits in 123 us and the random permutation in 262, but the scatter of
+ * `filter` in 32, and in 7.2 at 2^20, where they leave half of the device idle.
+ *
+ * Generated definitions expected: ACC_ELT, ACC_NCOMP, ACC_FOR_COMPONENTS, ACC_ENV_PARAMS, ACC_ENV_ASSUME, ACC_OUT_PARAMS,
+ * ACC_OUT_SIZE, ACC_GET(ix), ACC_PERMUTATION(ix), ACC_OWN_FIELDS, ACC_OWN_LOAD(sv, ix), ACC_OWN_WITHIN(past), ACC_GET_OWN(ix),
+ * ACC_PERMUTATION_OWN(ix), ACC_BLOCK, ACC_BATCH, ACC_SMALL.
+ */
+
+#define ACC_TILE (ACC_BLOCK * ACC_BATCH)
+#define ACC_CLAIMED (ACC_NCOMP > 1 || sizeof(ACC_ELT) > 8)       /* what no single store of at most 8 bytes writes */
+
+/* Names the kernels share.  A tile that reaches past the end reads the last source there (`in`): no test per element
+ * stands in front of a read. */
+#define ACC_SCATTER_NAMES                                                                                                      \
+  typedef ACC_ELT T;                                                                                                           \
+  ACC_ENV_ASSUME                                                                                                               \
+  struct own { ACC_OWN_FIELDS };                                                                                               \
+  auto get      = [&](const Int64 ix) -> T { return (ACC_GET(ix)); };                                                          \
+  auto perm     = [&](const Int64 ix) -> Int64 { return (Int64)(ACC_PERMUTATION(ix)); };                                       \
+  auto get_own  = [&](const Int64 ix, const own &acc_sv) -> T { (void)ix; (void)acc_sv; return (ACC_GET_OWN(ix)); };           \
+  auto perm_own = [&](const Int64 ix, const own &acc_sv) -> Int64 { (void)ix; (void)acc_sv; return (Int64)(ACC_PERMUTATION_OWN(ix)); }; \
+  (void)get; (void)get_own;                                                                                                    \
+  const Int64 ntarget = (ACC_OUT_SIZE);                                                                                        \
+  const Int64 ix0 = first + (Int64)blockIdx.x * ACC_TILE + threadIdx.x;                                                        \
+  auto in = [&](const int k) -> Int64 { return acc_min<Int64>(ix0 + k * ACC_BLOCK, past - 1); };
+
+extern "C" __global__ void __launch_bounds__(ACC_BLOCK)
+permute_claim(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 first, const Int64 past, unsigned int *__restrict__ winner ACC_GUARD_PARAM)
+{
+  ACC_GUARD_CHECK
+  ACC_SCATTER_NAMES
+  Int64 j[ACC_BATCH];
+  if (ACC_OWN_WITHIN(past)) {
+    own sv[ACC_BATCH];
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) { ACC_OWN_LOAD(sv[k], in(k)) }
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) j[k] = perm_own(in(k), sv[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) j[k] = perm(in(k));
+  }
+#pragma unroll
+  for (int k = 0; k < ACC_BATCH; ++k)
+    if (ix0 + k * ACC_BLOCK < past && j[k] >= 0 && j[k] < ntarget) winner[j[k]] = (unsigned int)(ix0 + k * ACC_BLOCK - first);
+}
+
+extern "C" __global__ void __launch_bounds__(ACC_BLOCK)
+permute(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 first, const Int64 past, const unsigned int *__restrict__ winner ACC_GUARD_PARAM)
+{
+  ACC_GUARD_CHECK
+  ACC_SCATTER_NAMES
+  Int64 j[ACC_BATCH];
+  T x[ACC_BATCH];
+  bool mine[ACC_BATCH];
+  if (ACC_OWN_WITHIN(past)) {
+    own sv[ACC_BATCH];
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) { ACC_OWN_LOAD(sv[k], in(k)) }
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) {
+      j[k] = perm_own(in(k), sv[k]);
+      x[k] = get_own(in(k), sv[k]);
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) {
+      j[k] = perm(in(k));
+      x[k] = get(in(k));
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < ACC_BATCH; ++k) mine[k] = ix0 + k * ACC_BLOCK < past && j[k] >= 0 && j[k] < ntarget;
+  if (ACC_CLAIMED) {
+    unsigned int w[ACC_BATCH];
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) w[k] = winner[mine[k] ? j[k] : 0];
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) mine[k] = mine[k] && w[k] == (unsigned int)(ix0 + k * ACC_BLOCK - first);
+  }
+#pragma unroll
+  for (int k = 0; k < ACC_BATCH; ++k)
+    if (mine[k]) ACC_SET(arrOut, j[k], x[k]);
+}
+
+/* `count` elements of one component, in 16-byte pieces where both arrays lie on such boundaries */
+template <typename C>
+ACC_DEV void acc_copy_component(C *__restrict__ dst, const C *__restrict__ src, const Int64 count, const Int64 lane, const Int64 lanes)
+{
+  typedef unsigned int acc_u4 __attribute__((ext_vector_type(4)));
+  if (((((unsigned long long)dst) | ((unsigned long long)src)) & 15u) == 0u) {
+    const Int64 bytes = count * (Int64)sizeof(C), pieces = bytes / 16;
+    for (Int64 i = lane; i < pieces; i += lanes) ((acc_u4 *)dst)[i] = __builtin_nontemporal_load((const acc_u4 *)src + i);
+    for (Int64 i = pieces * 16 + lane; i < bytes; i += lanes) ((unsigned char *)dst)[i] = ((const unsigned char *)src)[i];
+  } else {
+    for (Int64 i = lane; i < count; i += lanes) dst[i] = src[i];
+  }
+}
+
+extern "C" __global__ void __launch_bounds__(256)
+permute_fill(ACC_OUT_ARRAY(arrTo), ACC_CONST_ARRAY(arrFrom), const Int64 count ACC_GUARD_PARAM)
+{
+  ACC_GUARD_CHECK
+  const Int64 lane = (Int64)blockIdx.x * 256 + threadIdx.x, lanes = (Int64)gridDim.x * 256;
+#define ACC_COPY_ONE(c, type) acc_copy_component<type>(arrTo_##c, arrFrom_##c, count, lane, lanes);
+  ACC_FOR_COMPONENTS(ACC_COPY_ONE)
+}
+
+/* One workgroup: the defaults, a wait until they have arrived, the sources.  Below a few thousand elements a call is
+ * what its launches cost. */
+extern "C" __global__ void __launch_bounds__(1024)
+permute_small(ACC_ENV_PARAMS ACC_OUT_PARAMS, ACC_CONST_ARRAY(arrFrom), const int copy, const Int64 n ACC_GUARD_PARAM)
+{
+  ACC_GUARD_CHECK
+  typedef ACC_ELT T;
+  ACC_ENV_ASSUME
+  __shared__ unsigned int s_winner[ACC_CLAIMED ? ACC_SMALL : 1];
+  auto get  = [&](const Int64 ix) -> T { return (ACC_GET(ix)); };
+  auto perm = [&](const Int64 ix) -> Int64 { return (Int64)(ACC_PERMUTATION(ix)); };
+  const Int64 ntarget = (ACC_OUT_SIZE);
+  const int tid = (int)threadIdx.x;
+  constexpr int MOST = (ACC_SMALL + 1023) / 1024;
+  Int64 j[MOST];
+#pragma unroll
+  for (int k = 0; k < MOST; ++k) {
+    const Int64 ix = tid + k * 1024;
+    j[k] = ix < n ? perm(ix) : -1;
+    if (j[k] >= ntarget) j[k] = -1;
+    if (ACC_CLAIMED && j[k] >= 0) s_winner[j[k]] = (unsigned int)ix;
+  }
+  if (copy) {
+#define ACC_COPY_SMALL(c, type) acc_copy_component<type>(arrOut_##c, arrFrom_##c, ntarget, tid, 1024);
+    ACC_FOR_COMPONENTS(ACC_COPY_SMALL)
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       /* every wave's part has arrived before any wave stores over it */
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < MOST; ++k) {
+    const Int64 ix = tid + k * 1024;
+    if (j[k] < 0) continue;
+    if (ACC_CLAIMED && s_winner[j[k]] != (unsigned int)ix) continue;
+    ACC_SET(arrOut, j[k], get(ix));
+  }
+}

@@ -806,6 +806,62 @@ int acc_exec_scan_noalloc(acc_skel s, const acc_array *env, int64_t n, const acc
   return scan_core(s, env, n, out, total, stream, true, "acc_exec_scan_noalloc");
 }
 
+namespace {
+
+// `permute const`, the combination that is the new value (skel_scatter.h): the defaults go to the result, the sources
+// are stored over them.
+int permute_const(acc_skel_s *s, const acc_array *env, int64_t n_src, const acc_array &defaults, const acc_array &out, bool copy_defaults, hipStream_t st)
+{
+  Args args;
+  bool aligned = true;
+  ACC_TRY(push_env(s, env, &args, &aligned));
+  push_out(out, &args, &aligned);
+  const int v = aligned ? 0 : 1;
+  ACC_TRY(s->ensure_variant(v));
+  const acc::Variant &var = s->variants[v];
+  const int64_t ntarget = array_size(out);
+  bool ignore = true;
+  if (n_src <= acc::SCATTER_SMALL && ntarget <= acc::SCATTER_SMALL) {
+    push_ptrs(&defaults, s->ncomp(), &args, &ignore);
+    args.i32(copy_defaults ? 1 : 0);
+    args.i64(n_src);
+    ACC_HIP_TRY(launch_kernel(var.fn_finish, 1, 1, 1, 1024, 1, 1, 0, st, args.data(), nullptr));
+    return ACC_OK;
+  }
+  if (copy_defaults) {
+    Args f;
+    push_ptrs(&out, s->ncomp(), &f, &ignore);
+    push_ptrs(&defaults, s->ncomp(), &f, &ignore);
+    f.i64(ntarget);
+    const int64_t pieces = (ntarget * s->spec.vec_size + 15) / 16;      // 16 bytes a lane
+    const int64_t grid = std::min<int64_t>((pieces + 255) / 256, (int64_t)1 << 20);
+    ACC_HIP_TRY(launch_kernel(var.fn_fill, static_cast<unsigned>(grid), 1, 1, 256, 1, 1, 0, st, f.data(), nullptr));
+  }
+  acc::ScratchRef winner;
+  const bool claimed = s->ncomp() > 1 || s->spec.elt_size > 8;           // as ACC_CLAIMED
+  if (claimed) ACC_TRY(s->ctx->scratch_acquire((size_t)ntarget * 4, st, acc::SCRATCH_FOLD, &winner));
+  // indices in `winner` are 32 bits wide: a longer source goes piece by piece, the later ones over the earlier
+  int rc = ACC_OK;
+  for (int64_t first = 0; first < n_src && rc == ACC_OK; first += (int64_t)1 << 32) {
+    const int64_t past = std::min<int64_t>(n_src, first + ((int64_t)1 << 32));
+    const int64_t tile = (int64_t)s->spec.block * s->spec.unroll;
+    const unsigned grid = static_cast<unsigned>((past - first + tile - 1) / tile);
+    Args piece = args;
+    piece.i64(first);
+    piece.i64(past);
+    piece.ptr(reinterpret_cast<uint64_t>(winner.ptr));
+    for (hipFunction_t fn : {claimed ? var.fn_claim : nullptr, var.fn}) {
+      if (!fn || rc != ACC_OK) continue;
+      hipError_t e = launch_kernel(fn, grid, 1, 1, static_cast<unsigned>(s->spec.block), 1, 1, 0, st, piece.data(), nullptr);
+      if (e != hipSuccess) rc = acc::fail_hip(e, "hipModuleLaunchKernel(permute const)");
+    }
+  }
+  s->ctx->scratch_release(winner, st);
+  return rc;
+}
+
+}  // namespace
+
 int acc_exec_permute(acc_skel s, const acc_array *env, int64_t n_src, const acc_array *defaults, const acc_array *out, acc_stream stream)
 {
   if (!s) return fail(ACC_ERR_INVALID, "acc_exec_permute: NULL skeleton");
@@ -835,6 +891,7 @@ int acc_exec_permute(acc_skel s, const acc_array *env, int64_t n_src, const acc_
     return ACC_OK;
   };
   if (n_src == 0 || ntarget == 0) return plain_copy();
+  if (s->spec.permute_replace) return permute_const(s, env, n_src, *defaults, *out, copy_defaults, st);
 
   // A combination without an atomic instruction of its own on few targets: compare-and-swap loops on the result
   // meet on those few addresses (16 M Float32 `max` updates on 1000 targets: 16.6 ms), the tables in LDS of the
@@ -854,35 +911,6 @@ int acc_exec_permute(acc_skel s, const acc_array *env, int64_t n_src, const acc_
                       ntarget >= s->knobs.permute_fp_tables_from && ntarget <= s->knobs.permute_fp_tables_to;
   const bool generic_few = !s->spec.permute_locked && (s->spec.combine_hint == ACC_COMBINE_GENERIC || fp_add) && lds_table_fits &&
                            s->knobs.permute_generic_lds != 0;
-  if (s->spec.permute_locked && s->spec.permute_replace && n_src <= (int64_t)0xffffffffLL) {
-    // `permute const` of an element that no single store covers: nothing is read or locked.  A scalar of one or two
-    // bytes is stored; of a tuple the source whose index stays in the target's word of a table wins, whole
-    // (skel_permute.h, permute_claim / permute_place).
-    ACC_TRY(plain_copy());
-    Args pargs;
-    bool al = true;
-    ACC_TRY(push_env(s, env, &pargs, &al));
-    push_out(*out, &pargs, &al);
-    pargs.i64(n_src);
-    const int pv = al ? 0 : 1;
-    ACC_TRY(s->ensure_variant(pv));
-    acc::ScratchRef wblk;
-    const bool tuple = s->ncomp() > 1 || esz > 8;      // (what no single store of at most 8 bytes writes)
-    if (tuple) ACC_TRY(s->ctx->scratch_acquire((size_t)ntarget * 4, st, acc::SCRATCH_FOLD, &wblk));
-    pargs.ptr(reinterpret_cast<uint64_t>(wblk.ptr));
-    const int64_t pgrid = acc_launch_grid(n_src, 256 * 4, s->ctx->props.multiProcessorCount, 32);
-    int prc = ACC_OK;
-    if (tuple) {
-      hipError_t ce = launch_kernel(s->variants[pv].fn_claim, static_cast<unsigned>(pgrid), 1, 1, 256, 1, 1, 0, st, pargs.data(), nullptr);
-      if (ce != hipSuccess) prc = acc::fail_hip(ce, "hipModuleLaunchKernel(permute_claim)");
-    }
-    if (prc == ACC_OK) {
-      hipError_t pe = launch_kernel(s->variants[pv].fn_place, static_cast<unsigned>(pgrid), 1, 1, 256, 1, 1, 0, st, pargs.data(), nullptr);
-      if (pe != hipSuccess) prc = acc::fail_hip(pe, "hipModuleLaunchKernel(permute_place)");
-    }
-    s->ctx->scratch_release(wblk, st);
-    return prc;
-  }
   if (s->spec.permute_locked || generic_few) {
     // elements no atomic covers: a lock per target (the reference's lock array, Execute.hs:402-405)
     ACC_TRY(plain_copy());

@@ -9,6 +9,8 @@
 #include <cctype>
 #include <cstdlib>
 #include <cstring>
+#include <regex>
+#include <set>
 #include <sstream>
 
 #include "skeleton.hpp"
@@ -121,6 +123,41 @@ static const char *kind_name(int kind)
   static const char *names[] = {"map", "generate", "transform", "fold", "fold1", "foldSeg", "fold1Seg", "scanl",
                                 "scanl1", "scanl'", "scanr", "scanr1", "scanr'", "permute", "stencil", "stencil2"};
   return (kind >= 0 && kind < ACC_SKEL_KIND_COUNT) ? names[kind] : "?";
+}
+
+// ---- operands read at the element's own index ---------------------------------
+// A fragment reads most of its operands at the consuming skeleton's own linear index: `acc_stream(arrIn<k>_<c>, ix)` or
+// `arrIn<k>_<c>[ix]`.  A template that asks for the operands of a whole batch before it looks at the first (a read
+// inside one branch of a conditional is otherwise waited for where it stands, one element after the other) gets them
+// from here: `texts` with those reads replaced by members of `acc_sv`, and the arrays they named, in order.
+struct OwnRead {
+  int array, comp;
+  bool operator<(const OwnRead &o) const { return array != o.array ? array < o.array : comp < o.comp; }
+};
+static std::set<OwnRead> take_own_reads(const std::vector<EnvSig> &env, const std::vector<std::string *> &texts)
+{
+  static const std::regex own("acc_stream\\(\\s*arrIn(\\d+)_(\\d+)\\s*,\\s*ix\\s*\\)|\\barrIn(\\d+)_(\\d+)\\s*\\[\\s*ix\\s*\\]");
+  std::set<OwnRead> reads;
+  for (std::string *text : texts) {
+    std::string out;
+    auto at = text->cbegin();
+    for (std::sregex_iterator m(text->cbegin(), text->cend(), own), end; m != end; ++m) {
+      const bool streamed = (*m)[1].matched;
+      const std::string k = (*m)[streamed ? 1 : 3].str(), c = (*m)[streamed ? 2 : 4].str();
+      const OwnRead r = {k.size() > 6 ? -1 : std::atoi(k.c_str()), c.size() > 6 ? -1 : std::atoi(c.c_str())};
+      out.append(at, (*m)[0].first);
+      if (r.array >= 0 && r.array < (int)env.size() && r.comp >= 0 && r.comp < env[r.array].ncomp) {
+        reads.insert(r);
+        out += "acc_sv.s" + std::to_string(r.array) + "_" + std::to_string(r.comp);
+      } else {
+        out += (*m)[0].str();                 // (no array of the instance: the compiler will say so)
+      }
+      at = (*m)[0].second;
+    }
+    out.append(at, text->cend());
+    *text = out;
+  }
+  return reads;
 }
 
 // ---- the generator -------------------------------------------------------------
@@ -268,7 +305,30 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
       o << "#define ACC_OUT_PARAMS " << out_params(sp.out_rank, sp.elt_type) << "\n";
       o << "#define ACC_OUT_SIZE " << out_size(sp.out_rank) << "\n";
       o << "#define ACC_PERMUTATION(ix) " << sp.permutation << "\n";
-      o << "#define ACC_COMBINE_HINT " << (sp.permute_replace && !sp.permute_locked ? 7 : sp.combine_hint) << "\n";
+      if (sp.permute_replace) {
+        std::ostringstream from;
+        const int nc = sp.comp_types.empty() ? 1 : (int)sp.comp_types.size();
+        for (int i = 0; i < nc; ++i) from << (i ? ", const " : "const ") << (sp.comp_types.empty() ? std::string("ACC_ELT") : sp.comp_types[i]) << " *__restrict__ name##_" << (nc - 1 - i);
+        o << "#define ACC_CONST_ARRAY(name) " << from.str() << "\n";
+        o << "#define ACC_BLOCK " << sp.block << "\n#define ACC_BATCH " << sp.unroll << "\n#define ACC_SMALL " << acc::SCATTER_SMALL << "\n";
+        std::string pre_get = sp.get, pre_perm = sp.permutation;
+        const std::set<OwnRead> reads = take_own_reads(sp.env, {&pre_get, &pre_perm});
+        std::ostringstream fields, loads, lengths;
+        for (const OwnRead &r : reads) {
+          const EnvSig &e = sp.env[r.array];
+          const std::string id = std::to_string(r.array) + "_" + std::to_string(r.comp);
+          fields << e.type[r.comp] << " s" << id << "; ";
+          loads << "(sv).s" << id << " = " << "acc_stream(arrIn" << id << ", (ix)); ";
+          lengths << " && (past) <= (Int64)1";
+          for (int d = e.rank - 1; d >= 0; --d) lengths << " * shIn" << r.array << "_" << d;
+        }
+        o << "#define ACC_OWN_FIELDS " << fields.str() << "\n#define ACC_OWN_LOAD(sv, ix) " << loads.str() << "\n";
+        o << "#define ACC_OWN_WITHIN(past) (true" << lengths.str() << ")\n";
+        o << "#define ACC_GET_OWN(ix) " << pre_get << "\n#define ACC_PERMUTATION_OWN(ix) " << pre_perm << "\n";
+        tmpl = "skel_scatter.h";
+        break;
+      }
+      o << "#define ACC_COMBINE_HINT " << sp.combine_hint << "\n";
       o << "#define ACC_PERMUTE_LOCKED " << (sp.permute_locked ? 1 : 0) << "\n";
       o << "#define ACC_PERMUTE_WINDOWS " << (sp.permute_windows ? 1 : 0) << "\n";
       o << "#define ACC_PERMUTE_NARROW " << (sp.permute_narrow ? 1 : 0) << "\n";
@@ -641,6 +701,11 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
       sp->block = tune("permute.block", 1024);
       sp->merge_waves = std::max(4, std::min(16, tune("permute.merge_waves", 4)));
       sp->unroll = tune("permute.unroll", 2);
+      if (sp->permute_replace) {
+        sp->block = tune("scatter.block", 256);
+        // elements a lane holds at a time, fewer of wide ones (a tuple of sixteen Float64 is 32 registers)
+        sp->unroll = std::max(1, tune("scatter.batch", sp->elt_size <= 32 ? 8 : (sp->elt_size <= 64 ? 4 : 2)));
+      }
       break;
     case ACC_SKEL_STENCIL:
     case ACC_SKEL_STENCIL2: {
@@ -811,7 +876,7 @@ namespace acc {
 SkelSpec spec_of_variant(const SkelSpec &base, int v)
 {
   SkelSpec spec = base;
-  if (spec.kind == ACC_SKEL_PERMUTE) {
+  if (spec.kind == ACC_SKEL_PERMUTE && !spec.permute_replace) {
     if (v >= 2 && v < 4) spec.permute_locked = true;
     if (v >= 4 && v < 6) spec.permute_windows = true;
     if (v >= 6) spec.permute_narrow = true;
@@ -915,7 +980,7 @@ int acc_skel_s::ensure_variant(int v)
                          ((spec.kind == ACC_SKEL_FOLD || spec.kind == ACC_SKEL_FOLD1) && spec.out_rank > 0);
   const bool two_kernels = ((spec.kind == ACC_SKEL_FOLD || spec.kind == ACC_SKEL_FOLD1) && spec.out_rank == 0) ||
                            spec.kind == ACC_SKEL_PERMUTE || segmented;
-  const std::string second = entry_name + (spec.kind == ACC_SKEL_PERMUTE ? (spec.permute_locked ? "_join" : "_merge") : segmented ? "_team" : "_finish");
+  const std::string second = entry_name + (spec.kind == ACC_SKEL_PERMUTE ? (spec.permute_replace ? "_small" : spec.permute_locked ? "_join" : "_merge") : segmented ? "_team" : "_finish");
   if (two_kernels) {
     e = hipModuleGetFunction(&var.fn_finish, var.module, second.c_str());
     if (e != hipSuccess) {
@@ -924,7 +989,7 @@ int acc_skel_s::ensure_variant(int v)
       return acc::fail_hip(e, ("hipModuleGetFunction(" + second + ")").c_str());
     }
   }
-  if ((spec.kind == ACC_SKEL_PERMUTE && !spec.permute_locked) || segmented) {
+  if ((spec.kind == ACC_SKEL_PERMUTE && (!spec.permute_locked || spec.permute_replace)) || segmented) {
     const std::string third = entry_name + (segmented ? "_join" : "_fill");
     e = hipModuleGetFunction(&var.fn_fill, var.module, third.c_str());
     if (e != hipSuccess) {
@@ -933,15 +998,12 @@ int acc_skel_s::ensure_variant(int v)
       return acc::fail_hip(e, ("hipModuleGetFunction(" + third + ")").c_str());
     }
   }
-  if (spec.kind == ACC_SKEL_PERMUTE && spec.permute_locked) {
-    // `permute const` without locks: see skel_permute.h
-    for (const char *name : {"permute_claim", "permute_place"}) {
-      e = hipModuleGetFunction(name[8] == 'c' ? &var.fn_claim : &var.fn_place, var.module, name);
-      if (e != hipSuccess) {
-        (void)hipModuleUnload(var.module);
-        var.module = nullptr;
-        return acc::fail_hip(e, (std::string("hipModuleGetFunction(") + name + ")").c_str());
-      }
+  if (spec.kind == ACC_SKEL_PERMUTE && spec.permute_replace) {
+    e = hipModuleGetFunction(&var.fn_claim, var.module, "permute_claim");
+    if (e != hipSuccess) {
+      (void)hipModuleUnload(var.module);
+      var.module = nullptr;
+      return acc::fail_hip(e, "hipModuleGetFunction(permute_claim)");
     }
   }
   if ((spec.kind == ACC_SKEL_FOLDSEG || spec.kind == ACC_SKEL_FOLD1SEG) && spec.out_rank <= 1) {
@@ -1000,7 +1062,7 @@ static int variant_count(const acc::SkelSpec &sp)
   const bool stencil = sp.kind == ACC_SKEL_STENCIL || sp.kind == ACC_SKEL_STENCIL2;
   if ((sp.kind == ACC_SKEL_FOLDSEG || sp.kind == ACC_SKEL_FOLD1SEG) && sp.out_rank <= 1) return 8;
   if (sp.map_tiled) return 4;
-  return sp.kind == ACC_SKEL_PERMUTE ? 8 : (stencil ? (sp.stencil_nd ? 2 : 8) : ((sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
+  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : 8) : ((sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
 }
 
 extern "C" {
