@@ -33,10 +33,20 @@
  * index function does).  A wave takes a tile of 32 x 32 elements, its lanes 8 across and 8 down with a block of 4 x 4
  * each: a row of the tile is written in a run of 128 bytes (Float32), and a source read along the tile's columns is
  * read in runs of 128 bytes too (the four elements a lane reads down a column are consecutive there, and so are the
- * eight lanes below one another).  Tiles are numbered along the rows of the result, the waves of a workgroup side by
- * side.  (A workgroup that evaluates a tile of 64 x 64 down its columns, passes it through LDS and writes it along its
- * rows -- runs of 256 bytes both ways, but the direction of the source fixed -- transposes no faster: 8192 x 8192
- * Float32 in 123-130 us against 123-125, and 281 in runs.)
+ * eight lanes below one another).  (A workgroup that evaluates a tile of 64 x 64 down its columns, passes it through
+ * LDS and writes it along its rows -- runs of 256 bytes both ways, but the direction of the source fixed -- transposes
+ * no faster, and neither do lanes with blocks of 8 x 8 or 2 x 2: 5003 x 3001 Float32 in 40 and 36 us against 31.)
+ *
+ * What bounds it: the memory side, once the index arithmetic is out of the way.  The place of every element is known
+ * here before the fragment asks for it, so the compiler is told what `ix % shOut_0` and `ix / shOut_0` come to: it then
+ * drops the fragment's divisions (two 64-bit ones an element, some 3000 instructions a lane) and sees that the four
+ * elements down a column lie side by side in the source, which become one 128-bit access.  Where
+ * the rows of the result are no whole cache lines, a run leaves a piece of a line at both ends: the four waves of a
+ * workgroup then take two tiles by two and a die takes one contiguous run of the workgroups, so that the pieces meet in
+ * one L2.  Rows of whole lines have no pieces; dealing their workgroups out over the dies, four tiles side by side, is
+ * the faster order.  Transposes in us, dealt out with divisions / without / two by two on one die: 5003 x 3001 Float32
+ * 46.5 / 37.1 / 31.0 (3.9 TB/s; 1.2 times the source is read, 1.08 times the result written); 4000 x 4000 31.9 / 28.1 /
+ * 29.6; 8192 x 8192 125 / 118 / 131; 7001 x 2500 Float64 89.3 / - / 72.6.
  */
 #ifndef ACC_TT
 #define ACC_TT 4                                      /* a lane's block is ACC_TT x ACC_TT */
@@ -49,34 +59,50 @@ ACC_ENTRY(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_GUARD_PARAM)
   ACC_GUARD_CHECK
   typedef ACC_ELT T;
   ACC_ENV_ASSUME
-  auto get = [&](const Int64 ix) -> T { return (ACC_GET(ix)); };
+  /* the element at `ix`, which is column `acc_c` of row `acc_r` of the result's rows taken as one list */
+  auto get_at = [&](const Int64 ix, const Int64 acc_r, const Int64 acc_c) -> T {
+    __builtin_assume(ix % shOut_0 == acc_c);
+    __builtin_assume(ix / shOut_0 == acc_r);
+    return (ACC_GET(ix));
+  };
 
   /* The tiles' second dimension is the second innermost one of the result, or one further out (ACC_TILE_H its
-   * extent, ACC_TILE_STRIDE the elements between neighbours along it: a volume turned so that its innermost
+   * extent, ACC_TILE_MIDS the rows between neighbours along it: a volume turned so that its innermost
    * dimension becomes its outermost reads its source along that one).  What lies between that dimension and the
    * innermost (`mids` rows for every place along it) and outside it (`outers`) is walked tile by tile. */
-  const Int64 w = shOut_0, h = ACC_TILE_H, stride = ACC_TILE_STRIDE;
+  const Int64 w = shOut_0, h = ACC_TILE_H, mids = ACC_TILE_MIDS, stride = mids * w;
   const Int64 n = (ACC_OUT_SIZE);
-  const Int64 mids = w > 0 ? stride / w : 0, outers = (h > 0 && stride > 0) ? n / (h * stride) : 0;
-  const Int64 tiles_x = (w + ACC_TSIDE - 1) / ACC_TSIDE, tiles_y = (h + ACC_TSIDE - 1) / ACC_TSIDE;
-  const Int64 tiles = tiles_x * tiles_y * mids * outers;
+  const Int64 outers = (h > 0 && stride > 0) ? n / (h * stride) : 0;
   const int lane = acc_lane();
   const int lx = lane & 7, ly = lane >> 3;
-  const Int64 wave = (Int64)blockIdx.x * (ACC_BLOCK / ACC_WAVE) + (Int64)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const Int64 step = (Int64)gridDim.x * (ACC_BLOCK / ACC_WAVE);
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  /* a workgroup's waves: two by two tiles, or side by side where the result is no taller than one and where its rows
+   * are whole cache lines (the driver counts the workgroups by the same rule) */
+  constexpr int WAVES = ACC_BLOCK / ACC_WAVE;
+  const bool whole_lines = (w * ACC_TILE_ELT_BYTES) % 128 == 0;
+  const int down = (WAVES % 2 == 0 && h > ACC_TSIDE && !whole_lines) ? 2 : 1, across = WAVES / down;
+  const Int64 groups_x = (w + across * ACC_TSIDE - 1) / (across * ACC_TSIDE), groups_y = (h + down * ACC_TSIDE - 1) / (down * ACC_TSIDE);
+  const Int64 groups = groups_x * groups_y * mids * outers;
+  /* the quotient of numbers no larger than the array has elements: in 32 bits where it has fewer than 2^31 */
+  const bool narrow = n < 0x7fffffff;
+  auto divide = [&](const Int64 a, const Int64 b) -> Int64 {
+    return narrow ? (Int64)((unsigned int)a / (unsigned int)b) : a / b;
+  };
 
-  for (Int64 tile = wave; tile < tiles; tile += step) {
-    const Int64 tx = tile % tiles_x, ty = (tile / tiles_x) % tiles_y, plane = tile / (tiles_x * tiles_y);
-    const Int64 mid = plane % mids, outer = plane / mids;
+  for (Int64 group = whole_lines ? (Int64)blockIdx.x : acc_xcd_contiguous_block(); group < groups; group += gridDim.x) {
+    const Int64 g1 = divide(group, groups_x), gx = group - g1 * groups_x;
+    const Int64 plane = divide(g1, groups_y), gy = g1 - plane * groups_y;
+    const Int64 outer = divide(plane, mids), mid = plane - outer * mids;
+    const Int64 tx = gx * across + (down == 2 ? wave >> 1 : wave), ty = gy * down + (down == 2 ? wave & 1 : 0);
     const Int64 x = tx * ACC_TSIDE + lx * ACC_TT, y = ty * ACC_TSIDE + ly * ACC_TT;
-    const Int64 base = ((outer * h + y) * mids + mid) * w + x;
+    const Int64 row = (outer * h + y) * mids + mid, base = row * w + x;
     if ((tx + 1) * ACC_TSIDE <= w && (ty + 1) * ACC_TSIDE <= h) {
       T v[ACC_TT][ACC_TT];
       /* down the columns first: what a transposed source holds side by side */
 #pragma unroll
       for (int k = 0; k < ACC_TT; ++k)
 #pragma unroll
-        for (int i = 0; i < ACC_TT; ++i) v[i][k] = get(base + i * stride + k);
+        for (int i = 0; i < ACC_TT; ++i) v[i][k] = get_at(base + i * stride + k, row + i * mids, x + k);
 #pragma unroll
       for (int i = 0; i < ACC_TT; ++i)
 #pragma unroll
@@ -86,7 +112,7 @@ ACC_ENTRY(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_GUARD_PARAM)
       for (int i = 0; i < ACC_TT; ++i)
 #pragma unroll
         for (int k = 0; k < ACC_TT; ++k)
-          if (x + k < w && y + i < h) ACC_SET(arrOut, base + i * stride + k, get(base + i * stride + k));
+          if (x + k < w && y + i < h) ACC_SET(arrOut, base + i * stride + k, get_at(base + i * stride + k, row + i * mids, x + k));
     }
   }
 }

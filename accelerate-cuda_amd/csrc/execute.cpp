@@ -285,13 +285,15 @@ int acc_exec_map(acc_skel s, const acc_array *env, const acc_array *out, acc_str
   ACC_TRY(s->ensure_variant(v));
   if (in_tiles) {
     // a wave per tile of 32 x 32 elements of the innermost dimension and the second innermost one, or the one that
-    // ACC_FLAG_TILE_DIM names (skel_map.h)
+    // ACC_FLAG_TILE_DIM names, two tiles by two a workgroup or side by side, as skel_map.h numbers them
     const int rank = s->spec.out_rank;
     const int64_t side = 8 * (int64_t)s->spec.map_tile_block;
     const int64_t w = out->shape[rank - 1], h = out->shape[rank - 1 - s->spec.map_tile_dim];
-    const int64_t tiles = ((w + side - 1) / side) * ((h + side - 1) / side) * (n / (w * h));
     const int64_t waves = s->variants[v].block / 64;
-    return launch(s, v, std::min<int64_t>((tiles + waves - 1) / waves, (int64_t)1 << 22), 0, static_cast<hipStream_t>(stream), &args);
+    const bool whole_lines = (w * std::max(1, s->spec.elt_size)) % 128 == 0;
+    const int64_t down = (waves % 2 == 0 && h > side && !whole_lines) ? 2 : 1, across = waves / down;
+    const int64_t groups = ((w + across * side - 1) / (across * side)) * ((h + down * side - 1) / (down * side)) * (n / (w * h));
+    return launch(s, v, std::min<int64_t>(groups, (int64_t)1 << 22), 0, static_cast<hipStream_t>(stream), &args);
   }
   // streaming with no reuse: one short-lived workgroup per tile keeps the most loads in flight
   const int64_t grid = acc_launch_grid(n, s->elements_per_block(), resident(s, v), s->knobs.map_oversub);

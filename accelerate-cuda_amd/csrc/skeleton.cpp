@@ -244,9 +244,11 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
       o << "#define ACC_BLOCK " << sp.block << "\n#define ACC_VEC " << vec << "\n#define ACC_UNROLL " << sp.unroll << "\n";
       o << "#define ACC_MAP_TILED " << (sp.map_tiled ? 1 : 0) << "\n#define ACC_TT " << sp.map_tile_block << "\n";
       if (sp.map_tiled) {
-        // the tiles' second dimension: its extent, and the elements between neighbours along it
-        o << "#define ACC_TILE_H shOut_" << sp.map_tile_dim << "\n#define ACC_TILE_STRIDE (";
-        for (int dd = 0; dd < sp.map_tile_dim; ++dd) o << (dd ? " * " : "") << "shOut_" << dd;
+        // the tiles' second dimension: its extent, and the rows between neighbours along it
+        o << "#define ACC_TILE_ELT_BYTES " << std::max(1, sp.elt_size) << "\n";
+        o << "#define ACC_TILE_H shOut_" << sp.map_tile_dim << "\n#define ACC_TILE_MIDS (";
+        if (sp.map_tile_dim == 1) o << "1";
+        for (int dd = 1; dd < sp.map_tile_dim; ++dd) o << (dd > 1 ? " * " : "") << "shOut_" << dd;
         o << ")\n";
       }
       tmpl = "skel_map.h";

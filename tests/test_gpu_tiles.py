@@ -1,0 +1,53 @@
+"""Maps in tiles (ACC_FLAG_TILED) at the sizes where the tiling changes form: one tile or two down a workgroup (32 and 33
+rows), the last tile of either direction full, one short and one over, more workgroups than one die takes; index
+fragments the compiler can resolve from the tile's place and ones it cannot.  The same map in runs is the oracle: moved
+whole numbers, equal in every element."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+FORMS = {
+    "transpose": "arrIn0_0[(ix % shOut_0) * shIn0_0 + (ix / shOut_0)]",
+    "from_index": "arrIn0_0[acc_from_index<2>({shOut_1, shOut_0}, ix).i[1] * shIn0_0 + acc_from_index<2>({shOut_1, shOut_0}, ix).i[0]]",
+    "mirrored": "arrIn0_0[((shOut_0 - 1 - ix % shOut_0)) * shIn0_0 + (shOut_1 - 1 - ix / shOut_0)] + (Int32)((ix + 1) % shOut_0)",
+}
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import acchip as A
+    return A.Context(0)
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+@pytest.mark.parametrize("shape", [(10, 33), (31, 64), (32, 65), (33, 63), (33, 129), (64, 64), (65, 127), (257, 511), (1000, 1003)])
+def test_tiles_against_runs(ctx, form, shape):
+    import acchip as A
+    print("tiled map", form, shape, flush=True)
+    h, w = shape
+    src = ctx.array(np.random.default_rng(h * w).integers(-1000, 1000, (w, h)).astype(np.int32))
+    results = []
+    for flags in (A.FLAG_TILED, 0):
+        sk = ctx.skeleton(A.SKEL_MAP, "Int32", env=[(2, "Int32")], out_rank=2, flags=flags, get=FORMS[form])
+        out = ctx.array(np.full(h * w + 3, 77, np.int32))
+        sk.map([src], out.desc(shape=(h, w)))
+        results.append(out.get())
+    assert np.array_equal(results[0], results[1])
+    assert np.array_equal(results[0][-3:], [77, 77, 77])
+    if form != "mirrored":
+        assert np.array_equal(results[0][:-3].reshape(h, w), src.get().T)
+
+
+@pytest.mark.parametrize("dim,shape", [(2, (33, 3, 65)), (2, (32, 2, 64)), (2, (70, 1, 40))])
+def test_tiles_of_an_outer_dimension(ctx, dim, shape):
+    """rank 3: the remainder and the quotient by the innermost extent where the tile's rows are not next to one another"""
+    import acchip as A
+    print("tiled map of rank 3", dim, shape, flush=True)
+    frag = "(Int32)((ix % shOut_0) * 1000003 + (ix / shOut_0) * 7 + ix)"
+    results = []
+    for flags in (A.FLAG_TILED | A.FLAG_TILE_DIM(dim), 0):
+        out = ctx.empty(shape, np.int32)
+        ctx.skeleton(A.SKEL_GENERATE, "Int32", env=[], out_rank=3, flags=flags, get=frag).map([], out)
+        results.append(out.get())
+    assert np.array_equal(results[0], results[1])
