@@ -691,6 +691,15 @@ int acc_exec_foldseg(acc_skel s, const acc_array *env, int64_t n, const acc_arra
 
 namespace {
 
+// A variant beyond the ones an earlier call of this size would have loaded: there already, or buildable now (a stream
+// under capture is no place to load a module).
+bool may_take(acc_skel s, int v, hipStream_t st)
+{
+  if (s->variant_ready(v)) return true;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(st, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+}
+
 // scanOp / scan1Op / scan'Op / scanCore, Execute.hs:328-392, as ONE launch.  `noalloc`: the tile descriptors live in
 // the library's file-scope device array instead of a block of the context's pool, and nothing may be allocated,
 // compiled or loaded on the way.
@@ -728,12 +737,22 @@ int scan_core(acc_skel s, const acc_array *env, int64_t n, const acc_array *out,
   // 8.1, 3 M + 3 14.8 -> 9.3; at 2^22 the two are level, 11.7 and 11.2, and so are 2^21 Float64, 12.0 and 13.2).
   const bool small = s->spec.scan_small_rows > 0 &&
                      n * (int64_t)s->spec.elt_size <= (int64_t)s->knobs.scan_small_below_kb * 1024;
+  // Above that and up to 48 MB: tiles of 12 rows a lane.  Of 32 rows there are fewer tiles than two for a compute unit,
+  // each a long way from its first load to its last store; of 4 so many that the chain of their totals takes longer than
+  // the data (us with 4 / 8 / 12 / 16 / 32 rows: Int32 4 M 11.3 / 9.9 / 10.9 / 10.9 / 14.3, 6 M 14.6 / 12.1 / 11.7 / 12.7 /
+  // 15.4, 12 M 29.5 / 20.2 / 18.8 / 18.6 / 21.0, 16 M 36.4 / 28.1 / 30.1 / 24.7 / 23.9; Float64 3 M 18.6 / 14.1 / 13.0 /
+  // 13.9 / 16.0).  A call that may not build the variant -- without allocations, or on a stream that is being captured --
+  // takes the large tile where the variant is not there yet.
+  const bool mid = !small && s->spec.scan_mid_rows > 0 && s->knobs.scan_small_below_kb > 0 &&
+                   n * (int64_t)s->spec.elt_size <= (int64_t)s->knobs.scan_mid_below_kb * 1024;
   int v = (aligned ? 0 : 1) + (small ? 2 : 0);
+  if (mid && (noalloc ? s->variant_ready(v + 4) : may_take(s, v + 4, st))) v += 4;
   if (noalloc) {
     // building a variant compiles and loads a module: not here
     if (!s->variant_ready(v))
       return fail(ACC_ERR_INVALID, "%s: the %s %s-tile variant of this instance is not loaded yet; run acc_exec_scan once on operands of the same alignment and of %s %d KB first",
-                  who, aligned ? "aligned" : "unaligned", small ? "small" : "large", small ? "at most" : "more than", s->knobs.scan_small_below_kb);
+                  who, aligned ? "aligned" : "unaligned", small ? "small" : "large", small ? "at most" : "more than",
+                  s->knobs.scan_small_below_kb);
   } else {
     ACC_TRY(s->ensure_variant(v));
   }

@@ -848,6 +848,8 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
         sp->block = tune("scan.block", sp->scan_shape_open ? 256 : 1024);
         sp->rows = tune("scan.rows", sp->scan_shape_open ? rows4 : sp->scan_rows_fallback);
         sp->scan_small_rows = std::max(0, std::min(tune("scan.small_rows", 4), 32));
+        sp->scan_mid_rows = std::max(0, std::min(tune("scan.mid_rows", 12), 32));
+        if (sp->scan_mid_rows >= sp->rows || sp->scan_small_rows == 0) sp->scan_mid_rows = 0;      // no smaller than the tile itself
         sp->scan_ticket = tune("scan.ticket", 0) != 0;
       }
       break;
@@ -904,9 +906,10 @@ SkelSpec spec_of_variant(const SkelSpec &base, int v)
   }
   // a scan's variants 2 and 3: a small tile, for arrays of a few tiles at most (a lone workgroup runs through the
   // instructions of all its rows one after the other whether the array fills them or not)
+  // ... 4 and 5: one between the two
   if (spec.scan_small_rows > 0 && v >= 2) {
     spec.block = std::min(spec.block, 256);
-    spec.rows = std::min(spec.rows, spec.scan_small_rows);
+    spec.rows = std::min(spec.rows, v >= 4 ? spec.scan_mid_rows : spec.scan_small_rows);
   }
   return spec;
 }
@@ -1064,7 +1067,7 @@ static int variant_count(const acc::SkelSpec &sp)
   const bool stencil = sp.kind == ACC_SKEL_STENCIL || sp.kind == ACC_SKEL_STENCIL2;
   if ((sp.kind == ACC_SKEL_FOLDSEG || sp.kind == ACC_SKEL_FOLD1SEG) && sp.out_rank <= 1) return 8;
   if (sp.map_tiled) return 4;
-  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : 8) : ((sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
+  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
 }
 
 extern "C" {

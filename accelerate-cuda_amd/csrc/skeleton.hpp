@@ -58,6 +58,7 @@ struct SkelSpec {
   bool foldseg_giants = false;          // a segmented fold's variants 4-7: very long segments are handed over to a second launch (skel_foldseg.h)
   bool fold_single = true;              // foldAll in one launch (the last workgroup collects), as generated into the kernel
   int scan_rows_fallback = 8;
+  int scan_mid_rows = 0;                // ... of its variants 4 and 5, for arrays between those and the full tile; 0: none
   int scan_small_rows = 0;              // rows a lane of a scan's small-tile variants (2 and 3); 0: none
   int scan_desc_stride = 16;            // 8-byte words between the tile descriptors of a scan, as generated into the kernel
   bool scan_ticket = false;             // measurement: tiles drawn from a counter instead of numbered by workgroup (knob scan.ticket)
@@ -104,7 +105,8 @@ struct acc_skel_s {
                               // [4], [5]: for a hinted permute over several LDS windows of targets;
                               // [6], [7]: for integer addition on a table of 16-bit counts in LDS;
                               // of a segmented fold [2], [3]: a longer staged chunk, [4]-[7]: the same four with the table of
-                              // jobs for very long segments; of a scan [2], [3]: small tiles;
+                              // jobs for very long segments; of a scan [2], [3]: small tiles,
+                              // [4], [5]: tiles between those and the full ones;
                               // of a stencil [2], [3] and [4], [5]: half and a quarter of the columns a lane, [6], [7]: an
                               // element a thread
   int hint_slot = -1;         // a segmented fold: its word among the context's hints (its segments were looked at: a very long one)
