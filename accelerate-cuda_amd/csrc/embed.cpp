@@ -27,6 +27,7 @@ ACC_EMBED(permute, "device/skel_permute.h")
 ACC_EMBED(scatter, "device/skel_scatter.h")
 ACC_EMBED(stencil, "device/skel_stencil.h")
 ACC_EMBED(stencil_nd, "device/skel_stencil_nd.h")
+ACC_EMBED(stencil_flat, "device/skel_stencil_flat.h")
 
 namespace acc {
 
@@ -43,6 +44,7 @@ const std::vector<EmbeddedHeader> &embedded_headers()
       {"skel_scatter.h", acc_embed_scatter_begin, acc_embed_scatter_end},
       {"skel_stencil.h", acc_embed_stencil_begin, acc_embed_stencil_end},
       {"skel_stencil_nd.h", acc_embed_stencil_nd_begin, acc_embed_stencil_nd_end},
+      {"skel_stencil_flat.h", acc_embed_stencil_flat_begin, acc_embed_stencil_flat_end},
   };
   return headers;
 }

@@ -1326,6 +1326,31 @@ static int stencil_once(acc_skel s, const acc_array *env, const acc_array *in, c
     const int64_t grid = acc_launch_grid(array_size(*out), s->spec.block, resident(s, v), s->knobs.map_oversub);
     return launch(s, v, grid, 0, st, &args);
   }
+  // A volume whose rows do not divide into strips takes variants 8 and 9, lanes over the vectors of a whole plane, where
+  // the instance has them (skel_stencil_flat.h; us in strips / so: 7 points Float32 300^3 77 / 55, 400^3 152 / 116,
+  // 200 x 200 x 300 28.3 / 18.4, 150^3 14.8 / 8.3, 40^3 7.8 / 6.4, 390 x 200 x 70 27.3 / 11.3; 27 points 100^3 12.3 / 6.1,
+  // 399 x 397 x 395 221 / 142; Float64 300^3 131 / 102).  Where every strip is whole, strips are the faster half of the
+  // time: 256 x 512 x 512 94.7 / 105.9 and 121 / 131 (27 points), 256^3 Float64 57.2 / 56.9 and 27 points 32.6 / 30.9.
+  const int64_t strip = (int64_t)64 * s->spec.svec;
+  if (s->spec.flat_rows > 0 && s->knobs.stencil_flat != 0 && w >= s->spec.svec && (w % strip != 0 || s->knobs.stencil_flat == 2)) {
+    const int64_t rows = s->spec.flat_rows, per_block = s->spec.block / 64, cus = s->ctx->props.multiProcessorCount;
+    const int64_t per_plane = (((w + s->spec.svec - 1) / s->spec.svec) * ((h + rows - 1) / rows) + 63) / 64;
+    // Planes a wave walks through: 16, halved to 4 while there are fewer than sixteen waves for a compute unit, and 2
+    // if there are then not even two (300^3 with 2 / 4 / 8 / 16 planes: - / 56 / 55 / 59 us; 150^3 9.3 / 8.3 / 8.8 / 13.2;
+    // 27 points on 100^3 6.1 / 8.0 / 11.1 / 18.0; every run reads 2 rz planes beyond its own).
+    int64_t walk = s->knobs.stencil_flat_walk;
+    auto waves = [&]() { return per_plane * ((planes + walk - 1) / walk); };
+    while (walk > 4 && waves() < 16 * cus) walk /= 2;
+    if (walk > 2 && waves() < 2 * cus) walk = 2;
+    // the kernel counts lanes and waves in 32 bits, and bytes within a plane of source and result
+    const int64_t widest = std::max(s->spec.elt_size, 8);
+    const int v = (aligned ? 0 : 1) + 8;
+    if (w * h * widest < ((int64_t)1 << 32) && planes < ((int64_t)1 << 30) && waves() < ((int64_t)1 << 30) && may_take(s, v, st)) {
+      ACC_TRY(s->ensure_variant(v));
+      args.i32(static_cast<int32_t>(walk));
+      return launch(s, v, (waves() + per_block - 1) / per_block, 0, st, &args);
+    }
+  }
   // one wave per strip of 256 columns x tile_h rows
   // (for 2-D the waves of a workgroup are stacked vertically, so the row count is rounded up to whole groups)
   const int64_t waves = s->spec.block / 64;

@@ -483,7 +483,7 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
       o << "#define ACC_TILE_H " << sp.tile_h << "\n#define ACC_PREFETCH " << sp.prefetch << "\n#define ACC_BLOCK " << sp.block << "\n";
       o << "#define ACC_TZ " << sp.tile_z << "\n";
       o << "#define ACC_ZMARCH " << sp.zmarch << "\n";
-      tmpl = "skel_stencil.h";
+      tmpl = sp.stencil_flat ? "skel_stencil_flat.h" : "skel_stencil.h";
       break;
     }
     default:
@@ -828,6 +828,15 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
       // the strip goes through planes
       sp->tile_h = sp->out_rank == 2 ? tune("stencil.tile_h", 4)
                  : (sp->out_rank == 3 ? (sp->zmarch ? tune("stencil.walk", 64) : tune("stencil.tile_h3", sp->tile_z > 1 ? 8 : 16)) : 1);
+      // The form for volumes whose rows do not divide into strips: two rows a lane, or one, as its windows stay within 192
+      // registers; of one array of 4- or 8-byte elements.  No plane is asked for ahead: a step's requests are enough
+      // (300^3, 7 points, two rows: 57.1 us with a plane ahead, 55.0 without; 300^3 Float64 68 and 60).
+      if (sp->zmarch && d->kind == ACC_SKEL_STENCIL && sp->stencil_in_comps.size() == 1 && type_size(sp->stencil_in_comps[0]) >= 4) {
+        sp->flat_prefetch = std::max(0, std::min(tune("stencil.flat_prefetch", 0), 4));
+        const int words = (type_size(sp->stencil_in_comps[0]) + 3) / 4;
+        for (int ty = std::min(tune("stencil.flat_rows", 2), 4); ty > 0 && sp->flat_rows == 0; --ty)
+          if ((2 * ry + ty) * (2 * rz + 1 + sp->flat_prefetch) * (sp->svec + 2 * rx) * words <= 192) sp->flat_rows = ty;
+      }
       if (sp->zmarch && 2 * rx * (2 * ry + sp->tile_z) > 64) return fail(ACC_ERR_INVALID, "stencil: strip too tall for its reach");
       if (sp->tile_h < 1 || sp->prefetch < 0 || sp->prefetch > 8 || sp->tile_z < 1 || sp->tile_z > 8) return fail(ACC_ERR_INVALID, "stencil: bad tile shape");
       break;
@@ -903,6 +912,15 @@ SkelSpec spec_of_variant(const SkelSpec &base, int v)
   } else if ((spec.kind == ACC_SKEL_STENCIL || spec.kind == ACC_SKEL_STENCIL2) && v >= 2 && !spec.stencil_nd) {
     spec.svec = std::max(1, spec.svec >> (v / 2));
     spec.tile_w = 64 * spec.svec;
+  }
+  // ... and 8 and 9: lanes over the vectors of a whole plane
+  if (spec.kind == ACC_SKEL_STENCIL && v >= 8) {
+    spec.stencil_flat = true;
+    spec.stencil_nd = false;
+    spec.svec = base.svec;
+    spec.tile_w = 64 * spec.svec;
+    spec.tile_z = spec.flat_rows;
+    spec.prefetch = spec.flat_prefetch;
   }
   // a scan's variants 2 and 3: a small tile, for arrays of a few tiles at most (a lone workgroup runs through the
   // instructions of all its rows one after the other whether the array fills them or not)
@@ -1067,7 +1085,7 @@ static int variant_count(const acc::SkelSpec &sp)
   const bool stencil = sp.kind == ACC_SKEL_STENCIL || sp.kind == ACC_SKEL_STENCIL2;
   if ((sp.kind == ACC_SKEL_FOLDSEG || sp.kind == ACC_SKEL_FOLD1SEG) && sp.out_rank <= 1) return 8;
   if (sp.map_tiled) return 4;
-  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
+  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : sp.flat_rows > 0 ? 10 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
 }
 
 extern "C" {
@@ -1169,7 +1187,7 @@ int acc_skel_source(acc_skel s, int variant, const char **source)
 int acc_skel_preview(const acc_skel_desc *desc, int variant, const char **source, const char **entry)
 {
   static thread_local std::string text, name;
-  if (!source || variant < 0 || variant > 7) return fail(ACC_ERR_INVALID, "acc_skel_preview: bad argument");
+  if (!source || variant < 0 || variant > 9) return fail(ACC_ERR_INVALID, "acc_skel_preview: bad argument");
   acc::SkelSpec sp;
   ACC_TRY(acc::make_spec(desc, acc::default_tuning(), &sp));
   // beyond 1: a permute's forms (to 7), a stencil's fewer columns a lane (to 5), a scan's small tiles and a segmented

@@ -1,0 +1,56 @@
+"""3-D stencils with the lanes over the vectors of a plane (variants 8 and 9) at the sizes where that changes form: rows
+of a whole number of vectors and not, a last band of one row, a last wave partly beyond the plane, one run of planes and
+several, runs cut short, volumes thinner than the stencil's reach; every boundary condition.  The element-a-thread
+template is the reference: the same operations in the same order on one element, equal in every bit."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+STAR = [(0, 0, 0), (-1, 0, 0), (1, 0, 0), (0, -1, 0), (0, 1, 0), (0, 0, -1), (0, 0, 1)]
+BOX = [(a, b, c) for a in (-1, 0, 1) for b in (-1, 0, 1) for c in (-1, 0, 1)]
+ODD = [(0, 0, 2), (-1, 1, -2), (1, 0, 1), (0, -1, 0)]                    # lopsided, two columns away
+SHAPES = [(5, 7, 20), (3, 2, 17), (2, 1, 19), (17, 9, 33), (33, 16, 64), (40, 31, 101), (9, 130, 260), (70, 3, 258)]
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    import acchip as A
+    return A.Context(0)
+
+
+@pytest.mark.parametrize("boundary", ["clamp", "mirror", "wrap", "constant"])
+@pytest.mark.parametrize("ctype,dt,taps", [("float", np.float32, STAR), ("float", np.float32, BOX), ("double", np.float64, STAR),
+                                           ("Int32", np.int32, ODD), ("Int64", np.int64, BOX)])
+def test_against_an_element_a_thread(ctx, boundary, ctype, dt, taps):
+    import acchip as A
+    fn = " + ".join("(%s)%d * t%d" % (ctype, 3 + k % 5, k) for k in range(len(taps)))
+    desc = dict(out_rank=3, taps=taps, boundary=boundary, stencil_fn=fn, boundary_constant="(%s)7" % ctype if boundary == "constant" else None)
+    assert "skel_stencil_flat.h" in A.preview(A.make_desc(A.SKEL_STENCIL, ctype, **desc), 8)[1]
+    flat = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+    with A.tuning("stencil.nd=1,stencil.flat=0,stencil.thin_3d=1000000", ctx):
+        each = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+    rng = np.random.default_rng(3)
+    for shape in SHAPES:
+        # (mirrored and wrapped taps are defined where the volume spans the stencil)
+        if boundary in ("mirror", "wrap") and min(shape) < 3:
+            continue
+        n = int(np.prod(shape))
+        for shift in (0, 1):                                             # operands off the 16-byte boundary: variant 9
+            print(ctype, len(taps), boundary, shape, shift, flush=True)
+            x = rng.integers(-50, 50, n + shift).astype(dt)
+            src, got = ctx.array(x), []
+            for sk in (flat, each):
+                out = ctx.array(np.full(n + shift + 3, 77, dt))
+                sk.stencil(None, _Part(src, shape, shift), _Part(out, shape, shift))
+                got.append(out.get())
+            assert np.array_equal(got[0], got[1]), (shape, shift)
+            assert np.all(got[0][shift + n:] == 77) and np.all(got[0][:shift] == 77)
+
+
+class _Part(object):
+    def __init__(self, arr, shape, off):
+        self.d = arr.desc(shape=shape, offset_elems=off)
+
+    def desc(self):
+        return self.d
