@@ -520,78 +520,77 @@ ACC_FS_CAT_(ACC_FOLDSEG_ENTRY, _rows)(ACC_ENV_PARAMS
   }
 }
 
-/* ---- rows that lie across memory: a lane per row, whatever the length ------
- * <entry>_across, for an element function that, where the ROW index moves by one, reads neighbouring addresses --
- * the fold of a transposed matrix (sums down its columns), of a matrix product written as a fold over
- * `zipWith (*)` of two replicated operands, one of them transposed (ACC_FLAG_TILED says so: the host cannot see it).
- * A team of lanes along such a row asks for 64 cache lines with every load; a lane per row, neighbouring rows in
- * neighbouring lanes, asks for one.  Lane t takes piece t / rows of row t % rows: with fewer rows than the device
- * has lanes the rows are cut into `split` pieces of consecutive elements, whose values <entry>_join puts together in
- * order; with split == 1 the lane writes the row's result itself.  Every piece is folded in index order, eight
- * elements requested before the first is used.                                                                   */
-#define ACC_ACROSS_UNROLL 8
-extern "C" __global__ void __launch_bounds__(ACC_BLOCK)
-ACC_FS_CAT_(ACC_FOLDSEG_ENTRY, _across)(ACC_ENV_PARAMS
-                                        const Int64 shOut_0, ACC_OUT_ARRAY(arrOut),
-                                        ACC_SEG_PARAMS,
-                                        const Int64 split, ACC_ELT *__restrict__ part, int *__restrict__ part_ok ACC_GUARD_PARAM)
+/* ---- rows that lie across memory: neighbouring rows in neighbouring lanes, whatever the length ------
+ * <entry>_across and <entry>_across_wide (skel_fold_across.h, a row and several rows a lane), for an element function
+ * that, where the ROW index moves by one, reads neighbouring addresses -- the fold of a transposed matrix (sums down its
+ * columns), of a matrix product written as a fold over `zipWith (*)` of two replicated operands, one of them transposed
+ * (ACC_FLAG_TILED says so: the host cannot see it).  A team of lanes along such a row asks for 64 cache lines with every
+ * load.                                                                                                        */
+/* the folds of elements [k0, k1), not none, of the R rows `row`: in C runs side by side, the first of them
+ * beginning with the seed if SEEDED */
+template <int R, int C, bool SEEDED, typename T, typename Get, typename F>
+ACC_DEV void acc_across_piece(Get get, F f, const Int64 (&row)[R], const Int64 k0, const Int64 k1, const T &seed, T (&out)[R])
 {
-  ACC_GUARD_CHECK
-  typedef ACC_ELT T;
-  ACC_ENV_ASSUME
-  auto get = ACC_GET_AT_ROW_COL;
-  auto f   = [&](const T &x, const T &y) -> T { return (ACC_COMBINE(x, y)); };
-  (void)shIn_1;
-  const Int64 rows = shOut_0, len = shIn_0;
-  const Int64 piece = (len + split - 1) / split;
-  for (Int64 t = (Int64)blockIdx.x * ACC_BLOCK + threadIdx.x; t < rows * split; t += (Int64)gridDim.x * ACC_BLOCK) {
-    const Int64 p = t / rows, row = t - p * rows;
-    const Int64 k0 = acc_min<Int64>(p * piece, len), k1 = acc_min<Int64>(k0 + piece, len);
-    if (k0 >= k1) {                                        /* (a last piece without elements; the host launches no empty rows) */
-      if (split > 1) part_ok[row * split + p] = 0;
-      continue;
-    }
-    T x[ACC_ACROSS_UNROLL];
-#if ACC_HAS_SEED
-    const T seed = (ACC_SEED);
-#endif
-#if ACC_FOLD_RIGHT
-    /* x0 (+) (x1 (+) (... (x_last (+) z))), as the other entries associate a row */
-    T acc = get(row, k1 - 1);
-#if ACC_HAS_SEED
-    if (split == 1) acc = f(acc, seed);
-#endif
-    Int64 k = k1 - 1;
-    for (; k - ACC_ACROSS_UNROLL >= k0; k -= ACC_ACROSS_UNROLL) {
+  constexpr int WORDS = (int)((sizeof(T) + 3) / 4);
+  constexpr int WANT = 64 / (C * R * WORDS), U = WANT > 8 ? 8 : (WANT < 2 ? 2 : WANT);
+  /* run c is elements c h to (c + 1) h - 1, the last one to the end, counted from the end that is folded first */
+  const Int64 n = k1 - k0, h = n / C;
+  auto at = [&](const Int64 i) -> Int64 { return ACC_FOLD_RIGHT ? k1 - 1 - i : k0 + i; };
+  auto join = [&](const T &acc, const T &v) -> T { return ACC_FOLD_RIGHT ? f(v, acc) : f(acc, v); };
+  T acc[C][R];
+  auto batch = [&](const Int64 i, auto first_c, auto whole_c) {
+    constexpr bool first = decltype(first_c)::value, whole = decltype(whole_c)::value;
+    T x[C][U][R];
+    /* (every element is asked for before one is used, past the end of a run its last one) */
 #pragma unroll
-      for (int u = 0; u < ACC_ACROSS_UNROLL; ++u) x[u] = get(row, k - 1 - u);
+    for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int u = 0; u < ACC_ACROSS_UNROLL; ++u) acc = f(x[u], acc);
-    }
-    for (; k > k0; --k) acc = f(get(row, k - 1), acc);
-#else
-    T acc = get(row, k0);
-    Int64 k = k0 + 1;
-    for (; k + ACC_ACROSS_UNROLL <= k1; k += ACC_ACROSS_UNROLL) {
+      for (int c = 0; c < C; ++c) {
+        const Int64 len = c == C - 1 ? n - c * h : h;
+        const Int64 k = at(c * h + (whole ? i + u : acc_min<Int64>(i + u, len - 1)));
 #pragma unroll
-      for (int u = 0; u < ACC_ACROSS_UNROLL; ++u) x[u] = get(row, k + u);
+        for (int r = 0; r < R; ++r) x[c][u][r] = get(row[r], k);
+      }
 #pragma unroll
-      for (int u = 0; u < ACC_ACROSS_UNROLL; ++u) acc = f(acc, x[u]);
-    }
-    for (; k < k1; ++k) acc = f(acc, get(row, k));
-#endif
-    if (split > 1) {
-      part[row * split + p] = acc;
-      part_ok[row * split + p] = 1;
-    } else {
-#if ACC_HAS_SEED && !ACC_FOLD_RIGHT
-      ACC_PUT(arrOut, row, f(acc, seed));                  /* ((x0 (+) x1) (+) ... x_last) (+) z */
-#else
-      ACC_PUT(arrOut, row, acc);
-#endif
-    }
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const Int64 len = c == C - 1 ? n - c * h : h;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+          if (first && u == 0) acc[c][r] = (SEEDED && c == 0) ? join(seed, x[c][0][r]) : x[c][0][r];
+          else if (whole || i + u < len) acc[c][r] = join(acc[c][r], x[c][u][r]);
+        }
+      }
+  };
+  /* (C > 1 only for pieces of at least C elements) */
+  Int64 i = 0;
+  if (U <= h) batch(0, acc_bool<true>(), acc_bool<true>());
+  else        batch(0, acc_bool<true>(), acc_bool<false>());
+  for (i = U; i + U <= h; i += U) batch(i, acc_bool<false>(), acc_bool<true>());
+  for (; i < n - (C - 1) * h; i += U) batch(i, acc_bool<false>(), acc_bool<false>());
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    out[r] = acc[0][r];
+#pragma unroll
+    for (int c = 1; c < C; ++c) out[r] = join(out[r], acc[c][r]);
   }
 }
+
+/* two entries, so that one row a lane keeps its few registers (70 against
+ * 148 for Float32: in one entry a matrix product of 1024 x 1024 took 296 us, 261 with registers to spare and 252 so) */
+#define ACC_ACROSS_ENTRY _across
+#define ACC_ACROSS_R 1
+#include "skel_fold_across.h"
+#undef ACC_ACROSS_ENTRY
+#undef ACC_ACROSS_R
+#if ACC_ACROSS_ROWS > 1
+#define ACC_ACROSS_ENTRY _across_wide
+#define ACC_ACROSS_R ACC_ACROSS_ROWS
+#include "skel_fold_across.h"
+#undef ACC_ACROSS_ENTRY
+#undef ACC_ACROSS_R
+#endif
 #endif /* ACC_SEG_UNIFORM */
 
 /* ---- long segments: a team of lanes per segment ---------------------------

@@ -476,17 +476,24 @@ int launch_segmented(acc_skel_s *s, int v, Args *args, const acc_array *env, con
 }
 
 // A fold along the innermost dimension whose element function reads neighbouring addresses where the ROW moves by one
-// (ACC_FLAG_TILED: the fold of a transposed matrix, a matrix product written as a fold): a lane per row, neighbouring
-// rows in neighbouring lanes (<entry>_across) -- a team of lanes along such a row asks for 64 cache lines with every
-// load (sums down the columns of 4096 x 4096 Int32: 0.9 ms).  With fewer rows than the device has lanes the rows are
-// cut into pieces of at least `fold.across_min_piece` elements, joined in order by <entry>_join.
+// (ACC_FLAG_TILED: the fold of a transposed matrix, a matrix product written as a fold): neighbouring rows in
+// neighbouring lanes (<entry>_across) -- a team of lanes along such a row asks for 64 cache lines with every load (sums
+// down the columns of 4096 x 4096 Int32: 0.9 ms).  With fewer rows than the device has lanes the rows are cut into
+// pieces of at least `fold.across_min_piece` elements: as many as a workgroup has room for beside one another (`subs`),
+// and `split` times that, joined in order by <entry>_join, until there is a workgroup for every compute unit (two, of
+// lanes with one row each).  Neither more nor in between: 312 workgroups, 56 units with two of them, take 19.9 us for the
+// columns of 20000 x 1000, 256 take 18.3 and 512 18.9.  Below 4096 rows a lane takes several (1000 rows 18.3 us against
+// 22.0 with one, 4096 rows 15.3 and 14.6; the product of two 128 x 128 matrices, 16384 rows, 12 and 7: there several
+// rows read one element of the left operand each).
 int launch_across(acc_skel_s *s, int v, Args *args, const acc_array *env, const acc_array *out, int64_t rows, int64_t inner, hipStream_t st)
 {
-  const int64_t cus = s->ctx->props.multiProcessorCount;
-  const int64_t lanes = cus * 2048;
-  int64_t split = 1;
-  if (rows < lanes)
-    split = std::max<int64_t>(1, std::min<int64_t>({lanes / rows, inner / std::max(1, s->knobs.fold_across_min_piece), s->knobs.foldseg_max_split}));
+  const int64_t cus = s->ctx->props.multiProcessorCount, block = s->spec.block;
+  const int64_t wide = rows < s->knobs.fold_across_wide_below ? acc::across_rows(s->spec) : 1, lanes = (rows + wide - 1) / wide;
+  const int64_t pieces = rows < cus * 2048 ? inner / std::max(1, s->knobs.fold_across_min_piece) : 1;
+  // lanes side by side: a wave's worth or, of rows that are not cut, a workgroup's; spread evenly over the workgroups
+  const int64_t most = pieces > 1 ? 64 : block, chunks = (lanes + most - 1) / most, chunk = (lanes + chunks - 1) / chunks;
+  const int64_t subs = std::max<int64_t>(1, std::min(block / chunk, pieces));
+  const int64_t split = std::max<int64_t>(1, std::min<int64_t>({(wide > 1 ? 1 : 2) * cus / chunks, pieces / subs, s->knobs.foldseg_max_split}));
   acc::ScratchRef blk;
   uint64_t part = 0, part_ok = 0;
   if (split > 1) {
@@ -500,10 +507,12 @@ int launch_across(acc_skel_s *s, int v, Args *args, const acc_array *env, const 
   first.i64(split);
   first.ptr(part);
   first.ptr(part_ok);
-  const int64_t grid = acc_launch_grid(rows * split, s->spec.block, cus, 4 * (2048 / s->spec.block));
+  first.i32(static_cast<int32_t>(chunk));
+  first.i32(static_cast<int32_t>(subs));
+  const int64_t grid = std::min<int64_t>(chunks * split, (int64_t)1 << 22);
   int rc = s->ctx->make_current();
   if (rc == ACC_OK) {
-    hipError_t e = launch_kernel(s->variants[v].fn_across, static_cast<unsigned>(grid), 1, 1, static_cast<unsigned>(s->spec.block), 1, 1, 0, st,
+    hipError_t e = launch_kernel(wide > 1 ? s->variants[v].fn_across_wide : s->variants[v].fn_across, static_cast<unsigned>(grid), 1, 1, static_cast<unsigned>(s->spec.block), 1, 1, 0, st,
                                  first.data(), nullptr);
     if (e != hipSuccess) rc = acc::fail_hip(e, "hipModuleLaunchKernel(fold, a lane a row)");
   }

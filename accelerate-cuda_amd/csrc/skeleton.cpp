@@ -162,6 +162,9 @@ static std::set<OwnRead> take_own_reads(const std::vector<EnvSig> &env, const st
 
 // ---- the generator -------------------------------------------------------------
 
+// neighbouring rows a lane of a fold's <entry>_across takes: 16 bytes of them, no more than four
+int across_rows(const SkelSpec &sp) { return std::max(1, std::min(4, 16 / std::max(1, sp.elt_size))); }
+
 int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::string *source)
 {
   const Tuning &knobs = *sp.tuning;
@@ -258,7 +261,7 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
       if (sp.out_rank > 0) {
         // along the innermost dimension: the segmented fold over rows of one length
         *entry = sp.has_seed ? "fold" : "fold1";
-        o << "#define ACC_SEG_UNIFORM 1\n";
+        o << "#define ACC_SEG_UNIFORM 1\n#define ACC_ACROSS_ROWS " << across_rows(sp) << "\n";
         o << "#define ACC_TROUNDS " << tune("foldseg.team_rounds", 3) << "\n";
         if (tuned("foldseg.pad")) o << "#define ACC_PAD_ON " << (tune("foldseg.pad", 1) ? 1 : 0) << "\n";
         if (tuned("foldseg.wide")) o << "#define ACC_WIDE " << std::max(1, tune("foldseg.wide", 256)) << "\n";
@@ -1053,6 +1056,15 @@ int acc_skel_s::ensure_variant(int v)
       (void)hipModuleUnload(var.module);
       var.module = nullptr;
       return acc::fail_hip(e, ("hipModuleGetFunction(" + across + ")").c_str());
+    }
+    if (acc::across_rows(spec) > 1) {
+      const std::string wide = across + "_wide";
+      e = hipModuleGetFunction(&var.fn_across_wide, var.module, wide.c_str());
+      if (e != hipSuccess) {
+        (void)hipModuleUnload(var.module);
+        var.module = nullptr;
+        return acc::fail_hip(e, ("hipModuleGetFunction(" + wide + ")").c_str());
+      }
     }
   }
   (void)hipFuncGetAttribute(&var.num_regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, var.fn);

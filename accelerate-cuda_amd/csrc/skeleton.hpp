@@ -78,6 +78,7 @@ struct Variant {
   hipFunction_t fn_rows = nullptr;     // fold along the innermost dimension: _rows, a lane per short row
   hipFunction_t fn_claim = nullptr;    // a permute whose combination is the new value: permute_claim (skel_scatter.h)
   hipFunction_t fn_across = nullptr;   // fold along the innermost dimension: _across, a lane per row of any length
+  hipFunction_t fn_across_wide = nullptr;   // ... _across_wide, several rows a lane (elements of at most 8 bytes)
   hipFunction_t fn_sweep = nullptr;    // a segmented fold's variants 4-7: _sweep, the segments that were handed over;
                                        // its variants 0-3: _probe, a look at the segment lengths
   int num_regs = 0;
@@ -91,6 +92,7 @@ struct Variant {
 
 int type_size(const std::string &t);
 int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp);
+int across_rows(const SkelSpec &sp);
 int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::string *source);
 SkelSpec spec_of_variant(const SkelSpec &base, int variant);
 std::vector<std::string> compile_options(const SkelSpec &sp);
