@@ -29,6 +29,7 @@ ACC_EMBED(scatter, "device/skel_scatter.h")
 ACC_EMBED(stencil, "device/skel_stencil.h")
 ACC_EMBED(stencil_nd, "device/skel_stencil_nd.h")
 ACC_EMBED(stencil_flat, "device/skel_stencil_flat.h")
+ACC_EMBED(stencil_pair, "device/skel_stencil_pair.h")
 
 namespace acc {
 
@@ -47,6 +48,7 @@ const std::vector<EmbeddedHeader> &embedded_headers()
       {"skel_stencil.h", acc_embed_stencil_begin, acc_embed_stencil_end},
       {"skel_stencil_nd.h", acc_embed_stencil_nd_begin, acc_embed_stencil_nd_end},
       {"skel_stencil_flat.h", acc_embed_stencil_flat_begin, acc_embed_stencil_flat_end},
+      {"skel_stencil_pair.h", acc_embed_stencil_pair_begin, acc_embed_stencil_pair_end},
   };
   return headers;
 }

@@ -1398,6 +1398,31 @@ static int stencil_once(acc_skel s, const acc_array *env, const acc_array *in, c
   return launch(s, (aligned ? 0 : 1) + 2 * narrow, (strips_x * bands * zbands + waves - 1) / waves, 0, st, &args);
 }
 
+// Two applications of a stencil in one launch (skel_stencil_pair.h), where the instance and the shape allow: false if not,
+// and nothing has been done.
+static bool stencil_pair(acc_skel s, const acc_array *env, const acc_array *in, const acc_array *out, hipStream_t st, int *rc)
+{
+  if (s->spec.pair_rows <= 0 || s->knobs.stencil_pair == 0 || array_size(*out) == 0) return false;
+  const int64_t w = out->shape[1], h = out->shape[0], owned = (int64_t)62 * s->spec.svec, esz = s->spec.elt_size;
+  const int64_t strips = (w + owned - 1) / owned, bands = (h + s->spec.pair_rows - 1) / s->spec.pair_rows;
+  if ((w != owned && w < owned + s->spec.svec) || h < 3 || w >= (1 << 30) || h >= (1 << 30) || strips * bands >= (1 << 30)) return false;
+  const int v = 10 + ((aligned16(in->ptr[0]) && aligned16(out->ptr[0]) && w * esz % 16 == 0) ? 0 : 1);
+  if (!may_take(s, v, st)) return false;
+  *rc = [&]() -> int {
+    ACC_RUN_SCOPE(s, st);
+    Args args;
+    bool aligned = true;
+    ACC_TRY(push_env(s, env, &args, &aligned));
+    push_out(*out, &args, &aligned);
+    push_ptrs(in, in->ncomp, &args, &aligned);
+    args.i32(0);
+    ACC_TRY(s->ensure_variant(v));
+    const int64_t per_block = s->spec.block / 64;
+    return launch(s, v, (strips * bands + per_block - 1) / per_block, 0, st, &args);
+  }();
+  return true;
+}
+
 static int stencil_check(acc_skel s, const acc_array *in, const acc_array *out)
 {
   if (!s) return fail(ACC_ERR_INVALID, "acc_exec_stencil: NULL skeleton");
@@ -1440,8 +1465,21 @@ int acc_exec_stencil_iterate(acc_skel s, const acc_array *env, const acc_array *
   ACC_TRY(stencil_check(s, a, b));
   if (iters < 0) return fail(ACC_ERR_INVALID, "stencil: negative iteration count");
   const acc_array *src = a, *dst = b;
-  for (int32_t i = 0; i < iters; ++i) {
-    ACC_TRY(stencil_once(s, env, src, nullptr, dst, static_cast<hipStream_t>(stream)));
+  // Two applications a launch as often as leaves every result where one a launch would: an even number of pairs, so that
+  // the arrays have changed places as often, and at least one application by itself at the end, whose source is then the
+  // result before the last.
+  int32_t pairs = 2 * ((std::max(iters, 1) - 1) / 4);
+  for (int32_t i = 0; i < iters;) {
+    const bool two = pairs > 0;
+    int rc = ACC_OK;
+    if (two && !stencil_pair(s, env, src, dst, static_cast<hipStream_t>(stream), &rc)) {
+      pairs = 0;
+      continue;
+    }
+    if (!two) rc = stencil_once(s, env, src, nullptr, dst, static_cast<hipStream_t>(stream));
+    ACC_TRY(rc);
+    i += two ? 2 : 1;
+    pairs -= two ? 1 : 0;
     std::swap(src, dst);
   }
   if (result_in_b) *result_in_b = (iters & 1);

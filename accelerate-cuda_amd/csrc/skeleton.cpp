@@ -477,7 +477,7 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
       }
       o << "#define ACC_STENCIL_FN " << sp.stencil_fn << "\n";
       o << "#define ACC_XCD_REMAP " << tune("stencil.xcd_remap", 0) << "\n";
-      o << "#define ACC_STENCIL_NT " << tune("stencil.nt", 1) << "\n";
+      o << "#define ACC_STENCIL_NT " << (sp.stencil_pair ? tune("stencil.pair_nt", 0) : tune("stencil.nt", 1)) << "\n";
       o << "#define ACC_SCHED_BARRIER " << tune("stencil.sched_barrier", 3) << "\n";
       o << "#define ACC_SVEC " << sp.svec << "\n";
       o << "#define ACC_SHIFT_MIN " << tune("stencil.shift_min", sp.zmarch ? 1 : 24 * sp.svec) << "\n";
@@ -486,7 +486,7 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
       o << "#define ACC_TILE_H " << sp.tile_h << "\n#define ACC_PREFETCH " << sp.prefetch << "\n#define ACC_BLOCK " << sp.block << "\n";
       o << "#define ACC_TZ " << sp.tile_z << "\n";
       o << "#define ACC_ZMARCH " << sp.zmarch << "\n";
-      tmpl = sp.stencil_flat ? "skel_stencil_flat.h" : "skel_stencil.h";
+      tmpl = sp.stencil_pair ? "skel_stencil_pair.h" : sp.stencil_flat ? "skel_stencil_flat.h" : "skel_stencil.h";
       break;
     }
     default:
@@ -840,6 +840,14 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
         for (int ty = std::min(tune("stencil.flat_rows", 2), 4); ty > 0 && sp->flat_rows == 0; --ty)
           if ((2 * ry + ty) * (2 * rz + 1 + sp->flat_prefetch) * (sp->svec + 2 * rx) * words <= 192) sp->flat_rows = ty;
       }
+      // Two applications a launch, for calls that make many: of one array of 4- or 8-byte elements whose result is its
+      // source the next time, with taps no more than a row and a column away and nothing else to read.
+      if (sp->out_rank == 2 && d->kind == ACC_SKEL_STENCIL && sp->stencil_in_comps.size() == 1 && sp->comp_types.empty() &&
+          sp->stencil_in_comps[0] == sp->elt_type && sp->env.empty() && type_size(sp->elt_type) >= 4) {
+        int far = 0;
+        for (size_t k = 0; k < sp->tap_dx.size(); ++k) far = std::max({far, std::abs(sp->tap_dx[k]), std::abs(sp->tap_dy[k])});
+        if (far <= 1 && sp->svec >= 2 && sp->svec <= 4) sp->pair_rows = std::max(0, std::min(tune("stencil.pair_rows", 4), 16));
+      }
       if (sp->zmarch && 2 * rx * (2 * ry + sp->tile_z) > 64) return fail(ACC_ERR_INVALID, "stencil: strip too tall for its reach");
       if (sp->tile_h < 1 || sp->prefetch < 0 || sp->prefetch > 8 || sp->tile_z < 1 || sp->tile_z > 8) return fail(ACC_ERR_INVALID, "stencil: bad tile shape");
       break;
@@ -916,8 +924,14 @@ SkelSpec spec_of_variant(const SkelSpec &base, int v)
     spec.svec = std::max(1, spec.svec >> (v / 2));
     spec.tile_w = 64 * spec.svec;
   }
-  // ... and 8 and 9: lanes over the vectors of a whole plane
-  if (spec.kind == ACC_SKEL_STENCIL && v >= 8) {
+  // ... 10 and 11: two applications a launch; and 8 and 9: lanes over the vectors of a whole plane
+  if (spec.kind == ACC_SKEL_STENCIL && v >= 10) {
+    spec.stencil_pair = true;
+    spec.stencil_nd = false;
+    spec.svec = base.svec;
+    spec.tile_w = 62 * spec.svec;
+    spec.tile_h = spec.pair_rows;
+  } else if (spec.kind == ACC_SKEL_STENCIL && v >= 8) {
     spec.stencil_flat = true;
     spec.stencil_nd = false;
     spec.svec = base.svec;
@@ -1097,7 +1111,7 @@ static int variant_count(const acc::SkelSpec &sp)
   const bool stencil = sp.kind == ACC_SKEL_STENCIL || sp.kind == ACC_SKEL_STENCIL2;
   if ((sp.kind == ACC_SKEL_FOLDSEG || sp.kind == ACC_SKEL_FOLD1SEG) && sp.out_rank <= 1) return 8;
   if (sp.map_tiled) return 4;
-  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : sp.flat_rows > 0 ? 10 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
+  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : sp.pair_rows > 0 ? 12 : sp.flat_rows > 0 ? 10 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
 }
 
 extern "C" {
@@ -1199,7 +1213,7 @@ int acc_skel_source(acc_skel s, int variant, const char **source)
 int acc_skel_preview(const acc_skel_desc *desc, int variant, const char **source, const char **entry)
 {
   static thread_local std::string text, name;
-  if (!source || variant < 0 || variant > 9) return fail(ACC_ERR_INVALID, "acc_skel_preview: bad argument");
+  if (!source || variant < 0 || variant > 11) return fail(ACC_ERR_INVALID, "acc_skel_preview: bad argument");
   acc::SkelSpec sp;
   ACC_TRY(acc::make_spec(desc, acc::default_tuning(), &sp));
   // beyond 1: a permute's forms (to 7), a stencil's fewer columns a lane (to 5), a scan's small tiles and a segmented

@@ -38,6 +38,8 @@ struct SkelSpec {
   int boundary2 = 0;
   std::string boundary2_constant, stencil_in2_type;
   std::vector<int> tap2_dz, tap2_dy, tap2_dx;
+  bool stencil_pair = false;            // a stencil's variants 10 and 11: two applications a launch (skel_stencil_pair.h)
+  int pair_rows = 0;                    // ... their rows a strip; 0: no such variants
   bool stencil_flat = false;            // a stencil's variants 8 and 9: lanes over the vectors of a plane (skel_stencil_flat.h)
   int flat_rows = 0, flat_prefetch = 0; // ... their rows a lane and planes asked for ahead; 0 rows: no such variants
   bool stencil_nd = false;              // an element a thread (skel_stencil_nd.h): rank > 3, or taps further away than the strips' windows hold
@@ -104,7 +106,7 @@ struct acc_skel_s {
   acc::SkelSpec spec;
   acc::Knobs knobs;           // what the drivers read of the tuning table
   std::string entry;
-  acc::Variant variants[10];  // [0] pointers 16-byte aligned, [1] no assumption; [2], [3]: the same for the
+  acc::Variant variants[12];  // [0] pointers 16-byte aligned, [1] no assumption; [2], [3]: the same for the
                               // table-in-LDS form of a permute whose combination has no atomic instruction;
                               // [4], [5]: for a hinted permute over several LDS windows of targets;
                               // [6], [7]: for integer addition on a table of 16-bit counts in LDS;
