@@ -7,6 +7,7 @@ library has not been built.
 """
 import ctypes as C
 import os
+import struct
 import subprocess
 
 import numpy as np
@@ -48,6 +49,13 @@ class AccError(RuntimeError):
 class acc_array(C.Structure):
     _fields_ = [("rank", C.c_int32), ("ncomp", C.c_int32),
                 ("shape", C.c_int64 * MAX_RANK), ("ptr", C.c_uint64 * MAX_COMP)]
+
+
+# the bytes of an acc_array of one component, by rank: a field at a time through ctypes costs three times as much, and
+# three such descriptors were half of a small call's host time
+_ARRAY = [struct.Struct("@ii%dq%dxQ%dx" % (r, 8 * (MAX_RANK - r), 8 * (MAX_COMP - 1))).pack for r in range(MAX_RANK + 1)]
+_array_from = acc_array.from_buffer_copy
+assert len(_ARRAY[0](0, 1, 0)) == C.sizeof(acc_array)
 
 
 class acc_env_sig(C.Structure):
@@ -343,13 +351,9 @@ class DeviceArray(object):
         self.ptr = ptr
 
     def desc(self, shape=None, offset_elems=0):
-        a = acc_array()
         shape = self.shape if shape is None else tuple(shape)
-        a.rank, a.ncomp = len(shape), 1
-        for i, s in enumerate(shape):
-            a.shape[i] = s
-        a.ptr[0] = self.ptr + offset_elems * self.dtype.itemsize
-        return a
+        ptr = self.ptr + offset_elems * self.dtype.itemsize if offset_elems else self.ptr
+        return _array_from(_ARRAY[len(shape)](len(shape), 1, *shape, ptr))
 
     def get(self, out=None):
         """the array on the host; `out`: a C-contiguous array of the same shape and type to fill instead of a new one"""
@@ -581,13 +585,19 @@ class MemTable(object):
             self.handle = None
 
 
+_plain_desc = DeviceArray.desc
+
+
 def _env(arrays):
     if not arrays:
         return None
-    env = (acc_array * len(arrays))()
-    for k, a in enumerate(arrays):
-        env[k] = a if isinstance(a, acc_array) else a.desc()
-    return env
+    parts = []
+    for a in arrays:
+        if getattr(type(a), "desc", None) is _plain_desc:                  # a DeviceArray: its descriptor's bytes straight away
+            parts.append(_ARRAY[len(a.shape)](len(a.shape), 1, *a.shape, a.ptr))
+        else:
+            parts.append(bytes(a if isinstance(a, acc_array) else a.desc()))
+    return (acc_array * len(parts)).from_buffer_copy(b"".join(parts))
 
 
 class Skeleton(object):

@@ -10,7 +10,6 @@
 #include <algorithm>
 #include <cstdlib>
 #include <cstring>
-#include <deque>
 
 #include "skeleton.hpp"
 
@@ -37,7 +36,7 @@ class Args {
   void u32(uint32_t v) { push(&v, sizeof(v)); }
   void i32(int32_t v) { push(&v, sizeof(v)); }
   void ptr(uint64_t v) { push(&v, sizeof(v)); }
-  size_t count() const { return slots_.size(); }
+  size_t count() const { return count_; }
   // the arguments as HIP wants them, the guard's address appended for a guarded instance
   void **data()
   {
@@ -50,9 +49,14 @@ class Args {
   // (for a launch whose last arguments are not 8-byte slots: the caller appends them, then the guard)
   void **data_without_guard()
   {
-    ptrs_.clear();
-    for (uint64_t &s : slots_) ptrs_.push_back(&s);
-    return ptrs_.data();
+    uint64_t *slot = count_ <= FEW ? few_ : many_.data();
+    void **ptr = few_ptrs_;
+    if (count_ > FEW) {
+      many_ptrs_.resize(count_);
+      ptr = many_ptrs_.data();
+    }
+    for (size_t k = 0; k < count_; ++k) ptr[k] = slot + k;
+    return ptr;
   }
 
  private:
@@ -60,10 +64,22 @@ class Args {
   {
     uint64_t s = 0;
     std::memcpy(&s, p, n);
-    slots_.push_back(s);
+    if (count_ < FEW) {
+      few_[count_++] = s;
+      return;
+    }
+    if (count_ == FEW) many_.assign(few_, few_ + FEW);
+    many_.push_back(s);
+    ++count_;
   }
-  std::deque<uint64_t> slots_;
-  std::vector<void *> ptrs_;
+  // (in place as far as any but the longest lists go: a call's host side is a few microseconds, and as long as a small
+  // array's whole call)
+  static constexpr size_t FEW = 40;
+  size_t count_ = 0;
+  uint64_t few_[FEW];
+  void *few_ptrs_[FEW];
+  std::vector<uint64_t> many_;
+  std::vector<void *> many_ptrs_;
   bool guard_pushed_ = false;
 };
 
