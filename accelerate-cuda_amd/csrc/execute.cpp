@@ -718,9 +718,11 @@ namespace {
 
 // A variant beyond the ones an earlier call of this size would have loaded: there already, or buildable now (a stream
 // under capture is no place to load a module).
+// (A weak reference: a runtime without the call has no capture either.)
+#pragma weak hipStreamIsCapturing
 bool may_take(acc_skel s, int v, hipStream_t st)
 {
-  if (s->variant_ready(v)) return true;
+  if (s->variant_ready(v) || !hipStreamIsCapturing) return true;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   return hipStreamIsCapturing(st, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
 }
