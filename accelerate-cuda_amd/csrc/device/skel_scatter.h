@@ -26,21 +26,24 @@
  *
  * The operands that the fragments read at the element's own index (ACC_OWN_*, all of them arrays at least `past` long)
  * are asked for ahead of everything else, for the whole batch: `filter` reads a place only where the element stays, and a
- * read behind such a test is waited for on the spot, one element after the other.
+ * read behind such a test is waited for on the spot, one element after the other.  Everything else that the element
+ * function reads is read for sources that stay only: what it makes of one that is dropped need not exist.
  *
- * Measured with the operands in HBM, 2^24 Int32 sources, defaults included, before (stores of device scope, a lane four
- * elements side by side, reads behind tests) and now: half of them kept in order 64 us -> 43, a sorting pass by 4 bits
- * 146 -> 79, by 8 bits 356 -> 176, a random permutation 392 -> 344, all of them on 10 targets of 2^24 9.7 ms -> 0.05;
- * the scatter of `filter` (flag, place and value of 2^24 read, half stored) 98 -> 27, at 2^20 9.4 -> 4.0.  A lane takes 8
- * elements (ACC_BATCH): 32 do the sorting pass by 8 bits in 123 us and the random permutation in 262, but the scatter of
- * `filter` in 32, and in 7.2 at 2^20, where they leave half of the device idle.
+ * Measured with the operands in HBM, 2^24 Int32 sources, defaults included, through the atomics template (stores of device
+ * scope, a lane four elements side by side, reads behind tests) and now: half of them kept in order 64 us -> 49, a sorting
+ * pass by 4 bits 146 -> 77, by 8 bits 356 -> 161, a random permutation 392 -> 286, all of them on 10 targets of 2^24 9.7 ms
+ * -> 0.05; the scatter of `filter` (flag, place and value of 2^24 read, half stored) 98 -> 27, at 2^20 9.4 -> 4.0.  A lane
+ * takes 8 elements (ACC_BATCH): 32 do the sorting pass by 8 bits in 123 us and the random permutation in 262, but the
+ * scatter of `filter` in 32, and in 7.2 at 2^20, where they leave half of the device idle.  Pairs of Int32, two launches:
+ * 115 / 218 / 595 / 1240 us.
  *
  * Generated definitions expected: ACC_ELT, ACC_NCOMP, ACC_FOR_COMPONENTS, ACC_ENV_PARAMS, ACC_ENV_ASSUME, ACC_OUT_PARAMS,
  * ACC_OUT_SIZE, ACC_GET(ix), ACC_PERMUTATION(ix), ACC_OWN_FIELDS, ACC_OWN_LOAD(sv, ix), ACC_OWN_WITHIN(past), ACC_GET_OWN(ix),
- * ACC_PERMUTATION_OWN(ix), ACC_BLOCK, ACC_BATCH, ACC_SMALL.
+ * ACC_GET_TOTAL, ACC_PERMUTATION_OWN(ix), ACC_BLOCK, ACC_BATCH, ACC_SMALL.
  */
 
 #define ACC_TILE (ACC_BLOCK * ACC_BATCH)
+#define ACC_AHEAD (ACC_GET_TOTAL && ACC_NCOMP == 1)               /* elements worked out with the targets */
 #define ACC_CLAIMED (ACC_NCOMP > 1 || sizeof(ACC_ELT) > 8)       /* what no single store of at most 8 bytes writes */
 
 /* Names the kernels share.  A tile that reaches past the end reads the last source there (`in`): no test per element
@@ -84,9 +87,14 @@ permute(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 first, const Int64 past, cons
 {
   ACC_GUARD_CHECK
   ACC_SCATTER_NAMES
+  /* The element function of a source that is dropped may have no value -- the index it reads through may be any number.
+   * One that only calculates with the source's own operands has (ACC_GET_TOTAL).  Of any other a lane that stores nothing
+   * works out the element of a source of its wave that stays: behind a test every read would be waited for on the spot
+   * (2^24 Int32 through an index, half of them kept in order: 65.6 us behind tests, 59 so). */
   Int64 j[ACC_BATCH];
   T x[ACC_BATCH];
   bool mine[ACC_BATCH];
+#if ACC_AHEAD
   if (ACC_OWN_WITHIN(past)) {
     own sv[ACC_BATCH];
 #pragma unroll
@@ -98,11 +106,25 @@ permute(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 first, const Int64 past, cons
     }
   } else {
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) {
-      j[k] = perm(in(k));
-      x[k] = get(in(k));
-    }
+    for (int k = 0; k < ACC_BATCH; ++k) j[k] = perm(in(k));
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k)
+      if (j[k] >= 0 && j[k] < ntarget) x[k] = get(in(k));
   }
+#else
+  own sv[ACC_BATCH];
+  const bool whole = ACC_OWN_WITHIN(past);
+  if (whole) {
+    asm volatile("");          /* (a request shared with the other form would be made, and waited for, ahead of the branch) */
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) { ACC_OWN_LOAD(sv[k], in(k)) }
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) j[k] = perm_own(in(k), sv[k]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) j[k] = perm(in(k));
+  }
+#endif
 #pragma unroll
   for (int k = 0; k < ACC_BATCH; ++k) mine[k] = ix0 + k * ACC_BLOCK < past && j[k] >= 0 && j[k] < ntarget;
   if (ACC_CLAIMED) {
@@ -112,6 +134,28 @@ permute(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 first, const Int64 past, cons
 #pragma unroll
     for (int k = 0; k < ACC_BATCH; ++k) mine[k] = mine[k] && w[k] == (unsigned int)(ix0 + k * ACC_BLOCK - first);
   }
+#if !ACC_AHEAD
+  Int64 stays = -1;
+  own of_stays;
+#pragma unroll
+  for (int k = ACC_BATCH - 1; k >= 0; --k) {
+    const unsigned long long here = __ballot(mine[k]);
+    if (here != 0ull) {
+      const int lane = __builtin_ctzll(here);
+      stays = acc_readlane(in(k), lane);
+      of_stays = acc_readlane(sv[k], lane);
+    }
+  }
+  if (stays < 0) return;                                   /* (the whole wave) */
+  if (whole) {
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k)
+      x[k] = ACC_GET_TOTAL ? get_own(in(k), sv[k]) : get_own(mine[k] ? in(k) : stays, mine[k] ? sv[k] : of_stays);
+  } else {
+#pragma unroll
+    for (int k = 0; k < ACC_BATCH; ++k) x[k] = get(mine[k] ? in(k) : stays);
+  }
+#endif
 #pragma unroll
   for (int k = 0; k < ACC_BATCH; ++k)
     if (mine[k]) ACC_SET(arrOut, j[k], x[k]);

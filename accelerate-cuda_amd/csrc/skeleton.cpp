@@ -160,6 +160,32 @@ static std::set<OwnRead> take_own_reads(const std::vector<EnvSig> &env, const st
   return reads;
 }
 
+// Whether a fragment, its own reads taken out, has a value whatever they hold: arithmetic on them, on the index and on
+// extents, without a call, another read or a division.
+static bool only_calculates(const std::string &text)
+{
+  static const std::set<std::string> plain = {"ix", "acc_elt", "acc_sv", "Int8", "Int16", "Int32", "Int64", "Word8", "Word16", "Word32", "Word64",
+                                              "float", "double", "int", "unsigned", "char", "short", "long", "bool", "true", "false"};
+  static const std::regex field("s\\d+_\\d+|shIn\\d+_\\d+|shOut_\\d+");
+  for (size_t k = 0; k < text.size();) {
+    const unsigned char c = static_cast<unsigned char>(text[k]);
+    if (std::isdigit(c)) {                   // (a number, with whatever letters and points belong to it)
+      while (k < text.size() && (std::isalnum(static_cast<unsigned char>(text[k])) || text[k] == '.')) ++k;
+    } else if (std::isalpha(c) || c == '_') {
+      size_t end = k;
+      while (end < text.size() && (std::isalnum(static_cast<unsigned char>(text[end])) || text[end] == '_')) ++end;
+      const std::string name = text.substr(k, end - k);
+      if (!plain.count(name) && !std::regex_match(name, field)) return false;
+      for (k = end; k < text.size() && std::isspace(static_cast<unsigned char>(text[k])); ++k) {}
+      if (k < text.size() && (text[k] == '(' || (text[k] == '{' && name != "acc_elt"))) return false;
+    } else {
+      if (!std::isspace(c) && !std::strchr("+-*<>=!&|^~?:,.(){}", c)) return false;
+      ++k;
+    }
+  }
+  return true;
+}
+
 // ---- the generator -------------------------------------------------------------
 
 // neighbouring rows a lane of a fold's <entry>_across takes: 16 bytes of them, no more than four
@@ -329,6 +355,7 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
         }
         o << "#define ACC_OWN_FIELDS " << fields.str() << "\n#define ACC_OWN_LOAD(sv, ix) " << loads.str() << "\n";
         o << "#define ACC_OWN_WITHIN(past) (true" << lengths.str() << ")\n";
+        o << "#define ACC_GET_TOTAL " << (sp.preamble.empty() && only_calculates(pre_get) ? 1 : 0) << "\n";
         o << "#define ACC_GET_OWN(ix) " << pre_get << "\n#define ACC_PERMUTATION_OWN(ix) " << pre_perm << "\n";
         tmpl = "skel_scatter.h";
         break;

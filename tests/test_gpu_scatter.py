@@ -84,3 +84,34 @@ def test_an_operand_shorter_than_the_source(A, ctx, n):
     empty = ctx.empty(0, np.int32)
     sk.permute([empty, empty], n, out, out)
     assert np.array_equal(out.get(), np.arange(n, dtype=np.int32))
+
+
+@pytest.mark.parametrize("n", [3000, 9000])
+@pytest.mark.parametrize("elt", ["Word8", "Int32", "Int32, Int8"])
+def test_the_element_of_a_source_that_is_dropped_is_not_evaluated(A, ctx, elt, n):
+    """a gather through an index that is only good where the source stays -- elsewhere it leads to elements in front of the
+    ones meant, which are there -- and a mark wherever the element function is evaluated"""
+    rng = np.random.default_rng(n)
+    places = rng.permutation(n + 60).astype(np.int32)[:n]
+    places[rng.random(n) < 0.4] = -1
+    places[1000:2100] = -1                                             # (waves that keep nothing)
+    kept = (places >= 0) & (places < n)
+    through = np.where(kept, rng.integers(50, 100, n), rng.integers(0, 50, n)).astype(np.int32)
+    values, marks = rng.integers(0, 100, 100).astype(np.int32), ctx.array(np.zeros(n, np.int32))
+    comps = [t.strip() for t in elt.split(",")]
+    value = "({ ((Int32 *)arrIn3_0)[ix] = 1; arrIn0_0[arrIn1_0[ix]]; })"
+    get = "(%s)%s" % (comps[0], value) if len(comps) == 1 else "acc_elt{%s, (Int8)(ix %% 100)}" % value
+    sk = ctx.skeleton(A.SKEL_PERMUTE, elt, env=[(1, "Int32")] * 4, out_rank=1, get=get, combine="x" if len(comps) == 1 else "acc_elt{x.a1, x.a0}",
+                      permutation="(Int64)arrIn2_0[ix]")
+    dts = [{"Word8": np.uint8, "Int32": np.int32, "Int8": np.int8}[t] for t in comps]
+    make = (lambda k: ctx.array(np.full(n, k, dts[0]))) if len(comps) == 1 else (lambda k: ctx.tuple_array(*[np.full(n, k, d) for d in dts]))
+    out = make(0)
+    sk.permute([ctx.array(values), ctx.array(through), ctx.array(places), marks], n, make(77), out)
+    assert np.array_equal(marks.get() != 0, kept)
+    got = out.get() if len(comps) > 1 else [out.get()]
+    want = np.full(n, 77, np.int64)
+    want[places[kept]] = values[through[kept]]
+    assert np.array_equal(got[0].astype(np.int64), want)
+    if len(comps) > 1:
+        want[places[kept]] = np.flatnonzero(kept) % 100
+        assert np.array_equal(got[1].astype(np.int64), want)
