@@ -38,13 +38,24 @@
  * 115 / 218 / 595 / 1240 us.
  *
  * Generated definitions expected: ACC_ELT, ACC_NCOMP, ACC_FOR_COMPONENTS, ACC_ENV_PARAMS, ACC_ENV_ASSUME, ACC_OUT_PARAMS,
- * ACC_OUT_SIZE, ACC_GET(ix), ACC_PERMUTATION(ix), ACC_OWN_FIELDS, ACC_OWN_LOAD(sv, ix), ACC_OWN_WITHIN(past), ACC_GET_OWN(ix),
- * ACC_GET_TOTAL, ACC_PERMUTATION_OWN(ix), ACC_BLOCK, ACC_BATCH, ACC_SMALL.
+ * ACC_OUT_SIZE, ACC_GET(ix), ACC_PERMUTATION(ix), ACC_OWN_NAMES, ACC_OWN_FIELDS, ACC_OWN_LOAD(sv, ix), ACC_OWN_WITHIN(past),
+ * ACC_GET_OWN(ix), ACC_GET_TOTAL, ACC_PERMUTATION_OWN(ix), ACC_BLOCK, ACC_BATCH, ACC_SMALL.
  */
 
 #define ACC_TILE (ACC_BLOCK * ACC_BATCH)
 #define ACC_AHEAD (ACC_GET_TOTAL && ACC_NCOMP == 1)               /* elements worked out with the targets */
 #define ACC_CLAIMED (ACC_NCOMP > 1 || sizeof(ACC_ELT) > 8)       /* what no single store of at most 8 bytes writes */
+
+/* What stands in a fragment for a read of an operand at the element's own index: `v`, asked for ahead of the tests, where
+ * the array and the index named there are the element's own, as they are unless the fragment gives one of the names to
+ * something of its own; there it is the read that was written. */
+template <typename T, typename I>
+ACC_DEV const T &acc_own_value(const T *a, const I ix, const T *own_a, const Int64 own_ix, const T &v)
+{
+  return a == own_a && (Int64)ix == own_ix ? v : a[ix];
+}
+template <typename A, typename I, typename T>
+ACC_DEV decltype(auto) acc_own_value(const A &a, const I ix, const T *, const Int64, const T &) { return a[ix]; }
 
 /* Names the kernels share.  A tile that reaches past the end reads the last source there (`in`): no test per element
  * stands in front of a read. */
@@ -54,8 +65,9 @@
   struct own { ACC_OWN_FIELDS };                                                                                               \
   auto get      = [&](const Int64 ix) -> T { return (ACC_GET(ix)); };                                                          \
   auto perm     = [&](const Int64 ix) -> Int64 { return (Int64)(ACC_PERMUTATION(ix)); };                                       \
-  auto get_own  = [&](const Int64 ix, const own &acc_sv) -> T { (void)ix; (void)acc_sv; return (ACC_GET_OWN(ix)); };           \
-  auto perm_own = [&](const Int64 ix, const own &acc_sv) -> Int64 { (void)ix; (void)acc_sv; return (Int64)(ACC_PERMUTATION_OWN(ix)); }; \
+  ACC_OWN_NAMES                                                                                                                \
+  auto get_own  = [&](const Int64 ix, const own &acc_sv) -> T { const Int64 acc_own_ix = ix; (void)acc_own_ix; (void)acc_sv; return (ACC_GET_OWN(ix)); }; \
+  auto perm_own = [&](const Int64 ix, const own &acc_sv) -> Int64 { const Int64 acc_own_ix = ix; (void)acc_own_ix; (void)acc_sv; return (Int64)(ACC_PERMUTATION_OWN(ix)); }; \
   (void)get; (void)get_own;                                                                                                    \
   const Int64 ntarget = (ACC_OUT_SIZE);                                                                                        \
   const Int64 ix0 = first + (Int64)blockIdx.x * ACC_TILE + threadIdx.x;                                                        \

@@ -9,7 +9,6 @@
 #include <cctype>
 #include <cstdlib>
 #include <cstring>
-#include <regex>
 #include <set>
 #include <sstream>
 
@@ -129,32 +128,90 @@ static const char *kind_name(int kind)
 // A fragment reads most of its operands at the consuming skeleton's own linear index: `acc_stream(arrIn<k>_<c>, ix)` or
 // `arrIn<k>_<c>[ix]`.  A template that asks for the operands of a whole batch before it looks at the first (a read
 // inside one branch of a conditional is otherwise waited for where it stands, one element after the other) gets them
-// from here: `texts` with those reads replaced by members of `acc_sv`, and the arrays they named, in order.
+// from here: `texts` with those reads replaced, and the arrays they named, in order.
+//
+// A name may mean something else inside a fragment than outside it -- `ix` may be a lambda's parameter there.  It takes a
+// declaration, and so a semicolon: in a fragment with one, what takes a read's place compares the array and the index it
+// names with the element's own before it gives the value that was asked for (acc_own_value, skel_scatter.h).  What cannot
+// be put so is left alone: a fragment that takes addresses, and every fragment under a preamble that defines macros.
 struct OwnRead {
   int array, comp;
   bool operator<(const OwnRead &o) const { return array != o.array ? array < o.array : comp < o.comp; }
 };
-static std::set<OwnRead> take_own_reads(const std::vector<EnvSig> &env, const std::vector<std::string *> &texts)
+static bool in_name(char c) { return std::isalnum(static_cast<unsigned char>(c)) || c == '_'; }
+static size_t past_spaces(const std::string &t, size_t k)
 {
-  static const std::regex own("acc_stream\\(\\s*arrIn(\\d+)_(\\d+)\\s*,\\s*ix\\s*\\)|\\barrIn(\\d+)_(\\d+)\\s*\\[\\s*ix\\s*\\]");
+  while (k < t.size() && std::isspace(static_cast<unsigned char>(t[k]))) ++k;
+  return k;
+}
+// the character in front of place k that is no space, or 0
+static char before(const std::string &t, size_t k)
+{
+  while (k > 0 && std::isspace(static_cast<unsigned char>(t[k - 1]))) --k;
+  return k > 0 ? t[k - 1] : '\0';
+}
+static bool takes_an_address(const std::string &t)
+{
+  for (size_t k = 0; k < t.size(); ++k) {
+    if (t[k] != '&') continue;
+    if (k + 1 < t.size() && t[k + 1] == '&') { ++k; continue; }
+    const char c = before(t, k);
+    if (c == '[' && past_spaces(t, k + 1) < t.size() && t[past_spaces(t, k + 1)] == ']') continue;      // [&]
+    if (!in_name(c) && c != ')' && c != ']') return true;
+  }
+  return false;
+}
+// the read that begins at place k of the text, if one does: its array and the place behind it
+static bool own_read_at(const std::string &t, size_t k, OwnRead *read, size_t *past)
+{
+  auto word = [&](const char *w) {
+    const size_t n = std::strlen(w);
+    k = past_spaces(t, k);
+    if (t.compare(k, n, w) != 0 || (in_name(w[n - 1]) && k + n < t.size() && in_name(t[k + n]))) return false;
+    k += n;
+    return true;
+  };
+  auto number = [&](int *n) {
+    const size_t first = k;
+    for (*n = 0; k < t.size() && std::isdigit(static_cast<unsigned char>(t[k])) && k - first < 6; ++k) *n = 10 * *n + (t[k] - '0');
+    return k > first;
+  };
+  const bool streamed = word("acc_stream");
+  if (streamed && !word("(")) return false;
+  k = past_spaces(t, k);
+  if (t.compare(k, 5, "arrIn") != 0) return false;
+  k += 5;
+  if (!number(&read->array) || k >= t.size() || t[k] != '_') return false;
+  ++k;
+  if (!number(&read->comp) || (k < t.size() && in_name(t[k]))) return false;
+  if (!word(streamed ? "," : "[") || !word("ix") || !word(streamed ? ")" : "]")) return false;
+  *past = k;
+  return true;
+}
+// `values`: the names of the values in place of the reads (for a look at what else a fragment does)
+static std::set<OwnRead> take_own_reads(const SkelSpec &sp, const std::vector<std::string *> &texts, bool values = false)
+{
   std::set<OwnRead> reads;
+  if (sp.preamble.find('#') != std::string::npos) return reads;
   for (std::string *text : texts) {
+    if (takes_an_address(*text)) continue;
+    const bool declares = text->find(';') != std::string::npos;
     std::string out;
-    auto at = text->cbegin();
-    for (std::sregex_iterator m(text->cbegin(), text->cend(), own), end; m != end; ++m) {
-      const bool streamed = (*m)[1].matched;
-      const std::string k = (*m)[streamed ? 1 : 3].str(), c = (*m)[streamed ? 2 : 4].str();
-      const OwnRead r = {k.size() > 6 ? -1 : std::atoi(k.c_str()), c.size() > 6 ? -1 : std::atoi(c.c_str())};
-      out.append(at, (*m)[0].first);
-      if (r.array >= 0 && r.array < (int)env.size() && r.comp >= 0 && r.comp < env[r.array].ncomp) {
-        reads.insert(r);
-        out += "acc_sv.s" + std::to_string(r.array) + "_" + std::to_string(r.comp);
-      } else {
-        out += (*m)[0].str();                 // (no array of the instance: the compiler will say so)
+    for (size_t k = 0; k < text->size();) {
+      OwnRead r;
+      size_t past = 0;
+      const char c = before(*text, k);
+      const bool member = c == '.' || (c == '>' && text->find("->") != std::string::npos) || (c == ':' && text->find("::") != std::string::npos);
+      if (!in_name((*text)[k]) || (k > 0 && in_name((*text)[k - 1])) || member || !own_read_at(*text, k, &r, &past) ||
+          r.array >= (int)sp.env.size() || r.comp >= sp.env[r.array].ncomp) {
+        out.push_back((*text)[k++]);
+        continue;
       }
-      at = (*m)[0].second;
+      const std::string id = std::to_string(r.array) + "_" + std::to_string(r.comp);
+      reads.insert(r);
+      out += values || !declares ? "acc_sv.s" + id : "acc_own_value(arrIn" + id + ", ix, acc_own_arr" + id + ", acc_own_ix, acc_sv.s" + id + ")";
+      k = past;
     }
-    out.append(at, text->cend());
     *text = out;
   }
   return reads;
@@ -166,7 +223,11 @@ static bool only_calculates(const std::string &text)
 {
   static const std::set<std::string> plain = {"ix", "acc_elt", "acc_sv", "Int8", "Int16", "Int32", "Int64", "Word8", "Word16", "Word32", "Word64",
                                               "float", "double", "int", "unsigned", "char", "short", "long", "bool", "true", "false"};
-  static const std::regex field("s\\d+_\\d+|shIn\\d+_\\d+|shOut_\\d+");
+  auto field = [](const std::string &name) {         // s<k>_<c>, shIn<k>_<d>, shOut_<d>
+    const size_t at = name.find_first_of("0123456789");
+    const std::string head = name.substr(0, at);
+    return at != std::string::npos && (head == "s" || head == "shIn" || head == "shOut_");
+  };
   for (size_t k = 0; k < text.size();) {
     const unsigned char c = static_cast<unsigned char>(text[k]);
     if (std::isdigit(c)) {                   // (a number, with whatever letters and points belong to it)
@@ -175,7 +236,7 @@ static bool only_calculates(const std::string &text)
       size_t end = k;
       while (end < text.size() && (std::isalnum(static_cast<unsigned char>(text[end])) || text[end] == '_')) ++end;
       const std::string name = text.substr(k, end - k);
-      if (!plain.count(name) && !std::regex_match(name, field)) return false;
+      if (!plain.count(name) && !field(name)) return false;
       for (k = end; k < text.size() && std::isspace(static_cast<unsigned char>(text[k])); ++k) {}
       if (k < text.size() && (text[k] == '(' || (text[k] == '{' && name != "acc_elt"))) return false;
     } else {
@@ -343,19 +404,22 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
         o << "#define ACC_CONST_ARRAY(name) " << from.str() << "\n";
         o << "#define ACC_BLOCK " << sp.block << "\n#define ACC_BATCH " << sp.unroll << "\n#define ACC_SMALL " << acc::SCATTER_SMALL << "\n";
         std::string pre_get = sp.get, pre_perm = sp.permutation;
-        const std::set<OwnRead> reads = take_own_reads(sp.env, {&pre_get, &pre_perm});
-        std::ostringstream fields, loads, lengths;
+        std::string rest = sp.get;
+        take_own_reads(sp, {&rest}, true);
+        const std::set<OwnRead> reads = take_own_reads(sp, {&pre_get, &pre_perm});
+        std::ostringstream fields, loads, lengths, names;
         for (const OwnRead &r : reads) {
           const EnvSig &e = sp.env[r.array];
           const std::string id = std::to_string(r.array) + "_" + std::to_string(r.comp);
           fields << e.type[r.comp] << " s" << id << "; ";
+          names << "const " << e.type[r.comp] << " *const acc_own_arr" << id << " = arrIn" << id << "; (void)acc_own_arr" << id << "; ";
           loads << "(sv).s" << id << " = " << "acc_stream(arrIn" << id << ", (ix)); ";
           lengths << " && (past) <= (Int64)1";
           for (int d = e.rank - 1; d >= 0; --d) lengths << " * shIn" << r.array << "_" << d;
         }
-        o << "#define ACC_OWN_FIELDS " << fields.str() << "\n#define ACC_OWN_LOAD(sv, ix) " << loads.str() << "\n";
+        o << "#define ACC_OWN_NAMES " << names.str() << "\n#define ACC_OWN_FIELDS " << fields.str() << "\n#define ACC_OWN_LOAD(sv, ix) " << loads.str() << "\n";
         o << "#define ACC_OWN_WITHIN(past) (true" << lengths.str() << ")\n";
-        o << "#define ACC_GET_TOTAL " << (sp.preamble.empty() && only_calculates(pre_get) ? 1 : 0) << "\n";
+        o << "#define ACC_GET_TOTAL " << (sp.preamble.empty() && only_calculates(rest) ? 1 : 0) << "\n";
         o << "#define ACC_GET_OWN(ix) " << pre_get << "\n#define ACC_PERMUTATION_OWN(ix) " << pre_perm << "\n";
         tmpl = "skel_scatter.h";
         break;

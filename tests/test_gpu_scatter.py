@@ -115,3 +115,17 @@ def test_the_element_of_a_source_that_is_dropped_is_not_evaluated(A, ctx, elt, n
     if len(comps) > 1:
         want[places[kept]] = np.flatnonzero(kept) % 100
         assert np.array_equal(got[1].astype(np.int64), want)
+
+
+@pytest.mark.parametrize("n", [4000, 70001])
+def test_a_fragment_with_an_index_of_its_own(A, ctx, n):
+    """`ix` inside the lambda is not the element's index"""
+    rng = np.random.default_rng(n)
+    a, b, places = rng.integers(0, 100, n).astype(np.int32), rng.permutation(n).astype(np.int32), rng.permutation(n).astype(np.int32)
+    sk = ctx.skeleton(A.SKEL_PERMUTE, "Int32", env=[(1, "Int32")] * 3, out_rank=1, combine="x", permutation="(Int64)acc_stream(arrIn2_0, ix)",
+                      get="[&](Int64 ix) { return arrIn0_0[ix]; }((Int64)arrIn1_0[ix]) * 1000 + arrIn0_0[ix]")
+    out = ctx.empty(n, np.int32)
+    sk.permute([ctx.array(a), ctx.array(b), ctx.array(places)], n, ctx.array(np.zeros(n, np.int32)), out)
+    want = np.zeros(n, np.int32)
+    want[places] = a[b] * 1000 + a
+    assert np.array_equal(out.get(), want)

@@ -120,3 +120,54 @@ def test_which_element_functions_are_worked_out_ahead(A):
                 "({ Int32 a = arrIn0_0[ix]; while (a > 9) a -= arrIn1_0[ix]; a; })", "*(arrIn0_0 + arrIn1_0[ix])", "acc_stream(arrIn0_0, arrIn1_0[ix])"):
         assert not total(get), get
     assert not total("arrIn0_0[ix]", preamble="#define V 1")
+
+
+def _next(a):
+    return np.append(a[1:], 0)
+
+
+REBOUND = [
+    # (fragment, preamble, its value from the arrays a and b and the index i)
+    ("[&](Int64 ix) { return arrIn0_0[ix]; }((Int64)arrIn1_0[ix])", None, lambda a, b, i: a[b]),
+    ("[&](Int64 ix) { return acc_stream(arrIn0_0, ix) + arrIn1_0[ix]; }(ix / 2)", None, lambda a, b, i: a[i // 2] + b[i // 2]),
+    ("({ Int32 s = arrIn1_0[ix]; for (Int64 ix = 0; ix < 3; ++ix) s += arrIn0_0[ix]; s; })", None, lambda a, b, i: b + a[:3].sum()),
+    ("({ const unsigned char ix = 7; arrIn0_0[ix]; })", None, lambda a, b, i: 0 * i + a[7]),
+    ("({ const Int32 *arrIn0_0 = arrIn1_0; arrIn0_0[ix]; })", None, lambda a, b, i: b),
+    ("({ struct { const Int32 *arrIn0_0; } s = {arrIn1_0}; s.arrIn0_0[ix]; })", None, lambda a, b, i: b),
+    ("({ const Int32 *p = &arrIn0_0[ix]; ix + 1 < shIn0_0 ? p[1] : 0; })", None, lambda a, b, i: _next(a)),
+    ("({ auto &v = arrIn0_0[ix]; v + (3 & arrIn1_0[ix]); })", None, lambda a, b, i: a + (3 & b)),
+    ("AT(arrIn1_0[ix]) + arrIn0_0[ix]", "#define AT(i) [&](Int64 ix) { return arrIn0_0[ix]; }(i)", lambda a, b, i: a[b] + a),
+    ("not_acc_stream(arrIn0_0, ix)", "ACC_DEV Int32 not_acc_stream(const Int32 *p, Int64 ix) { return p[ix] + 1; }", lambda a, b, i: a + 1),
+]
+
+
+@pytest.mark.parametrize("fragment,preamble,value", REBOUND)
+@pytest.mark.parametrize("where", ["get", "permutation"])
+def test_names_that_a_fragment_gives_to_something_of_its_own(A, tmp_path, fragment, preamble, value, where):
+    n = 3000
+    rng = np.random.default_rng(1)
+    a, b = rng.integers(0, n, n).astype(np.int32), rng.permutation(n).astype(np.int32)
+    places, want = rng.permutation(n).astype(np.int32), np.full(n, -5, np.int32)
+    v = value(a, b, np.arange(n))
+    out = [want.copy()]
+    if where == "get":
+        scatter(A, tmp_path, "Int32", ["Int32"] * 3, [a, b, places], n, out, get=fragment, combine="x", permutation="(Int64)arrIn2_0[ix]", preamble=preamble)
+        want[places] = v
+        assert np.array_equal(out[0], want)
+    else:                                                    # (of several sources on one target any: they bring their target)
+        scatter(A, tmp_path, "Int32", ["Int32"] * 2, [a, b], n, out, get=fragment, combine="x", permutation="(Int64)(%s)" % fragment, preamble=preamble)
+        v = v[(v >= 0) & (v < n)]
+        want[v] = v
+        assert np.array_equal(out[0], want)
+
+
+def test_reads_at_the_own_index_are_taken_ahead(A):
+    """... of the fragments as the front end and the other code generators write them"""
+    def own(get, **more):
+        d = A.make_desc(A.SKEL_PERMUTE, "Int32", env=[(1, "Int32"), (2, ["Int32", "float"])], out_rank=1, get=get, combine="x", permutation="(Int64)arrIn0_0[ix]", **more)
+        return [line for line in A.preview(d)[1].splitlines() if line.startswith("#define ACC_OWN_FIELDS")][0][len("#define ACC_OWN_FIELDS"):].split()
+    assert own("arrIn0_0 [ ix ]") == ["Int32", "s0_0;"]
+    assert own("(Int32)(acc_stream( arrIn1_1 ,ix ) * 2.0f) & 3 & arrIn1_0[ix]") == ["Int32", "s0_0;", "Int32", "s1_0;", "float", "s1_1;"]
+    assert own("[&] { const Int32 v = arrIn1_0[ix]; return v * v; }()") == ["Int32", "s0_0;", "Int32", "s1_0;"]
+    assert own("arrIn1_0[ix + 1] + arrIn1_0[(ix)]") == ["Int32", "s0_0;"]
+    assert own("*(&arrIn1_0[ix])") == ["Int32", "s0_0;"] and own("1", preamble="#define V 1") == []
