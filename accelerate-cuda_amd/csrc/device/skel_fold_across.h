@@ -20,84 +20,84 @@ extern "C" __global__ void __launch_bounds__(ACC_BLOCK)
 ACC_FS_CAT_(ACC_FOLDSEG_ENTRY, ACC_ACROSS_ENTRY)(ACC_ENV_PARAMS
                                                 const Int64 shOut_0, ACC_OUT_ARRAY(arrOut),
                                                 ACC_SEG_PARAMS,
-                                                const Int64 split, ACC_ELT *__restrict__ part, int *__restrict__ part_ok,
-                                                const int chunk, const int subs ACC_GUARD_PARAM)
+                                                const Int64 acc_split, ACC_ELT *__restrict__ acc_part, int *__restrict__ acc_part_ok,
+                                                const int acc_chunk, const int acc_subs ACC_GUARD_PARAM)
 {
   ACC_GUARD_CHECK
   typedef ACC_ELT T;
-  constexpr int R = ACC_ACROSS_R;
+  constexpr int acc_R = ACC_ACROSS_R;
   ACC_ENV_ASSUME
-  auto get = ACC_GET_AT_ROW_COL;
-  auto f   = [&](const T &x, const T &y) -> T { return (ACC_COMBINE(x, y)); };
+  auto acc_get = ACC_GET_AT_ROW_COL;
+  auto acc_f   = [&](const T &x, const T &y) -> T { return (ACC_COMBINE(x, y)); };
   (void)shIn_1;
-  const Int64 rows = shOut_0, len = shIn_0;
+  const Int64 acc_rows = shOut_0, acc_len = shIn_0;
   /* (in bytes: an element type may have members with initialisers of their own) */
-  __shared__ __align__(16) unsigned char s_raw[ACC_BLOCK * R * sizeof(T)];
-  __shared__ int s_ok[ACC_BLOCK];
-  T *s_val = (T *)s_raw;
+  __shared__ __align__(16) unsigned char acc_s_raw[ACC_BLOCK * acc_R * sizeof(T)];
+  __shared__ int acc_s_ok[ACC_BLOCK];
+  T *acc_s_val = (T *)acc_s_raw;
 #if ACC_HAS_SEED
-  const T seed = (ACC_SEED);
+  const T acc_seed = (ACC_SEED);
 #else
-  const T seed = T();
+  const T acc_seed = T();
 #endif
 
-  const Int64 lanes = (rows + R - 1) / R, chunks = (lanes + chunk - 1) / chunk;
-  const int sub = (int)threadIdx.x / chunk, side = (int)threadIdx.x - sub * chunk;
-  const Int64 pieces = split * subs, piece = (len + pieces - 1) / pieces;
-  for (Int64 b = blockIdx.x; b < chunks * split; b += gridDim.x) {       /* (the same number of turns in every thread) */
-    const Int64 run = b / chunks, first = (b - run * chunks) * chunk * R + side;
-    const bool mine = sub < subs && first < rows;
-    Int64 row[R];                                        /* past the last one: that one again, not written */
+  const Int64 lanes = (acc_rows + acc_R - 1) / acc_R, chunks = (lanes + acc_chunk - 1) / acc_chunk;
+  const int sub = (int)threadIdx.x / acc_chunk, side = (int)threadIdx.x - sub * acc_chunk;
+  const Int64 pieces = acc_split * acc_subs, piece = (acc_len + pieces - 1) / pieces;
+  for (Int64 b = blockIdx.x; b < chunks * acc_split; b += gridDim.x) {       /* (the same number of turns in every thread) */
+    const Int64 run = b / chunks, first = (b - run * chunks) * acc_chunk * acc_R + side;
+    const bool mine = sub < acc_subs && first < acc_rows;
+    Int64 row[acc_R];                                        /* past the last one: that one again, not written */
 #pragma unroll
-    for (int r = 0; r < R; ++r) row[r] = acc_min<Int64>(first + r * chunk, rows - 1);
-    const Int64 k0 = acc_min<Int64>((run * subs + sub) * piece, len), k1 = acc_min<Int64>(k0 + piece, len);
-    T v[R];
+    for (int r = 0; r < acc_R; ++r) row[r] = acc_min<Int64>(first + r * acc_chunk, acc_rows - 1);
+    const Int64 k0 = acc_min<Int64>((run * acc_subs + sub) * piece, acc_len), k1 = acc_min<Int64>(k0 + piece, acc_len);
+    T v[acc_R];
     bool ok = mine && k0 < k1;
     if (ok) {
       /* (from the right a row in one piece begins with the seed, x0 (+) (x1 (+) (... (x_last (+) z))), as the other
        * entries associate a row; from the left the seed comes last) */
-      if (pieces == 1)       acc_across_piece<R, 1, ACC_FOLD_RIGHT && ACC_HAS_SEED, T>(get, f, row, k0, k1, seed, v);
-      else if (k1 - k0 >= 4) acc_across_piece<R, 2, false, T>(get, f, row, k0, k1, seed, v);
-      else                   acc_across_piece<R, 1, false, T>(get, f, row, k0, k1, seed, v);
+      if (pieces == 1)       acc_across_piece<acc_R, 1, ACC_FOLD_RIGHT && ACC_HAS_SEED, T>(acc_get, acc_f, row, k0, k1, acc_seed, v);
+      else if (k1 - k0 >= 4) acc_across_piece<acc_R, 2, false, T>(acc_get, acc_f, row, k0, k1, acc_seed, v);
+      else                   acc_across_piece<acc_R, 1, false, T>(acc_get, acc_f, row, k0, k1, acc_seed, v);
     }
     /* the pieces of a row meet: neighbours in order, then neighbours of those */
-    if (subs > 1) {
+    if (acc_subs > 1) {
       __syncthreads();                                   /* (the turn before has read) */
-      s_ok[threadIdx.x] = ok;
+      acc_s_ok[threadIdx.x] = ok;
       if (ok) {
 #pragma unroll
-        for (int r = 0; r < R; ++r) s_val[threadIdx.x * R + r] = v[r];
+        for (int r = 0; r < acc_R; ++r) acc_s_val[threadIdx.x * acc_R + r] = v[r];
       }
-      for (int apart = 1; apart < subs; apart *= 2) {
+      for (int apart = 1; apart < acc_subs; apart *= 2) {
         __syncthreads();
-        const int other = (int)threadIdx.x + apart * chunk;
-        if (sub < subs && (sub & (2 * apart - 1)) == 0 && sub + apart < subs && s_ok[other]) {
+        const int other = (int)threadIdx.x + apart * acc_chunk;
+        if (sub < acc_subs && (sub & (2 * apart - 1)) == 0 && sub + apart < acc_subs && acc_s_ok[other]) {
 #pragma unroll
-          for (int r = 0; r < R; ++r) {
-            const T w = s_val[other * R + r];
-            v[r] = ok ? f(v[r], w) : w;
-            s_val[threadIdx.x * R + r] = v[r];
+          for (int r = 0; r < acc_R; ++r) {
+            const T w = acc_s_val[other * acc_R + r];
+            v[r] = ok ? acc_f(v[r], w) : w;
+            acc_s_val[threadIdx.x * acc_R + r] = v[r];
           }
           ok = true;
-          s_ok[threadIdx.x] = 1;
+          acc_s_ok[threadIdx.x] = 1;
         }
       }
     }
     if (!mine || sub != 0) continue;
-    if (split > 1) {
+    if (acc_split > 1) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (first + r * chunk >= rows) break;
-        if (ok) part[row[r] * split + run] = v[r];
-        part_ok[row[r] * split + run] = ok;
+      for (int r = 0; r < acc_R; ++r) {
+        if (first + r * acc_chunk >= acc_rows) break;
+        if (ok) acc_part[row[r] * acc_split + run] = v[r];
+        acc_part_ok[row[r] * acc_split + run] = ok;
       }
     } else {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (first + r * chunk >= rows) break;
+      for (int r = 0; r < acc_R; ++r) {
+        if (first + r * acc_chunk >= acc_rows) break;
 #if ACC_HAS_SEED
         /* ((x0 (+) x1) (+) ... x_last) (+) z; a row in one piece from the right has its seed already */
-        ACC_PUT(arrOut, row[r], (ACC_FOLD_RIGHT && pieces == 1) ? v[r] : f(v[r], seed));
+        ACC_PUT(arrOut, row[r], (ACC_FOLD_RIGHT && pieces == 1) ? v[r] : acc_f(v[r], acc_seed));
 #else
         ACC_PUT(arrOut, row[r], v[r]);
 #endif

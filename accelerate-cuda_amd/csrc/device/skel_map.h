@@ -60,7 +60,7 @@ ACC_ENTRY(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_GUARD_PARAM)
   typedef ACC_ELT T;
   ACC_ENV_ASSUME
   /* the element at `ix`, which is column `acc_c` of row `acc_r` of the result's rows taken as one list */
-  auto get_at = [&](const Int64 ix, const Int64 acc_r, const Int64 acc_c) -> T {
+  auto acc_get_at = [&](const Int64 ix, const Int64 acc_r, const Int64 acc_c) -> T {
     __builtin_assume(ix % shOut_0 == acc_c);
     __builtin_assume(ix / shOut_0 == acc_r);
     return (ACC_GET(ix));
@@ -102,7 +102,7 @@ ACC_ENTRY(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_GUARD_PARAM)
 #pragma unroll
       for (int k = 0; k < ACC_TT; ++k)
 #pragma unroll
-        for (int i = 0; i < ACC_TT; ++i) v[i][k] = get_at(base + i * stride + k, row + i * mids, x + k);
+        for (int i = 0; i < ACC_TT; ++i) v[i][k] = acc_get_at(base + i * stride + k, row + i * mids, x + k);
 #pragma unroll
       for (int i = 0; i < ACC_TT; ++i)
 #pragma unroll
@@ -112,7 +112,7 @@ ACC_ENTRY(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_GUARD_PARAM)
       for (int i = 0; i < ACC_TT; ++i)
 #pragma unroll
         for (int k = 0; k < ACC_TT; ++k)
-          if (x + k < w && y + i < h) ACC_SET(arrOut, base + i * stride + k, get_at(base + i * stride + k, row + i * mids, x + k));
+          if (x + k < w && y + i < h) ACC_SET(arrOut, base + i * stride + k, acc_get_at(base + i * stride + k, row + i * mids, x + k));
     }
   }
 }

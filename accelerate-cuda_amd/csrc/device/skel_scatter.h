@@ -59,43 +59,43 @@ ACC_DEV decltype(auto) acc_own_value(const A &a, const I ix, const T *, const In
 
 /* Names the kernels share.  A tile that reaches past the end reads the last source there (`in`): no test per element
  * stands in front of a read. */
-#define ACC_SCATTER_NAMES                                                                                                      \
-  typedef ACC_ELT T;                                                                                                           \
-  ACC_ENV_ASSUME                                                                                                               \
-  struct own { ACC_OWN_FIELDS };                                                                                               \
-  auto get      = [&](const Int64 ix) -> T { return (ACC_GET(ix)); };                                                          \
-  auto perm     = [&](const Int64 ix) -> Int64 { return (Int64)(ACC_PERMUTATION(ix)); };                                       \
-  ACC_OWN_NAMES                                                                                                                \
-  auto get_own  = [&](const Int64 ix, const own &acc_sv) -> T { const Int64 acc_own_ix = ix; (void)acc_own_ix; (void)acc_sv; return (ACC_GET_OWN(ix)); }; \
-  auto perm_own = [&](const Int64 ix, const own &acc_sv) -> Int64 { const Int64 acc_own_ix = ix; (void)acc_own_ix; (void)acc_sv; return (Int64)(ACC_PERMUTATION_OWN(ix)); }; \
-  (void)get; (void)get_own;                                                                                                    \
-  const Int64 ntarget = (ACC_OUT_SIZE);                                                                                        \
-  const Int64 ix0 = first + (Int64)blockIdx.x * ACC_TILE + threadIdx.x;                                                        \
-  auto in = [&](const int k) -> Int64 { return acc_min<Int64>(ix0 + k * ACC_BLOCK, past - 1); };
+#define ACC_SCATTER_NAMES                                                                                                           \
+  typedef ACC_ELT T;                                                                                                                \
+  ACC_ENV_ASSUME                                                                                                                    \
+  struct acc_own { ACC_OWN_FIELDS };                                                                                                \
+  auto acc_get      = [&](const Int64 ix) -> T { return (ACC_GET(ix)); };                                                           \
+  auto acc_perm     = [&](const Int64 ix) -> Int64 { return (Int64)(ACC_PERMUTATION(ix)); };                                        \
+  ACC_OWN_NAMES                                                                                                                     \
+  auto acc_get_own  = [&](const Int64 ix, const acc_own &acc_sv) -> T { const Int64 acc_own_ix = ix; (void)acc_own_ix; (void)acc_sv; return (ACC_GET_OWN(ix)); }; \
+  auto acc_perm_own = [&](const Int64 ix, const acc_own &acc_sv) -> Int64 { const Int64 acc_own_ix = ix; (void)acc_own_ix; (void)acc_sv; return (Int64)(ACC_PERMUTATION_OWN(ix)); }; \
+  (void)acc_get; (void)acc_get_own;                                                                                                 \
+  const Int64 acc_ntarget = (ACC_OUT_SIZE);                                                                                         \
+  const Int64 acc_ix0 = acc_first + (Int64)blockIdx.x * ACC_TILE + threadIdx.x;                                                     \
+  auto acc_in = [&](const int k) -> Int64 { return acc_min<Int64>(acc_ix0 + k * ACC_BLOCK, acc_past - 1); };
 
 extern "C" __global__ void __launch_bounds__(ACC_BLOCK)
-permute_claim(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 first, const Int64 past, unsigned int *__restrict__ winner ACC_GUARD_PARAM)
+permute_claim(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 acc_first, const Int64 acc_past, unsigned int *__restrict__ acc_winner ACC_GUARD_PARAM)
 {
   ACC_GUARD_CHECK
   ACC_SCATTER_NAMES
   Int64 j[ACC_BATCH];
-  if (ACC_OWN_WITHIN(past)) {
-    own sv[ACC_BATCH];
+  if (ACC_OWN_WITHIN(acc_past)) {
+    acc_own sv[ACC_BATCH];
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) { ACC_OWN_LOAD(sv[k], in(k)) }
+    for (int k = 0; k < ACC_BATCH; ++k) { ACC_OWN_LOAD(sv[k], acc_in(k)) }
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) j[k] = perm_own(in(k), sv[k]);
+    for (int k = 0; k < ACC_BATCH; ++k) j[k] = acc_perm_own(acc_in(k), sv[k]);
   } else {
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) j[k] = perm(in(k));
+    for (int k = 0; k < ACC_BATCH; ++k) j[k] = acc_perm(acc_in(k));
   }
 #pragma unroll
   for (int k = 0; k < ACC_BATCH; ++k)
-    if (ix0 + k * ACC_BLOCK < past && j[k] >= 0 && j[k] < ntarget) winner[j[k]] = (unsigned int)(ix0 + k * ACC_BLOCK - first);
+    if (acc_ix0 + k * ACC_BLOCK < acc_past && j[k] >= 0 && j[k] < acc_ntarget) acc_winner[j[k]] = (unsigned int)(acc_ix0 + k * ACC_BLOCK - acc_first);
 }
 
 extern "C" __global__ void __launch_bounds__(ACC_BLOCK)
-permute(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 first, const Int64 past, const unsigned int *__restrict__ winner ACC_GUARD_PARAM)
+permute(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 acc_first, const Int64 acc_past, const unsigned int *__restrict__ acc_winner ACC_GUARD_PARAM)
 {
   ACC_GUARD_CHECK
   ACC_SCATTER_NAMES
@@ -107,54 +107,54 @@ permute(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 first, const Int64 past, cons
   T x[ACC_BATCH];
   bool mine[ACC_BATCH];
 #if ACC_AHEAD
-  if (ACC_OWN_WITHIN(past)) {
-    own sv[ACC_BATCH];
+  if (ACC_OWN_WITHIN(acc_past)) {
+    acc_own sv[ACC_BATCH];
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) { ACC_OWN_LOAD(sv[k], in(k)) }
+    for (int k = 0; k < ACC_BATCH; ++k) { ACC_OWN_LOAD(sv[k], acc_in(k)) }
 #pragma unroll
     for (int k = 0; k < ACC_BATCH; ++k) {
-      j[k] = perm_own(in(k), sv[k]);
-      x[k] = get_own(in(k), sv[k]);
+      j[k] = acc_perm_own(acc_in(k), sv[k]);
+      x[k] = acc_get_own(acc_in(k), sv[k]);
     }
   } else {
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) j[k] = perm(in(k));
+    for (int k = 0; k < ACC_BATCH; ++k) j[k] = acc_perm(acc_in(k));
 #pragma unroll
     for (int k = 0; k < ACC_BATCH; ++k)
-      if (j[k] >= 0 && j[k] < ntarget) x[k] = get(in(k));
+      if (j[k] >= 0 && j[k] < acc_ntarget) x[k] = acc_get(acc_in(k));
   }
 #else
-  own sv[ACC_BATCH];
-  const bool whole = ACC_OWN_WITHIN(past);
+  acc_own sv[ACC_BATCH];
+  const bool whole = ACC_OWN_WITHIN(acc_past);
   if (whole) {
     asm volatile("");          /* (a request shared with the other form would be made, and waited for, ahead of the branch) */
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) { ACC_OWN_LOAD(sv[k], in(k)) }
+    for (int k = 0; k < ACC_BATCH; ++k) { ACC_OWN_LOAD(sv[k], acc_in(k)) }
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) j[k] = perm_own(in(k), sv[k]);
+    for (int k = 0; k < ACC_BATCH; ++k) j[k] = acc_perm_own(acc_in(k), sv[k]);
   } else {
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) j[k] = perm(in(k));
+    for (int k = 0; k < ACC_BATCH; ++k) j[k] = acc_perm(acc_in(k));
   }
 #endif
 #pragma unroll
-  for (int k = 0; k < ACC_BATCH; ++k) mine[k] = ix0 + k * ACC_BLOCK < past && j[k] >= 0 && j[k] < ntarget;
+  for (int k = 0; k < ACC_BATCH; ++k) mine[k] = acc_ix0 + k * ACC_BLOCK < acc_past && j[k] >= 0 && j[k] < acc_ntarget;
   if (ACC_CLAIMED) {
     unsigned int w[ACC_BATCH];
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) w[k] = winner[mine[k] ? j[k] : 0];
+    for (int k = 0; k < ACC_BATCH; ++k) w[k] = acc_winner[mine[k] ? j[k] : 0];
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) mine[k] = mine[k] && w[k] == (unsigned int)(ix0 + k * ACC_BLOCK - first);
+    for (int k = 0; k < ACC_BATCH; ++k) mine[k] = mine[k] && w[k] == (unsigned int)(acc_ix0 + k * ACC_BLOCK - acc_first);
   }
 #if !ACC_AHEAD
   Int64 stays = -1;
-  own of_stays;
+  acc_own of_stays;
 #pragma unroll
   for (int k = ACC_BATCH - 1; k >= 0; --k) {
     const unsigned long long here = __ballot(mine[k]);
     if (here != 0ull) {
       const int lane = __builtin_ctzll(here);
-      stays = acc_readlane(in(k), lane);
+      stays = acc_readlane(acc_in(k), lane);
       of_stays = acc_readlane(sv[k], lane);
     }
   }
@@ -162,10 +162,10 @@ permute(ACC_ENV_PARAMS ACC_OUT_PARAMS, const Int64 first, const Int64 past, cons
   if (whole) {
 #pragma unroll
     for (int k = 0; k < ACC_BATCH; ++k)
-      x[k] = ACC_GET_TOTAL ? get_own(in(k), sv[k]) : get_own(mine[k] ? in(k) : stays, mine[k] ? sv[k] : of_stays);
+      x[k] = ACC_GET_TOTAL ? acc_get_own(acc_in(k), sv[k]) : acc_get_own(mine[k] ? acc_in(k) : stays, mine[k] ? sv[k] : of_stays);
   } else {
 #pragma unroll
-    for (int k = 0; k < ACC_BATCH; ++k) x[k] = get(mine[k] ? in(k) : stays);
+    for (int k = 0; k < ACC_BATCH; ++k) x[k] = acc_get(mine[k] ? acc_in(k) : stays);
   }
 #endif
 #pragma unroll
@@ -199,27 +199,27 @@ permute_fill(ACC_OUT_ARRAY(arrTo), ACC_CONST_ARRAY(arrFrom), const Int64 count A
 /* One workgroup: the defaults, a wait until they have arrived, the sources.  Below a few thousand elements a call is
  * what its launches cost. */
 extern "C" __global__ void __launch_bounds__(1024)
-permute_small(ACC_ENV_PARAMS ACC_OUT_PARAMS, ACC_CONST_ARRAY(arrFrom), const int copy, const Int64 n ACC_GUARD_PARAM)
+permute_small(ACC_ENV_PARAMS ACC_OUT_PARAMS, ACC_CONST_ARRAY(arrFrom), const int acc_copy, const Int64 acc_n ACC_GUARD_PARAM)
 {
   ACC_GUARD_CHECK
   typedef ACC_ELT T;
   ACC_ENV_ASSUME
-  __shared__ unsigned int s_winner[ACC_CLAIMED ? ACC_SMALL : 1];
-  auto get  = [&](const Int64 ix) -> T { return (ACC_GET(ix)); };
-  auto perm = [&](const Int64 ix) -> Int64 { return (Int64)(ACC_PERMUTATION(ix)); };
-  const Int64 ntarget = (ACC_OUT_SIZE);
+  __shared__ unsigned int acc_s_winner[ACC_CLAIMED ? ACC_SMALL : 1];
+  auto acc_get  = [&](const Int64 ix) -> T { return (ACC_GET(ix)); };
+  auto acc_perm = [&](const Int64 ix) -> Int64 { return (Int64)(ACC_PERMUTATION(ix)); };
+  const Int64 acc_ntarget = (ACC_OUT_SIZE);
   const int tid = (int)threadIdx.x;
   constexpr int MOST = (ACC_SMALL + 1023) / 1024;
   Int64 j[MOST];
 #pragma unroll
   for (int k = 0; k < MOST; ++k) {
     const Int64 ix = tid + k * 1024;
-    j[k] = ix < n ? perm(ix) : -1;
-    if (j[k] >= ntarget) j[k] = -1;
-    if (ACC_CLAIMED && j[k] >= 0) s_winner[j[k]] = (unsigned int)ix;
+    j[k] = ix < acc_n ? acc_perm(ix) : -1;
+    if (j[k] >= acc_ntarget) j[k] = -1;
+    if (ACC_CLAIMED && j[k] >= 0) acc_s_winner[j[k]] = (unsigned int)ix;
   }
-  if (copy) {
-#define ACC_COPY_SMALL(c, type) acc_copy_component<type>(arrOut_##c, arrFrom_##c, ntarget, tid, 1024);
+  if (acc_copy) {
+#define ACC_COPY_SMALL(c, type) acc_copy_component<type>(arrOut_##c, arrFrom_##c, acc_ntarget, tid, 1024);
     ACC_FOR_COMPONENTS(ACC_COPY_SMALL)
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       /* every wave's part has arrived before any wave stores over it */
   }
@@ -228,7 +228,7 @@ permute_small(ACC_ENV_PARAMS ACC_OUT_PARAMS, ACC_CONST_ARRAY(arrFrom), const int
   for (int k = 0; k < MOST; ++k) {
     const Int64 ix = tid + k * 1024;
     if (j[k] < 0) continue;
-    if (ACC_CLAIMED && s_winner[j[k]] != (unsigned int)ix) continue;
-    ACC_SET(arrOut, j[k], get(ix));
+    if (ACC_CLAIMED && acc_s_winner[j[k]] != (unsigned int)ix) continue;
+    ACC_SET(arrOut, j[k], acc_get(ix));
   }
 }

@@ -115,67 +115,67 @@ stencil(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk ACC_GU
   ACC_GUARD_CHECK
   typedef ACC_ELT T;
   ACC_ENV_ASSUME
-  const int d = (int)shOut_2, h = (int)shOut_1, w = (int)shOut_0;
+  const int acc_d = (int)shOut_2, acc_h = (int)shOut_1, acc_w = (int)shOut_0;
   /* (the driver counts the waves by the same numbers, all of them within 32 bits) */
-  const unsigned int vectors = ((unsigned int)w + ACC_SVEC - 1) / ACC_SVEC, bands = ((unsigned int)h + ACC_TZ - 1) / ACC_TZ;
-  const unsigned int per_plane = vectors * bands, waves = (per_plane + ACC_WAVE - 1) / ACC_WAVE;
-  const unsigned int number = (unsigned int)acc_xcd_contiguous_block() * (ACC_BLOCK / ACC_WAVE) +
+  const unsigned int acc_vectors = ((unsigned int)acc_w + ACC_SVEC - 1) / ACC_SVEC, acc_bands = ((unsigned int)acc_h + ACC_TZ - 1) / ACC_TZ;
+  const unsigned int acc_per_plane = acc_vectors * acc_bands, acc_waves = (acc_per_plane + ACC_WAVE - 1) / ACC_WAVE;
+  const unsigned int acc_number = (unsigned int)acc_xcd_contiguous_block() * (ACC_BLOCK / ACC_WAVE) +
                               (unsigned int)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const unsigned int run = number / waves;
-  const int z0 = (int)run * acc_walk;
-  if (z0 >= d) return;                                   /* whole wave leaves together */
-  const int planes = acc_min(acc_walk, d - z0);
+  const unsigned int acc_run = acc_number / acc_waves;
+  const int acc_z0 = (int)acc_run * acc_walk;
+  if (acc_z0 >= acc_d) return;                                   /* whole wave leaves together */
+  const int acc_planes = acc_min(acc_walk, acc_d - acc_z0);
   /* (lanes beyond the last vector of a plane do the last one again) */
-  const unsigned int id = acc_min<unsigned int>((number - run * waves) * ACC_WAVE + (unsigned int)acc_lane(), per_plane - 1);
-  const int y = (int)(id / vectors) * ACC_TZ;
-  const int x = acc_min((int)(id % vectors) * ACC_SVEC, w - ACC_SVEC);
+  const unsigned int acc_id = acc_min<unsigned int>((acc_number - acc_run * acc_waves) * ACC_WAVE + (unsigned int)acc_lane(), acc_per_plane - 1);
+  const int acc_y = (int)(acc_id / acc_vectors) * ACC_TZ;
+  const int acc_x = acc_min((int)(acc_id % acc_vectors) * ACC_SVEC, acc_w - ACC_SVEC);
 
-#define ACC_DECLARE_A(c, CT, OUTSIDE, arg)                                         \
-  acc_flat_source<CT, ACC_BOUNDARY> a##c;                                          \
-  a##c.base = (const char *)arrStencil_##c;                                        \
-  a##c.plane_bytes = (Int64)h * w * (Int64)sizeof(CT);                             \
-  a##c.d = d; a##c.z0 = z0; a##c.outside = (CT)OUTSIDE;                            \
-  a##c.place(x, y, w, h);
+#define ACC_DECLARE_A(c, CT, OUTSIDE, arg)                                                          \
+  acc_flat_source<CT, ACC_BOUNDARY> acc_a##c;                                                       \
+  acc_a##c.base = (const char *)arrStencil_##c;                                                     \
+  acc_a##c.plane_bytes = (Int64)acc_h * acc_w * (Int64)sizeof(CT);                                  \
+  acc_a##c.d = acc_d; acc_a##c.z0 = acc_z0; acc_a##c.outside = (CT)OUTSIDE;                         \
+  acc_a##c.place(acc_x, acc_y, acc_w, acc_h);
   ACC_SRC1_COMPONENTS(ACC_DECLARE_A, 0)
 #undef ACC_DECLARE_A
-#define ACC_CALL_A(c, CT, OUTSIDE, call) a##c.call;
+#define ACC_CALL_A(c, CT, OUTSIDE, call) acc_a##c.call;
 #define ACC_EACH(call) do { ACC_SRC1_COMPONENTS(ACC_CALL_A, call) } while (0)
 
-  const int total = planes + 2 * ACC_RADIUS_Z;
+  const int acc_total = acc_planes + 2 * ACC_RADIUS_Z;
 #pragma unroll
-  for (int rho = 0; rho < ACC_RING - 1; ++rho) ACC_EACH(fetch(acc_min(rho, total - 1), rho));
+  for (int acc_rho = 0; acc_rho < ACC_RING - 1; ++acc_rho) ACC_EACH(fetch(acc_min(acc_rho, acc_total - 1), acc_rho));
   __builtin_amdgcn_sched_barrier(0);                     /* (every request ahead of anything that waits for one) */
 
-  for (int zb = 0; zb < planes; zb += ACC_RING) {
+  for (int acc_zb = 0; acc_zb < acc_planes; acc_zb += ACC_RING) {
 #pragma unroll
-    for (int s = 0; s < ACC_RING; ++s) {
-      const int z = zb + s;
-      if (z < planes) {
+    for (int acc_s = 0; acc_s < ACC_RING; ++acc_s) {
+      const int acc_z = acc_zb + acc_s;
+      if (acc_z < acc_planes) {
         /* asked for without a test -- a load under a condition is waited for on the spot: past the end of the run the
          * last plane again, into a slot nothing reads any more */
-        ACC_EACH(fetch(acc_min(z + ACC_RING - 1, total - 1), (s + ACC_RING - 1) % ACC_RING));
+        ACC_EACH(fetch(acc_min(acc_z + ACC_RING - 1, acc_total - 1), (acc_s + ACC_RING - 1) % ACC_RING));
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int py = 0; py < ACC_TZ; ++py) {
-          acc_out_vec res;
+        for (int acc_py = 0; acc_py < ACC_TZ; ++acc_py) {
+          acc_out_vec acc_res;
 #pragma unroll
-          for (int k = 0; k < ACC_SVEC; ++k) {
-#define ACC_WINDOW_READ(c, dz, dy, dx) a##c.ring[py + ACC_RADIUS_Y + (dy)][(s + ACC_RADIUS_Z + (dz)) % ACC_RING].e[ACC_RADIUS_X + k + (dx)]
+          for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) {
+#define ACC_WINDOW_READ(c, dz, dy, dx) acc_a##c.ring[acc_py + ACC_RADIUS_Y + (dy)][(acc_s + ACC_RADIUS_Z + (dz)) % ACC_RING].e[ACC_RADIUS_X + acc_k + (dx)]
             ACC_STENCIL_TAPS1(ACC_WINDOW_READ)
 #undef ACC_WINDOW_READ
-            res.v[k] = (T)(ACC_STENCIL_FN);
+            acc_res.v[acc_k] = (T)(ACC_STENCIL_FN);
           }
-          if (ACC_TZ > 1 && y + py >= h) continue;       /* the last band of rows may be short */
-#define ACC_STORE_COMPONENT(c, CT)                                                   \
-          {                                                                          \
-            typedef CT acc_out_native __attribute__((ext_vector_type(ACC_SVEC)));    \
+          if (ACC_TZ > 1 && acc_y + acc_py >= acc_h) continue;       /* the last band of rows may be short */
+#define ACC_STORE_COMPONENT(c, CT)                                                                  \
+          {                                                                                         \
+            typedef CT acc_out_native __attribute__((ext_vector_type(ACC_SVEC)));                   \
             typedef acc_out_native acc_out_stored __attribute__((aligned(ACC_ALIGNED ? ACC_SVEC * sizeof(CT) : alignof(CT)))); \
-            char *plane = (char *)arrOut_##c + (Int64)(z0 + z) * ((Int64)h * w * (Int64)sizeof(CT)); \
-            const unsigned int at = ((unsigned int)(y + py) * (unsigned int)w + (unsigned int)x) * (unsigned int)sizeof(CT); \
-            acc_out_native nv;                                                       \
-            _Pragma("unroll") for (int k = 0; k < ACC_SVEC; ++k) nv[k] = ACC_COMPONENT(res.v[k], c); \
+            char *plane = (char *)arrOut_##c + (Int64)(acc_z0 + acc_z) * ((Int64)acc_h * acc_w * (Int64)sizeof(CT)); \
+            const unsigned int at = ((unsigned int)(acc_y + acc_py) * (unsigned int)acc_w + (unsigned int)acc_x) * (unsigned int)sizeof(CT); \
+            acc_out_native nv;                                                                      \
+            _Pragma("unroll") for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) nv[acc_k] = ACC_COMPONENT(acc_res.v[acc_k], c); \
             if (ACC_STENCIL_NT & 1) __builtin_nontemporal_store(nv, (acc_out_stored *)(plane + at)); \
-            else                    *(acc_out_stored *)(plane + at) = nv;            \
+            else                    *(acc_out_stored *)(plane + at) = nv;                           \
           }
           ACC_FOR_COMPONENTS(ACC_STORE_COMPONENT)
 #undef ACC_STORE_COMPONENT

@@ -61,52 +61,52 @@ stencil(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk ACC_GU
   typedef ACC_ELT T;
   ACC_ENV_ASSUME
   (void)acc_walk;
-  const int h = (int)shOut_1, w = (int)shOut_0;
-  const int lane = acc_lane();
-  const unsigned int strips = ((unsigned int)w + ACC_OWNED * ACC_SVEC - 1) / (ACC_OWNED * ACC_SVEC);
-  const unsigned int number = (unsigned int)acc_xcd_contiguous_block() * (ACC_BLOCK / ACC_WAVE) +
+  const int acc_h = (int)shOut_1, acc_w = (int)shOut_0;
+  const int acc_me = acc_lane();
+  const unsigned int acc_strips = ((unsigned int)acc_w + ACC_OWNED * ACC_SVEC - 1) / (ACC_OWNED * ACC_SVEC);
+  const unsigned int acc_number = (unsigned int)acc_xcd_contiguous_block() * (ACC_BLOCK / ACC_WAVE) +
                               (unsigned int)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const int y0 = (int)(number / strips) * ACC_TILE_H;
-  if (y0 >= h) return;                                   /* whole wave leaves together */
+  const int acc_y0 = (int)(acc_number / acc_strips) * ACC_TILE_H;
+  if (acc_y0 >= acc_h) return;                                   /* whole wave leaves together */
   /* the last strip ends at the right edge, and the one before it leaves a whole vector for its outermost lane: the
    * outermost lanes are inside the array, or outside, with all their columns */
-  const int nth = (int)(number % strips), last_x0 = w - ACC_OWNED * ACC_SVEC;
-  const int x0 = nth == (int)strips - 1 ? last_x0 : acc_min(nth * (ACC_OWNED * ACC_SVEC), last_x0 - ACC_SVEC);
-  const int gx = x0 + (lane - 1) * ACC_SVEC;             /* this lane's first column */
+  const int acc_nth = (int)(acc_number % acc_strips), acc_last_x0 = acc_w - ACC_OWNED * ACC_SVEC;
+  const int acc_x0 = acc_nth == (int)acc_strips - 1 ? acc_last_x0 : acc_min(acc_nth * (ACC_OWNED * ACC_SVEC), acc_last_x0 - ACC_SVEC);
+  const int acc_gx = acc_x0 + (acc_me - 1) * ACC_SVEC;             /* this lane's first column */
   /* where it reads: its own columns; outside the array the other end of the row, or the nearest vector inside */
-  const int from = ACC_BOUNDARY == ACC_B_WRAP ? (gx < 0 ? gx + w : (gx >= w ? gx - w : gx)) : acc_max(0, acc_min(gx, w - ACC_SVEC));
-  const bool at_left = gx == 0, at_right = gx + ACC_SVEC == w;
+  const int acc_from = ACC_BOUNDARY == ACC_B_WRAP ? (acc_gx < 0 ? acc_gx + acc_w : (acc_gx >= acc_w ? acc_gx - acc_w : acc_gx)) : acc_max(0, acc_min(acc_gx, acc_w - ACC_SVEC));
+  const bool acc_at_left = acc_gx == 0, acc_at_right = acc_gx + ACC_SVEC == acc_w;
 #define ACC_OUTSIDE_OF(c, CT, OUTSIDE, arg) const T acc_outside = (T)OUTSIDE;
   ACC_SRC1_COMPONENTS(ACC_OUTSIDE_OF, 0)
 #undef ACC_OUTSIDE_OF
 
-  auto load = [&](const int y) -> acc_pair_own {         /* y inside the array */
+  auto acc_load = [&](const int y) -> acc_pair_own {         /* y inside the array */
     struct __attribute__((aligned(ACC_ALIGNED ? ACC_SVEC * sizeof(T) : alignof(T)))) vec { T v[ACC_SVEC]; };
-    const vec own = *(const vec *)(arrStencil_0 + (Int64)y * w + from);
+    const vec own = *(const vec *)(arrStencil_0 + (Int64)y * acc_w + acc_from);
     acc_pair_own r;
 #pragma unroll
-    for (int k = 0; k < ACC_SVEC; ++k) r.v[k] = own.v[k];
+    for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) r.v[acc_k] = own.v[acc_k];
     return r;
   };
-  auto all_outside = [&]() -> acc_pair_own {
+  auto acc_all_outside = [&]() -> acc_pair_own {
     acc_pair_own r;
 #pragma unroll
-    for (int k = 0; k < ACC_SVEC; ++k) r.v[k] = acc_outside;
+    for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) r.v[acc_k] = acc_outside;
     return r;
   };
   /* a row with the columns beside each lane's own */
-  auto widen = [&](const acc_pair_own &own, auto xedge_c) -> acc_pair_row {
+  auto acc_widen = [&](const acc_pair_own &own, auto xedge_c) -> acc_pair_row {
     constexpr bool xedge = decltype(xedge_c)::value && ACC_BOUNDARY != ACC_B_WRAP;
     acc_pair_row r;
 #pragma unroll
-    for (int k = 0; k < ACC_SVEC; ++k) r.e[ACC_RX + k] = own.v[k];
+    for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) r.e[ACC_RX + acc_k] = own.v[acc_k];
     if (ACC_RX > 0) {
       T l = acc_wave_shift_up1(own.v[ACC_SVEC - 1]), t = acc_dpp<ACC_DPP_WAVE_SHL1, 0xf>(own.v[0], own.v[0]);
       if (xedge) {
         const T beyond_l = ACC_BOUNDARY == ACC_B_CONSTANT ? acc_outside : own.v[ACC_BOUNDARY == ACC_B_MIRROR ? 1 : 0];
         const T beyond_r = ACC_BOUNDARY == ACC_B_CONSTANT ? acc_outside : own.v[ACC_BOUNDARY == ACC_B_MIRROR ? ACC_SVEC - 2 : ACC_SVEC - 1];
-        l = at_left ? beyond_l : l;
-        t = at_right ? beyond_r : t;
+        l = acc_at_left ? beyond_l : l;
+        t = acc_at_right ? beyond_r : t;
       }
       r.e[0] = l;
       r.e[ACC_WW - 1] = t;
@@ -114,40 +114,40 @@ stencil(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk ACC_GU
     return r;
   };
   /* one application: rows[0 .. 2 ry] are the rows it reads */
-  auto apply = [&](const acc_pair_row (&rows)[ACC_NR]) -> acc_pair_own {
-    acc_pair_own res;
+  auto acc_apply = [&](const acc_pair_row (&acc_rows)[ACC_NR]) -> acc_pair_own {
+    acc_pair_own acc_res;
 #pragma unroll
-    for (int k = 0; k < ACC_SVEC; ++k) {
-#define ACC_WINDOW_READ(c, dz, dy, dx) rows[ACC_RY + (dy)].e[ACC_RX + k + (dx)]
+    for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) {
+#define ACC_WINDOW_READ(c, dz, dy, dx) acc_rows[ACC_RY + (dy)].e[ACC_RX + acc_k + (dx)]
       ACC_STENCIL_TAPS1(ACC_WINDOW_READ)
 #undef ACC_WINDOW_READ
-      res.v[k] = (T)(ACC_STENCIL_FN);
+      acc_res.v[acc_k] = (T)(ACC_STENCIL_FN);
     }
-    return res;
+    return acc_res;
   };
-  auto store = [&](const int y, const acc_pair_own &res) {
-    if (lane == 0 || lane == ACC_WAVE - 1) return;
+  auto acc_put = [&](const int y, const acc_pair_own &acc_res) {
+    if (acc_me == 0 || acc_me == ACC_WAVE - 1) return;
     typedef T acc_out_native __attribute__((ext_vector_type(ACC_SVEC)));
     typedef acc_out_native acc_out_stored __attribute__((aligned(ACC_ALIGNED ? ACC_SVEC * sizeof(T) : alignof(T))));
     acc_out_native nv;
 #pragma unroll
-    for (int k = 0; k < ACC_SVEC; ++k) nv[k] = res.v[k];
-    acc_out_stored *dst = (acc_out_stored *)(arrOut_0 + (Int64)y * w + gx);
+    for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) nv[acc_k] = acc_res.v[acc_k];
+    acc_out_stored *dst = (acc_out_stored *)(arrOut_0 + (Int64)y * acc_w + acc_gx);
     if (ACC_STENCIL_NT & 1) __builtin_nontemporal_store(nv, dst);
     else                    *dst = nv;
   };
 
-  auto run = [&](auto xedge_c, auto yedge_c) {
+  auto acc_run = [&](auto xedge_c, auto yedge_c) {
     constexpr bool yedge = decltype(yedge_c)::value;
     constexpr int READ_ROWS = ACC_TILE_H + 4 * ACC_RY, MID_ROWS = ACC_TILE_H + 2 * ACC_RY;
     acc_pair_own src[READ_ROWS];
     acc_pair_row above[ACC_NR], between[ACC_NR];
     if (!yedge) {
 #pragma unroll
-      for (int i = 0; i < READ_ROWS; ++i) src[i] = load(y0 - 2 * ACC_RY + i);
+      for (int i = 0; i < READ_ROWS; ++i) src[i] = acc_load(acc_y0 - 2 * ACC_RY + i);
       __builtin_amdgcn_sched_barrier(0);                 /* (every request ahead of anything that waits for one) */
 #pragma unroll
-      for (int i = 0; i < ACC_NR - 1; ++i) above[i + 1] = widen(src[i], xedge_c);
+      for (int i = 0; i < ACC_NR - 1; ++i) above[i + 1] = acc_widen(src[i], xedge_c);
     }
 #pragma unroll
     for (int m = 0; m < MID_ROWS; ++m) {
@@ -155,28 +155,28 @@ stencil(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk ACC_GU
       if (!yedge) {
 #pragma unroll
         for (int i = 0; i < ACC_NR - 1; ++i) above[i] = above[i + 1];
-        above[ACC_NR - 1] = widen(src[m + ACC_NR - 1], xedge_c);
-        mid = apply(above);
+        above[ACC_NR - 1] = acc_widen(src[m + ACC_NR - 1], xedge_c);
+        mid = acc_apply(above);
       } else {
         /* the row in between that the boundary condition puts here, and the rows that one is made of */
-        const int want = y0 - ACC_RY + m, at = acc_pair_boundary(want, h);
+        const int want = acc_y0 - ACC_RY + m, at = acc_pair_boundary(want, acc_h);
 #pragma unroll
         for (int i = 0; i < ACC_NR; ++i) {
           const int y = at - ACC_RY + i;
-          const acc_pair_own read = load(acc_pair_boundary(y, h));
-          above[i] = widen((ACC_BOUNDARY == ACC_B_CONSTANT && (y < 0 || y >= h)) ? all_outside() : read, xedge_c);
+          const acc_pair_own read = acc_load(acc_pair_boundary(y, acc_h));
+          above[i] = acc_widen((ACC_BOUNDARY == ACC_B_CONSTANT && (y < 0 || y >= acc_h)) ? acc_all_outside() : read, xedge_c);
         }
-        mid = apply(above);
-        if (ACC_BOUNDARY == ACC_B_CONSTANT && (want < 0 || want >= h)) mid = all_outside();
+        mid = acc_apply(above);
+        if (ACC_BOUNDARY == ACC_B_CONSTANT && (want < 0 || want >= acc_h)) mid = acc_all_outside();
       }
 #pragma unroll
       for (int i = 0; i < ACC_NR - 1; ++i) between[i] = between[i + 1];
-      between[ACC_NR - 1] = widen(mid, xedge_c);
-      const int y = y0 + m - 2 * ACC_RY;
-      if (m >= 2 * ACC_RY && (!yedge || y < h)) store(y, apply(between));
+      between[ACC_NR - 1] = acc_widen(mid, xedge_c);
+      const int y = acc_y0 + m - 2 * ACC_RY;
+      if (m >= 2 * ACC_RY && (!yedge || y < acc_h)) acc_put(y, acc_apply(between));
     }
   };
-  if (y0 < 2 * ACC_RY || y0 + ACC_TILE_H + 2 * ACC_RY > h) run(acc_bool<true>(), acc_bool<true>());
-  else if (x0 < ACC_SVEC || x0 + (ACC_OWNED + 1) * ACC_SVEC > w) run(acc_bool<true>(), acc_bool<false>());
-  else run(acc_bool<false>(), acc_bool<false>());
+  if (acc_y0 < 2 * ACC_RY || acc_y0 + ACC_TILE_H + 2 * ACC_RY > acc_h) acc_run(acc_bool<true>(), acc_bool<true>());
+  else if (acc_x0 < ACC_SVEC || acc_x0 + (ACC_OWNED + 1) * ACC_SVEC > acc_w) acc_run(acc_bool<true>(), acc_bool<false>());
+  else acc_run(acc_bool<false>(), acc_bool<false>());
 }

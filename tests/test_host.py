@@ -122,6 +122,35 @@ def test_variants_by_shape_of_scans_stencils_and_maps_compile(A, tmp_path):
     assert "#define ACC_MAP_TILED 0" in A.preview(vector, 0)[1]
 
 
+def test_templates_leave_a_preamble_its_names(A, tmp_path):
+    """a description may declare functions of its own; what a template calls its parameters and locals where a fragment
+    stands must not hide them (the names below are ones that the form of the instance for any other shape takes)"""
+    A.lib().acc_cache_set_dir(str(tmp_path).encode())
+    nine = [(a, b) for a in (-1, 0, 1) for b in (-1, 0, 1)]
+    seven = [(0, 0, 0), (-1, 0, 0), (1, 0, 0), (0, -1, 0), (0, 1, 0), (0, 0, -1), (0, 0, 1)]
+
+    def check(names, variants, **d):
+        names = names.split()
+        pre = " ".join("ACC_DEV Int32 %s(Int32 v) { return v; }" % n for n in names)
+        calls = "%s%%s%s" % ("".join(n + "(" for n in names), ")" * len(names))
+        desc = A.make_desc(preamble=pre, **{k: v.replace("CALL", calls % "1") if isinstance(v, str) else v for k, v in d.items()})
+        for v in variants:
+            assert A.compile_source(A.preview(desc, v)[1]) > 2000, (d, v)
+
+    I = (1, "Int32")
+    scatter = "own get perm get_own perm_own ntarget ix0 in first past winner copy n s_winner tid"
+    check(scatter, (0, 1), kind=A.SKEL_PERMUTE, elt="Int32", env=[I, I], out_rank=1, get="arrIn0_0[ix] + CALL", combine="x", permutation="(Int64)arrIn1_0[ix] * CALL")
+    check(scatter, (0,), kind=A.SKEL_PERMUTE, elt="Int32, Int8", env=[I, I], out_rank=1, get="acc_elt{arrIn0_0[ix], (Int8)CALL}", combine="acc_elt{x.a1, x.a0}",
+          permutation="(Int64)arrIn1_0[ix] * CALL")
+    check("strips number nth last_x0 from at_left at_right load all_outside widen apply store", (0, 1, 2, 4, 6, 10, 11), kind=A.SKEL_STENCIL, elt="Int32", out_rank=2, taps=nine,
+          boundary="constant", boundary_constant="CALL", stencil_fn="t0 + t1 + CALL * t8")
+    check("vectors per_plane waves number planes id x rho zb z py", (0, 1, 2, 4, 6, 8, 9), kind=A.SKEL_STENCIL, elt="Int32", out_rank=3, taps=seven,
+          boundary="constant", boundary_constant="CALL", stencil_fn="t0 + t1 + CALL * t6")
+    check("s_raw s_ok R chunk subs lanes chunks", (0, 1), kind=A.SKEL_FOLD, elt="Int32", env=[(2, "Int32")], out_rank=1, flags=A.FLAG_TILED,
+          get="arrIn0_0[acc_col * shIn0_0 + acc_row] + CALL", combine="x + CALL * y", seed="CALL")
+    check("get_at", (0, 1, 2, 3), kind=A.SKEL_MAP, elt="Int32", env=[(2, "Int32")], out_rank=2, flags=A.FLAG_TILED, get="arrIn0_0[(ix % shOut_0) * shIn0_0 + (ix / shOut_0)] + CALL")
+
+
 def test_every_scalar_primitive_compiles_for_every_type(A, tmp_path):
     """acc_prim.h: one map per element type naming every primitive that type has
     (CodeGen.hs:406-476); what they compute is checked on the GPU"""

@@ -137,6 +137,7 @@ REBOUND = [
     ("({ const Int32 *p = &arrIn0_0[ix]; ix + 1 < shIn0_0 ? p[1] : 0; })", None, lambda a, b, i: _next(a)),
     ("({ auto &v = arrIn0_0[ix]; v + (3 & arrIn1_0[ix]); })", None, lambda a, b, i: a + (3 & b)),
     ("AT(arrIn1_0[ix]) + arrIn0_0[ix]", "#define AT(i) [&](Int64 ix) { return arrIn0_0[ix]; }(i)", lambda a, b, i: a[b] + a),
+    ("arrIn0_0[ix] + first * past + copy", "static const Int32 first = 2, past = 3, copy = 4;", lambda a, b, i: a + 10),
     ("not_acc_stream(arrIn0_0, ix)", "ACC_DEV Int32 not_acc_stream(const Int32 *p, Int64 ix) { return p[ix] + 1; }", lambda a, b, i: a + 1),
 ]
 
