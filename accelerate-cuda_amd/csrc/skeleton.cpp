@@ -987,7 +987,7 @@ using acc::fail;
 // ---- acc_skel_s ----------------------------------------------------------------
 
 namespace acc {
-// what variant v of an instance is generated from (variants beyond 1 exist for permute only)
+// what variant v of an instance is generated from
 SkelSpec spec_of_variant(const SkelSpec &base, int v)
 {
   SkelSpec spec = base;
@@ -1205,6 +1205,18 @@ static int variant_count(const acc::SkelSpec &sp)
   return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : sp.pair_rows > 0 ? 12 : sp.flat_rows > 0 ? 10 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
 }
 
+// ... one of which is left out: of a 2-D stencil with two applications a launch (10 and 11) the form that 3-D ones have at 8 and 9
+static bool variant_exists(const acc::SkelSpec &sp, int v)
+{
+  return v >= 0 && v < variant_count(sp) && !(sp.pair_rows > 0 && (v == 8 || v == 9));
+}
+
+static int no_such_variant(const char *who, const acc::SkelSpec &sp)
+{
+  if (!variant_exists(sp, 8) && variant_exists(sp, 10)) return fail(ACC_ERR_INVALID, "%s: this kind of skeleton has variants 0 to 7, 10 and 11", who);
+  return fail(ACC_ERR_INVALID, "%s: this kind of skeleton has variants 0 to %d", who, variant_count(sp) - 1);
+}
+
 extern "C" {
 
 int acc_skel_create_async(acc_context ctx, const acc_skel_desc *desc, acc_skel *out)
@@ -1240,8 +1252,7 @@ int acc_skel_create(acc_context ctx, const acc_skel_desc *desc, acc_skel *out)
 int acc_skel_prefetch(acc_skel s, int variant)
 {
   if (!s) return fail(ACC_ERR_INVALID, "acc_skel_prefetch: NULL skeleton");
-  if (variant < 0 || variant >= variant_count(s->spec))
-    return fail(ACC_ERR_INVALID, "acc_skel_prefetch: this kind of skeleton has variants 0 to %d", variant_count(s->spec) - 1);
+  if (!variant_exists(s->spec, variant)) return no_such_variant("acc_skel_prefetch", s->spec);
   // (the locked form of a permute is only generated for elements the atomic template does not take, and the other way round)
   if (s->spec.kind == ACC_SKEL_PERMUTE && s->spec.permute_locked && variant >= 2)
     return fail(ACC_ERR_INVALID, "acc_skel_prefetch: a permute under locks has variants 0 and 1");
@@ -1304,13 +1315,10 @@ int acc_skel_source(acc_skel s, int variant, const char **source)
 int acc_skel_preview(const acc_skel_desc *desc, int variant, const char **source, const char **entry)
 {
   static thread_local std::string text, name;
-  if (!source || variant < 0 || variant > 11) return fail(ACC_ERR_INVALID, "acc_skel_preview: bad argument");
+  if (!source || variant < 0) return fail(ACC_ERR_INVALID, "acc_skel_preview: bad argument");
   acc::SkelSpec sp;
   ACC_TRY(acc::make_spec(desc, acc::default_tuning(), &sp));
-  // beyond 1: a permute's forms (to 7), a stencil's fewer columns a lane (to 5), a scan's small tiles and a segmented
-  // fold's longer chunk (2 and 3)
-  const int most = variant_count(sp) - 1;
-  if (variant > most) return fail(ACC_ERR_INVALID, "acc_skel_preview: this kind of skeleton has variants 0 to %d", most);
+  if (!variant_exists(sp, variant)) return no_such_variant("acc_skel_preview", sp);
   ACC_TRY(acc::generate_source(acc::spec_of_variant(sp, variant), (variant & 1) == 0, &name, &text));
   *source = text.c_str();
   if (entry) *entry = name.c_str();

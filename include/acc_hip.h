@@ -408,12 +408,17 @@ int acc_skel_source(acc_skel s, int variant, const char **source);
  * string stays valid until the calling thread's next call of this function.
  * A permute has further forms the driver chooses between by the number of
  * targets, at variant + 2 (tables under locks in LDS), + 4 (several LDS
- * windows of targets), + 6 (16-bit counts in LDS, integer addition); a scan
- * its small tiles and a segmented fold its longer staged chunk at + 2; a
- * segmented fold of a vector the forms that hand segments far longer than
- * the rest over to a second launch at + 4; a stencil half and a quarter of
- * the columns a lane at + 2 and + 4, and an element a thread (for arrays of
- * a few columns) at + 6; a map in tiles the map in runs at + 2                */
+ * windows of targets), + 6 (16-bit counts in LDS, integer addition), but for
+ * one that stores the new values (`combine`); a scan its small tiles at + 2 and
+ * tiles between those and the full ones at + 4, a segmented fold its longer
+ * staged chunk at + 2; a segmented fold of a vector the forms that hand
+ * segments far longer than the rest over to a second launch at + 4; a stencil
+ * half and a quarter of the columns a lane at + 2 and + 4, an element a thread
+ * (for arrays of a few columns) at + 6, one in three dimensions lanes over the
+ * vectors of a whole plane at + 8 (where its windows allow), one in two
+ * dimensions two applications a launch at + 10 (where acc_exec_stencil_iterate
+ * may make them); a map in tiles the map in runs at + 2.  A variant that an
+ * instance does not have is ACC_ERR_INVALID.                                  */
 int acc_skel_preview(const acc_skel_desc *desc, int variant, const char **source, const char **entry);
 /* compile only (no GPU needed): used by the build check */
 int acc_skel_compile_only(const char *target, const acc_skel_desc *desc, size_t *code_size);

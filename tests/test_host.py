@@ -122,6 +122,35 @@ def test_variants_by_shape_of_scans_stencils_and_maps_compile(A, tmp_path):
     assert "#define ACC_MAP_TILED 0" in A.preview(vector, 0)[1]
 
 
+def test_every_variant_there_is_compiles_and_no_other_is_accepted(A, tmp_path):
+    A.lib().acc_cache_set_dir(str(tmp_path).encode())
+    cross = [(-1, 0), (0, -1), (0, 0), (0, 1), (1, 0)]
+    star = [(0, 0, 0), (-1, 0, 0), (1, 0, 0), (0, -1, 0), (0, 1, 0), (0, 0, -1), (0, 0, 1)]
+    I = (1, "Int32")
+
+    def stencil(taps, rank, elt="Int32", **more):
+        return A.make_desc(A.SKEL_STENCIL, elt, out_rank=rank, taps=taps, boundary="clamp", stencil_fn=" + ".join("t%d" % k for k in range(len(taps))), **more)
+    cases = [
+        (stencil(cross, 2), list(range(8)) + [10, 11]),
+        (stencil(cross, 2, elt="Int8"), range(8)), (stencil([(0, -1), (0, 0)], 1), range(8)),
+        (stencil(star, 3), range(10)), (stencil(star, 3, elt="Int8"), range(8)), (stencil([(0, 0, 0), (0, 1, 0)], 3), range(8)),
+        (A.make_desc(A.SKEL_SCANL1, "Int32", env=[I], get="arrIn0_0[ix]", combine="x + y"), range(6)),
+        (A.make_desc(A.SKEL_PERMUTE, "Int32", env=[I], out_rank=1, get="1", combine="x", permutation="(Int64)arrIn0_0[ix]"), range(2)),
+        (A.make_desc(A.SKEL_MAP, "Int32", env=[I], out_rank=1, get="arrIn0_0[ix]"), range(2)),
+    ]
+    wide = stencil([(0, -2), (0, 0)], 2)                # (accepted, but not taken: fewer columns a lane than the taps reach)
+    for desc, there in cases + [(wide, range(8))]:
+        for v in range(-1, 14):
+            if v in there and desc is wide:
+                A.preview(desc, v)
+            elif v in there:
+                assert A.compile_source(A.preview(desc, v)[1]) > 2000, (desc.kind, v)
+            else:
+                with pytest.raises(A.AccError) as e:
+                    A.preview(desc, v)
+                assert e.value.code == A.ERR_INVALID
+
+
 def test_templates_leave_a_preamble_its_names(A, tmp_path):
     """a description may declare functions of its own; what a template calls its parameters and locals where a fragment
     stands must not hide them (the names below are ones that the form of the instance for any other shape takes)"""
