@@ -520,12 +520,13 @@ ACC_FS_CAT_(ACC_FOLDSEG_ENTRY, _rows)(ACC_ENV_PARAMS
   }
 }
 
+#if ACC_ACROSS_ROWS > 0
 /* ---- rows that lie across memory: neighbouring rows in neighbouring lanes, whatever the length ------
  * <entry>_across and <entry>_across_wide (skel_fold_across.h, a row and several rows a lane), for an element function
  * that, where the ROW index moves by one, reads neighbouring addresses -- the fold of a transposed matrix (sums down its
  * columns), of a matrix product written as a fold over `zipWith (*)` of two replicated operands, one of them transposed
  * (ACC_FLAG_TILED says so: the host cannot see it).  A team of lanes along such a row asks for 64 cache lines with every
- * load.                                                                                                        */
+ * load.  Only instances that launch them have them (ACC_ACROSS_ROWS): they are a third of the code of a fold along rows. */
 /* the folds of elements [k0, k1), not none, of the R rows `row`: in C runs side by side, the first of them
  * beginning with the seed if SEEDED */
 template <int R, int C, bool SEEDED, typename T, typename Get, typename F>
@@ -591,6 +592,7 @@ ACC_DEV void acc_across_piece(Get get, F f, const Int64 (&row)[R], const Int64 k
 #undef ACC_ACROSS_ENTRY
 #undef ACC_ACROSS_R
 #endif
+#endif /* ACC_ACROSS_ROWS > 0 */
 #endif /* ACC_SEG_UNIFORM */
 
 /* ---- long segments: a team of lanes per segment ---------------------------

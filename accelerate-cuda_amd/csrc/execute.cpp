@@ -606,7 +606,7 @@ int acc_exec_fold(acc_skel s, const acc_array *env, int32_t in_rank, const int64
                                            0, st, args.data(), nullptr);
       return e == hipSuccess ? ACC_OK : acc::fail_hip(e, "hipModuleLaunchKernel(fold, short rows)");
     }
-    if (s->knobs.fold_across == 1 || (s->knobs.fold_across == 2 && s->spec.fold_across))
+    if (s->spec.fold_across)
       return launch_across(s, v, &args, env, out, rows, inner, st);
     return launch_segmented(s, v, &args, env, out, rows, rows * inner, st);
   }

@@ -348,7 +348,7 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
       if (sp.out_rank > 0) {
         // along the innermost dimension: the segmented fold over rows of one length
         *entry = sp.has_seed ? "fold" : "fold1";
-        o << "#define ACC_SEG_UNIFORM 1\n#define ACC_ACROSS_ROWS " << across_rows(sp) << "\n";
+        o << "#define ACC_SEG_UNIFORM 1\n#define ACC_ACROSS_ROWS " << (sp.fold_across ? across_rows(sp) : 0) << "\n";
         o << "#define ACC_TROUNDS " << tune("foldseg.team_rounds", 3) << "\n";
         if (tuned("foldseg.pad")) o << "#define ACC_PAD_ON " << (tune("foldseg.pad", 1) ? 1 : 0) << "\n";
         if (tuned("foldseg.wide")) o << "#define ACC_WIDE " << std::max(1, tune("foldseg.wide", 256)) << "\n";
@@ -705,7 +705,9 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
   if (sp->map_tile_dim == 0) sp->map_tile_dim = 1;
   if (sp->map_tiled && sp->map_tile_dim >= d->out_rank)
     return fail(ACC_ERR_INVALID, "%s: ACC_FLAG_TILE_DIM(%d) on a result of rank %d", kind_name(d->kind), sp->map_tile_dim, d->out_rank);
-  sp->fold_across = (d->flags & ACC_FLAG_TILED) != 0 && d->out_rank >= 1 && (d->kind == ACC_SKEL_FOLD || d->kind == ACC_SKEL_FOLD1);
+  const int across = tune("fold.across", 2);              // 2: where the flag says so, 1: every fold along rows, 0: none
+  sp->fold_across = (across == 1 || (across == 2 && (d->flags & ACC_FLAG_TILED) != 0)) && d->out_rank >= 1 &&
+                    (d->kind == ACC_SKEL_FOLD || d->kind == ACC_SKEL_FOLD1);
   sp->out_rank = d->out_rank;
   if (sp->out_rank < 0 || sp->out_rank > ACC_MAX_RANK) return fail(ACC_ERR_INVALID, "bad out_rank %d", d->out_rank);
   for (int k = 0; k < d->n_env; ++k) {
@@ -1155,20 +1157,22 @@ int acc_skel_s::ensure_variant(int v)
       var.module = nullptr;
       return acc::fail_hip(e, ("hipModuleGetFunction(" + rows + ")").c_str());
     }
-    const std::string across = entry_name + "_across";
-    e = hipModuleGetFunction(&var.fn_across, var.module, across.c_str());
-    if (e != hipSuccess) {
-      (void)hipModuleUnload(var.module);
-      var.module = nullptr;
-      return acc::fail_hip(e, ("hipModuleGetFunction(" + across + ")").c_str());
-    }
-    if (acc::across_rows(spec) > 1) {
-      const std::string wide = across + "_wide";
-      e = hipModuleGetFunction(&var.fn_across_wide, var.module, wide.c_str());
+    if (spec.fold_across) {
+      const std::string across = entry_name + "_across";
+      e = hipModuleGetFunction(&var.fn_across, var.module, across.c_str());
       if (e != hipSuccess) {
         (void)hipModuleUnload(var.module);
         var.module = nullptr;
-        return acc::fail_hip(e, ("hipModuleGetFunction(" + wide + ")").c_str());
+        return acc::fail_hip(e, ("hipModuleGetFunction(" + across + ")").c_str());
+      }
+      if (acc::across_rows(spec) > 1) {
+        const std::string wide = across + "_wide";
+        e = hipModuleGetFunction(&var.fn_across_wide, var.module, wide.c_str());
+        if (e != hipSuccess) {
+          (void)hipModuleUnload(var.module);
+          var.module = nullptr;
+          return acc::fail_hip(e, ("hipModuleGetFunction(" + wide + ")").c_str());
+        }
       }
     }
   }

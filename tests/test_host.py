@@ -151,6 +151,18 @@ def test_every_variant_there_is_compiles_and_no_other_is_accepted(A, tmp_path):
                 assert e.value.code == A.ERR_INVALID
 
 
+def test_a_fold_has_the_kernels_for_rows_across_memory_where_it_launches_them(A, tmp_path):
+    A.lib().acc_cache_set_dir(str(tmp_path).encode())
+
+    def size(flags, knobs=""):
+        with A.tuning(knobs):
+            src = A.preview(A.make_desc(A.SKEL_FOLD, "float", env=[(2, "float")], out_rank=1, get="arrIn0_0[ix]", combine="x + y", seed="0.0f", flags=flags))[1]
+        return A.compile_source(src)
+    plain, tiled = size(0), size(A.FLAG_TILED)
+    assert plain < 0.7 * tiled
+    assert size(0, "fold.across=1") == tiled and size(A.FLAG_TILED, "fold.across=0") == plain
+
+
 def test_templates_leave_a_preamble_its_names(A, tmp_path):
     """a description may declare functions of its own; what a template calls its parameters and locals where a fragment
     stands must not hide them (the names below are ones that the form of the instance for any other shape takes)"""
