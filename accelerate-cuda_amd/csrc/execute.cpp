@@ -768,18 +768,15 @@ int scan_core(acc_skel s, const acc_array *env, int64_t n, const acc_array *out,
   // each a long way from its first load to its last store; of 4 so many that the chain of their totals takes longer than
   // the data (us with 4 / 8 / 12 / 16 / 32 rows: Int32 4 M 11.3 / 9.9 / 10.9 / 10.9 / 14.3, 6 M 14.6 / 12.1 / 11.7 / 12.7 /
   // 15.4, 12 M 29.5 / 20.2 / 18.8 / 18.6 / 21.0, 16 M 36.4 / 28.1 / 30.1 / 24.7 / 23.9; Float64 3 M 18.6 / 14.1 / 13.0 /
-  // 13.9 / 16.0).  A call that may not build the variant -- without allocations, or on a stream that is being captured --
-  // takes the large tile where the variant is not there yet.
+  // 13.9 / 16.0).  The variant is loaded together with the large tile's (acc_skel_s::ensure_variant).
   const bool mid = !small && s->spec.scan_mid_rows > 0 && s->knobs.scan_small_below_kb > 0 &&
                    n * (int64_t)s->spec.elt_size <= (int64_t)s->knobs.scan_mid_below_kb * 1024;
-  int v = (aligned ? 0 : 1) + (small ? 2 : 0);
-  if (mid && (noalloc ? s->variant_ready(v + 4) : may_take(s, v + 4, st))) v += 4;
+  const int v = (aligned ? 0 : 1) + (small ? 2 : mid ? 4 : 0);
   if (noalloc) {
     // building a variant compiles and loads a module: not here
     if (!s->variant_ready(v))
       return fail(ACC_ERR_INVALID, "%s: the %s %s-tile variant of this instance is not loaded yet; run acc_exec_scan once on operands of the same alignment and of %s %d KB first",
-                  who, aligned ? "aligned" : "unaligned", small ? "small" : "large", small ? "at most" : "more than",
-                  s->knobs.scan_small_below_kb);
+                  who, aligned ? "aligned" : "unaligned", small ? "small" : "large", small ? "at most" : "more than", s->knobs.scan_small_below_kb);
   } else {
     ACC_TRY(s->ensure_variant(v));
   }

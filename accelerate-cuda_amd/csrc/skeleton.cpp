@@ -1037,7 +1037,7 @@ SkelSpec spec_of_variant(const SkelSpec &base, int v)
   // ... 4 and 5: one between the two
   if (spec.scan_small_rows > 0 && v >= 2) {
     spec.block = std::min(spec.block, 256);
-    spec.rows = std::min(spec.rows, v >= 4 ? spec.scan_mid_rows : spec.scan_small_rows);
+    spec.rows = v >= 4 ? spec.scan_mid_rows : std::min(spec.rows, spec.scan_small_rows);
   }
   return spec;
 }
@@ -1049,6 +1049,8 @@ static int make_job(acc_skel_s *s, int v, std::shared_ptr<acc::CompileJob> *out)
   acc::Variant &var = s->variants[v];
   const acc::SkelSpec spec = acc::spec_of_variant(s->spec, v);
   ACC_TRY(acc::generate_source(spec, (v & 1) == 0, &var.entry, &var.source));
+  var.block = spec.block;      // the shape that is in the text: a scan's may change before the code is loaded
+  var.rows = spec.rows;
   if (s->entry.empty()) s->entry = var.entry;      // the same for every variant; set once, before the instance is shared
   auto job = std::make_shared<acc::CompileJob>();
   job->target = s->ctx->arch;
@@ -1083,6 +1085,21 @@ bool acc_skel_s::variant_compiled(int v)
 }
 
 int acc_skel_s::ensure_variant(int v)
+{
+  // A scan's full tile and the middle one are loaded together: which of the two a call takes depends on the size of its
+  // arrays alone then, and not on what was called before -- under capture and without allocations nothing can be built,
+  // and sums of floating numbers would be associated by the tile that happens to be there.
+  const int other = other_of_pair(v);
+  {
+    std::lock_guard<std::mutex> lock(mu);
+    if (variants[v].ready && (other < 0 || variants[other].ready)) return ACC_OK;
+  }
+  if (other >= 0) ACC_TRY(start_variant(other));
+  ACC_TRY(load_variant(v));
+  return other >= 0 ? load_variant(other) : ACC_OK;
+}
+
+int acc_skel_s::load_variant(int v)
 {
   // two threads may meet here on the first launch that needs the unaligned variant
   std::unique_lock<std::mutex> lock(mu);
@@ -1177,8 +1194,6 @@ int acc_skel_s::ensure_variant(int v)
     }
   }
   (void)hipFuncGetAttribute(&var.num_regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, var.fn);
-  var.block = spec.block;
-  var.rows = spec.rows;
   if (this->spec.scan_shape_open && v < 2) {
     // the first build of a scan decides its tile shape: see make_spec
     this->spec.scan_shape_open = false;
@@ -1188,12 +1203,12 @@ int acc_skel_s::ensure_variant(int v)
       this->spec.block = 1024;
       this->spec.rows = this->spec.scan_rows_fallback;
       lock.unlock();
-      return ensure_variant(v);
+      return load_variant(v);
     }
   }
   (void)hipFuncGetAttribute(&var.static_lds, HIP_FUNC_ATTRIBUTE_SHARED_SIZE_BYTES, var.fn);
   int bpc = 0;
-  e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, var.fn, spec.block, 0);
+  e = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, var.fn, var.block, 0);
   if (e != hipSuccess || bpc < 1) { (void)hipGetLastError(); bpc = 1; }
   var.blocks_per_cu = bpc;
   var.ready = true;
@@ -1237,7 +1252,8 @@ int acc_skel_create_async(acc_context ctx, const acc_skel_desc *desc, acc_skel *
     s->hint_slot = static_cast<int>(ctx->next_hint.fetch_add(1) % acc::HINT_WORDS);
     __atomic_store_n(const_cast<uint32_t *>(ctx->status_host) + acc::STATUS_WORDS + s->hint_slot, 0u, __ATOMIC_RELAXED);
   }
-  const int rc = s->start_variant(0);     // the other variants are built when a call first needs them
+  int rc = s->start_variant(0);           // the other variants are built when a call first needs them
+  if (rc == ACC_OK && s->other_of_pair(0) >= 0) rc = s->start_variant(s->other_of_pair(0));
   if (rc != ACC_OK) { delete s; return rc; }
   *out = s;
   return ACC_OK;
@@ -1272,17 +1288,8 @@ int acc_skel_wait(acc_skel s)
 int acc_skel_poll(acc_skel s, int *ready)
 {
   if (!s || !ready) return fail(ACC_ERR_INVALID, "acc_skel_poll: NULL argument");
-  std::shared_ptr<acc::CompileJob> job;
-  {
-    std::lock_guard<std::mutex> lock(s->mu);
-    if (s->variants[0].ready) { *ready = 1; return ACC_OK; }
-    job = s->variants[0].job;
-  }
-  *ready = 0;
-  if (job) {
-    std::lock_guard<std::mutex> lock(job->mu);
-    *ready = job->done ? 1 : 0;
-  }
+  const int other = s->other_of_pair(0);
+  *ready = s->variant_compiled(0) && (other < 0 || s->variant_compiled(other)) ? 1 : 0;
   return ACC_OK;
 }
 

@@ -86,8 +86,8 @@ struct Variant {
   int num_regs = 0;
   int static_lds = 0;
   int blocks_per_cu = 1;
-  int block = 0;                       // workgroup size and rows a lane of this variant was built with (a scan's small
-  int rows = 0;                        // variant differs from the instance's)
+  int block = 0;                       // workgroup size and rows a lane of this variant is built with (a scan's small
+  int rows = 0;                        // variant differs from the instance's), from the moment its text is made
   std::shared_ptr<CompileJob> job;     // its compilation, once started: in the background, or by the thread that needs it
   std::string entry;                   // the main kernel's name in `job`'s code
 };
@@ -122,6 +122,9 @@ struct acc_skel_s {
 
   // variant v compiled, loaded and measured; compiles on the calling thread unless a job for it is under way
   int ensure_variant(int v);
+  int load_variant(int v);             // ... that one alone
+  // the variant that is loaded together with v, or -1: a scan's full tile and its middle one
+  int other_of_pair(int v) const { return spec.scan_mid_rows == 0 || v == 2 || v == 3 ? -1 : (v < 2 ? v + 4 : v - 4); }
   // start variant v's compilation on the worker pool (nothing if it has been started or is ready)
   int start_variant(int v);
   bool variant_ready(int v) { std::lock_guard<std::mutex> lock(mu); return variants[v].ready; }

@@ -479,10 +479,9 @@ int acc_exec_scan(acc_skel s, const acc_array *env, int64_t n, const acc_array *
  *     (32768 Int32 each: 2^28 elements); more is ACC_ERR_INVALID;
  *   - the variant that acc_exec_scan takes for such operands must have been loaded already, else ACC_ERR_INVALID.
  *     There are six: for operands aligned to 16 bytes or not, and for arrays of at most 12 MB (scanned in tiles
- *     an eighth the size), of at most 48 MB (in tiles of three eighths) or more.  acc_skel_create loads the one for
- *     large aligned arrays, a first acc_exec_scan on operands of the same alignment and of a size in the same range
- *     each of the others.  (Between 12 and 48 MB the large tile does where that is the one there is; sums of floating
- *     numbers may then be associated otherwise than acc_exec_scan does.)
+ *     an eighth the size), of at most 48 MB (in tiles of three eighths) or more.  The last two are loaded together:
+ *     for aligned operands by acc_skel_create; for others, as the one for small arrays, by a first acc_exec_scan on
+ *     operands of the same alignment and on the same side of 12 MB;
  *   - every call on a device shares that device's array: calls that overlap in time on one device, from any
  *     stream, thread or context, race.  Calls ordered on one stream are fine.  A call of more tiles than the device
  *     holds at once must not overlap ANY other scan of that size on the device either, acc_exec_scan's included:
@@ -491,7 +490,9 @@ int acc_exec_scan(acc_skel s, const acc_array *env, int64_t n, const acc_array *
  *   - a call makes two launches: a small kernel that counts the launch's tag in the array's header, and the scan,
  *     which reads it there.  A graph that records the call therefore gets a fresh tag at every replay; were the tag
  *     an argument of the recorded launch, a replay would take the descriptors its predecessor left for its own.
- * Results are those of acc_exec_scan on the same variant, bit for bit.                                      */
+ * Results are those of acc_exec_scan, in every bit where the operator is associative in every bit.  (Sums of floating
+ * numbers are associated across tiles by what a tile finds finished when it looks back, and differ in their last bits
+ * from one call to the next, of either entry point.)                                                          */
 #define ACC_NOALLOC_MAX_TILES 8192
 int acc_exec_scan_noalloc(acc_skel s, const acc_array *env, int64_t n, const acc_array *out,
                           const acc_array *total, acc_stream stream);

@@ -54,6 +54,72 @@ def test_middle_tile(ctx, kind, ctype, dt):
                 assert int(tot.get().reshape(-1)[0]) == int(np.array(total).astype(dt))
 
 
+@pytest.mark.parametrize("ctype,dt", [("float", np.float32), ("double", np.float64)])
+def test_the_tile_does_not_depend_on_what_was_called_before(ctx, ctype, dt):
+    """An instance that has run nothing yet takes the same tile without allocations, and recorded into a graph, as
+    acc_exec_scan does; so does one whose unaligned form was first wanted for an array of another size.  Sums of floating
+    numbers tell the tile: what the first one holds is associated by its shape alone (further on by what the look-back
+    finds finished, which differs from call to call)."""
+    import ctypes as C
+
+    import acchip as A
+    size = np.dtype(dt).itemsize
+    n, large = (20 << 20) // size + 3, (49 << 20) // size
+    rng = np.random.default_rng(1)
+    x = rng.standard_normal(large + 1).astype(dt)
+    src, stream, first = ctx.array(x), ctx.stream(), TILE * 4 // size
+
+    def fresh():
+        return ctx.skeleton(A.SKEL_SCANL1, ctype, env=[(1, ctype)], get="arrIn0_0[ix]", combine="x + y", wait=True)
+    for shift in (0, 1):
+        usual = fresh()
+        want, got, out = ctx.empty(n, dt), ctx.empty(n, dt), ctx.empty(large, dt)
+        env = [_Part(src, shift, n)]
+        usual.scan(env, n, want, stream=stream)
+        sk = fresh()
+        if shift:                                                  # (the unaligned form is loaded by a first call)
+            sk.scan([_Part(src, shift, large)], large, out, stream=stream)
+        print(ctype, shift, "without allocations", flush=True)
+        sk.scan(env, n, got, stream=stream, noalloc=True)
+        ctx.sync()
+        assert np.array_equal(got.get()[:first], want.get()[:first]), shift
+        # the other way round: a call of this size first
+        sk = fresh()
+        sk.scan(env, n, got, stream=stream)
+        usual.scan([_Part(src, shift, large)], large, out, stream=stream)
+        ctx.sync()
+        ref = out.get()
+        sk.scan([_Part(src, shift, large)], large, out, stream=stream, noalloc=True)
+        ctx.sync()
+        assert np.array_equal(out.get()[:first], ref[:first]), shift
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(C.c_void_p), C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [C.c_void_p, C.c_void_p]
+    hip.hipGraphExecDestroy.argtypes = hip.hipGraphDestroy.argtypes = [C.c_void_p]
+    usual, sk = fresh(), fresh()
+    env = [_Part(src, 0, n)]
+    want, got = ctx.empty(n, dt), ctx.empty(n, dt)
+    graph, graph_exec = C.c_void_p(), C.c_void_p()
+    ctx.sync()
+    assert hip.hipStreamBeginCapture(stream, 2) == 0
+    try:
+        sk.scan(env, n, got, stream=stream, noalloc=True)
+    finally:
+        rc = hip.hipStreamEndCapture(stream, C.byref(graph))
+    assert rc == 0 and graph.value and hip.hipGraphInstantiate(C.byref(graph_exec), graph, None, None, 0) == 0
+    for replay in range(3):
+        print(ctype, "replay", replay, flush=True)
+        src.set(rng.standard_normal(large + 1).astype(dt))
+        assert hip.hipGraphLaunch(graph_exec, stream) == 0
+        usual.scan(env, n, want, stream=stream)
+        ctx.sync()
+        assert np.array_equal(got.get()[:first], want.get()[:first]) and np.allclose(got.get(), want.get(), rtol=0, atol=1e-2)
+    hip.hipGraphExecDestroy(graph_exec)
+    hip.hipGraphDestroy(graph)
+
+
 class _Part(object):
     def __init__(self, arr, off, count):
         self.d = arr.desc(shape=(count,), offset_elems=off)
