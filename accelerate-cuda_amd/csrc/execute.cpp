@@ -716,15 +716,18 @@ int acc_exec_foldseg(acc_skel s, const acc_array *env, int64_t n, const acc_arra
 
 namespace {
 
-// A variant beyond the ones an earlier call of this size would have loaded: there already, or buildable now (a stream
-// under capture is no place to load a module).
+// A variant that makes what another one of the instance makes too: whether it is there, or can be had now (a stream under
+// capture is no place to load a module).  Where it cannot be built the call goes on with the other.
 // (A weak reference: a runtime without the call has no capture either.)
 #pragma weak hipStreamIsCapturing
 bool may_take(acc_skel s, int v, hipStream_t st)
 {
-  if (s->variant_ready(v) || !hipStreamIsCapturing) return true;
-  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(st, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone;
+  if (s->variant_ready(v)) return true;
+  if (hipStreamIsCapturing) {
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
+  }
+  return s->ensure_variant(v) == ACC_OK;
 }
 
 // scanOp / scan1Op / scan'Op / scanCore, Execute.hs:328-392, as ONE launch.  `noalloc`: the tile descriptors live in
@@ -1370,7 +1373,6 @@ static int stencil_once(acc_skel s, const acc_array *env, const acc_array *in, c
     const int64_t widest = std::max(s->spec.elt_size, 8);
     const int v = (aligned ? 0 : 1) + 8;
     if (w * h * widest < ((int64_t)1 << 32) && planes < ((int64_t)1 << 30) && waves() < ((int64_t)1 << 30) && may_take(s, v, st)) {
-      ACC_TRY(s->ensure_variant(v));
       args.i32(static_cast<int32_t>(walk));
       return launch(s, v, (waves() + per_block - 1) / per_block, 0, st, &args);
     }
@@ -1431,7 +1433,6 @@ static bool stencil_pair(acc_skel s, const acc_array *env, const acc_array *in, 
     push_out(*out, &args, &aligned);
     push_ptrs(in, in->ncomp, &args, &aligned);
     args.i32(0);
-    ACC_TRY(s->ensure_variant(v));
     const int64_t per_block = s->spec.block / 64;
     return launch(s, v, (strips * bands + per_block - 1) / per_block, 0, st, &args);
   }();

@@ -56,3 +56,71 @@ def test_pairs_against_single_applications(ctx, boundary, ctype, dt, taps):
                 got.append((res is pb, a.get(), b.get()))
             assert got[0][0] == got[1][0]
             assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][2], got[1][2]), (shape, shift, iters)
+
+
+@pytest.mark.parametrize("what,rank,shape", [("acc_pair_own", 2, (40, 300)), ("acc_flat_source", 3, (5, 7, 700))])
+def test_a_form_that_cannot_be_built_leaves_the_call_to_another(ctx, what, rank, shape):
+    """a preamble that takes a name which only this form's template has: the form does not compile, the others do"""
+    import acchip as A
+    taps = CROSS if rank == 2 else [(0, 0, 0), (-1, 0, 0), (1, 0, 0), (0, -1, 0), (0, 1, 0), (0, 0, -1), (0, 0, 1)]
+    desc = dict(out_rank=rank, taps=taps, boundary="clamp", stencil_fn=" + ".join("%d * t%d" % (k + 2, k) for k in range(len(taps))))
+    broken = A.make_desc(A.SKEL_STENCIL, "Int32", preamble="#define %s 1" % what, **desc)
+    with pytest.raises(A.AccError):
+        A.compile_source(A.preview(broken, 10 if rank == 2 else 8)[1])
+    x = np.random.default_rng(2).integers(-50, 50, shape).astype(np.int32)
+    got = []
+    for preamble in (None, "#define %s 1" % what):
+        sk = ctx.skeleton(A.SKEL_STENCIL, "Int32", preamble=preamble, wait=True, **desc)
+        for _ in range(2):
+            a, b = ctx.array(x), ctx.empty(shape, np.int32)
+            if rank == 2:
+                got.append(sk.stencil_iterate(None, a, b, 6).get())
+            else:
+                sk.stencil(None, a, b)
+                got.append(b.get())
+    assert all(np.array_equal(g, got[0]) for g in got)
+
+
+@pytest.mark.parametrize("rank,shape", [(2, (40, 300)), (3, (5, 7, 700))])
+def test_recorded_before_the_form_is_loaded(ctx, rank, shape):
+    """under capture nothing is built: the graph holds the form that is there, and its results are the same"""
+    import ctypes as C
+
+    import acchip as A
+    taps = CROSS if rank == 2 else [(0, 0, 0), (-1, 0, 0), (1, 0, 0), (0, -1, 0), (0, 1, 0), (0, 0, -1), (0, 0, 1)]
+    desc = dict(out_rank=rank, taps=taps, boundary="mirror", stencil_fn=" + ".join("%d * t%d" % (k + 2, k) for k in range(len(taps))))
+    sk = ctx.skeleton(A.SKEL_STENCIL, "Int32", wait=True, **desc)
+    hip = C.CDLL("libamdhip64.so")
+    hip.hipStreamBeginCapture.argtypes = [C.c_void_p, C.c_int]
+    hip.hipStreamEndCapture.argtypes = [C.c_void_p, C.POINTER(C.c_void_p)]
+    hip.hipGraphInstantiate.argtypes = [C.POINTER(C.c_void_p), C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
+    hip.hipGraphLaunch.argtypes = [C.c_void_p, C.c_void_p]
+    hip.hipGraphExecDestroy.argtypes = hip.hipGraphDestroy.argtypes = [C.c_void_p]
+    stream, rng = ctx.stream(), np.random.default_rng(2)
+    a, b = ctx.empty(shape, np.int32), ctx.empty(shape, np.int32)
+
+    def call(x, y):
+        if rank == 2:
+            return sk.stencil_iterate(None, x, y, 5, stream=stream)
+        sk.stencil(None, x, y, stream=stream)
+        return y
+    graph, graph_exec = C.c_void_p(), C.c_void_p()
+    ctx.sync()
+    assert hip.hipStreamBeginCapture(stream, 2) == 0
+    try:
+        res = call(a, b)
+    finally:
+        rc = hip.hipStreamEndCapture(stream, C.byref(graph))
+    assert rc == 0 and graph.value and hip.hipGraphInstantiate(C.byref(graph_exec), graph, None, None, 0) == 0
+    for replay in range(4):
+        print(rank, "replay", replay, flush=True)
+        x = rng.integers(-50, 50, shape).astype(np.int32)
+        a.set(x)
+        assert hip.hipGraphLaunch(graph_exec, stream) == 0
+        ctx.sync()
+        got = res.get()
+        eager = call(ctx.array(x), ctx.empty(shape, np.int32))          # (the form is built and taken from here on)
+        ctx.sync()
+        assert np.array_equal(got, eager.get()), replay
+    hip.hipGraphExecDestroy(graph_exec)
+    hip.hipGraphDestroy(graph)
