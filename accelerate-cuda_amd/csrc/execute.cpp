@@ -718,16 +718,15 @@ namespace {
 
 // A variant that makes what another one of the instance makes too: whether it is there, or can be had now (a stream under
 // capture is no place to load a module).  Where it cannot be built the call goes on with the other.
-// (A weak reference: a runtime without the call has no capture either.)
-#pragma weak hipStreamIsCapturing
 bool may_take(acc_skel s, int v, hipStream_t st)
 {
   if (s->variant_ready(v)) return true;
-  if (hipStreamIsCapturing) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(st, &capture) != hipSuccess || capture != hipStreamCaptureStatusNone) return false;
+  hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &capture) != hipSuccess) {
+    (void)hipGetLastError();      // (answered by the other form: no later call is to find this error)
+    return false;
   }
-  return s->ensure_variant(v) == ACC_OK;
+  return capture == hipStreamCaptureStatusNone && s->ensure_variant(v) == ACC_OK;
 }
 
 // scanOp / scan1Op / scan'Op / scanCore, Execute.hs:328-392, as ONE launch.  `noalloc`: the tile descriptors live in
