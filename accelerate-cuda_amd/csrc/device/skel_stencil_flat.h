@@ -18,9 +18,9 @@
  * come out of the L2: a die takes one contiguous run of the workgroups.
  *
  * What bounds it: the memory side.  7 points on 300^3 Float32, 216 MB: 77 us in strips, which read 1.86 and wrote 1.32
- * times what they had to; 55 us (3.9 TB/s) here, reading 1.07 and writing 1.00 times, with half the vector instructions.
- * (The same launch on operands that the memory-side cache holds: 39 us.)  Non-temporal stores 57.1, ordinary ones 60.0;
- * workgroups of 1024 64, of 64 63.
+ * times what they had to; 54.6 us (4.0 TB/s) here, reading 1.11 and writing 1.06 times, with less than half the vector
+ * instructions.  (The same launch on operands that the memory-side cache holds: 35 us.)  Non-temporal stores, a wave
+ * through 8 planes, 57.1 us, ordinary ones 60.0; workgroups of 1024 64, of 64 63.
  *
  * Generated definitions expected: those of skel_stencil.h, for ACC_STENCIL_RANK 3 and one source; the planes of source
  * and result are smaller than 4 GB (the driver sees to it), the rows no shorter than a vector.

@@ -908,6 +908,7 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
         // (2 ry + rows of them side by side, 2 rz + 1 + prefetch planes deep); within 192 for elements of two words or
         // more, which would otherwise get strips one row tall that read every row three times (Float64, 7 points,
         // 256 x 512 x 512: 249.5 us; two rows tall, 207 registers, 231.5).
+        sp->reach_z = rz;
         sp->zmarch = (rz > 0 && 2 * rx * (2 * ry + 1) <= 64) ? (tune("stencil.zmarch", 1) ? 1 : 0) : 0;
         if (sp->zmarch) {
           for (int ty = 4; ty > 1 && planes_per_strip == 1; --ty)

@@ -46,7 +46,7 @@ struct SkelSpec {
   std::vector<int> tap_off, tap2_off;   // ... its taps: n_taps rows of out_rank offsets, outermost dimension first
   int tile_w = 256, tile_h = 4, prefetch = 3;
   int svec = 4;                         // stencils: columns a lane holds of every row (tile_w = 64 of them)
-  int reach_x = 0;                      // stencils: the furthest a tap reaches to either side
+  int reach_x = 0, reach_z = 0;         // stencils: the furthest a tap reaches to either side, and across planes
   int tile_z = 1;                       // rank-3 stencils: result planes per strip (rows per strip where the strip walks through planes)
   int zmarch = 0;                       // rank-3 stencils: strips tile_z rows tall walk through tile_h planes
   // tuning

@@ -758,6 +758,12 @@ def main():
             tr = ctx.skeleton(A.SKEL_MAP, "float", env=[(2, "float")], out_rank=2, flags=flags, get="arrIn0_0[(ix % shOut_0) * shIn0_0 + (ix / shOut_0)]")
             one("transpose 8192 x 8192 Float32 " + name, lambda: A.check(L.acc_exec_map(tr.handle, se, C.byref(dd), stream)), 8 * side * side)
         assert np.array_equal(dst.get(), wl.stencil_image(side, side).T), "transpose mismatch"
+        # (rows that are no whole cache lines on either side)
+        odd = np.arange(5003 * 3001, dtype=np.float32).reshape(5003, 3001)
+        so, do = ctx.array(odd), ctx.empty((3001, 5003), np.float32)
+        oe, od_ = A._env([so]), do.desc()
+        one("transpose 5003 x 3001 Float32 in tiles (ACC_FLAG_TILED)", lambda: A.check(L.acc_exec_map(tr.handle, oe, C.byref(od_), stream)), 8 * odd.size)
+        assert np.array_equal(do.get(), odd.T), "transpose mismatch"
         del src, dst
         # (a result of two rows or two columns: most of every tile would lie outside it, so the tiled instance goes in runs)
         for shape in ((1 << 23, 2), (2, 1 << 23)):

@@ -54,3 +54,45 @@ class _Part(object):
 
     def desc(self):
         return self.d
+
+
+@pytest.mark.parametrize("walk", [1, 2, 3, 4, 8, 16, 20])
+@pytest.mark.parametrize("ctype,dt,taps", [("float", np.float32, BOX), ("double", np.float64, STAR), ("Int32", np.int32, ODD)])
+def test_walks_through_several_planes(ctx, ctype, dt, taps, walk):
+    """the ring of planes goes round several times and the last run is cut short: depths round one and two walks, the walk
+    given (left to itself it is the shortest there is at these sizes)"""
+    import acchip as A
+    fn = " + ".join("(%s)%d * t%d" % (ctype, 3 + k % 5, k) for k in range(len(taps)))
+    desc = dict(out_rank=3, taps=taps, stencil_fn=fn)
+    rng = np.random.default_rng(4)
+    for boundary in ("clamp", "constant", "wrap"):
+        desc.update(boundary=boundary, boundary_constant="(%s)7" % ctype if boundary == "constant" else None)
+        with A.tuning("stencil.flat=2,stencil.thin_3d=0,stencil.flat_walk=%d" % walk, ctx):
+            flat = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+        with A.tuning("stencil.nd=1", ctx):
+            each = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+        for depth in sorted({max(3, d) for d in (walk - 1, walk, walk + 1, 2 * walk + 1, 3 * walk)}):
+            for h, w in ((5, 22), (6, 131)):
+                print(ctype, boundary, walk, depth, h, w, flush=True)
+                src, got = ctx.array(rng.integers(-50, 50, (depth, h, w)).astype(dt)), []
+                for sk in (flat, each):
+                    out = ctx.empty((depth, h, w), dt)
+                    sk.stencil(None, src, out)
+                    got.append(out.get())
+                assert np.array_equal(got[0], got[1]), (boundary, depth, h, w)
+
+
+@pytest.mark.parametrize("shape", [(83, 84, 300), (160, 150, 150)])
+def test_the_walk_the_driver_chooses(ctx, shape):
+    """volumes for which it is more than the shortest (5 and 8 planes on 256 compute units)"""
+    import acchip as A
+    desc = dict(out_rank=3, taps=BOX, boundary="mirror", stencil_fn=" + ".join("%d * t%d" % (3 + k % 5, k) for k in range(len(BOX))))
+    flat = ctx.skeleton(A.SKEL_STENCIL, "Int32", wait=True, **desc)
+    with A.tuning("stencil.nd=1", ctx):
+        each = ctx.skeleton(A.SKEL_STENCIL, "Int32", wait=True, **desc)
+    src, got = ctx.array(np.random.default_rng(4).integers(-50, 50, shape).astype(np.int32)), []
+    for sk in (flat, each):
+        out = ctx.empty(shape, np.int32)
+        sk.stencil(None, src, out)
+        got.append(out.get())
+    assert np.array_equal(got[0], got[1])
