@@ -330,7 +330,8 @@ typedef struct acc_skel_desc {
                                        `acc_elt{x.a<n-1>, ..., x.a0}` for a tuple: `permute const`, the
                                        scatter of a compaction or of a sorting pass -- stores the new
                                        values and reads and locks nothing; of several sources on one
-                                       target one wins whole */
+                                       target one wins whole, and `get` is evaluated for sources that
+                                       stay only */
   const char        *seed;          /* NULL for the seedless kinds                           */
   const char        *permutation;   /* permute: linear target index of source `ix`, or
                                        ACC_IGNORE (-1) to drop the element                   */
@@ -521,7 +522,9 @@ int acc_exec_stencil2(acc_skel s, const acc_array *env, const acc_array *in1, co
  * a; *result_in_b tells where the last application wrote, the other array then
  * holds what that one read.  (A 2-D stencil of one array of 4- or 8-byte elements
  * with taps next to the element goes two applications a launch, but for the last
- * ones; the results are the same.)                                            */
+ * ones; the results are the same.  The variant that does -- 10, or 11 off the
+ * 16-byte boundary -- is compiled by the first call of five or more applications,
+ * a fifth of a second, unless acc_skel_prefetch has.)                         */
 int acc_exec_stencil_iterate(acc_skel s, const acc_array *env, const acc_array *a, const acc_array *b,
                              int32_t iters, acc_stream stream, int32_t *result_in_b);
 
