@@ -103,6 +103,7 @@ void set_default_tuning(TuningPtr t);
   X(scan_small_below_kb, "scan.small_below_kb", 12288)                                                                 \
   X(scan_mid_below_kb, "scan.mid_below_kb", 49152)                                                                     \
   X(stencil_pair, "stencil.pair", 1)                                                                                    \
+  X(stencil_pair_walk, "stencil.pair_walk", 0)                                                                          \
   X(stencil_flat, "stencil.flat", 1)                                                                     \
   X(stencil_flat_walk, "stencil.flat_walk", 0)                                                                         \
   X(stencil_half_strips, "stencil.half_strips", 1)                                                                     \

@@ -1451,14 +1451,23 @@ static int stencil_once(acc_skel s, const acc_array *env, const acc_array *in, c
   return launch(s, (aligned ? 0 : 1) + 2 * narrow, (strips_x * bands * zbands + waves - 1) / waves, 0, st, &args);
 }
 
-// Two applications of a stencil in one launch (skel_stencil_pair.h), where the instance and the shape allow: false if not,
-// and nothing has been done.
-static bool stencil_pair(acc_skel s, const acc_array *env, const acc_array *in, const acc_array *out, hipStream_t st, int *rc)
+// Three or four applications of a stencil in one launch (skel_stencil_pair.h), where the instance and the shape allow: false
+// if not, and nothing has been done.
+static bool stencil_many(acc_skel s, int levels, const acc_array *env, const acc_array *in, const acc_array *out, hipStream_t st, int *rc)
 {
-  if (s->spec.pair_rows <= 0 || s->knobs.stencil_pair == 0 || array_size(*out) == 0) return false;
-  const int64_t w = out->shape[1], h = out->shape[0], owned = (int64_t)62 * s->spec.svec, esz = s->spec.elt_size;
-  const int64_t strips = (w + owned - 1) / owned, bands = (h + s->spec.pair_rows - 1) / s->spec.pair_rows;
-  if ((w != owned && w < owned + s->spec.svec) || h < 3 || w >= (1 << 30) || h >= (1 << 30) || strips * bands >= (1 << 30)) return false;
+  if (!s->spec.pair_form || s->knobs.stencil_pair == 0 || array_size(*out) == 0) return false;
+  // lanes at either side of a strip whose columns go wrong, and the columns of a strip (as the kernel has them)
+  const int64_t svec = s->spec.svec, outer = s->spec.reach_x > 0 ? (levels + svec - 1) / svec : 1, owned = (64 - 2 * outer) * svec;
+  const int64_t w = out->shape[1], h = out->shape[0], esz = s->spec.elt_size;
+  if ((w != owned && w < owned + outer * svec) || h < 3 || w >= (1 << 30) || h >= (1 << 30)) return false;
+  const int64_t strips = (w + owned - 1) / owned;
+  // rows a wave walks through: 28, or fewer, down to 4, as long as that leaves a compute unit fewer than eight waves (the
+  // rows above and below are read and worked out for every walk anew: 3000 x 3000 Float32 in 28 / 20 / 12 / 8 rows 24.5 /
+  // 22.4 / 25.0 / 23.3 us for four applications, 1024 x 1024 in 16 / 8 / 4 rows 14.2 / 9.9 / 9.2, 300 x 300 13.5 / 9.1 / 6.3)
+  int64_t walk = s->knobs.stencil_pair_walk;
+  if (walk <= 0) walk = std::max<int64_t>(4, std::min<int64_t>(28, h * strips / (8 * (int64_t)s->ctx->props.multiProcessorCount)));
+  const int64_t bands = (h + walk - 1) / walk;
+  if (strips * bands >= (1 << 30)) return false;
   const int v = 10 + ((aligned16(in->ptr[0]) && aligned16(out->ptr[0]) && w * esz % 16 == 0) ? 0 : 1);
   if (!may_take(s, v, st)) return false;
   *rc = [&]() -> int {
@@ -1468,9 +1477,12 @@ static bool stencil_pair(acc_skel s, const acc_array *env, const acc_array *in, 
     ACC_TRY(push_env(s, env, &args, &aligned));
     push_out(*out, &args, &aligned);
     push_ptrs(in, in->ncomp, &args, &aligned);
-    args.i32(0);
-    const int64_t per_block = s->spec.block / 64;
-    return launch(s, v, (strips * bands + per_block - 1) / per_block, 0, st, &args);
+    args.i32(static_cast<int32_t>(walk));
+    const int64_t per_block = s->spec.block / 64, grid = (strips * bands + per_block - 1) / per_block;
+    ACC_TRY(s->ctx->make_current());
+    const acc::Variant &var = s->variants[v];
+    ACC_HIP_TRY(launch_kernel(levels == 4 ? var.fn : var.fn_three, static_cast<unsigned>(grid), 1, 1, static_cast<unsigned>(var.block), 1, 1, 0, st, args.data(), nullptr));
+    return ACC_OK;
   }();
   return true;
 }
@@ -1517,21 +1529,31 @@ int acc_exec_stencil_iterate(acc_skel s, const acc_array *env, const acc_array *
   ACC_TRY(stencil_check(s, a, b));
   if (iters < 0) return fail(ACC_ERR_INVALID, "stencil: negative iteration count");
   const acc_array *src = a, *dst = b;
-  // Two applications a launch as often as leaves every result where one a launch would: an even number of pairs, so that
-  // the arrays have changed places as often, and at least one application by itself at the end, whose source is then the
-  // result before the last.
-  int32_t pairs = 2 * ((std::max(iters, 1) - 1) / 4);
+  // Four and three applications a launch as often as leaves every result where one a launch would: an even number of
+  // fours, so that the arrays have changed places as often (a three changes them as three single ones do), and at least
+  // one application by itself at the end, whose source is then the result before the last.  Of these splits the one that
+  // takes least: of large arrays a four takes about 1.35 times a single application, a three 1.25 times.
+  const int32_t many = std::max(iters, 1) - 1;
+  int32_t fours = 0, threes = 0;
+  for (int32_t q = many / 4 / 2 * 2, least = -1; q >= 0 && q > many / 4 - 8; q -= 2) {
+    const int32_t t = (many - 4 * q) / 3, cost = 27 * q + 25 * t + 20 * (many - 4 * q - 3 * t);
+    if (least >= 0 && cost >= least) continue;
+    least = cost;
+    fours = q;
+    threes = t;
+  }
   for (int32_t i = 0; i < iters;) {
-    const bool two = pairs > 0;
+    const int32_t levels = fours > 0 ? 4 : threes > 0 ? 3 : 1;
     int rc = ACC_OK;
-    if (two && !stencil_pair(s, env, src, dst, static_cast<hipStream_t>(stream), &rc)) {
-      pairs = 0;
+    if (levels > 1 && !stencil_many(s, levels, env, src, dst, static_cast<hipStream_t>(stream), &rc)) {
+      fours = threes = 0;                // (never after the first: what one launch has taken the others find there)
       continue;
     }
-    if (!two) rc = stencil_once(s, env, src, nullptr, dst, static_cast<hipStream_t>(stream));
+    if (levels == 1) rc = stencil_once(s, env, src, nullptr, dst, static_cast<hipStream_t>(stream));
     ACC_TRY(rc);
-    i += two ? 2 : 1;
-    pairs -= two ? 1 : 0;
+    i += levels;
+    fours -= levels == 4 ? 1 : 0;
+    threes -= levels == 3 ? 1 : 0;
     std::swap(src, dst);
   }
   if (result_in_b) *result_in_b = (iters & 1);

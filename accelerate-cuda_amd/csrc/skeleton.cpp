@@ -934,13 +934,13 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
         for (int ty = std::min(tune("stencil.flat_rows", 2), 4); ty > 0 && sp->flat_rows == 0; --ty)
           if ((2 * ry + ty) * (2 * rz + 1 + sp->flat_prefetch) * (sp->svec + 2 * rx) * words <= 192) sp->flat_rows = ty;
       }
-      // Two applications a launch, for calls that make many: of one array of 4- or 8-byte elements whose result is its
+      // Three or four applications a launch, for calls that make many: of one array of 4- or 8-byte elements whose result is its
       // source the next time, with taps no more than a row and a column away and nothing else to read.
       if (sp->out_rank == 2 && d->kind == ACC_SKEL_STENCIL && sp->stencil_in_comps.size() == 1 && sp->comp_types.empty() &&
           sp->stencil_in_comps[0] == sp->elt_type && sp->env.empty() && type_size(sp->elt_type) >= 4) {
         int far = 0;
         for (size_t k = 0; k < sp->tap_dx.size(); ++k) far = std::max({far, std::abs(sp->tap_dx[k]), std::abs(sp->tap_dy[k])});
-        if (far <= 1 && sp->svec >= 2 && sp->svec <= 4) sp->pair_rows = std::max(0, std::min(tune("stencil.pair_rows", 4), 16));
+        sp->pair_form = far <= 1 && sp->svec >= 2 && sp->svec <= 4;
       }
       if (sp->zmarch && 2 * rx * (2 * ry + sp->tile_z) > 64) return fail(ACC_ERR_INVALID, "stencil: strip too tall for its reach");
       if (sp->tile_h < 1 || sp->prefetch < 0 || sp->prefetch > 8 || sp->tile_z < 1 || sp->tile_z > 8) return fail(ACC_ERR_INVALID, "stencil: bad tile shape");
@@ -1018,13 +1018,13 @@ SkelSpec spec_of_variant(const SkelSpec &base, int v)
     spec.svec = std::max(1, spec.svec >> (v / 2));
     spec.tile_w = 64 * spec.svec;
   }
-  // ... 10 and 11: two applications a launch; and 8 and 9: lanes over the vectors of a whole plane
+  // ... 10 and 11: three or four applications a launch; and 8 and 9: lanes over the vectors of a whole plane
   if (spec.kind == ACC_SKEL_STENCIL && v >= 10) {
     spec.stencil_pair = true;
     spec.stencil_nd = false;
     spec.svec = base.svec;
     spec.tile_w = 62 * spec.svec;
-    spec.tile_h = spec.pair_rows;
+    spec.tile_h = 1;
   } else if (spec.kind == ACC_SKEL_STENCIL && v >= 8) {
     spec.stencil_flat = true;
     spec.stencil_nd = false;
@@ -1194,6 +1194,15 @@ int acc_skel_s::load_variant(int v)
       }
     }
   }
+  if (spec.stencil_pair) {
+    const std::string three = entry_name + "_three";
+    e = hipModuleGetFunction(&var.fn_three, var.module, three.c_str());
+    if (e != hipSuccess) {
+      (void)hipModuleUnload(var.module);
+      var.module = nullptr;
+      return acc::fail_hip(e, ("hipModuleGetFunction(" + three + ")").c_str());
+    }
+  }
   (void)hipFuncGetAttribute(&var.num_regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, var.fn);
   if (this->spec.scan_shape_open && v < 2) {
     // the first build of a scan decides its tile shape: see make_spec
@@ -1222,13 +1231,13 @@ static int variant_count(const acc::SkelSpec &sp)
   const bool stencil = sp.kind == ACC_SKEL_STENCIL || sp.kind == ACC_SKEL_STENCIL2;
   if ((sp.kind == ACC_SKEL_FOLDSEG || sp.kind == ACC_SKEL_FOLD1SEG) && sp.out_rank <= 1) return 8;
   if (sp.map_tiled) return 4;
-  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : sp.pair_rows > 0 ? 12 : sp.flat_rows > 0 ? 10 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
+  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : sp.pair_form ? 12 : sp.flat_rows > 0 ? 10 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
 }
 
 // ... one of which is left out: of a 2-D stencil with two applications a launch (10 and 11) the form that 3-D ones have at 8 and 9
 static bool variant_exists(const acc::SkelSpec &sp, int v)
 {
-  return v >= 0 && v < variant_count(sp) && !(sp.pair_rows > 0 && (v == 8 || v == 9));
+  return v >= 0 && v < variant_count(sp) && !(sp.pair_form && (v == 8 || v == 9));
 }
 
 static int no_such_variant(const char *who, const acc::SkelSpec &sp)

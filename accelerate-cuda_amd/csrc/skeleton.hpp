@@ -38,8 +38,8 @@ struct SkelSpec {
   int boundary2 = 0;
   std::string boundary2_constant, stencil_in2_type;
   std::vector<int> tap2_dz, tap2_dy, tap2_dx;
-  bool stencil_pair = false;            // a stencil's variants 10 and 11: two applications a launch (skel_stencil_pair.h)
-  int pair_rows = 0;                    // ... their rows a strip; 0: no such variants
+  bool stencil_pair = false;            // a stencil's variants 10 and 11: three or four applications a launch (skel_stencil_pair.h)
+  bool pair_form = false;               // ... whether there are any
   bool stencil_flat = false;            // a stencil's variants 8 and 9: lanes over the vectors of a plane (skel_stencil_flat.h)
   int flat_rows = 0, flat_prefetch = 0; // ... their rows a lane and planes asked for ahead; 0 rows: no such variants
   bool stencil_nd = false;              // an element a thread (skel_stencil_nd.h): rank > 3, or taps further away than the strips' windows hold
@@ -81,6 +81,7 @@ struct Variant {
   hipFunction_t fn_claim = nullptr;    // a permute whose combination is the new value: permute_claim (skel_scatter.h)
   hipFunction_t fn_across = nullptr;   // fold along the innermost dimension: _across, a lane per row of any length
   hipFunction_t fn_across_wide = nullptr;   // ... _across_wide, several rows a lane (elements of at most 8 bytes)
+  hipFunction_t fn_three = nullptr;    // a stencil's variants 10 and 11: three applications a launch (fn makes four)
   hipFunction_t fn_sweep = nullptr;    // a segmented fold's variants 4-7: _sweep, the segments that were handed over;
                                        // its variants 0-3: _probe, a look at the segment lengths
   int num_regs = 0;

@@ -58,6 +58,32 @@ def test_pairs_against_single_applications(ctx, boundary, ctype, dt, taps):
             assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][2], got[1][2]), (shape, shift, iters)
 
 
+@pytest.mark.parametrize("boundary", ["clamp", "mirror", "wrap", "constant"])
+@pytest.mark.parametrize("ctype,dt,taps", [("float", np.float32, BOX), ("double", np.float64, BOX), ("Int32", np.int32, CROSS), ("float", np.float32, COLUMNS)])
+def test_walks_and_counts(ctx, boundary, ctype, dt, taps):
+    """every count of applications whose launches split differently, walks that end amid the steps written out, inside the
+    array and cut short by its end; one application a launch is the reference, bit by bit"""
+    import acchip as A
+    fn = " + ".join("(%s)%s * t%d" % (ctype, (3 + 2 * k) if dt == np.int32 else repr(0.07 * (k + 1) - 0.2), k) for k in range(len(taps)))
+    desc = dict(out_rank=2, taps=taps, boundary=boundary, stencil_fn=fn, boundary_constant="(%s)7" % ctype if boundary == "constant" else None)
+    with A.tuning("stencil.pair=0", ctx):
+        ones = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+    own = 60 * (16 // np.dtype(dt).itemsize)
+    rng = np.random.default_rng(7)
+    for walk, shape, counts in ((0, (29, 2 * own + 9), range(1, 15)), (28, (90, own + 24), (4, 9)), (5, (37, 2 * own - 8), (4, 9)), (1, (6, own + 16), (5, 9))):
+        with A.tuning("stencil.pair_walk=%d" % walk, ctx):
+            many = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+        for iters in counts:
+            print(ctype, len(taps), boundary, walk, shape, iters, flush=True)
+            x = rng.integers(-50, 50, shape).astype(dt)
+            got = []
+            for sk in (many, ones):
+                a, b = ctx.array(x), ctx.array(np.full(shape, 77, dt))
+                res = sk.stencil_iterate(None, a, b, iters)
+                got.append((res is b, a.get(), b.get()))
+            assert got[0][0] == got[1][0] and all(np.array_equal(got[0][k], got[1][k]) for k in (1, 2)), (walk, shape, iters)
+
+
 @pytest.mark.parametrize("what,rank,shape", [("acc_pair_own", 2, (40, 300)), ("acc_flat_source", 3, (5, 7, 700))])
 def test_a_form_that_cannot_be_built_leaves_the_call_to_another(ctx, what, rank, shape):
     """a preamble that takes a name which only this form's template has: the form does not compile, the others do"""
