@@ -105,7 +105,6 @@ void set_default_tuning(TuningPtr t);
   X(stencil_pair, "stencil.pair", 1)                                                                                    \
   X(stencil_pair_walk, "stencil.pair_walk", 0)                                                                          \
   X(stencil_flat, "stencil.flat", 1)                                                                     \
-  X(stencil_flat_walk, "stencil.flat_walk", 0)                                                                         \
   X(stencil_half_strips, "stencil.half_strips", 1)                                                                     \
   X(map_tiled_min_w, "map.tiled_min_w", 33)                                                                          \
   X(map_tiled_min_h, "map.tiled_min_h", 10)                                                                          \

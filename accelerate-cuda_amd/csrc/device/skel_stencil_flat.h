@@ -1,38 +1,44 @@
 /*
- * skel_stencil_flat.h -- 3-D stencils with taps in other planes, on volumes whose rows do not divide into strips.
+ * skel_stencil_flat.h -- 3-D stencils with taps in other planes, the lanes over the vectors of a plane.
  *
  * The strips of skel_stencil.h are 64 lanes of one row each: a row of 300 columns is two strips of 256 or three of 128,
- * of which a fifth of the lanes lie outside the volume, every strip ends amid a cache line that another one writes the
- * rest of, and what stands left and right of a strip is gathered for every plane anew.  Here the lanes are laid over the
- * vectors of a whole plane, row after row (bands of ACC_TZ rows): a wave takes 64 consecutive vectors wherever rows end
- * among them, so no lane is idle and consecutive waves read and write consecutive memory.  A wave walks through
- * `acc_walk` planes with the rows that its results read in registers, ACC_NZ rows side by side of 2 rz + 1 planes and
- * those asked for ahead, as the strips do.  What differs:
- *   - the columns left and right of a lane's vector are read by the lane itself, from the cache lines its neighbours
- *     read at the same time; no lane hands anything to another, so it does not matter where its neighbours are;
- *   - the boundary condition along rows and columns is worked out once, before the walk: it is the offset within a
- *     plane that each of the lane's reads goes to, the same in every plane;
- *   - the last vector of a row ends where the row ends (it overlaps its neighbour, whose columns it produces a second
- *     time, the same values).
- * The planes of a run that are read by the run before or after it, and the rows shared with the wave before or after,
- * come out of the L2: a die takes one contiguous run of the workgroups.
+ * of which a fifth of the lanes lie outside the volume, and every strip ends amid a cache line that another one writes the
+ * rest of.  Here the lanes are laid over the vectors of a whole plane, row after row: a wave takes 62 consecutive vectors
+ * wherever rows end among them, and one more at either end whose columns its neighbours ask for, so no lane is idle and
+ * consecutive waves read and write consecutive memory.  A wave makes ACC_FLAT_PLANES planes of the result, written out; it
+ * asks for the first ACC_FIRST planes it reads at once -- all of them for a stencil that reads few rows -- and for the others
+ * one by one.
+ *   - The columns left and right of a lane's vector come from the lanes beside it (DPP wave shifts), at the ends of a row
+ *     from the boundary condition; under `wrap` those lanes read the other end of the row, the others all ask for one
+ *     element.  (Taps two columns away are read by the lane itself, as all were: 300^3 with 7 points 51 us against 44.)
+ *   - The boundary condition along rows and columns is worked out once: it is the offset within a plane that each of the
+ *     lane's reads goes to, the same in every plane.
+ *   - The last vector of a row ends where the row ends (it overlaps its neighbour, whose columns it produces a second
+ *     time, the same values); the two hand each other what stands beside the other's columns.
+ *   - A die takes an eighth of every plane, the same one, so that the rows that neighbouring planes share are in its L2, and
+ *     all dies go through the volume together: what is in flight is a few planes, not the whole volume.  (Every die a run
+ *     of planes of its own: 47 us instead of 44.)
  *
- * What bounds it: the memory side.  7 points on 300^3 Float32, 216 MB: 77 us in strips, which read 1.86 and wrote 1.32
- * times what they had to; 54.6 us (4.0 TB/s) here, reading 1.11 and writing 1.06 times, with less than half the vector
- * instructions.  (The same launch on operands that the memory-side cache holds: 35 us.)  Non-temporal stores, a wave
- * through 8 planes, 57.1 us, ordinary ones 60.0; workgroups of 1024 64, of 64 63.
+ * What bounds it: the memory side; a copy of the same bytes takes 36 us.  300^3 Float32, 7 points: 77 us in strips, 54.4 in
+ * waves that walked through 8 planes and read the columns beside a vector themselves, 45.2 (4.8 TB/s) so; 27 points 97 /
+ * 64 / 51; Float64 131 / 103 / 88 and 167 / 118 / 113; 150^3 15.0 / 8.7 / 7.1.  Planes a wave, all at once / one asked for
+ * ahead: 2 49.7, 4 45.7 / 47.4, 8 - / 47.7; with 27 points 67.5, 58.4 / 57.5, - / 51.3.  Two rows a lane: 47.4, with 27
+ * points the same.  Ordinary stores instead of non-temporal ones: 47.8.
  *
- * Generated definitions expected: those of skel_stencil.h, for ACC_STENCIL_RANK 3 and one source; the planes of source
- * and result are smaller than 4 GB (the driver sees to it), the rows no shorter than a vector.
+ * Generated definitions expected: those of skel_stencil.h, for ACC_STENCIL_RANK 3 and one source of one component, and
+ * ACC_FLAT_PLANES, ACC_FLAT_SPREAD (waves of a plane for each die from which planes are dealt out over the dies); the planes of
+ * source and result are smaller than 4 GB (the driver sees to it), the rows no shorter than a vector.
  */
 
 #ifndef ACC_SVEC
 #define ACC_SVEC 4
 #endif
-#define ACC_NR    (2 * ACC_RADIUS_Z + 1)              /* planes a result depends on */
-#define ACC_RING  (ACC_NR + ACC_PREFETCH)             /* planes held in registers */
+#define ACC_NR    (2 * ACC_RADIUS_Z + ACC_FLAT_PLANES)    /* planes a wave reads */
+#define ACC_FIRST (2 * ACC_RADIUS_Z + 1 + ACC_PREFETCH) /* ... of them asked for at once */
 #define ACC_WW    (ACC_SVEC + 2 * ACC_RADIUS_X)       /* row window of one lane */
-#define ACC_NZ    (2 * ACC_RADIUS_Y + ACC_TZ)         /* rows held side by side */
+#define ACC_NZ    (2 * ACC_RADIUS_Y + 1)              /* rows read of each */
+#define ACC_GIVE  (ACC_RADIUS_X == 1 ? 1 : 0)         /* lanes hand each other the columns beside their own */
+#define ACC_OWNED (ACC_WAVE - 2 * ACC_GIVE)           /* lanes whose columns are stored */
 
 #define ACC_B_CLAMP 0
 #define ACC_B_MIRROR 1
@@ -48,11 +54,26 @@ ACC_DEV int acc_flat_boundary(int i, const int sz)
   return acc_max(0, acc_min(i, sz - 1));
 }
 
-/* one component of the source as a lane sees it */
+/* the neighbouring lane's value; a lane that has no neighbour gets zero (nobody looks) */
+#define ACC_DPP_WAVE_SHL1 0x130
+template <int CTRL, typename S>
+ACC_DEV S acc_flat_shift(const S &x)
+{
+  unsigned int s[acc_words<S>::n];
+  __builtin_memcpy(s, &x, sizeof(S));
+#pragma unroll
+  for (int w = 0; w < acc_words<S>::n; ++w) s[w] = (unsigned int)__builtin_amdgcn_update_dpp(0, (int)s[w], CTRL, 0xf, 0xf, true);
+  S r;
+  __builtin_memcpy(&r, s, sizeof(S));
+  return r;
+}
+
+/* the source as a lane sees it */
 template <typename S, int MODE>
 struct acc_flat_source {
   struct row { S e[ACC_WW]; };
   struct __attribute__((aligned(ACC_ALIGNED ? ACC_SVEC * sizeof(S) : alignof(S)))) vec { S v[ACC_SVEC]; };
+  static constexpr bool GIVE = ACC_GIVE != 0, ENDS = GIVE && MODE == ACC_B_WRAP;      /* ENDS: the other end of a row is read */
   static constexpr int SIDE = ACC_RADIUS_X > 0 ? ACC_RADIUS_X : 1;
 
   const char *base;
@@ -62,21 +83,33 @@ struct acc_flat_source {
   unsigned int row_at[ACC_NZ];         /* bytes from the start of a plane to each of the rows */
   unsigned int own;                    /* ... and from the start of a row to the vector and its neighbours */
   unsigned int left[SIDE], right[SIDE];
+  unsigned int end_at[ENDS ? ACC_NZ : 1];
   unsigned int rows_in, left_in, right_in;         /* constant boundary: which of them lie inside */
-  row ring[ACC_NZ][ACC_RING];
+  bool at_left, at_right;              /* the row begins, ends with this lane's vector */
+  int rest;                            /* columns of the last vector that are not the one's before it, where that is not all of them */
+  bool last, next_last;                /* ... this lane's vector, its right neighbour's is that one */
+  row window[ACC_NR][ACC_NZ];
+  S end[ENDS ? ACC_NR : 1][ENDS ? ACC_NZ : 1];
 
   ACC_DEV void place(const int x, const int y, const int w, const int h)
   {
     rows_in = left_in = right_in = 0;
+    at_left = x == 0;
+    at_right = x + ACC_SVEC == w;
+    rest = ACC_ALIGNED ? 0 : w % ACC_SVEC;
+    last = rest != 0 && at_right && !at_left;
+    next_last = rest != 0 && !at_right && x + 2 * ACC_SVEC > w;
 #pragma unroll
     for (int p = 0; p < ACC_NZ; ++p) {
       const int gy = y - ACC_RADIUS_Y + p;
       row_at[p] = (unsigned int)acc_flat_boundary<MODE>(gy, h) * (unsigned int)w * (unsigned int)sizeof(S);
       rows_in |= (gy >= 0 && gy < h ? 1u : 0u) << p;
+      /* (the lanes amid a row all ask for the plane's first element) */
+      if (ENDS) end_at[p] = at_left ? row_at[p] + (unsigned int)(w - 1) * (unsigned int)sizeof(S) : (at_right ? row_at[p] : 0u);
     }
     own = (unsigned int)x * (unsigned int)sizeof(S);
 #pragma unroll
-    for (int j = 0; j < ACC_RADIUS_X; ++j) {
+    for (int j = 0; j < (GIVE ? 0 : ACC_RADIUS_X); ++j) {
       const int l = x - ACC_RADIUS_X + j, r = x + ACC_SVEC + j;
       left[j] = (unsigned int)acc_flat_boundary<MODE>(l, w) * (unsigned int)sizeof(S);
       right[j] = (unsigned int)acc_flat_boundary<MODE>(r, w) * (unsigned int)sizeof(S);
@@ -84,24 +117,62 @@ struct acc_flat_source {
       right_in |= (r < w ? 1u : 0u) << j;
     }
   }
-  /* plane z0 - rz + rho into ring slot `slot` */
-  ACC_DEV void fetch(const int rho, const int slot)
+  /* ask for the rows of plane z0 - rz + i (those that no tap of the stencil reads are not asked for: the compiler sees) */
+  ACC_DEV void ask(const int i)
   {
-    const int gz = z0 - ACC_RADIUS_Z + rho;
-    const char *plane = base + (Int64)acc_flat_boundary<MODE>(gz, d) * plane_bytes;
+    const char *plane = base + (Int64)acc_flat_boundary<MODE>(z0 - ACC_RADIUS_Z + i, d) * plane_bytes;
+#pragma unroll
+    for (int p = 0; p < ACC_NZ; ++p) {
+      row &r = window[i][p];
+      const vec v = *(const vec *)(plane + (row_at[p] + own));
+#pragma unroll
+      for (int k = 0; k < ACC_SVEC; ++k) r.e[ACC_RADIUS_X + k] = v.v[k];
+#pragma unroll
+      for (int j = 0; j < (GIVE ? 0 : ACC_RADIUS_X); ++j) {
+        r.e[j] = *(const S *)(plane + (row_at[p] + left[j]));
+        r.e[ACC_RADIUS_X + ACC_SVEC + j] = *(const S *)(plane + (row_at[p] + right[j]));
+      }
+      if (ENDS) end[i][p] = *(const S *)(plane + end_at[p]);
+    }
+  }
+  /* what stands beside the lane's columns, and outside */
+  ACC_DEV void settle(const int i)
+  {
+    const int gz = z0 - ACC_RADIUS_Z + i;
     const bool plane_in = MODE != ACC_B_CONSTANT || (gz >= 0 && gz < d);
 #pragma unroll
     for (int p = 0; p < ACC_NZ; ++p) {
-      row &r = ring[p][slot];
-      const vec v = *(const vec *)(plane + (row_at[p] + own));
+      row &r = window[i][p];
       const bool in = plane_in && (MODE != ACC_B_CONSTANT || ((rows_in >> p) & 1u));
 #pragma unroll
-      for (int k = 0; k < ACC_SVEC; ++k) r.e[ACC_RADIUS_X + k] = in ? v.v[k] : outside;
+      for (int k = 0; k < ACC_SVEC; ++k) r.e[ACC_RADIUS_X + k] = in ? r.e[ACC_RADIUS_X + k] : outside;
+      if (GIVE) {
+        const S *v = &r.e[ACC_RADIUS_X];
+        /* what the neighbours get: the columns at the ends, or, where the last vector of a row overlaps the one before
+         * it, those that stand beside the other's */
+        S first = v[0], back = v[ACC_SVEC - 1];
+        if (!ACC_ALIGNED) {
+          S to_left = v[ACC_SVEC - 1], to_right = v[0];                            /* (rest 1) */
 #pragma unroll
-      for (int j = 0; j < ACC_RADIUS_X; ++j) {
-        const S l = *(const S *)(plane + (row_at[p] + left[j])), t = *(const S *)(plane + (row_at[p] + right[j]));
-        r.e[j] = (MODE != ACC_B_CONSTANT || (in && ((left_in >> j) & 1u))) ? l : outside;
-        r.e[ACC_RADIUS_X + ACC_SVEC + j] = (MODE != ACC_B_CONSTANT || (in && ((right_in >> j) & 1u))) ? t : outside;
+          for (int k = 2; k < ACC_SVEC; ++k) {
+            to_left = rest == k ? v[ACC_SVEC - k] : to_left;
+            to_right = rest == k ? v[k - 1] : to_right;
+          }
+          first = last ? to_left : first;
+          back = next_last ? to_right : back;
+        }
+        const S l = acc_flat_shift<ACC_DPP_WAVE_SHR1>(back), t = acc_flat_shift<ACC_DPP_WAVE_SHL1>(first);
+        const S beyond_l = MODE == ACC_B_CONSTANT ? outside : (MODE == ACC_B_WRAP ? end[ENDS ? i : 0][ENDS ? p : 0] : v[MODE == ACC_B_MIRROR && ACC_SVEC > 1 ? 1 : 0]);
+        const S beyond_r = MODE == ACC_B_CONSTANT ? outside : (MODE == ACC_B_WRAP ? (at_left ? v[0] : end[ENDS ? i : 0][ENDS ? p : 0]) : v[MODE == ACC_B_MIRROR && ACC_SVEC > 1 ? ACC_SVEC - 2 : ACC_SVEC - 1]);
+        r.e[0] = at_left ? beyond_l : l;
+        r.e[ACC_WW - 1] = at_right ? beyond_r : t;
+      } else {
+#pragma unroll
+        for (int j = 0; j < ACC_RADIUS_X; ++j) {
+          if (MODE != ACC_B_CONSTANT) break;
+          r.e[j] = (in && ((left_in >> j) & 1u)) ? r.e[j] : outside;
+          r.e[ACC_RADIUS_X + ACC_SVEC + j] = (in && ((right_in >> j) & 1u)) ? r.e[ACC_RADIUS_X + ACC_SVEC + j] : outside;
+        }
       }
     }
   }
@@ -115,19 +186,35 @@ stencil(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk ACC_GU
   ACC_GUARD_CHECK
   typedef ACC_ELT T;
   ACC_ENV_ASSUME
+  (void)acc_walk;
   const int acc_d = (int)shOut_2, acc_h = (int)shOut_1, acc_w = (int)shOut_0;
   /* (the driver counts the waves by the same numbers, all of them within 32 bits) */
-  const unsigned int acc_vectors = ((unsigned int)acc_w + ACC_SVEC - 1) / ACC_SVEC, acc_bands = ((unsigned int)acc_h + ACC_TZ - 1) / ACC_TZ;
-  const unsigned int acc_per_plane = acc_vectors * acc_bands, acc_waves = (acc_per_plane + ACC_WAVE - 1) / ACC_WAVE;
-  const unsigned int acc_number = (unsigned int)acc_xcd_contiguous_block() * (ACC_BLOCK / ACC_WAVE) +
-                              (unsigned int)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  const unsigned int acc_run = acc_number / acc_waves;
-  const int acc_z0 = (int)acc_run * acc_walk;
-  if (acc_z0 >= acc_d) return;                                   /* whole wave leaves together */
-  const int acc_planes = acc_min(acc_walk, acc_d - acc_z0);
-  /* (lanes beyond the last vector of a plane do the last one again) */
-  const unsigned int acc_id = acc_min<unsigned int>((acc_number - acc_run * acc_waves) * ACC_WAVE + (unsigned int)acc_lane(), acc_per_plane - 1);
-  const int acc_y = (int)(acc_id / acc_vectors) * ACC_TZ;
+  const unsigned int acc_vectors = ((unsigned int)acc_w + ACC_SVEC - 1) / ACC_SVEC, acc_per_plane = acc_vectors * (unsigned int)acc_h;
+  const unsigned int acc_waves = (acc_per_plane + ACC_OWNED - 1) / ACC_OWNED;
+  constexpr unsigned int acc_waves_of_block = ACC_BLOCK / ACC_WAVE;
+  const unsigned int acc_mine = (unsigned int)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  unsigned int acc_run, acc_nth;                       /* which planes, and which wave of them */
+  if (acc_waves >= 8 * ACC_FLAT_SPREAD) {
+    /* a die takes an eighth of every plane, and all dies go through the planes together */
+    const unsigned int acc_die = blockIdx.x % ACC_XCDS, acc_turn = blockIdx.x / ACC_XCDS;
+    const unsigned int acc_blocks = ((acc_waves + ACC_XCDS - 1) / ACC_XCDS + acc_waves_of_block - 1) / acc_waves_of_block;
+    const unsigned int acc_from = acc_waves * acc_die / ACC_XCDS, acc_to = acc_waves * (acc_die + 1) / ACC_XCDS;
+    acc_run = acc_turn / acc_blocks;
+    acc_nth = acc_from + (acc_turn - acc_run * acc_blocks) * acc_waves_of_block + acc_mine;
+    if (acc_nth >= acc_to) return;                               /* whole wave leaves together */
+  } else {
+    /* planes of a few waves: a die takes one contiguous run of them */
+    const unsigned int acc_number = (unsigned int)acc_xcd_contiguous_block() * acc_waves_of_block + acc_mine;
+    acc_run = acc_number / acc_waves;
+    acc_nth = acc_number - acc_run * acc_waves;
+  }
+  const int acc_z0 = (int)acc_run * ACC_FLAT_PLANES;
+  if (acc_z0 >= acc_d) return;
+  /* (lanes before the first and beyond the last vector of a plane do that one again, and store nothing) */
+  const int acc_place = (int)(acc_nth * ACC_OWNED) + acc_lane() - ACC_GIVE;
+  const bool acc_stores = (!ACC_GIVE || (acc_lane() > 0 && acc_lane() < ACC_WAVE - 1)) && acc_place < (int)acc_per_plane;
+  const unsigned int acc_id = (unsigned int)acc_max(0, acc_min(acc_place, (int)acc_per_plane - 1));
+  const int acc_y = (int)(acc_id / acc_vectors);
   const int acc_x = acc_min((int)(acc_id % acc_vectors) * ACC_SVEC, acc_w - ACC_SVEC);
 
 #define ACC_DECLARE_A(c, CT, OUTSIDE, arg)                                                          \
@@ -140,48 +227,40 @@ stencil(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk ACC_GU
 #undef ACC_DECLARE_A
 #define ACC_CALL_A(c, CT, OUTSIDE, call) acc_a##c.call;
 #define ACC_EACH(call) do { ACC_SRC1_COMPONENTS(ACC_CALL_A, call) } while (0)
-
-  const int acc_total = acc_planes + 2 * ACC_RADIUS_Z;
 #pragma unroll
-  for (int acc_rho = 0; acc_rho < ACC_RING - 1; ++acc_rho) ACC_EACH(fetch(acc_min(acc_rho, acc_total - 1), acc_rho));
+  for (int acc_i = 0; acc_i < acc_min(ACC_NR, ACC_FIRST); ++acc_i) ACC_EACH(ask(acc_i));
   __builtin_amdgcn_sched_barrier(0);                     /* (every request ahead of anything that waits for one) */
+#pragma unroll
+  for (int acc_i = 0; acc_i < 2 * ACC_RADIUS_Z; ++acc_i) ACC_EACH(settle(acc_i));
 
-  for (int acc_zb = 0; acc_zb < acc_planes; acc_zb += ACC_RING) {
 #pragma unroll
-    for (int acc_s = 0; acc_s < ACC_RING; ++acc_s) {
-      const int acc_z = acc_zb + acc_s;
-      if (acc_z < acc_planes) {
-        /* asked for without a test -- a load under a condition is waited for on the spot: past the end of the run the
-         * last plane again, into a slot nothing reads any more */
-        ACC_EACH(fetch(acc_min(acc_z + ACC_RING - 1, acc_total - 1), (acc_s + ACC_RING - 1) % ACC_RING));
-        __builtin_amdgcn_sched_barrier(0);
+  for (int acc_z = 0; acc_z < ACC_FLAT_PLANES; ++acc_z) {
+    if (acc_z0 + acc_z >= acc_d) return;                           /* the last run may be short */
+    if (acc_z + ACC_FIRST < ACC_NR) ACC_EACH(ask(acc_z + ACC_FIRST));
+    __builtin_amdgcn_sched_barrier(0);
+    ACC_EACH(settle(acc_z + 2 * ACC_RADIUS_Z));
+    acc_out_vec acc_res;
 #pragma unroll
-        for (int acc_py = 0; acc_py < ACC_TZ; ++acc_py) {
-          acc_out_vec acc_res;
-#pragma unroll
-          for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) {
-#define ACC_WINDOW_READ(c, dz, dy, dx) acc_a##c.ring[acc_py + ACC_RADIUS_Y + (dy)][(acc_s + ACC_RADIUS_Z + (dz)) % ACC_RING].e[ACC_RADIUS_X + acc_k + (dx)]
-            ACC_STENCIL_TAPS1(ACC_WINDOW_READ)
+    for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) {
+#define ACC_WINDOW_READ(c, dz, dy, dx) acc_a##c.window[acc_z + ACC_RADIUS_Z + (dz)][ACC_RADIUS_Y + (dy)].e[ACC_RADIUS_X + acc_k + (dx)]
+      ACC_STENCIL_TAPS1(ACC_WINDOW_READ)
 #undef ACC_WINDOW_READ
-            acc_res.v[acc_k] = (T)(ACC_STENCIL_FN);
-          }
-          if (ACC_TZ > 1 && acc_y + acc_py >= acc_h) continue;       /* the last band of rows may be short */
-#define ACC_STORE_COMPONENT(c, CT)                                                                  \
-          {                                                                                         \
-            typedef CT acc_out_native __attribute__((ext_vector_type(ACC_SVEC)));                   \
-            typedef acc_out_native acc_out_stored __attribute__((aligned(ACC_ALIGNED ? ACC_SVEC * sizeof(CT) : alignof(CT)))); \
-            char *plane = (char *)arrOut_##c + (Int64)(acc_z0 + acc_z) * ((Int64)acc_h * acc_w * (Int64)sizeof(CT)); \
-            const unsigned int at = ((unsigned int)(acc_y + acc_py) * (unsigned int)acc_w + (unsigned int)acc_x) * (unsigned int)sizeof(CT); \
-            acc_out_native nv;                                                                      \
-            _Pragma("unroll") for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) nv[acc_k] = ACC_COMPONENT(acc_res.v[acc_k], c); \
-            if (ACC_STENCIL_NT & 1) __builtin_nontemporal_store(nv, (acc_out_stored *)(plane + at)); \
-            else                    *(acc_out_stored *)(plane + at) = nv;                           \
-          }
-          ACC_FOR_COMPONENTS(ACC_STORE_COMPONENT)
-#undef ACC_STORE_COMPONENT
-        }
-      }
+      acc_res.v[acc_k] = (T)(ACC_STENCIL_FN);
     }
+    if (!acc_stores) continue;
+#define ACC_STORE_COMPONENT(c, CT)                                                                  \
+    {                                                                                               \
+      typedef CT acc_out_native __attribute__((ext_vector_type(ACC_SVEC)));                       \
+      typedef acc_out_native acc_out_stored __attribute__((aligned(ACC_ALIGNED ? ACC_SVEC * sizeof(CT) : alignof(CT)))); \
+      char *plane = (char *)arrOut_##c + (Int64)(acc_z0 + acc_z) * ((Int64)acc_h * acc_w * (Int64)sizeof(CT)); \
+      const unsigned int at = ((unsigned int)acc_y * (unsigned int)acc_w + (unsigned int)acc_x) * (unsigned int)sizeof(CT); \
+      acc_out_native nv;                                                                          \
+      _Pragma("unroll") for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) nv[acc_k] = ACC_COMPONENT(acc_res.v[acc_k], c); \
+      if (ACC_STENCIL_NT & 1) __builtin_nontemporal_store(nv, (acc_out_stored *)(plane + at));    \
+      else                    *(acc_out_stored *)(plane + at) = nv;                               \
+    }
+    ACC_FOR_COMPONENTS(ACC_STORE_COMPONENT)
+#undef ACC_STORE_COMPONENT
   }
 #undef ACC_EACH
 #undef ACC_CALL_A

@@ -1300,42 +1300,6 @@ int acc_exec_permute(acc_skel s, const acc_array *env, int64_t n_src, const acc_
   return rc;
 }
 
-// Planes that a wave of a stencil's variants 8 and 9 walks through (skel_stencil_flat.h), `per_plane` waves side by side.
-// 16, halved to 4 while there are fewer than sixteen waves for a compute unit, and 2 if there are then not even two; every
-// run reads 2 rz planes beyond its own.  Unless that number leaves a compute unit with workgroups to itself while the
-// others have ended: the launch takes as long as the unit with the most workgroups, a workgroup by itself 1.3 times what
-// it takes of one that is full, and where another number of planes shortens that by an eighth it is taken (us with 4 / 5 / 8 /
-// 9 / 18 planes: 7 points on 83 x 84 x 300 7.2 / 6.1 / 7.7 / 8.2 / 13, 27 points 10.9 / 8.8 / 11.7 / 12.7 / 22, on 222 x
-// 223 x 508 53 / 49 / 49 / 46 / 43, on 300^3 54 / 53 / 50 / 46 / 43).
-static int64_t flat_walk(acc_skel_s *s, int v, int64_t per_plane, int64_t planes)
-{
-  if (s->knobs.stencil_flat_walk > 0) return s->knobs.stencil_flat_walk;
-  const int64_t per_block = s->spec.block / 64, cus = s->ctx->props.multiProcessorCount, held = s->variants[v].blocks_per_cu;
-  auto waves = [&](int64_t walk) { return per_plane * ((planes + walk - 1) / walk); };
-  int64_t walk = 16;
-  while (walk > 4 && waves(walk) < 16 * cus) walk /= 2;
-  if (walk > 2 && waves(walk) < 2 * cus) walk = 2;
-  auto groups = [&](int64_t k) { return ((waves(k) + per_block - 1) / per_block + cus - 1) / cus; };
-  auto longest = [&](int64_t k) {
-    const int64_t last = groups(k) % held;
-    return (10 * (groups(k) - last) + (last == 1 ? 13 : 10 * last)) * (k + 2 * s->spec.reach_z);
-  };
-  if (groups(walk) <= 1) return walk;
-  const int64_t as_is = longest(walk);
-  int64_t best = as_is, at = walk;
-  for (int64_t k = 3; k <= 20; ++k) {
-    // (a unit with less to do than three workgroups waits for memory; with rows off the 16-byte boundary more of them pay:
-    // 391 x 234 x 242 37 us with 8 planes and 42 with 15)
-    if (groups(walk) == 2 ? groups(k) != 1 : ((v & 1) != 0 || groups(k) < 3)) continue;
-    const int64_t l = longest(k);
-    if (l < best) {
-      best = l;
-      at = k;
-    }
-  }
-  return best * 8 < as_is * 7 ? at : walk;
-}
-
 // `in2` is the second source of a stencil2, NULL for a stencil
 static int stencil_once(acc_skel s, const acc_array *env, const acc_array *in, const acc_array *in2, const acc_array *out, hipStream_t st)
 {
@@ -1388,29 +1352,27 @@ static int stencil_once(acc_skel s, const acc_array *env, const acc_array *in, c
     const int64_t grid = acc_launch_grid(array_size(*out), s->spec.block, resident(s, v), s->knobs.map_oversub);
     return launch(s, v, grid, 0, st, &args);
   }
-  // A volume whose rows do not divide into strips takes variants 8 and 9, lanes over the vectors of a whole plane, where
-  // the instance has them (skel_stencil_flat.h; us in strips / so: 7 points Float32 300^3 52 / 35, 400^3 151 / 116,
-  // 200 x 200 x 300 35 / 26, 150^3 12.5 / 7.7, 129 x 130 x 1500 31.9 / 31.2, 118 x 118 x 3000 84 / 80, 45 x 46 x 1000 7.7 /
-  // 6.2; 27 points 289 x 290 x 300 66 / 42, 158 x 159 x 1000 49 / 44, 64 x 65 x 500 10.0 / 8.9; Float64 300^3 130 / 101).
-  // Beyond 512 MB of source and result what counts is how much of the strips lies outside the array: a third 263 / 205 us
-  // (450 x 451 x 516), a fifth 223 / 199 (418 x 418 x 600; but 184 / 190, with 27 points 185 / 210, in two strips, 512 x
-  // 512 x 400), a tenth and less 187 / 198 (323 x 324 x 1000), 193 / 203 (273 x 274 x 1400), with 27 points 187 / 205, 195 /
-  // 216.  (27 points of Float64 win by half on average up to there, but lose a tenth in some shapes: 196 x 323 x 351 95 / 107.)
-  const int64_t half = (int64_t)32 * s->spec.svec, halves = (w + half - 1) / half;
-  const int64_t covered = half * (halves <= 3 ? halves : (halves + 1) / 2 * 2);        // columns of all strips (half ones up to three)
-  const bool small = array_size(*out) * (int64_t)(s->spec.elt_size + acc::type_size(s->spec.stencil_in_comps[0])) <= ((int64_t)512 << 20);
-  const bool idle = (covered - w) * 6 > covered && halves != 4;
-  if (s->spec.flat_rows > 0 && s->knobs.stencil_flat != 0 && w >= s->spec.svec &&
-      ((w % (2 * half) != 0 && (small || idle)) || s->knobs.stencil_flat == 2)) {
-    const int64_t rows = s->spec.flat_rows, per_block = s->spec.block / 64;
-    const int64_t per_plane = (((w + s->spec.svec - 1) / s->spec.svec) * ((h + rows - 1) / rows) + 63) / 64;
+  // A volume takes variants 8 and 9, lanes over the vectors of a whole plane, where the instance has them
+  // (skel_stencil_flat.h; us in strips / so, buffers that the memory-side cache does not hold: 7 points Float32 300^3 77 /
+  // 45.3, 256^3 30.6 / 28.4, 128 x 128 x 256 9.0 / 7.5, 300 x 512 x 512 135 / 131, 418 x 418 x 600 222 / 173, 273 x 274 x 1400
+  // 190 / 178; 27 points 256^3 36.5 / 31.7, 323 x 324 x 1000 226 / 192; Float64 400^3 248 / 217, 27 points 316 / 258).  Only
+  // where rows are whole strips and the arrays large, so that planes lie far apart, are strips ahead that walk through many
+  // of them: 512^3 195 / 231 (27 points 240 / 234), 256 x 512 x 512 Float64 192 / 243.
+  const bool small = array_size(*out) * (int64_t)(s->spec.elt_size + acc::type_size(s->spec.stencil_in_comps[0])) <= ((int64_t)768 << 20);
+  if (s->spec.flat_planes > 0 && s->knobs.stencil_flat != 0 && w >= s->spec.svec &&
+      (w % ((int64_t)64 * s->spec.svec) != 0 || small || s->knobs.stencil_flat == 2)) {
+    const int64_t deep = s->spec.flat_planes, per_block = s->spec.block / 64;
+    const int64_t owned = s->spec.reach_x == 1 ? 62 : 64;          // lanes that store: the others hand over columns
+    const int64_t per_plane = (((w + s->spec.svec - 1) / s->spec.svec) * h + owned - 1) / owned, runs = (planes + deep - 1) / deep;
     // the kernel counts lanes and waves in 32 bits, and bytes within a plane of source and result
     const int64_t widest = std::max(s->spec.elt_size, 8);
     const int v = (aligned ? 0 : 1) + 8;
-    if (w * h * widest < ((int64_t)1 << 32) && planes < ((int64_t)1 << 30) && per_plane * planes < ((int64_t)1 << 30) && may_take(s, v, st)) {
-      const int64_t walk = flat_walk(s, v, per_plane, planes);
-      args.i32(static_cast<int32_t>(walk));
-      return launch(s, v, (per_plane * ((planes + walk - 1) / walk) + per_block - 1) / per_block, 0, st, &args);
+    if (w * h * widest < ((int64_t)1 << 32) && planes < ((int64_t)1 << 30) && per_plane * 8 < ((int64_t)1 << 30) && (per_plane + 40) * planes < ((int64_t)1 << 30) &&
+        may_take(s, v, st)) {
+      args.i32(0);
+      // every die an eighth of every plane, or one after the other: as the kernel numbers them
+      const int64_t grid = per_plane >= 8 * acc::flat_spread ? 8 * (((per_plane + 7) / 8 + per_block - 1) / per_block) * runs : (per_plane * runs + per_block - 1) / per_block;
+      return launch(s, v, grid, 0, st, &args);
     }
   }
   // one wave per strip of 256 columns x tile_h rows

@@ -577,6 +577,7 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
       o << "#define ACC_TILE_H " << sp.tile_h << "\n#define ACC_PREFETCH " << sp.prefetch << "\n#define ACC_BLOCK " << sp.block << "\n";
       o << "#define ACC_TZ " << sp.tile_z << "\n";
       o << "#define ACC_ZMARCH " << sp.zmarch << "\n";
+      if (sp.stencil_flat) o << "#define ACC_FLAT_PLANES " << sp.flat_planes << "\n#define ACC_FLAT_SPREAD " << flat_spread << "\n";
       tmpl = sp.stencil_pair ? "skel_stencil_pair.h" : sp.stencil_flat ? "skel_stencil_flat.h" : "skel_stencil.h";
       break;
     }
@@ -925,14 +926,23 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
       // the strip goes through planes
       sp->tile_h = sp->out_rank == 2 ? tune("stencil.tile_h", 4)
                  : (sp->out_rank == 3 ? (sp->zmarch ? tune("stencil.walk", 64) : tune("stencil.tile_h3", sp->tile_z > 1 ? 8 : 16)) : 1);
-      // The form for volumes whose rows do not divide into strips: two rows a lane, or one, as its windows stay within 192
-      // registers; of one array of 4- or 8-byte elements.  No plane is asked for ahead: a step's requests are enough
-      // (300^3, 7 points, two rows: 57.1 us with a plane ahead, 55.0 without; 300^3 Float64 68 and 60).
+      // The form with the lanes over the vectors of a plane: of one array of 4- or 8-byte elements.  A result that reads few
+      // rows (the 7 points five) is made four planes a wave, every request at once; one that reads more, whose rows are worth
+      // keeping longer, eight with a plane asked for ahead (300^3 in us, 4 planes at once / 8 one ahead: 7 points Float32
+      // 45.7 / 47.7, Float64 93.7 / 95.8; 27 points 58.4 / 51.3 and 136 / 114).
       if (sp->zmarch && d->kind == ACC_SKEL_STENCIL && sp->stencil_in_comps.size() == 1 && type_size(sp->stencil_in_comps[0]) >= 4) {
-        sp->flat_prefetch = std::max(0, std::min(tune("stencil.flat_prefetch", 0), 4));
-        const int words = (type_size(sp->stencil_in_comps[0]) + 3) / 4;
-        for (int ty = std::min(tune("stencil.flat_rows", 2), 4); ty > 0 && sp->flat_rows == 0; --ty)
-          if ((2 * ry + ty) * (2 * rz + 1 + sp->flat_prefetch) * (sp->svec + 2 * rx) * words <= 192) sp->flat_rows = ty;
+        const int row = (sp->svec + 2 * rx) * ((type_size(sp->stencil_in_comps[0]) + 3) / 4), plane = (2 * ry + 1) * row;      // registers
+        std::set<std::pair<int, int>> one, four;
+        for (size_t k = 0; k < sp->tap_dx.size(); ++k)
+          for (int j = 0; j < 4; ++j) {
+            if (j == 0) one.insert({sp->tap_dz[k], sp->tap_dy[k]});
+            four.insert({sp->tap_dz[k] + j, sp->tap_dy[k]});
+          }
+        const bool at_once = one.size() <= 6 && (int)four.size() * row <= 112;
+        if ((2 * rz + 1) * plane <= 192) {
+          sp->flat_planes = std::max(1, std::min(tune("stencil.flat_walk", at_once ? 4 : 8), 16));
+          sp->flat_prefetch = std::max(0, tune("stencil.flat_prefetch", at_once ? sp->flat_planes : (2 * rz + 2) * plane <= 144 ? 1 : 0));
+        }
       }
       // Three or four applications a launch, for calls that make many: of one array of 4- or 8-byte elements whose result is its
       // source the next time, with taps no more than a row and a column away and nothing else to read.
@@ -1030,7 +1040,7 @@ SkelSpec spec_of_variant(const SkelSpec &base, int v)
     spec.stencil_nd = false;
     spec.svec = base.svec;
     spec.tile_w = 64 * spec.svec;
-    spec.tile_z = spec.flat_rows;
+    spec.tile_z = 1;
     spec.prefetch = spec.flat_prefetch;
   }
   // a scan's variants 2 and 3: a small tile, for arrays of a few tiles at most (a lone workgroup runs through the
@@ -1231,7 +1241,7 @@ static int variant_count(const acc::SkelSpec &sp)
   const bool stencil = sp.kind == ACC_SKEL_STENCIL || sp.kind == ACC_SKEL_STENCIL2;
   if ((sp.kind == ACC_SKEL_FOLDSEG || sp.kind == ACC_SKEL_FOLD1SEG) && sp.out_rank <= 1) return 8;
   if (sp.map_tiled) return 4;
-  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : sp.pair_form ? 12 : sp.flat_rows > 0 ? 10 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
+  return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : sp.pair_form ? 12 : sp.flat_planes > 0 ? 10 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
 }
 
 // ... one of which is left out: of a 2-D stencil with two applications a launch (10 and 11) the form that 3-D ones have at 8 and 9

@@ -41,7 +41,7 @@ struct SkelSpec {
   bool stencil_pair = false;            // a stencil's variants 10 and 11: three or four applications a launch (skel_stencil_pair.h)
   bool pair_form = false;               // ... whether there are any
   bool stencil_flat = false;            // a stencil's variants 8 and 9: lanes over the vectors of a plane (skel_stencil_flat.h)
-  int flat_rows = 0, flat_prefetch = 0; // ... their rows a lane and planes asked for ahead; 0 rows: no such variants
+  int flat_planes = 0, flat_prefetch = 0;   // ... the planes a wave produces, and those it asks for ahead; 0: no such variants
   bool stencil_nd = false;              // an element a thread (skel_stencil_nd.h): rank > 3, or taps further away than the strips' windows hold
   std::vector<int> tap_off, tap2_off;   // ... its taps: n_taps rows of out_rank offsets, outermost dimension first
   int tile_w = 256, tile_h = 4, prefetch = 3;
@@ -96,6 +96,7 @@ struct Variant {
 int type_size(const std::string &t);
 int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp);
 int across_rows(const SkelSpec &sp);
+constexpr int flat_spread = 8;          // waves of a plane that a die takes at least, in the form for volumes of skel_stencil_flat.h, for every die to take a share of every plane
 int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::string *source);
 SkelSpec spec_of_variant(const SkelSpec &base, int variant);
 std::vector<std::string> compile_options(const SkelSpec &sp);

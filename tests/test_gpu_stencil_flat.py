@@ -96,3 +96,27 @@ def test_the_walk_the_driver_chooses(ctx, shape):
         sk.stencil(None, src, out)
         got.append(out.get())
     assert np.array_equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("boundary", ["clamp", "mirror", "wrap", "constant"])
+@pytest.mark.parametrize("ctype,dt,taps", [("float", np.float32, BOX), ("double", np.float64, STAR), ("Int32", np.int32, STAR)])
+def test_planes_dealt_out_over_the_dies(ctx, boundary, ctype, dt, taps):
+    """every length that a row's last vector can have, in planes of just less and just more than the eight waves a die from
+    which every die takes a share of every plane, shares of unequal size among them"""
+    import acchip as A
+    fn = " + ".join("(%s)%d * t%d" % (ctype, 3 + k % 5, k) for k in range(len(taps)))
+    desc = dict(out_rank=3, taps=taps, boundary=boundary, stencil_fn=fn, boundary_constant="(%s)7" % ctype if boundary == "constant" else None)
+    with A.tuning("stencil.flat=2", ctx):
+        flat = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+    with A.tuning("stencil.nd=1", ctx):
+        each = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+    vec = 16 // np.dtype(dt).itemsize
+    rng = np.random.default_rng(5)
+    for d, h, w in [(5, 62, 64 * vec - k) for k in range(vec + 1)] + [(9, 66, 61 * vec - 1), (3, 71, 63 * vec + 1), (13, 131, 62 * vec)]:
+        print(ctype, boundary, d, h, w, flush=True)
+        src, got = ctx.array(rng.integers(-50, 50, (d, h, w)).astype(dt)), []
+        for sk in (flat, each):
+            out = ctx.array(np.full((d, h, w), 77, dt))
+            sk.stencil(None, src, out)
+            got.append(out.get())
+        assert np.array_equal(got[0], got[1]), (d, h, w)
