@@ -76,6 +76,8 @@ void set_default_tuning(TuningPtr t);
   X(foldseg_long_from, "foldseg.long_from", 8)                                                                         \
   X(foldseg_max_split, "foldseg.max_split", 4096)                                                                      \
   X(foldseg_oversub, "foldseg.oversub", 1 << 20)                                                                       \
+  X(foldseg_spread, "foldseg.spread", 16)                                                                              \
+  X(foldseg_spread_min, "foldseg.spread_min", 2048)                                                                    \
   X(foldseg_giants, "foldseg.giants", 2)                                                                               \
   X(foldseg_giant_chunks, "foldseg.giant_chunks", 4)                                                                   \
   X(foldseg_sweep_per_cu, "foldseg.sweep_per_cu", 4)                                                                   \

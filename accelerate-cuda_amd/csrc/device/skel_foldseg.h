@@ -6,8 +6,8 @@
  * 32-lane warp (one useful load per lane and a five-step shared-memory tree
  * for a 32-element row).  With 64-lane waves and short segments most of that
  * would idle, so the work is split the other way round:
- *   - a workgroup owns ACC_BLOCK consecutive segments, i.e. ONE contiguous
- *     range of the input;
+ *   - a workgroup owns ACC_BLOCK consecutive segments (down to an eighth of
+ *     that where there are few), i.e. ONE contiguous range of the input;
  *   - all its lanes stream that range through LDS in chunks of ACC_CHUNK
  *     elements, evaluating the (fused) producer with fully coalesced, 128-bit
  *     reads whatever the segment lengths are;
@@ -216,16 +216,19 @@ ACC_FOLDSEG_ENTRY(ACC_ENV_PARAMS
   constexpr int acc_pad_mask = decltype(padded_c)::value ? ~0 : 0;
   /* (seen by all at the first barrier of the first chunk) */
 
-  for (Int64 first = (Int64)blockIdx.x * ACC_BLOCK; first < nseg; first += (Int64)gridDim.x * ACC_BLOCK) {
-    const Int64 seg = first + tid;
-    const bool live = seg < nseg;
+  /* the segments of a workgroup: a lane each, or a half, a quarter, an eighth of its lanes where the grid is larger than
+   * a lane each would make it (few segments, and the host wants more workgroups for them) */
+  int acc_own = ACC_BLOCK;
+  while (acc_own > ACC_BLOCK / 8 && (Int64)gridDim.x * acc_own >= 2 * nseg) acc_own /= 2;
+  for (Int64 first = (Int64)blockIdx.x * acc_own; first < nseg; first += (Int64)gridDim.x * acc_own) {
+    const Int64 seg = first + tid, last = acc_min<Int64>(first + acc_own, nseg);
+    const bool live = seg < last;
     /* both ends of the lane's segment are asked for at once (a lane past the last segment asks for the last one's
      * and takes nothing) */
-    const Int64 seg_c = acc_min<Int64>(seg, nseg - 1);
+    const Int64 seg_c = acc_min<Int64>(seg, last - 1);
     const Int64 a_c = ACC_SEG_AT(seg_c), b_c = ACC_SEG_END(seg_c);
     Int64 a = live ? a_c : 0;
     Int64 b = live ? b_c : 0;
-    const Int64 last = acc_min<Int64>(first + ACC_BLOCK, nseg);
     const Int64 lo = ACC_SEG_AT(first), hi = acc_min<Int64>(ACC_SEG_END(last - 1), n);
     bool handed = false;                             /* this lane's segment has been handed over (below) */
 
