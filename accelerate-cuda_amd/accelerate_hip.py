@@ -28,6 +28,7 @@ Everything runs on the GPU through the C ABI; there is no other execution path.
 """
 import collections
 import ctypes as C
+import math
 import numbers
 import re
 import threading
@@ -438,7 +439,7 @@ class _ResultPool(object):
 
     def array(self, shape, dtype):
         dtype = np.dtype(dtype)
-        size = int(np.prod(shape, dtype=np.int64))
+        size = math.prod(shape)
         nbytes = size * dtype.itemsize
         if nbytes < self.GRAIN or self.closed:
             return None
@@ -489,7 +490,7 @@ class _Resident(object):
         self.stream, self.ready = None, None          # where it was produced, and the event recorded behind that
         self.pending = None                           # the launch that will produce it, while that is put off (_Pending)
         with cx.lock:
-            cx.table.malloc(host, frozen)
+            cx.table.malloc(host, frozen, self.key)
             cx.live[self.key] = cx.live.get(self.key, 0) + 1
 
     def get(self):
@@ -499,11 +500,11 @@ class _Resident(object):
             self.pending.force()
         if self.ready is not None:
             A.check(A.lib().acc_event_sync(self.cx.ctx.handle, self.ready))
-        d = self.cx.table.acquire(self.host)
+        d = self.cx.table.acquire(self.host, key=self.key)
         try:
             return d.get(self.cx.results.array(self.shape, self.dtype))
         finally:
-            self.cx.table.release(self.host)
+            self.cx.table.release(self.host, key=self.key)
 
     def __del__(self):
         try:
@@ -515,7 +516,7 @@ class _Resident(object):
                 if cx.live[self.key] == 0:
                     del cx.live[self.key]
                     if cx.table.handle:
-                        cx.table.free(self.host)
+                        cx.table.free(self.host, self.key)
         except Exception:
             pass
 
@@ -669,7 +670,7 @@ class Context(object):
                 return None
             if isinstance(m, A.TupleArray):
                 return A.TupleArray([view(c) for c in m.comps])
-            d = self.table.acquire(m.host, stream)
+            d = self.table.acquire(m.host, stream, m.key)
             taken.append(m)
             return d
         try:
@@ -681,7 +682,7 @@ class Context(object):
                 m.stream = stream
         finally:
             for m in taken:
-                self.table.release(m.host, stream)
+                self.table.release(m.host, stream, m.key)
 
 
 def _elt(ctype):
@@ -961,10 +962,11 @@ def fold1Seg(f, a, seg_lengths, context=None):
 
 
 def _scan(kind, f, z, a, context):
-    cx = _context(context, a)
+    get = a.stream().text                # (written out once: where the scan runs is told by the arrays that it names)
+    cx = _context(context, get)
     if len(a.shape) != 1:
         raise TypeError("scans are over vectors")
-    arrays, sig, fr = _assemble(get=a.stream().text, combine=_combine(f, a.ctype).text,
+    arrays, sig, fr = _assemble(get=get, combine=_combine(f, a.ctype).text,
                                 seed=Exp.of(z, a.ctype).text if z is not None else None)
     sk = cx.skeleton(A.SCAN_KINDS[kind], _elt(a.ctype), sig, **fr)
     n = a.shape[0]

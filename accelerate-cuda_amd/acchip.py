@@ -6,6 +6,7 @@ the HIP skeletons in the shared library, and loading fails loudly if the
 library has not been built.
 """
 import ctypes as C
+import math
 import os
 import struct
 import subprocess
@@ -341,7 +342,7 @@ class DeviceArray(object):
 
     def __init__(self, ctx, shape, dtype, ptr=None, owner=True):
         self.ctx, self.shape, self.dtype = ctx, tuple(int(s) for s in shape), np.dtype(dtype)
-        self.size = int(np.prod(self.shape, dtype=np.int64)) if self.shape else 1
+        self.size = math.prod(self.shape)
         self.nbytes = self.size * self.dtype.itemsize
         self.owner = owner
         if ptr is None:
@@ -349,6 +350,13 @@ class DeviceArray(object):
             check(lib().acc_malloc(ctx.handle, self.nbytes, C.byref(p)))
             ptr = p.value
         self.ptr = ptr
+
+    @classmethod
+    def view(cls, ctx, shape, dtype, size, ptr):
+        """memory that somebody else owns, as an array: `shape` a tuple of ints, `dtype` a numpy dtype"""
+        a = cls.__new__(cls)
+        a.ctx, a.shape, a.dtype, a.size, a.nbytes, a.owner, a.ptr = ctx, shape, dtype, size, size * dtype.itemsize, False, ptr
+        return a
 
     def desc(self, shape=None, offset_elems=0):
         shape = self.shape if shape is None else tuple(shape)
@@ -361,7 +369,7 @@ class DeviceArray(object):
             out = np.empty(self.shape, dtype=self.dtype)
         assert out.flags.c_contiguous and out.dtype == self.dtype and out.size == self.size
         if self.nbytes:
-            check(lib().acc_memcpy_d2h(self.ctx.handle, out.ctypes.data_as(C.c_void_p), self.ptr, self.nbytes))
+            check(lib().acc_memcpy_d2h(self.ctx.handle, out.ctypes.data, self.ptr, self.nbytes))
         return out
 
     def set(self, host):
@@ -548,25 +556,28 @@ class MemTable(object):
         """address and length of the storage (a slice that starts where its parent starts is another array)"""
         return (host.ctypes.data ^ (host.nbytes * 0x9E3779B97F4A7C15)) & 0xFFFFFFFFFFFFFFFF
 
-    def malloc(self, host, frozen):
+    # (a caller that has an array's key at hand gives it: working it out is as dear as the call)
+    def malloc(self, host, frozen, key=None):
         """enter a C-contiguous host array; returns True if it was not in the table yet"""
         assert host.flags.c_contiguous
+        key = self.key(host) if key is None else key
         new = C.c_int()
-        check(lib().acc_memtable_malloc(self.handle, self.key(host), host.ctypes.data, host.nbytes, int(frozen), C.byref(new)))
-        self.hosts[self.key(host)] = host           # the table reads and writes this storage later
+        check(lib().acc_memtable_malloc(self.handle, key, host.ctypes.data, host.nbytes, int(frozen), C.byref(new)))
+        self.hosts[key] = host           # the table reads and writes this storage later
         return bool(new.value)
 
-    def acquire(self, host, stream=None):
+    def acquire(self, host, stream=None, key=None):
         p = C.c_uint64()
-        check(lib().acc_memtable_acquire(self.handle, self.key(host), stream, C.byref(p)))
-        return DeviceArray(self.ctx, host.shape, host.dtype, ptr=p.value, owner=False)
+        check(lib().acc_memtable_acquire(self.handle, self.key(host) if key is None else key, stream, C.byref(p)))
+        return DeviceArray.view(self.ctx, host.shape, host.dtype, host.size, p.value)
 
-    def release(self, host, stream=None):
-        check(lib().acc_memtable_release(self.handle, self.key(host), stream))
+    def release(self, host, stream=None, key=None):
+        check(lib().acc_memtable_release(self.handle, self.key(host) if key is None else key, stream))
 
-    def free(self, host):
-        check(lib().acc_memtable_free(self.handle, self.key(host)))
-        self.hosts.pop(self.key(host), None)
+    def free(self, host, key=None):
+        key = self.key(host) if key is None else key
+        check(lib().acc_memtable_free(self.handle, key))
+        self.hosts.pop(key, None)
 
     def insert_unmanaged(self, host, dev):
         check(lib().acc_memtable_insert_unmanaged(self.handle, self.key(host), dev.ptr, host.nbytes))
@@ -586,6 +597,47 @@ class MemTable(object):
 
 
 _plain_desc = DeviceArray.desc
+
+
+def _bytes(a):
+    """the descriptor of an array, or one that is given, as the bytes that the library reads"""
+    if getattr(type(a), "desc", None) is _plain_desc:                  # a DeviceArray: straight away
+        return _ARRAY[len(a.shape)](len(a.shape), 1, *a.shape, a.ptr)
+    return bytes(a if isinstance(a, acc_array) else a.desc())
+
+
+def _all(arrays):
+    """the descriptors of the free arrays, one behind the other (None: there are none)"""
+    if not arrays:
+        return None
+    return _bytes(arrays[0]) if len(arrays) == 1 else b"".join([_bytes(a) for a in arrays])
+
+
+_EXTENTS = [struct.Struct("@%dq" % r).pack for r in range(MAX_RANK + 1)]
+
+
+def _extents(shape):
+    return _EXTENTS[len(shape)](*shape) if len(shape) <= MAX_RANK else (C.c_int64 * len(shape))(*shape)
+
+
+class _Drivers(object):
+    """The drivers as the methods below call them: descriptors and extents as bytes, which are packed in a fraction of the
+    time that structures take (`lib()` has the drivers taking pointers to those).  The bytes live as long as the call, and
+    the library looks at them no longer."""
+    _P = C.c_void_p
+    _TYPES = {"acc_exec_map": (_P, _P, _P, _P), "acc_exec_fold": (_P, _P, C.c_int32, _P, _P, _P), "acc_exec_foldseg": (_P, _P, C.c_int64, _P, _P, _P),
+              "acc_exec_foldseg_nd": (_P, _P, C.c_int32, _P, _P, _P, _P), "acc_exec_scan": (_P, _P, C.c_int64, _P, _P, _P),
+              "acc_exec_scan_noalloc": (_P, _P, C.c_int64, _P, _P, _P), "acc_exec_permute": (_P, _P, C.c_int64, _P, _P, _P),
+              "acc_exec_stencil": (_P, _P, _P, _P, _P), "acc_exec_stencil2": (_P, _P, _P, _P, _P, _P),
+              "acc_exec_stencil_iterate": (_P, _P, _P, _P, C.c_int32, _P, _P)}
+
+    def __getattr__(self, name):               # (at its first call; an attribute of its own from then on)
+        f = C.CFUNCTYPE(C.c_int, *self._TYPES[name])((name, lib()))
+        setattr(self, name, f)
+        return f
+
+
+_drivers = _Drivers()
 
 
 def _env(arrays):
@@ -636,41 +688,48 @@ class Skeleton(object):
         return s.value.decode()
 
     def map(self, env, out, stream=None):
-        check(lib().acc_exec_map(self.handle, _env(env), C.byref(out if isinstance(out, acc_array) else out.desc()), stream))
+        rc = _drivers.acc_exec_map(self.handle, _all(env), _bytes(out), stream)
+        if rc:
+            check(rc)
 
     def fold(self, env, in_shape, out, stream=None):
         if isinstance(in_shape, int):
             in_shape = (in_shape,)
-        sh = (C.c_int64 * len(in_shape))(*in_shape)
-        check(lib().acc_exec_fold(self.handle, _env(env), len(in_shape), sh,
-                                  C.byref(out if isinstance(out, acc_array) else out.desc()), stream))
+        rc = _drivers.acc_exec_fold(self.handle, _all(env), len(in_shape), _extents(in_shape), _bytes(out), stream)
+        if rc:
+            check(rc)
 
     def foldseg(self, env, n, offsets, out, stream=None):
-        check(lib().acc_exec_foldseg(self.handle, _env(env), n, C.byref(offsets.desc()), C.byref(out.desc()), stream))
+        rc = _drivers.acc_exec_foldseg(self.handle, _all(env), n, _bytes(offsets), _bytes(out), stream)
+        if rc:
+            check(rc)
 
     def foldseg_nd(self, env, in_shape, offsets, out, stream=None):
-        sh = (C.c_int64 * len(in_shape))(*in_shape)
-        check(lib().acc_exec_foldseg_nd(self.handle, _env(env), len(in_shape), sh, C.byref(offsets.desc()), C.byref(out.desc()), stream))
+        check(_drivers.acc_exec_foldseg_nd(self.handle, _all(env), len(in_shape), _extents(in_shape), _bytes(offsets), _bytes(out), stream))
 
     def scan(self, env, n, out, total=None, stream=None, noalloc=False):
-        o = out if isinstance(out, acc_array) else out.desc()
-        t = None if total is None else C.byref(total if isinstance(total, acc_array) else total.desc(shape=()))
-        fn = lib().acc_exec_scan_noalloc if noalloc else lib().acc_exec_scan
-        check(fn(self.handle, _env(env), n, C.byref(o), t, stream))
+        t = None if total is None else _bytes(total) if isinstance(total, acc_array) or getattr(total, "shape", None) == () else bytes(total.desc(shape=()))
+        f = _drivers.acc_exec_scan_noalloc if noalloc else _drivers.acc_exec_scan
+        rc = f(self.handle, _all(env), n, _bytes(out), t, stream)
+        if rc:
+            check(rc)
 
     def permute(self, env, n_src, defaults, out, stream=None):
-        check(lib().acc_exec_permute(self.handle, _env(env), n_src, C.byref(defaults.desc()), C.byref(out.desc()), stream))
+        rc = _drivers.acc_exec_permute(self.handle, _all(env), n_src, _bytes(defaults), _bytes(out), stream)
+        if rc:
+            check(rc)
 
     def stencil(self, env, src, out, stream=None):
-        check(lib().acc_exec_stencil(self.handle, _env(env), C.byref(src.desc()), C.byref(out.desc()), stream))
+        rc = _drivers.acc_exec_stencil(self.handle, _all(env), _bytes(src), _bytes(out), stream)
+        if rc:
+            check(rc)
 
     def stencil2(self, env, src1, src2, out, stream=None):
-        check(lib().acc_exec_stencil2(self.handle, _env(env), C.byref(src1.desc()), C.byref(src2.desc()),
-                                      C.byref(out.desc()), stream))
+        check(_drivers.acc_exec_stencil2(self.handle, _all(env), _bytes(src1), _bytes(src2), _bytes(out), stream))
 
     def stencil_iterate(self, env, a, b, iters, stream=None):
         r = C.c_int32(0)
-        check(lib().acc_exec_stencil_iterate(self.handle, _env(env), C.byref(a.desc()), C.byref(b.desc()), iters, stream, C.byref(r)))
+        check(_drivers.acc_exec_stencil_iterate(self.handle, _all(env), _bytes(a), _bytes(b), iters, stream, C.byref(r)))
         return b if r.value else a
 
     def destroy(self):
