@@ -793,9 +793,10 @@ struct acc_merge_job {
  * LDS and wave q writes the targets of byte q -- one thread per target, so no atomics and nothing that must be in
  * the result beforehand -- and clears the carries it has taken (the table is all zero between launches).  `base` is
  * the defaults array, or the result itself where that was filled from the defaults before the main kernel (which
- * then also added to it directly).                                                                          */
+ * then also added to it directly).  It is a few round trips long: 256 rows in eight waves 4.6 us for 18 754 targets
+ * and 4.9 for 65 536, in four 5.4 and 4.9. */
 #ifndef ACC_MERGE_WAVES
-#define ACC_MERGE_WAVES 4
+#define ACC_MERGE_WAVES 8
 #endif
 static_assert(ACC_MERGE_WAVES >= 4 && ACC_MERGE_WAVES <= 16, "a wave for each byte of a row's word");
 extern "C" __global__ void __launch_bounds__(64 * ACC_MERGE_WAVES)
@@ -827,9 +828,17 @@ permute_merge(ACC_ENV_PARAMS ACC_OUT_PARAMS, const unsigned *__restrict__ dump, 
     c0 += even & 0xFFFFu; c2 += even >> 16;
     c1 += odd & 0xFFFFu;  c3 += odd >> 16;
   }
-  for (; r < nrows; r += waves) {
-    const unsigned w = __builtin_nontemporal_load(dump + (Int64)r * nd + col_c);
-    c0 += w & 0xFFu; c1 += (w >> 8) & 0xFFu; c2 += (w >> 16) & 0xFFu; c3 += w >> 24;
+  /* (the rows left over, the last one again for those that are not there: one by one they are a round trip each: 432 rows
+   * of 18 754 targets 11.5 us, 8.4 so) */
+  if (r < nrows) {
+    unsigned w[ACC_MERGE_BATCH];
+#pragma unroll
+    for (int k = 0; k < ACC_MERGE_BATCH; ++k) w[k] = __builtin_nontemporal_load(dump + (Int64)acc_min(r + waves * k, nrows - 1) * nd + col_c);
+#pragma unroll
+    for (int k = 0; k < ACC_MERGE_BATCH; ++k) {
+      const unsigned u = r + waves * k < nrows ? w[k] : 0u;
+      c0 += u & 0xFFu; c1 += (u >> 8) & 0xFFu; c2 += (u >> 16) & 0xFFu; c3 += u >> 24;
+    }
   }
   s_sum[wave][0][lane] = c0;
   s_sum[wave][1][lane] = c1;

@@ -1088,11 +1088,11 @@ int acc_exec_permute(acc_skel s, const acc_array *env, int64_t n_src, const acc_
     }
     const int64_t nwords = (ntarget + 1) / 2;
     const size_t nlds = (size_t)nwords * 4;
-    int bpc = 0;
-    hipError_t oe = hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&bpc, s->variants[nv].fn, s->spec.block, nlds);
-    if (oe != hipSuccess || bpc < 1) { (void)hipGetLastError(); bpc = 1; }
+    // a workgroup a compute unit, whatever room a small table leaves for others: every one is a row that the merge reads (18 754
+    // targets, 3.5 M / 67 M sources: 11.7 + 11.5 us / 50.2 + 8.2 with as many as there is room for, 8.6 + 4.6 / 49.6 + 4.8
+    // so; 20 M on 30 000 targets 21.3 + 6.9 / 18.0 + 4.8)
     const int64_t cus_n = s->ctx->props.multiProcessorCount;
-    const int64_t ngrid = acc_launch_grid(n_src, s->elements_per_block(), cus_n, bpc);
+    const int64_t ngrid = acc_launch_grid(n_src, s->elements_per_block(), cus_n, 1);
     acc::ScratchRef nblk, cblk;
     ACC_TRY(s->ctx->scratch_acquire((size_t)ntarget * esz, st, acc::SCRATCH_CARRY, &cblk));
     const int64_t nd = (nwords + 1) / 2;             // words a workgroup's row of 8-bit counts takes

@@ -798,7 +798,7 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
       if (sp->combine_hint >= ACC_COMBINE_AND && !is_integer_type(sp->elt_type))
         return fail(ACC_ERR_INVALID, "permute: bitwise combine_hint on non-integer element type '%s'", sp->elt_type.c_str());
       sp->block = tune("permute.block", 1024);
-      sp->merge_waves = std::max(4, std::min(16, tune("permute.merge_waves", 4)));
+      sp->merge_waves = std::max(4, std::min(16, tune("permute.merge_waves", 8)));
       sp->unroll = tune("permute.unroll", 2);
       if (sp->permute_replace) {
         sp->block = tune("scatter.block", 256);
