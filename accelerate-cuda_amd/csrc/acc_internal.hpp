@@ -108,6 +108,7 @@ void set_default_tuning(TuningPtr t);
   X(stencil_pair_walk, "stencil.pair_walk", 0)                                                                          \
   X(stencil_flat, "stencil.flat", 1)                                                                     \
   X(stencil_half_strips, "stencil.half_strips", 1)                                                                     \
+  X(map_lines_from_mb, "map.lines_from_mb", 28)                                                                      \
   X(map_tiled_min_w, "map.tiled_min_w", 33)                                                                          \
   X(map_tiled_min_h, "map.tiled_min_h", 10)                                                                          \
   X(stencil_thin_2d, "stencil.thin_2d", 36)                                                                          \

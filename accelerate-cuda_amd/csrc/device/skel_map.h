@@ -40,82 +40,52 @@
  * What bounds it: the memory side, once the index arithmetic is out of the way.  The place of every element is known
  * here before the fragment asks for it, so the compiler is told what `ix % shOut_0` and `ix / shOut_0` come to: it then
  * drops the fragment's divisions (two 64-bit ones an element, some 3000 instructions a lane) and sees that the four
- * elements down a column lie side by side in the source, which become one 128-bit access.  Where
- * the rows of the result are no whole cache lines, a run leaves a piece of a line at both ends: the four waves of a
- * workgroup then take two tiles by two and a die takes one contiguous run of the workgroups, so that the pieces meet in
- * one L2.  Rows of whole lines have no pieces; dealing their workgroups out over the dies, four tiles side by side, is
- * the faster order.  Transposes in us, dealt out with divisions / without / two by two on one die: 5003 x 3001 Float32
- * 46.5 / 37.1 / 31.0 (3.9 TB/s; 1.2 times the source is read, 1.08 times the result written); 4000 x 4000 31.9 / 28.1 /
- * 29.6; 8192 x 8192 125 / 118 / 131; 7001 x 2500 Float64 89.3 / - / 72.6.
+ * elements down a column lie side by side in the source, which become one 128-bit access.
+ *
+ * Where the rows of the result are no whole cache lines, a run leaves a piece of a line at both ends, which the memory side
+ * takes as a read and a write of the line if the pieces do not meet in time.  Large results of 4- and 8-byte elements
+ * therefore go through LDS: a workgroup evaluates four tiles side by side, as ever, and writes of every row the lines that
+ * begin within the first 96 (Float64: 112) columns -- the rest of its columns it has for the sake of the last line, and its
+ * neighbour evaluates them again.  The lines leave in non-temporal stores.  Other such results are written as they stand:
+ * the four waves take two tiles by two and a die takes one contiguous run of the workgroups, so that the pieces meet in
+ * one L2.  Rows of whole lines have no pieces: their workgroups, four tiles side by side, are dealt out over the dies, and
+ * in large matrices lie one below the other and go down strips of eight, so that the source too is read in longer runs.
+ *
+ * Transposes in us, before (pieces in every size, divisions gone; whole lines row after row) and now: 5003 x 3001 Float32
+ * 30.4 / 20.7 on operands that the memory-side cache holds in part, 32.9 / 28.6 on those it does not (a copy 21.4); 8191^2
+ * 152 / 104; 7001 x 2500 Float64 73 / 60; 3891 x 2048 18.5 / 15.7; 8192^2, in strips, 118 / 100; 4096^2 28.8 and 28.8.  Small
+ * ones are the tiles at the ends, whose reads were waited for one by one behind a test and now are asked for at once:
+ * 1001 x 999 6.4 / 5.0, thirty planes of 501 x 400 14.9 / 14.2, 100 x 101 x 102 turned 9.4 / 6.2.
  */
 #ifndef ACC_TT
 #define ACC_TT 4                                      /* a lane's block is ACC_TT x ACC_TT */
 #endif
 #define ACC_TSIDE (8 * ACC_TT)                        /* a wave's tile is ACC_TSIDE x ACC_TSIDE */
+#define ACC_TILE_LINE (128 / ACC_TILE_ELT_BYTES)      /* elements of a cache line */
+#define ACC_TILE_PITCH (ACC_BLOCK / ACC_WAVE * ACC_TSIDE + 4)
 
-extern "C" __global__ void __launch_bounds__(ACC_BLOCK)
-ACC_ENTRY(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_GUARD_PARAM)
-{
-  ACC_GUARD_CHECK
-  typedef ACC_ELT T;
-  ACC_ENV_ASSUME
-  /* the element at `ix`, which is column `acc_c` of row `acc_r` of the result's rows taken as one list */
-  auto acc_get_at = [&](const Int64 ix, const Int64 acc_r, const Int64 acc_c) -> T {
-    __builtin_assume(ix % shOut_0 == acc_c);
-    __builtin_assume(ix / shOut_0 == acc_r);
-    return (ACC_GET(ix));
-  };
-
-  /* The tiles' second dimension is the second innermost one of the result, or one further out (ACC_TILE_H its
-   * extent, ACC_TILE_MIDS the rows between neighbours along it: a volume turned so that its innermost
-   * dimension becomes its outermost reads its source along that one).  What lies between that dimension and the
-   * innermost (`mids` rows for every place along it) and outside it (`outers`) is walked tile by tile. */
-  const Int64 w = shOut_0, h = ACC_TILE_H, mids = ACC_TILE_MIDS, stride = mids * w;
-  const Int64 n = (ACC_OUT_SIZE);
-  const Int64 outers = (h > 0 && stride > 0) ? n / (h * stride) : 0;
-  const int lane = acc_lane();
-  const int lx = lane & 7, ly = lane >> 3;
-  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-  /* a workgroup's waves: two by two tiles, or side by side where the result is no taller than one and where its rows
-   * are whole cache lines (the driver counts the workgroups by the same rule) */
-  constexpr int WAVES = ACC_BLOCK / ACC_WAVE;
-  const bool whole_lines = (w * ACC_TILE_ELT_BYTES) % 128 == 0;
-  const int down = (WAVES % 2 == 0 && h > ACC_TSIDE && !whole_lines) ? 2 : 1, across = WAVES / down;
-  const Int64 groups_x = (w + across * ACC_TSIDE - 1) / (across * ACC_TSIDE), groups_y = (h + down * ACC_TSIDE - 1) / (down * ACC_TSIDE);
-  const Int64 groups = groups_x * groups_y * mids * outers;
-  /* the quotient of numbers no larger than the array has elements: in 32 bits where it has fewer than 2^31 */
-  const bool narrow = n < 0x7fffffff;
-  auto divide = [&](const Int64 a, const Int64 b) -> Int64 {
-    return narrow ? (Int64)((unsigned int)a / (unsigned int)b) : a / b;
-  };
-
-  for (Int64 group = whole_lines ? (Int64)blockIdx.x : acc_xcd_contiguous_block(); group < groups; group += gridDim.x) {
-    const Int64 g1 = divide(group, groups_x), gx = group - g1 * groups_x;
-    const Int64 plane = divide(g1, groups_y), gy = g1 - plane * groups_y;
-    const Int64 outer = divide(plane, mids), mid = plane - outer * mids;
-    const Int64 tx = gx * across + (down == 2 ? wave >> 1 : wave), ty = gy * down + (down == 2 ? wave & 1 : 0);
-    const Int64 x = tx * ACC_TSIDE + lx * ACC_TT, y = ty * ACC_TSIDE + ly * ACC_TT;
-    const Int64 row = (outer * h + y) * mids + mid, base = row * w + x;
-    if ((tx + 1) * ACC_TSIDE <= w && (ty + 1) * ACC_TSIDE <= h) {
-      T v[ACC_TT][ACC_TT];
-      /* down the columns first: what a transposed source holds side by side */
-#pragma unroll
-      for (int k = 0; k < ACC_TT; ++k)
-#pragma unroll
-        for (int i = 0; i < ACC_TT; ++i) v[i][k] = acc_get_at(base + i * stride + k, row + i * mids, x + k);
-#pragma unroll
-      for (int i = 0; i < ACC_TT; ++i)
-#pragma unroll
-        for (int k = 0; k < ACC_TT; ++k) ACC_SET(arrOut, base + i * stride + k, v[i][k]);
-    } else {
-#pragma unroll
-      for (int i = 0; i < ACC_TT; ++i)
-#pragma unroll
-        for (int k = 0; k < ACC_TT; ++k)
-          if (x + k < w && y + i < h) ACC_SET(arrOut, base + i * stride + k, acc_get_at(base + i * stride + k, row + i * mids, x + k));
-    }
-  }
-}
+#define ACC_MAP_CAT2_(a, b) a##b
+#define ACC_MAP_CAT_(a, b) ACC_MAP_CAT2_(a, b)
+#define ACC_TILES_WHOLE 0
+#define ACC_TILES_PIECES 1
+#define ACC_TILES_LINES 2
+#define ACC_TILES_ENTRY ACC_ENTRY
+#define ACC_TILES_FORM ACC_TILES_WHOLE
+#include "skel_map_tiles.h"
+#undef ACC_TILES_ENTRY
+#undef ACC_TILES_FORM
+#define ACC_TILES_ENTRY ACC_MAP_CAT_(ACC_ENTRY, _pieces)
+#define ACC_TILES_FORM ACC_TILES_PIECES
+#include "skel_map_tiles.h"
+#undef ACC_TILES_ENTRY
+#undef ACC_TILES_FORM
+#if ACC_TILE_LINES
+#define ACC_TILES_ENTRY ACC_MAP_CAT_(ACC_ENTRY, _lines)
+#define ACC_TILES_FORM ACC_TILES_LINES
+#include "skel_map_tiles.h"
+#undef ACC_TILES_ENTRY
+#undef ACC_TILES_FORM
+#endif
 
 #else
 

@@ -23,6 +23,7 @@ ACC_EMBED(map, "device/skel_map.h")
 ACC_EMBED(fold, "device/skel_fold.h")
 ACC_EMBED(foldseg, "device/skel_foldseg.h")
 ACC_EMBED(fold_across, "device/skel_fold_across.h")
+ACC_EMBED(map_tiles, "device/skel_map_tiles.h")
 ACC_EMBED(scan, "device/skel_scan.h")
 ACC_EMBED(permute, "device/skel_permute.h")
 ACC_EMBED(scatter, "device/skel_scatter.h")
@@ -42,6 +43,7 @@ const std::vector<EmbeddedHeader> &embedded_headers()
       {"skel_fold.h", acc_embed_fold_begin, acc_embed_fold_end},
       {"skel_foldseg.h", acc_embed_foldseg_begin, acc_embed_foldseg_end},
       {"skel_fold_across.h", acc_embed_fold_across_begin, acc_embed_fold_across_end},
+      {"skel_map_tiles.h", acc_embed_map_tiles_begin, acc_embed_map_tiles_end},
       {"skel_scan.h", acc_embed_scan_begin, acc_embed_scan_end},
       {"skel_permute.h", acc_embed_permute_begin, acc_embed_permute_end},
       {"skel_scatter.h", acc_embed_scatter_begin, acc_embed_scatter_end},

@@ -301,15 +301,28 @@ int acc_exec_map(acc_skel s, const acc_array *env, const acc_array *out, acc_str
   ACC_TRY(s->ensure_variant(v));
   if (in_tiles) {
     // a wave per tile of 32 x 32 elements of the innermost dimension and the second innermost one, or the one that
-    // ACC_FLAG_TILE_DIM names, two tiles by two a workgroup or side by side, as skel_map.h numbers them
+    // ACC_FLAG_TILE_DIM names, as skel_map.h arranges them in a workgroup
     const int rank = s->spec.out_rank;
-    const int64_t side = 8 * (int64_t)s->spec.map_tile_block;
+    const int64_t side = 8 * (int64_t)s->spec.map_tile_block, esz = std::max(1, s->spec.elt_size);
     const int64_t w = out->shape[rank - 1], h = out->shape[rank - 1 - s->spec.map_tile_dim];
     const int64_t waves = s->variants[v].block / 64;
-    const bool whole_lines = (w * std::max(1, s->spec.elt_size)) % 128 == 0;
-    const int64_t down = (waves % 2 == 0 && h > side && !whole_lines) ? 2 : 1, across = waves / down;
-    const int64_t groups = ((w + across * side - 1) / (across * side)) * ((h + down * side - 1) / (down * side)) * (n / (w * h));
-    return launch(s, v, std::min<int64_t>(groups, (int64_t)1 << 22), 0, static_cast<hipStream_t>(stream), &args);
+    bool whole = (w * esz) % 128 == 0;
+    for (int c = 0; c < out->ncomp; ++c) whole = whole && out->ptr[c] % 128 == 0;
+    const bool strips = whole && n == w * h && n * esz >= acc::map_strips_from;
+    // Results of no whole lines, or that begin amid one, go out in lines from 28 MB on, where they do not stay in the
+    // memory-side cache (us as they stand / in lines: 5003 x 3001 Float32 33.8 / 28.5, 8191^2 148 / 104, 3891 x 2048 17.9 /
+    // 15.8, 7001 x 2500 Float64 77 / 60, with another operand read along the rows 3001 x 2999 29.4 / 27.6, 5003 x 3001 47 / 43;
+    // but 1001 x 999 4.6 / 5.6, 1500 x 1501 with another operand 8.5 / 10.3, thirty planes of 400 x 501 14.8 / 16.5).
+    const bool in_lines = s->spec.map_lines && !whole && n * esz >= s->knobs.map_lines_from_mb * ((int64_t)1 << 20);
+    const int64_t down = h <= side || in_lines ? 1 : (strips ? waves : (waves % 2 == 0 && !whole ? 2 : 1));
+    const int64_t columns = waves / down * side - (in_lines ? 128 / esz : 0);
+    const int64_t groups = ((w + columns - 1) / columns) * ((h + down * side - 1) / (down * side)) * (n / (w * h));
+    const int64_t grid = std::min<int64_t>(groups, (int64_t)1 << 22);
+    if (whole) return launch(s, v, grid, 0, static_cast<hipStream_t>(stream), &args);
+    ACC_TRY(s->ctx->make_current());
+    ACC_HIP_TRY(launch_kernel(in_lines ? s->variants[v].fn_lines : s->variants[v].fn_pieces, static_cast<unsigned>(grid), 1, 1,
+                              static_cast<unsigned>(s->variants[v].block), 1, 1, 0, static_cast<hipStream_t>(stream), args.data(), nullptr));
+    return ACC_OK;
   }
   // streaming with no reuse: one short-lived workgroup per tile keeps the most loads in flight
   const int64_t grid = acc_launch_grid(n, s->elements_per_block(), resident(s, v), s->knobs.map_oversub);

@@ -335,7 +335,7 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
       o << "#define ACC_MAP_TILED " << (sp.map_tiled ? 1 : 0) << "\n#define ACC_TT " << sp.map_tile_block << "\n";
       if (sp.map_tiled) {
         // the tiles' second dimension: its extent, and the rows between neighbours along it
-        o << "#define ACC_TILE_ELT_BYTES " << std::max(1, sp.elt_size) << "\n";
+        o << "#define ACC_TILE_ELT_BYTES " << std::max(1, sp.elt_size) << "\n#define ACC_TILE_LINES " << (sp.map_lines ? 1 : 0) << "\n#define ACC_TILE_STRIPS_FROM " << map_strips_from << "ll\n";
         o << "#define ACC_TILE_H shOut_" << sp.map_tile_dim << "\n#define ACC_TILE_MIDS (";
         if (sp.map_tile_dim == 1) o << "1";
         for (int dd = 1; dd < sp.map_tile_dim; ++dd) o << (dd > 1 ? " * " : "") << "shOut_" << dd;
@@ -759,6 +759,12 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
     case ACC_SKEL_MAP: case ACC_SKEL_GENERATE: case ACC_SKEL_TRANSFORM:
       sp->block = tune("map.block", 256);
       sp->unroll = tune("map.unroll", 1);
+      {
+        // (two waves' tiles at least side by side, and the tiles of a workgroup within 64 KB)
+        const int side = 8 * sp->map_tile_block, across = sp->block / 64 * side;
+        sp->map_lines = sp->map_tiled && sp->comp_types.empty() && (type_size(sp->elt_type) == 4 || type_size(sp->elt_type) == 8) && across >= 64 &&
+                        side * (across + 4) * sp->elt_size <= 65536 && tune("map.tiled_lines", 1) != 0;
+      }
       break;
     case ACC_SKEL_FOLD: case ACC_SKEL_FOLD1:
       sp->block = tune("fold.block", 256);
@@ -1202,6 +1208,16 @@ int acc_skel_s::load_variant(int v)
           return acc::fail_hip(e, ("hipModuleGetFunction(" + wide + ")").c_str());
         }
       }
+    }
+  }
+  if (spec.map_tiled) {
+    const std::string pieces = entry_name + "_pieces", lines = entry_name + "_lines";
+    e = hipModuleGetFunction(&var.fn_pieces, var.module, pieces.c_str());
+    if (e == hipSuccess && spec.map_lines) e = hipModuleGetFunction(&var.fn_lines, var.module, lines.c_str());
+    if (e != hipSuccess) {
+      (void)hipModuleUnload(var.module);
+      var.module = nullptr;
+      return acc::fail_hip(e, ("hipModuleGetFunction(" + (var.fn_pieces ? lines : pieces) + ")").c_str());
     }
   }
   if (spec.stencil_pair) {

@@ -58,6 +58,7 @@ struct SkelSpec {
   int map_tile_dim = 1;                 // ACC_FLAG_TILE_DIM: which dimension of the result, counted from the innermost, the tiles pair with it
   bool map_tiled = false;               // ACC_FLAG_TILED on a map of rank 2 or more: tiles of 32 x 32 elements, a wave each
   int map_tile_block = 4;               // ... a lane's share of a tile: a block of that many elements either way
+  bool map_lines = false;               // ... results whose rows are no whole cache lines go out through LDS, in whole lines
   bool guarded = false;                 // ACC_FLAG_GUARDED: every kernel takes the address of a loop's guard word last
   bool foldseg_giants = false;          // a segmented fold's variants 4-7: very long segments are handed over to a second launch (skel_foldseg.h)
   bool fold_single = true;              // foldAll in one launch (the last workgroup collects), as generated into the kernel
@@ -81,6 +82,8 @@ struct Variant {
   hipFunction_t fn_claim = nullptr;    // a permute whose combination is the new value: permute_claim (skel_scatter.h)
   hipFunction_t fn_across = nullptr;   // fold along the innermost dimension: _across, a lane per row of any length
   hipFunction_t fn_across_wide = nullptr;   // ... _across_wide, several rows a lane (elements of at most 8 bytes)
+  hipFunction_t fn_pieces = nullptr;   // a map in tiles: _pieces, for results whose rows are no whole cache lines
+  hipFunction_t fn_lines = nullptr;    // ... _lines, for large ones of elements of 4 and 8 bytes
   hipFunction_t fn_three = nullptr;    // a stencil's variants 10 and 11: three applications a launch (fn makes four)
   hipFunction_t fn_sweep = nullptr;    // a segmented fold's variants 4-7: _sweep, the segments that were handed over;
                                        // its variants 0-3: _probe, a look at the segment lengths
@@ -96,6 +99,7 @@ struct Variant {
 int type_size(const std::string &t);
 int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp);
 int across_rows(const SkelSpec &sp);
+constexpr int64_t map_strips_from = int64_t(128) << 20;     // bytes of a result of whole cache lines from which a map in tiles goes down strips of tiles
 constexpr int flat_spread = 8;          // waves of a plane that a die takes at least, in the form for volumes of skel_stencil_flat.h, for every die to take a share of every plane
 int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::string *source);
 SkelSpec spec_of_variant(const SkelSpec &base, int variant);

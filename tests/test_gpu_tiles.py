@@ -51,3 +51,53 @@ def test_tiles_of_an_outer_dimension(ctx, dim, shape):
         ctx.skeleton(A.SKEL_GENERATE, "Int32", env=[], out_rank=3, flags=flags, get=frag).map([], out)
         results.append(out.get())
     assert np.array_equal(results[0], results[1])
+
+
+@pytest.mark.parametrize("shape", [(70, 3, 65), (33, 40, 97), (5, 33, 130)])
+@pytest.mark.parametrize("dim", [1, 2])
+def test_volumes_in_whole_lines(ctx, dim, shape):
+    import acchip as A
+    frag = "(ix % shOut_0) * 1000003 + (ix / shOut_0) * 7 + ix"
+    results = []
+    with A.tuning("map.lines_from_mb=0", ctx):
+        for flags in (A.FLAG_TILED | A.FLAG_TILE_DIM(dim), 0):
+            out = ctx.empty(shape, np.int64)
+            ctx.skeleton(A.SKEL_GENERATE, "Int64", env=[], out_rank=3, flags=flags, get=frag, wait=True).map([], out)
+            results.append(out.get())
+    assert np.array_equal(results[0], results[1])
+
+
+def test_large_matrices_of_whole_lines(ctx):
+    """down strips of workgroups, from 128 MB of result on: a last strip of one row of them, a last tile short"""
+    import acchip as A
+    sk = ctx.skeleton(A.SKEL_MAP, "Int32", env=[(2, "Int32")], out_rank=2, flags=A.FLAG_TILED, get=FORMS["transpose"], wait=True)
+    for h, w in ((8 * 128 + 1, 32768), (32769, 1056), (8193, 4128)):
+        x = np.arange(h * w, dtype=np.int32).reshape(w, h)
+        out = ctx.array(np.full((h, w), 77, np.int32))
+        sk.map([ctx.array(x)], out)
+        assert np.array_equal(out.get(), x.T), (h, w)
+
+
+@pytest.mark.parametrize("ctype,dt", [("Int32", np.int32), ("double", np.float64), ("Int16", np.int16)])
+def test_tiles_in_whole_lines(ctx, ctype, dt):
+    """results whose rows are no whole cache lines go out in lines, those whose rows are down strips eight groups tall: widths
+    either side of what a workgroup writes, of whole lines, results that begin anywhere within a line"""
+    import acchip as A
+    get = FORMS["transpose"]
+    with A.tuning("map.lines_from_mb=0", ctx):
+        tiled, runs = [ctx.skeleton(A.SKEL_MAP, ctype, env=[(2, ctype)], out_rank=2, flags=f, get=get, wait=True) for f in (A.FLAG_TILED, 0)]
+    lines = np.dtype(dt).itemsize >= 4
+    assert ("#define ACC_TILE_LINES %d\n" % lines) in tiled.source(0)
+    rng = np.random.default_rng(13)
+    for h, w in [(10, 34), (33, 95), (32, 96), (31, 97), (40, 111), (33, 112), (33, 113), (100, 128), (33, 129), (65, 191), (64, 193), (35, 225), (1030, 160),
+                 (1024, 64), (1056, 96), (300, 1001)]:
+        x = rng.integers(-1000, 1000, (w, h)).astype(dt)
+        src = ctx.array(x)
+        for shift in (0, 1, 5, 31):
+            print(ctype, h, w, shift, flush=True)
+            for sk in (tiled, runs):
+                out = ctx.array(np.full(h * w + shift + 3, 77, dt))
+                sk.map([src], out.desc(shape=(h, w), offset_elems=shift))
+                got = out.get()
+                assert np.array_equal(got[shift:shift + h * w].reshape(h, w), x.T), (h, w, shift)
+                assert np.all(got[:shift] == 77) and np.all(got[shift + h * w:] == 77), (h, w, shift)
