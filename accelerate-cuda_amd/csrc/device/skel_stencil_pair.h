@@ -18,15 +18,20 @@
  * the array is its right end, and what stands above it its bottom, in between as well; such rows and columns are read and
  * worked out there.)
  *
- * What bounds it: memory -- waves that walk copy at 5.4 TB/s at best, 100 us for 8192 x 8192 Float32 -- and the rows that
- * neighbouring walks both read, with the vector units close behind (15 instructions an element and application of 3 x 3,
- * 105 us for four).  3 x 3 on 8192 x 8192 Float32: four applications 118 us and three 112, one by itself 88; two a launch,
- * in strips that asked for all their rows at once, 96.  Ten in a call, two of them by themselves: 884 us one a launch,
- * 554 in pairs, 412 so.  4000 x 4000 Float64 56 / 61 (46 one by itself), 3000 x 3000 Float32 22 / 19 (17), 300 x 300 6.3 /
- * 6.4 (5.6: launches count).  Walks of 28 rows: of 16 / 20 / 32 / 40 / 70 rows four take 127 / 123 / 124 / 122 / 122 us
- * (5000 x 8191: 61 / 59 / 62 / 63 / 62, and 61); shorter ones where the array would give too few waves (the driver's
- * rule).  Six rows ahead instead of three: the same.  Non-temporal stores: 8192 x 8192 the same, arrays that the memory-side
- * cache holds a tenth slower.
+ * Every second band of walks goes up from its last row instead of down from its first, so that of two walks that read
+ * the same rows both begin or both end with them, at about the same time and in one L2 (a die takes one contiguous run of
+ * the walks; walks at the upper and lower edge all go down).  All of them down, 8192 x 8192 Float32, 3 x 3: four
+ * applications 119 us and now 116, three 112 and now 107; 5 points 118 / 114 and now 112 / 107; 5003 x 8000 75 / 72 and now
+ * 70 / 66; 7001 x 5002 Float64 125 / 118 and now 123 / 116; arrays that the memory-side cache holds the same.
+ *
+ * What bounds it: memory -- waves that walk copy at 5.4 TB/s at best, 100 us for 8192 x 8192 Float32 -- with the vector
+ * units close behind (15 instructions an element and application of 3 x 3, 105 us for four).  3 x 3 on 8192 x 8192
+ * Float32: four applications 116 us and three 107, one by itself 88; two a launch, in strips that asked for all their rows
+ * at once, 96.  Ten in a call, two of them by themselves: 884 us one a launch, 554 in pairs, 405 so.  3001 x 5000 Float64
+ * 56 / 58 (43 one by itself), 3000 x 3000 Float32 24 / 20 (17), 300 x 300 6.4 / 6.2 (4.5: launches count).  Walks of 28
+ * rows: of 16 / 20 / 24 / 32 / 36 / 40 rows four take 126 / 121 / 119 / 117 / 120 / 118 us (4001 x 8191: 59 / 59 / 59 /
+ * 61 / 59 / 61, and 59); shorter ones where the array would give too few waves (the driver's rule).  Six rows ahead instead
+ * of three: the same.  Non-temporal stores: 8192 x 8192 the same, arrays that the memory-side cache holds a tenth slower.
  *
  * Generated definitions expected: those of skel_stencil.h, for ACC_STENCIL_RANK 2, one source of one component of the
  * result's type, no arrays in the environment, taps at most one row and one column away; rows as long as a strip, or at
@@ -140,19 +145,20 @@ ACC_DEV void acc_applications(ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk
     else                    *dst = nv;
   };
 
-  auto acc_run = [&](auto xedge_c, auto acc_yedge_c) {
-    constexpr bool acc_yedge = decltype(acc_yedge_c)::value;
-    const int acc_first = acc_y0 - acc_levels * ACC_RY;              /* the row of the source that the walk begins with */
+  auto acc_run = [&](auto xedge_c, auto acc_yedge_c, auto acc_up_c) {
+    constexpr bool acc_yedge = decltype(acc_yedge_c)::value, acc_up = decltype(acc_up_c)::value;
+    /* the row of the source that the walk begins with */
+    const int acc_first = acc_up ? acc_y1 - 1 + acc_levels * ACC_RY : acc_y0 - acc_levels * ACC_RY;
     const int acc_rows = acc_y1 - acc_y0 + 2 * acc_levels * ACC_RY;  /* ... and how many it takes */
     /* the source's row that stands for row y, which may lie outside (what is asked for beyond the walk is not looked at) */
     auto acc_row_of = [&](const int y) -> int {
       if (acc_yedge && ACC_BOUNDARY == ACC_B_WRAP) return ((y % acc_h) + acc_h) % acc_h;
-      return acc_yedge ? acc_max(0, acc_min(y, acc_h - 1)) : acc_min(y, acc_h - 1);
+      return acc_yedge ? acc_max(0, acc_min(y, acc_h - 1)) : acc_up ? acc_max(0, y) : acc_min(y, acc_h - 1);
     };
     acc_pair_own acc_ahead[ACC_AHEAD];
     acc_pair_row acc_window[acc_levels][ACC_NR];                     /* of the source and of what lies between: the rows that the next application reads */
 #pragma unroll
-    for (int i = 0; i < ACC_AHEAD; ++i) acc_ahead[i] = acc_load(acc_row_of(acc_first + i));
+    for (int i = 0; i < ACC_AHEAD; ++i) acc_ahead[i] = acc_load(acc_row_of(acc_first + (acc_up ? -i : i)));
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int acc_l = 0; acc_l < acc_levels; ++acc_l)
@@ -167,7 +173,7 @@ ACC_DEV void acc_applications(ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk
         const int acc_s = acc_base + acc_u;
         if (acc_s >= acc_rows) return;
         acc_pair_own acc_next = acc_ahead[acc_u];
-        acc_ahead[acc_u] = acc_load(acc_row_of(acc_first + acc_s + ACC_AHEAD));
+        acc_ahead[acc_u] = acc_load(acc_row_of(acc_first + (acc_up ? -1 : 1) * (acc_s + ACC_AHEAD)));
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int acc_l = 0; acc_l < acc_levels; ++acc_l) {
@@ -195,20 +201,22 @@ ACC_DEV void acc_applications(ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk
           acc_pair_own acc_res;
 #pragma unroll
           for (int acc_k = 0; acc_k < ACC_SVEC; ++acc_k) {
-#define ACC_WINDOW_READ(c, dz, dy, dx) acc_rows_of[(acc_u + 1 + ACC_RY + (dy)) % ACC_NR].e[ACC_RX + acc_k + (dx)]
+#define ACC_WINDOW_READ(c, dz, dy, dx) acc_rows_of[(acc_u + 1 + ACC_RY + (acc_up ? -(dy) : (dy))) % ACC_NR].e[ACC_RX + acc_k + (dx)]
             ACC_STENCIL_TAPS1(ACC_WINDOW_READ)
 #undef ACC_WINDOW_READ
             acc_res.v[acc_k] = (T)(ACC_STENCIL_FN);
           }
           acc_next = acc_res;
-          if (acc_l == acc_levels - 1) acc_put(acc_y0 + acc_s - 2 * acc_levels * ACC_RY, acc_res);
+          if (acc_l == acc_levels - 1) acc_put(acc_up ? acc_y1 - 1 - (acc_s - 2 * acc_levels * ACC_RY) : acc_y0 + acc_s - 2 * acc_levels * ACC_RY, acc_res);
         }
       }
     }
   };
-  if (acc_y0 < acc_levels * ACC_RY || acc_y1 + acc_levels * ACC_RY > acc_h) acc_run(acc_bool<true>(), acc_bool<true>());
-  else if (acc_x0 < acc_outer * ACC_SVEC || acc_x0 + acc_owned + acc_outer * ACC_SVEC > acc_w) acc_run(acc_bool<true>(), acc_bool<false>());
-  else acc_run(acc_bool<false>(), acc_bool<false>());
+  const bool acc_goes_up = ((acc_number / acc_strips) & 1) != 0;
+  if (acc_y0 < acc_levels * ACC_RY || acc_y1 + acc_levels * ACC_RY > acc_h) acc_run(acc_bool<true>(), acc_bool<true>(), acc_bool<false>());
+  else if (acc_x0 < acc_outer * ACC_SVEC || acc_x0 + acc_owned + acc_outer * ACC_SVEC > acc_w) acc_run(acc_bool<true>(), acc_bool<false>(), acc_bool<false>());
+  else if (acc_goes_up) acc_run(acc_bool<false>(), acc_bool<false>(), acc_bool<true>());
+  else acc_run(acc_bool<false>(), acc_bool<false>(), acc_bool<false>());
 }
 
 extern "C" __global__ void __launch_bounds__(ACC_BLOCK)

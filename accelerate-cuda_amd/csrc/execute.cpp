@@ -1516,7 +1516,7 @@ int acc_exec_stencil_iterate(acc_skel s, const acc_array *env, const acc_array *
   // Four and three applications a launch as often as leaves every result where one a launch would: an even number of
   // fours, so that the arrays have changed places as often (a three changes them as three single ones do), and at least
   // one application by itself at the end, whose source is then the result before the last.  Of these splits the one that
-  // takes least: of large arrays a four takes about 1.35 times a single application, a three 1.25 times.
+  // takes least: of large arrays a four takes 1.25 to 1.4 times a single application, a three 1.15 to 1.3.
   const int32_t many = std::max(iters, 1) - 1;
   int32_t fours = 0, threes = 0;
   for (int32_t q = many / 4 / 2 * 2, least = -1; q >= 0 && q > many / 4 - 8; q -= 2) {

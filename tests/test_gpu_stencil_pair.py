@@ -84,6 +84,32 @@ def test_walks_and_counts(ctx, boundary, ctype, dt, taps):
             assert got[0][0] == got[1][0] and all(np.array_equal(got[0][k], got[1][k]) for k in (1, 2)), (walk, shape, iters)
 
 
+@pytest.mark.parametrize("boundary", ["clamp", "wrap"])
+@pytest.mark.parametrize("ctype,dt,taps", [("float", np.float32, BOX), ("double", np.float64, CROSS), ("Int32", np.int32, ROWS), ("Int64", np.int64, COLUMNS)])
+def test_walks_that_go_up(ctx, boundary, ctype, dt, taps):
+    """strips inside the array, whose every second walk goes up: walks shorter than what the launch reads beyond them, of as
+    many rows as are asked for ahead and of one more, and a last one of a single row; equal to one application a launch"""
+    import acchip as A
+    fn = " + ".join("(%s)%s * t%d" % (ctype, (3 + 2 * k) if np.issubdtype(dt, np.integer) else repr(0.07 * (k + 1) - 0.2), k) for k in range(len(taps)))
+    desc = dict(out_rank=2, taps=taps, boundary=boundary, stencil_fn=fn)
+    with A.tuning("stencil.pair=0", ctx):
+        ones = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+    own = 60 * (16 // np.dtype(dt).itemsize)
+    rng = np.random.default_rng(11)
+    for walk, h in ((1, 16), (3, 31), (4, 33), (28, 141)):
+        with A.tuning("stencil.pair_walk=%d" % walk, ctx):
+            many = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+        for iters in (4, 9):                              # a three and one by itself; two fours and one
+            print(ctype, len(taps), boundary, walk, h, iters, flush=True)
+            x = rng.integers(-50, 50, (h, 4 * own + 9)).astype(dt)
+            got = []
+            for sk in (many, ones):
+                a, b = ctx.array(x), ctx.array(np.full(x.shape, 77, dt))
+                res = sk.stencil_iterate(None, a, b, iters)
+                got.append((res is b, a.get(), b.get()))
+            assert got[0][0] == got[1][0] and all(np.array_equal(got[0][k], got[1][k]) for k in (1, 2)), (walk, h, iters)
+
+
 @pytest.mark.parametrize("what,rank,shape", [("acc_pair_own", 2, (40, 300)), ("acc_flat_source", 3, (5, 7, 700))])
 def test_a_form_that_cannot_be_built_leaves_the_call_to_another(ctx, what, rank, shape):
     """a preamble that takes a name which only this form's template has: the form does not compile, the others do"""
