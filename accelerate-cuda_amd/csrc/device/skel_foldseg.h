@@ -179,6 +179,10 @@ ACC_DEV unsigned int acc_giant_edge_slot(const Int64 n, const int job) { return 
 
 #endif
 
+/* where index `ix` of the source lies in the chunk [cs, ce), counted from its start: the start for one before it, the end
+ * for one behind it, however far away */
+ACC_DEV int acc_place_in_chunk(const Int64 ix, const Int64 cs, const Int64 ce) { return ix < cs ? 0 : ix > ce ? (int)(ce - cs) : (int)(ix - cs); }
+
 extern "C" __global__ void __launch_bounds__(ACC_BLOCK)
 ACC_FOLDSEG_ENTRY(ACC_ENV_PARAMS
                   const Int64 shOut_0, ACC_OUT_ARRAY(arrOut),
@@ -224,12 +228,15 @@ ACC_FOLDSEG_ENTRY(ACC_ENV_PARAMS
     const Int64 seg = first + tid, last = acc_min<Int64>(first + acc_own, nseg);
     const bool live = seg < last;
     /* both ends of the lane's segment are asked for at once (a lane past the last segment asks for the last one's
-     * and takes nothing) */
+     * and takes nothing: an empty segment where that one ends) */
     const Int64 seg_c = acc_min<Int64>(seg, last - 1);
     const Int64 a_c = ACC_SEG_AT(seg_c), b_c = ACC_SEG_END(seg_c);
-    Int64 a = live ? a_c : 0;
-    Int64 b = live ? b_c : 0;
     const Int64 lo = ACC_SEG_AT(first), hi = acc_min<Int64>(ACC_SEG_END(last - 1), n);
+    Int64 a = live ? a_c : b_c, b = b_c;
+    /* the block's elements are no more than 2^31 apart, as they all but always are: where a lane's segment lies in a chunk
+     * is then a difference of 32 bits wherever the two are.  (With both ends tested in 64 bits in every block, segments of
+     * 2 elements took 25.3 us instead of 24.9, of 4 20.4 instead of 19.9.) */
+    const bool near = hi - lo < 0x7fff0000;
     bool handed = false;                             /* this lane's segment has been handed over (below) */
 
     T acc = T();
@@ -288,7 +295,9 @@ ACC_FOLDSEG_ENTRY(ACC_ENV_PARAMS
           for (int k = 0; k < ACC_VEC; ++k) s_val[ACC_PAD((u * ACC_BLOCK + tid) * ACC_VEC + k)] = v[u][k];
         }
       /* this lane's segment, as far as it lies in the chunk */
-      int p0 = (int)(acc_max(a, cs) - cs), p1 = (int)(acc_min(b, ce) - cs);
+      int p0, p1;
+      if (near) { p0 = (int)(acc_max(a, cs) - cs); p1 = (int)(acc_min(b, ce) - cs); }
+      else      { p0 = acc_place_in_chunk(a, cs, ce); p1 = acc_place_in_chunk(b, cs, ce); }
       /* One lane a segment serialises a long segment on its lane while the rest of the workgroup waits: among a
        * million short segments a single one of 2^23 elements took 130-200 ms.  A stretch of ACC_WIDE elements or more
        * of one segment in a chunk is therefore folded by the whole workgroup: every lane a run of consecutive

@@ -82,3 +82,36 @@ def test_rows(ctx, right):
             out = ctx.empty(rows, np.uint32)
             sk.fold([ctx.array(x)], (rows, w), out)
             assert np.array_equal(out.get(), chain(x.ravel(), np.arange(rows + 1) * w, affine, SEED)), (rows, w)
+
+
+@pytest.mark.parametrize("right", [False, True])
+@pytest.mark.parametrize("giants", [0, 1])
+def test_beyond_2_31_elements(ctx, giants, right):
+    """short segments of a source of more than 2^31 elements (none of them in memory: an element is its index), a last
+    workgroup that has lanes without a segment"""
+    import acchip as A
+    rng = np.random.default_rng(13)
+    nseg, last, first = (1 << 25) + 77, 90, (1 << 31) + 1005
+    lens = rng.integers(0, 100, last)
+    lens[last - 20], lens[last - 7] = 700, 0
+    offs = np.full(nseg + 1, first, np.int64)
+    offs[nseg - last + 1:] += np.cumsum(lens)
+    print(nseg, first, flush=True)
+    with A.tuning("foldseg.giants=%d" % giants, ctx):
+        sk = ctx.skeleton(A.SKEL_FOLDSEG, "Int64", env=[], get="ix", combine="x + y", seed="5", seg_type="Int64",
+                          flags=A.FLAG_FOLD_RIGHT if right else 0, wait=True)
+    out = ctx.empty(nseg, np.int64)
+    sk.foldseg([], int(offs[-1]) + 3, ctx.array(offs), out)
+    got = out.get()
+    assert np.all(got[:nseg - last] == 5)
+    assert got[nseg - last:].tolist() == [5 + sum(range(int(a), int(b))) for a, b in zip(offs[nseg - last:-1], offs[nseg - last + 1:])]
+
+
+def test_rows_beyond_2_31_elements(ctx):
+    import acchip as A
+    rows, w = (1 << 26) + 77, 33
+    sk = ctx.skeleton(A.SKEL_FOLD, "Int64", env=[], out_rank=1, get="ix", combine="x + y", seed="0", wait=True)
+    out = ctx.empty(rows, np.int64)
+    print(rows, w, flush=True)
+    sk.fold([], (rows, w), out)
+    assert np.array_equal(out.get(), w * (w * np.arange(rows, dtype=np.int64)) + w * (w - 1) // 2)
