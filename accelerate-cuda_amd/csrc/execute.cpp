@@ -399,6 +399,33 @@ int launch_sweep(acc_skel_s *s, int lv, Args *common, const acc::ScratchRef &job
   return e == hipSuccess ? ACC_OK : acc::fail_hip(e, "hipModuleLaunchKernel(segmented fold, sweep)");
 }
 
+// Segments a workgroup: one for each of its lanes, or a half, a quarter, an eighth of them, the least that leaves it more
+// than 1024 elements.  A workgroup goes through its chunks one after the other, a round trip or, of a gather, two each, and
+// more of them run side by side (us with a lane each / so: rows of 64, 1000 of them 15.4 / 4.4, 67352 of 83 24.6 / 7.9,
+// 8000 of 100 29.9 / 7.7; sparse matrices of 1000 rows of 64 21.0 / 5.1, 18251 of 95 33 / 13).  Once there are more than
+// eight for a compute unit, which is what it holds, every chunk counts whether it is full or not.  Then no more of them in
+// all than a lane a segment would make, or, where every workgroup has a single one, of no gathers, and so nothing to wait
+// for in between, a third more: 359769 rows of 20 take 8.2 us in two chunks a workgroup of 128, in one of 64, half full, 10.6,
+// and 9.3 in two of 256; 765249 of 10, one chunk either way, 9.0 in workgroups of 256 and 11.8 of 128; 300000 of 50 18.0 in
+// five chunks of 256, 18.9 in two of 64 (rows of a matrix 13.6 / 15.5); but 200000 of 70 21.0 in six and 14.6 in one of 32,
+// 524287 of 40 21.4 in four and 17.3 in one of 64.  (Sparse matrices: 250000 rows of 33 43.6 in three of 256, 46.6 in one of
+// 64; 262143 of 64 84 in three of 128, 92 in one of 32.)  And no more workgroups than 32 for a compute unit, 20 where
+// elements are gathered: 10^6 rows of 30, 61 of them, 27.3 and 25.9 in 256, the sparse matrix of 524287 rows of 40, 32 of
+// them, 109.3 and 102.7 in 128.
+int64_t segments_a_workgroup(const acc_skel_s *s, int lv, int64_t nseg, int64_t avg)
+{
+  const int64_t lanes = s->spec.block, chunk = (lv & 2) ? s->spec.chunk_long : s->spec.chunk;
+  const int64_t spread = s->knobs.foldseg_spread * s->ctx->props.multiProcessorCount;
+  const bool streams = s->spec.get_streams;
+  auto chunks = [&](int64_t own) { return (own * avg + chunk - 1) / chunk; };
+  for (int64_t own = lanes / 8; own < lanes; own *= 2) {
+    if (2 * own * avg <= s->knobs.foldseg_spread_min || 4 * nseg > (streams ? 8 : 5) * own * spread) continue;
+    const int64_t in_all = chunks(own) * (lanes / own);
+    if (2 * nseg <= own * spread || 100 * in_all <= (streams && chunks(own) == 1 ? 134 : 115) * chunks(lanes)) return own;
+  }
+  return lanes;
+}
+
 // `args`: the parameters every kernel of the template begins with (free arrays, result, segments).  `giants`: the
 // segments are a vector's (the kernels of rows and of arrays of rank > 1 know no table).
 int launch_segmented(acc_skel_s *s, int v, Args *args, const acc_array *env, const acc_array *out, int64_t nseg, int64_t n,
@@ -416,15 +443,7 @@ int launch_segmented(acc_skel_s *s, int v, Args *args, const acc_array *env, con
     }
     GiantsPlan plan;
     if (giants) ACC_TRY(plan_giants(s, lv, &plan));
-    // Segments a workgroup: one for each of its lanes, halved, down to an eighth of them, as long as there are then fewer
-    // than sixteen workgroups for a compute unit and each has more than 1024 elements (a workgroup goes through its chunks
-    // one after the other, a round trip or, of a gather, two each).  us with a lane each / so: rows of 64, 1000 of them 13.1 /
-    // 6.4, 67352 of 83 15.6 / 7.0, 8000 of 100 18.0 / 6.2; sparse matrices of 1000 rows of 100 36.6 / 9.2, 30000 of 60
-    // (skewed) 49 / 22, 10754 of 19 15.1 / 8.8, 283671 of 83 156 / 134, 262144 of 128 199 / 181.  At 32 for a compute unit
-    // 262144 rows of 100 take 26.8 us instead of 24.4, the matrix of 2^20 rows of 32 201 instead of 190; from 512
-    // elements 100000 rows of 24 take 7.4 instead of 5.4.
-    int64_t own = s->spec.block;
-    while (own > s->spec.block / 8 && nseg < own * s->knobs.foldseg_spread * s->ctx->props.multiProcessorCount && own * avg > s->knobs.foldseg_spread_min) own /= 2;
+    const int64_t own = segments_a_workgroup(s, lv, nseg, avg);
     if (!plan.hand_over) {
       const int64_t grid = acc_launch_grid(nseg, own, resident(s, lv), s->knobs.foldseg_oversub);
       int rc = launch(s, lv, grid, 0, st, args);

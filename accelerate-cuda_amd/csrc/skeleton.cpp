@@ -247,6 +247,14 @@ static bool only_calculates(const std::string &text)
   return true;
 }
 
+// whether the element function is arithmetic on reads at the element's own index, for all that its text says: no gather
+static bool only_streams(const SkelSpec &sp)
+{
+  std::string rest = sp.get;
+  take_own_reads(sp, {&rest}, true);
+  return sp.preamble.empty() && only_calculates(rest);
+}
+
 // ---- the generator -------------------------------------------------------------
 
 // neighbouring rows a lane of a fold's <entry>_across takes: 16 bytes of them, no more than four
@@ -404,8 +412,6 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
         o << "#define ACC_CONST_ARRAY(name) " << from.str() << "\n";
         o << "#define ACC_BLOCK " << sp.block << "\n#define ACC_BATCH " << sp.unroll << "\n#define ACC_SMALL " << acc::SCATTER_SMALL << "\n";
         std::string pre_get = sp.get, pre_perm = sp.permutation;
-        std::string rest = sp.get;
-        take_own_reads(sp, {&rest}, true);
         const std::set<OwnRead> reads = take_own_reads(sp, {&pre_get, &pre_perm});
         std::ostringstream fields, loads, lengths, names;
         for (const OwnRead &r : reads) {
@@ -419,7 +425,7 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
         }
         o << "#define ACC_OWN_NAMES " << names.str() << "\n#define ACC_OWN_FIELDS " << fields.str() << "\n#define ACC_OWN_LOAD(sv, ix) " << loads.str() << "\n";
         o << "#define ACC_OWN_WITHIN(past) (true" << lengths.str() << ")\n";
-        o << "#define ACC_GET_TOTAL " << (sp.preamble.empty() && only_calculates(rest) ? 1 : 0) << "\n";
+        o << "#define ACC_GET_TOTAL " << (only_streams(sp) ? 1 : 0) << "\n";
         o << "#define ACC_GET_OWN(ix) " << pre_get << "\n#define ACC_PERMUTATION_OWN(ix) " << pre_perm << "\n";
         tmpl = "skel_scatter.h";
         break;
@@ -774,12 +780,14 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
         sp->block = tune("foldseg.block", 256);
         sp->chunk = segmented_chunk(*sp);
         sp->chunk_long = segmented_chunk(*sp, true);
+        sp->get_streams = only_streams(*sp);
       }
       break;
     case ACC_SKEL_FOLDSEG: case ACC_SKEL_FOLD1SEG:
       sp->block = tune("foldseg.block", 256);
       sp->chunk = segmented_chunk(*sp);
       sp->chunk_long = segmented_chunk(*sp, true);
+      sp->get_streams = only_streams(*sp);
       break;
     case ACC_SKEL_PERMUTE:
       if (sp->permutation.empty()) return fail(ACC_ERR_INVALID, "permute: `permutation` fragment missing");

@@ -53,6 +53,7 @@ struct SkelSpec {
   int block = 256, unroll = 4, rows = 4, chunk = 4096;
   int merge_waves = 8;                  // permute of 16-bit counts: waves of a workgroup of permute_merge
   int chunk_long = 0;                   // segmented folds: the staged chunk of variants 2 and 3 (segments of 8 elements or more on average); 0: none
+  bool get_streams = false;             // segmented folds: the element function reads its operands at the element's own index and no others
   bool fold_across = false;             // ACC_FLAG_TILED on a fold along the innermost dimension: neighbouring rows are neighbours in memory
   bool permute_replace = false;         // permute whose combination is spelt `x` (the new value): skel_scatter.h
   int map_tile_dim = 1;                 // ACC_FLAG_TILE_DIM: which dimension of the result, counted from the innermost, the tiles pair with it
