@@ -40,6 +40,9 @@
 #define ACC_GIVE  (ACC_RADIUS_X == 1 ? 1 : 0)         /* lanes hand each other the columns beside their own */
 #define ACC_OWNED (ACC_WAVE - 2 * ACC_GIVE)           /* lanes whose columns are stored */
 
+/* what is known of a vector's address */
+#define ACC_FLAT_ALIGN(S) (ACC_ALIGNED ? (ACC_SVEC * sizeof(S) < 16 ? ACC_SVEC * sizeof(S) : 16) : alignof(S))
+
 #define ACC_B_CLAMP 0
 #define ACC_B_MIRROR 1
 #define ACC_B_WRAP 2
@@ -71,8 +74,10 @@ ACC_DEV S acc_flat_shift(const S &x)
 /* the source as a lane sees it */
 template <typename S, int MODE>
 struct acc_flat_source {
+  /* rows begin on 16-byte boundaries in an aligned instance: whole vectors then, unless a vector is longer than that */
+  static constexpr bool WHOLE = ACC_ALIGNED && ACC_SVEC * sizeof(S) <= 16;
   struct row { S e[ACC_WW]; };
-  struct __attribute__((aligned(ACC_ALIGNED ? ACC_SVEC * sizeof(S) : alignof(S)))) vec { S v[ACC_SVEC]; };
+  struct __attribute__((aligned(ACC_FLAT_ALIGN(S)))) vec { S v[ACC_SVEC]; };
   static constexpr bool GIVE = ACC_GIVE != 0, ENDS = GIVE && MODE == ACC_B_WRAP;      /* ENDS: the other end of a row is read */
   static constexpr int SIDE = ACC_RADIUS_X > 0 ? ACC_RADIUS_X : 1;
 
@@ -96,7 +101,7 @@ struct acc_flat_source {
     rows_in = left_in = right_in = 0;
     at_left = x == 0;
     at_right = x + ACC_SVEC == w;
-    rest = ACC_ALIGNED ? 0 : w % ACC_SVEC;
+    rest = WHOLE ? 0 : w % ACC_SVEC;
     last = rest != 0 && at_right && !at_left;
     next_last = rest != 0 && !at_right && x + 2 * ACC_SVEC > w;
 #pragma unroll
@@ -151,7 +156,7 @@ struct acc_flat_source {
         /* what the neighbours get: the columns at the ends, or, where the last vector of a row overlaps the one before
          * it, those that stand beside the other's */
         S first = v[0], back = v[ACC_SVEC - 1];
-        if (!ACC_ALIGNED) {
+        if (!WHOLE) {
           S to_left = v[ACC_SVEC - 1], to_right = v[0];                            /* (rest 1) */
 #pragma unroll
           for (int k = 2; k < ACC_SVEC; ++k) {
@@ -162,8 +167,10 @@ struct acc_flat_source {
           back = next_last ? to_right : back;
         }
         const S l = acc_flat_shift<ACC_DPP_WAVE_SHR1>(back), t = acc_flat_shift<ACC_DPP_WAVE_SHL1>(first);
-        const S beyond_l = MODE == ACC_B_CONSTANT ? outside : (MODE == ACC_B_WRAP ? end[ENDS ? i : 0][ENDS ? p : 0] : v[MODE == ACC_B_MIRROR && ACC_SVEC > 1 ? 1 : 0]);
-        const S beyond_r = MODE == ACC_B_CONSTANT ? outside : (MODE == ACC_B_WRAP ? (at_left ? v[0] : end[ENDS ? i : 0][ENDS ? p : 0]) : v[MODE == ACC_B_MIRROR && ACC_SVEC > 1 ? ACC_SVEC - 2 : ACC_SVEC - 1]);
+        /* (the columns next to the first and the last: with one column a lane, where there are any, the neighbours hold them) */
+        const S second = ACC_SVEC > 1 ? v[ACC_SVEC > 1 ? 1 : 0] : (at_right ? v[0] : t), last_but_one = ACC_SVEC > 1 ? v[ACC_SVEC > 1 ? ACC_SVEC - 2 : 0] : (at_left ? v[0] : l);
+        const S beyond_l = MODE == ACC_B_CONSTANT ? outside : (MODE == ACC_B_WRAP ? end[ENDS ? i : 0][ENDS ? p : 0] : (MODE == ACC_B_MIRROR ? second : v[0]));
+        const S beyond_r = MODE == ACC_B_CONSTANT ? outside : (MODE == ACC_B_WRAP ? (at_left ? v[0] : end[ENDS ? i : 0][ENDS ? p : 0]) : (MODE == ACC_B_MIRROR ? last_but_one : v[ACC_SVEC - 1]));
         r.e[0] = at_left ? beyond_l : l;
         r.e[ACC_WW - 1] = at_right ? beyond_r : t;
       } else {
@@ -251,7 +258,7 @@ stencil(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk ACC_GU
 #define ACC_STORE_COMPONENT(c, CT)                                                                  \
     {                                                                                               \
       typedef CT acc_out_native __attribute__((ext_vector_type(ACC_SVEC)));                       \
-      typedef acc_out_native acc_out_stored __attribute__((aligned(ACC_ALIGNED ? ACC_SVEC * sizeof(CT) : alignof(CT)))); \
+      typedef acc_out_native acc_out_stored __attribute__((aligned(ACC_FLAT_ALIGN(CT))));         \
       char *plane = (char *)arrOut_##c + (Int64)(acc_z0 + acc_z) * ((Int64)acc_h * acc_w * (Int64)sizeof(CT)); \
       const unsigned int at = ((unsigned int)acc_y * (unsigned int)acc_w + (unsigned int)acc_x) * (unsigned int)sizeof(CT); \
       acc_out_native nv;                                                                          \

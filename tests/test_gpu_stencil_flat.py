@@ -120,3 +120,28 @@ def test_planes_dealt_out_over_the_dies(ctx, boundary, ctype, dt, taps):
             sk.stencil(None, src, out)
             got.append(out.get())
         assert np.array_equal(got[0], got[1]), (d, h, w)
+
+
+@pytest.mark.parametrize("boundary", ["clamp", "mirror", "wrap", "constant"])
+@pytest.mark.parametrize("svec,ctype,dt,taps", [(1, "float", np.float32, BOX), (1, "double", np.float64, STAR), (2, "Int32", np.int32, STAR),
+                                                (4, "double", np.float64, STAR), (8, "float", np.float32, STAR), (8, "Int64", np.int64, BOX)])
+def test_columns_a_lane(ctx, boundary, svec, ctype, dt, taps):
+    """as many as stencil.svec says: one, whose neighbours stand with other lanes where the boundary mirrors them, and more
+    than 16 bytes of them, of which rows that begin on a 16-byte boundary need not be a whole number"""
+    import acchip as A
+    fn = " + ".join("(%s)%d * t%d" % (ctype, 3 + k % 5, k) for k in range(len(taps)))
+    desc = dict(out_rank=3, taps=taps, boundary=boundary, stencil_fn=fn, boundary_constant="(%s)7" % ctype if boundary == "constant" else None)
+    with A.tuning("stencil.flat=2,stencil.thin_3d=0,stencil.svec=%d" % svec, ctx):
+        assert "skel_stencil_flat.h" in A.preview(A.make_desc(A.SKEL_STENCIL, ctype, **desc), 8)[1] or svec * np.dtype(dt).itemsize > 32
+        flat = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+    with A.tuning("stencil.nd=1", ctx):
+        each = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+    rng = np.random.default_rng(5)
+    for d, h, w in ((5, 7, 20), (9, 5, 36), (3, 6, 61), (4, 62, 64), (6, 70, 130), (3, 3, 16), (4, 9, 260)):
+        print(svec, ctype, boundary, d, h, w, flush=True)
+        src, got = ctx.array(rng.integers(-50, 50, (d, h, w)).astype(dt)), []
+        for sk in (flat, each):
+            out = ctx.array(np.full((d, h, w), 77, dt))
+            sk.stencil(None, src, out)
+            got.append(out.get())
+        assert np.array_equal(got[0], got[1]), (d, h, w)
