@@ -1341,6 +1341,34 @@ int acc_exec_permute(acc_skel s, const acc_array *env, int64_t n_src, const acc_
   return rc;
 }
 
+// Whether a volume that could go by the vectors of whole planes (skel_stencil_flat.h) is better off in strips that walk through
+// many planes: `both` the bytes of an element of source and result.  us in strips / by vectors, 7 and 27 points Float32, then
+// 7 and 27 points Float64 of half the columns or other sizes as given:
+//   - By vectors what the memory-side cache holds a good part of (200 x 512 x 512 55 / 50, 127 / 62; 60 x 1024 x 1024 64 / 61,
+//     118 / 74; Float64 50 x 512 x 1024 53 / 52, 89 / 58), and rows that leave much of a strip outside the array (400^3 Float64
+//     244 / 218, 356 / 228; 418 x 418 x 600 220 / 169, 252 / 183; 250 x 900 x 900 377 / 346, 375 / 371).
+//   - Rows of whole strips: in strips from 768 MB on (512^3 194 / 222, 203 / 234; 50 x 1000 x 1024 Float64 145 / 172, 178 / 192),
+//     and from 512 MB on where planes lie far apart: a result that reads few rows from planes of 2 MB on (150 x 512 x 1024
+//     108 / 134, 75 x 1024 x 1024 100 / 130; Float64 170 x 512 x 512 136 / 149, 75 x 512 x 1024 101 / 137; but 360 x 512 x 512
+//     158 / 150), one that reads many from 2^19 elements and 576 MB on (180 x 512 x 1024 153 / 178, 75 x 1024 x 1024 144 / 165,
+//     Float64 75 x 512 x 1024 144 / 161; but 130 x 512 x 1024 133 / 105, 170 x 512 x 512 Float64 196 / 164).
+//   - Rows of nearly whole strips (a twentieth outside at most) in strips from 512 MB and planes of 3.5 MB on: Float64 that
+//     reads few rows (45 x 1000 x 1000 134 / 153, 300 x 700 x 760 501 / 560, 500 x 640 x 1000 983 / 1143; with 27 points 164 / 167,
+//     632 / 610, 1186 / 1208: left), Float32 that reads many (90 x 1000 x 1000 158 / 167, 200 x 1200 x 1000 415 / 459, 1000^3 1658 /
+//     1816), and Float32 that reads few up to planes of 6 MB (135 / 149, 407 / 416, 1647 / 1718; but 150 x 1500 x 2040 966 / 846,
+//     100 x 3000 x 2500 1427 / 1353).  Smaller planes go either way (510^3 222 / 219, 228 / 233; 600 x 512 x 500 279 / 251, 337 /
+//     263; 600 x 400 x 1000 396 / 415, 406 / 442; 300 x 700 x 760 271 / 260, 331 / 288).
+static bool volume_in_strips(const acc_skel_s *s, int64_t w, int64_t h, int64_t planes, int64_t both)
+{
+  const int64_t half = (int64_t)32 * s->spec.svec, halves = (w + half - 1) / half;
+  const int64_t covered = half * (halves <= 3 ? halves : (halves + 1) / 2 * 2);        // columns of all strips (half ones up to three)
+  const int64_t kb = w * h * both / 1024 * planes, plane_kb = w * h * both / 2048;
+  const bool few = s->spec.flat_prefetch >= s->spec.flat_planes, wide = both >= 16;
+  if (kb <= 512 * 1024) return false;
+  if (w % (2 * half) == 0) return kb > 768 * 1024 || (few ? plane_kb >= 2048 : kb > 576 * 1024 && w * h >= (1 << 19));
+  return (covered - w) * 20 <= covered && plane_kb >= 3584 && (few ? wide || plane_kb <= 6144 : !wide);
+}
+
 // `in2` is the second source of a stencil2, NULL for a stencil
 static int stencil_once(acc_skel s, const acc_array *env, const acc_array *in, const acc_array *in2, const acc_array *out, hipStream_t st)
 {
@@ -1394,14 +1422,9 @@ static int stencil_once(acc_skel s, const acc_array *env, const acc_array *in, c
     return launch(s, v, grid, 0, st, &args);
   }
   // A volume takes variants 8 and 9, lanes over the vectors of a whole plane, where the instance has them
-  // (skel_stencil_flat.h; us in strips / so, buffers that the memory-side cache does not hold: 7 points Float32 300^3 77 /
-  // 45.3, 256^3 30.6 / 28.4, 128 x 128 x 256 9.0 / 7.5, 300 x 512 x 512 135 / 131, 418 x 418 x 600 222 / 173, 273 x 274 x 1400
-  // 190 / 178; 27 points 256^3 36.5 / 31.7, 323 x 324 x 1000 226 / 192; Float64 400^3 248 / 217, 27 points 316 / 258).  Only
-  // where rows are whole strips and the arrays large, so that planes lie far apart, are strips ahead that walk through many
-  // of them: 512^3 195 / 231 (27 points 240 / 234), 256 x 512 x 512 Float64 192 / 243.
-  const bool small = array_size(*out) * (int64_t)(s->spec.elt_size + acc::type_size(s->spec.stencil_in_comps[0])) <= ((int64_t)768 << 20);
+  // (skel_stencil_flat.h) and volume_in_strips does not say otherwise.
   if (s->spec.flat_planes > 0 && s->knobs.stencil_flat != 0 && w >= s->spec.svec &&
-      (w % ((int64_t)64 * s->spec.svec) != 0 || small || s->knobs.stencil_flat == 2)) {
+      (s->knobs.stencil_flat == 2 || !volume_in_strips(s, w, h, planes, s->spec.elt_size + acc::type_size(s->spec.stencil_in_comps[0])))) {
     const int64_t deep = s->spec.flat_planes, per_block = s->spec.block / 64;
     const int64_t owned = s->spec.reach_x == 1 ? 62 : 64;          // lanes that store: the others hand over columns
     const int64_t per_plane = (((w + s->spec.svec - 1) / s->spec.svec) * h + owned - 1) / owned, runs = (planes + deep - 1) / deep;

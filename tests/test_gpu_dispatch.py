@@ -31,3 +31,32 @@ def test_segments_a_workgroup(ctx, nseg, mean, own, get):
     out = ctx.empty(nseg, np.int32)
     sk.foldseg([], nseg * mean, ctx.array((np.arange(nseg + 1) * mean).astype(np.int32)), out)
     assert np.array_equal(out.get(), np.arange(nseg) // own)
+
+
+SEVEN = [(0, 0, 0), (-1, 0, 0), (1, 0, 0), (0, -1, 0), (0, 1, 0), (0, 0, -1), (0, 0, 1)]
+BOX = [(z, y, x) for z in (-1, 0, 1) for y in (-1, 0, 1) for x in (-1, 0, 1)]
+
+
+@pytest.mark.parametrize("ctype,dt,taps,shape,strips", [
+    # 512 MB of source and result at most
+    ("Int32", np.int32, SEVEN, (60, 1024, 1024), False), ("Int32", np.int32, BOX, (60, 1000, 1000), False),
+    # whole strips: planes far apart, or near each other
+    ("Int32", np.int32, SEVEN, (131, 512, 1024), True), ("Int32", np.int32, SEVEN, (257, 512, 512), False), ("Int32", np.int32, BOX, (140, 512, 1024), False),
+    ("Int32", np.int32, BOX, (150, 512, 1024), True), ("Int64", np.int64, BOX, (150, 512, 512), False), ("Int64", np.int64, SEVEN, (131, 512, 512), True),
+    ("Int64", np.int64, BOX, (75, 512, 1024), True), ("Int32", np.int32, SEVEN, (400, 512, 512), True),
+    # nearly whole ones, and rows that leave more of a strip outside
+    ("Int32", np.int32, SEVEN, (70, 1000, 1000), True), ("Int32", np.int32, SEVEN, (45, 1580, 1000), False), ("Int32", np.int32, BOX, (45, 1580, 1000), True),
+    ("Int32", np.int32, SEVEN, (80, 900, 970), False), ("Int64", np.int64, SEVEN, (66, 700, 760), True), ("Int64", np.int64, BOX, (66, 700, 760), False)])
+def test_volumes_in_strips_or_by_vectors(ctx, ctype, dt, taps, shape, strips):
+    import acchip as A
+    print(ctype, len(taps), shape, flush=True)
+    desc = dict(out_rank=3, taps=taps, boundary="clamp", stencil_fn="(%s)blockIdx.x + 0 * (%s)" % (ctype, " + ".join("t%d" % k for k in range(len(taps)))))
+    src, got = ctx.empty(shape, dt), []
+    out = ctx.empty(shape, dt)
+    for knobs in ("stencil.flat=1", "stencil.flat=0", "stencil.flat=2"):
+        with A.tuning(knobs, ctx):
+            sk = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+        sk.stencil(None, src, out)
+        got.append(out.get())
+    alike = [np.mean(got[0] == g) for g in got[1:]]            # (a last strip that overlaps its neighbour: either number)
+    assert alike[0 if strips else 1] > 0.98 and alike[1 if strips else 0] < 0.5, alike
