@@ -1,7 +1,8 @@
 /*
- * skel_stencil_pair.h -- three or four applications of a 2-D stencil in one launch, for a call that applies one many times
+ * skel_stencil_pair.h -- several applications of a 2-D stencil in one launch, for a call that applies one many times
  * (acc_exec_stencil_iterate): what lies between them stays in registers, and most of the arrays' trips through memory are
- * gone.
+ * gone.  Four, three and two (ACC_PAIR_LEVELS) are modules of their own, which are compiled at the same time: the three
+ * in one took 1.4 s, a module takes 0.75.
  *
  * A wave owns a strip of columns, 64 vectors of ACC_SVEC less the outermost ones on either side, and `acc_walk` rows of the
  * result.  It walks down the source from as many rows above them as there are applications (times ry) to as many below,
@@ -27,13 +28,15 @@
  * What bounds it: memory -- waves that walk copy at 5.4 TB/s at best, 100 us for 8192 x 8192 Float32 -- with the vector
  * units close behind (15 instructions an element and application of 3 x 3, 105 us for four).  3 x 3 on 8192 x 8192
  * Float32: four applications 116 us and three 107, one by itself 88; two a launch, in strips that asked for all their rows
- * at once, 96.  Ten in a call, two of them by themselves: 884 us one a launch, 554 in pairs, 405 so.  3001 x 5000 Float64
- * 56 / 58 (43 one by itself), 3000 x 3000 Float32 24 / 20 (17), 300 x 300 6.4 / 6.2 (4.5: launches count).  Walks of 28
+ * at once, 96.  Ten in a call, two of them by themselves: 884 us one a launch, 554 in pairs, 405 so.  Four, three, two and one by
+ * itself: 3000 x 3000 Float32 27.1 / 20.9 / 16.2 / 15.9, Float64 33.2 / 25.9 / 22.3 / 27.1, 500 x 500 Float32 7.2 / 5.8 / 4.8 / 3.2
+ * (launches count).  Two are there for calls of five and six on arrays that the memory-side cache holds: 3000 x 3000 Float64 77 /
+ * 68.5 and 108 / 100 without and with them.  Walks of 28
  * rows: of 16 / 20 / 24 / 32 / 36 / 40 rows four take 126 / 121 / 119 / 117 / 120 / 118 us (4001 x 8191: 59 / 59 / 59 /
  * 61 / 59 / 61, and 59); shorter ones where the array would give too few waves (the driver's rule).  Six rows ahead instead
  * of three: the same.  Non-temporal stores: 8192 x 8192 the same, arrays that the memory-side cache holds a tenth slower.
  *
- * Generated definitions expected: those of skel_stencil.h, for ACC_STENCIL_RANK 2, one source of one component of the
+ * Generated definitions expected: ACC_PAIR_LEVELS and those of skel_stencil.h, for ACC_STENCIL_RANK 2, one source of one component of the
  * result's type, no arrays in the environment, taps at most one row and one column away; rows as long as a strip, or at
  * least as much longer as the outermost lanes of one side are wide; three rows or more.
  */
@@ -53,14 +56,6 @@ static_assert(ACC_RADIUS_X <= 1 && ACC_RADIUS_Y <= 1 && ACC_SVEC >= 2, "a lane h
 #define ACC_B_MIRROR 1
 #define ACC_B_WRAP 2
 #define ACC_B_CONSTANT 3
-
-ACC_DEV int acc_pair_boundary(int i, const int sz)
-{
-  if (ACC_BOUNDARY == ACC_B_MIRROR) i = i < 0 ? -i : (i >= sz ? sz - (i - sz + 2) : i);
-  if (ACC_BOUNDARY == ACC_B_WRAP)   i = i < 0 ? sz + i : (i >= sz ? i - sz : i);
-  /* clamped in every mode: the maps assume the array spans the stencil; keep the address legal if not */
-  return acc_max(0, acc_min(i, sz - 1));
-}
 
 #define ACC_DPP_WAVE_SHL1 0x130
 /* the neighbouring lane's value; the lane that has no neighbour gets zero (nobody looks), which spares the move that a
@@ -223,12 +218,5 @@ extern "C" __global__ void __launch_bounds__(ACC_BLOCK)
 stencil(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk ACC_GUARD_PARAM)
 {
   ACC_GUARD_CHECK
-  acc_applications<4>(shOut_1, shOut_0, arrOut_0, arrStencil_0, acc_walk);
-}
-
-extern "C" __global__ void __launch_bounds__(ACC_BLOCK)
-stencil_three(ACC_ENV_PARAMS ACC_OUT_PARAMS ACC_SRC1_PARAMS, const int acc_walk ACC_GUARD_PARAM)
-{
-  ACC_GUARD_CHECK
-  acc_applications<3>(shOut_1, shOut_0, arrOut_0, arrStencil_0, acc_walk);
+  acc_applications<ACC_PAIR_LEVELS>(shOut_1, shOut_0, arrOut_0, arrStencil_0, acc_walk);
 }

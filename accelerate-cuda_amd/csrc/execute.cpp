@@ -759,16 +759,16 @@ namespace {
 
 // A variant that makes what another one of the instance makes too: whether it is there, or can be had now (a stream under
 // capture is no place to load a module).  Where it cannot be built the call goes on with the other.
-bool may_take(acc_skel s, int v, hipStream_t st)
+bool may_build(hipStream_t st)
 {
-  if (s->variant_ready(v)) return true;
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &capture) != hipSuccess) {
     (void)hipGetLastError();      // (answered by the other form: no later call is to find this error)
     return false;
   }
-  return capture == hipStreamCaptureStatusNone && s->ensure_variant(v) == ACC_OK;
+  return capture == hipStreamCaptureStatusNone;
 }
+bool may_take(acc_skel s, int v, hipStream_t st) { return s->variant_ready(v) || (may_build(st) && s->ensure_variant(v) == ACC_OK); }
 
 // scanOp / scan1Op / scan'Op / scanCore, Execute.hs:328-392, as ONE launch.  `noalloc`: the tile descriptors live in
 // the library's file-scope device array instead of a block of the context's pool, and nothing may be allocated,
@@ -1477,25 +1477,42 @@ static int stencil_once(acc_skel s, const acc_array *env, const acc_array *in, c
   return launch(s, (aligned ? 0 : 1) + 2 * narrow, (strips_x * bands * zbands + waves - 1) / waves, 0, st, &args);
 }
 
-// Three or four applications of a stencil in one launch (skel_stencil_pair.h), where the instance and the shape allow: false
-// if not, and nothing has been done.
-static bool stencil_many(acc_skel s, int levels, const acc_array *env, const acc_array *in, const acc_array *out, hipStream_t st, int *rc)
+// Two, three or four applications of a stencil in one launch (skel_stencil_pair.h): the waves' columns, rows and number, where
+// the instance and the shape allow; false if not.
+struct ManyPlan { int64_t walk, waves; };
+static bool plan_many(const acc_skel_s *s, int levels, const acc_array *out, ManyPlan *plan)
 {
   if (!s->spec.pair_form || s->knobs.stencil_pair == 0 || array_size(*out) == 0) return false;
   // lanes at either side of a strip whose columns go wrong, and the columns of a strip (as the kernel has them)
   const int64_t svec = s->spec.svec, outer = s->spec.reach_x > 0 ? (levels + svec - 1) / svec : 1, owned = (64 - 2 * outer) * svec;
-  const int64_t w = out->shape[1], h = out->shape[0], esz = s->spec.elt_size;
+  const int64_t w = out->shape[1], h = out->shape[0];
   if ((w != owned && w < owned + outer * svec) || h < 3 || w >= (1 << 30) || h >= (1 << 30)) return false;
   const int64_t strips = (w + owned - 1) / owned;
   // rows a wave walks through: 28, or fewer, down to 4, as long as that leaves a compute unit fewer than eight waves (the
   // rows above and below are read and worked out for every walk anew: 3000 x 3000 Float32 in 28 / 20 / 12 / 8 rows 24.5 /
   // 22.4 / 25.0 / 23.3 us for four applications, 1024 x 1024 in 16 / 8 / 4 rows 14.2 / 9.9 / 9.2, 300 x 300 13.5 / 9.1 / 6.3)
-  int64_t walk = s->knobs.stencil_pair_walk;
-  if (walk <= 0) walk = std::max<int64_t>(4, std::min<int64_t>(28, h * strips / (8 * (int64_t)s->ctx->props.multiProcessorCount)));
-  const int64_t bands = (h + walk - 1) / walk;
-  if (strips * bands >= (1 << 30)) return false;
-  const int v = 10 + ((aligned16(in->ptr[0]) && aligned16(out->ptr[0]) && w * esz % 16 == 0) ? 0 : 1);
-  if (!may_take(s, v, st)) return false;
+  plan->walk = s->knobs.stencil_pair_walk;
+  if (plan->walk <= 0) plan->walk = std::max<int64_t>(4, std::min<int64_t>(28, h * strips / (8 * (int64_t)s->ctx->props.multiProcessorCount)));
+  plan->waves = strips * ((h + plan->walk - 1) / plan->walk);
+  return plan->waves < (1 << 30);
+}
+
+// ... and the launch; false, with nothing done, where a form is not there and cannot be had.
+static bool stencil_many(acc_skel s, int levels, const acc_array *env, const acc_array *in, const acc_array *out, hipStream_t st, int *rc)
+{
+  ManyPlan plan;
+  if (!plan_many(s, levels, out, &plan)) return false;
+  const int64_t w = out->shape[1], esz = s->spec.elt_size;
+  // the forms for four, three and two are compiled at the same time and loaded together, four the last: which of them a call
+  // finds does not hang on what was called before
+  const int four = 10 + ((aligned16(in->ptr[0]) && aligned16(out->ptr[0]) && w * esz % 16 == 0) ? 0 : 1), v = four + 2 * (4 - levels);
+  if (!s->variant_ready(four)) {
+    if (!may_build(st)) return false;
+    for (int k = four; k < four + 6; k += 2)
+      if (s->start_variant(k) != ACC_OK) return false;
+    for (int k = four + 4; k >= four; k -= 2)
+      if (s->ensure_variant(k) != ACC_OK) return false;
+  }
   *rc = [&]() -> int {
     ACC_RUN_SCOPE(s, st);
     Args args;
@@ -1503,14 +1520,54 @@ static bool stencil_many(acc_skel s, int levels, const acc_array *env, const acc
     ACC_TRY(push_env(s, env, &args, &aligned));
     push_out(*out, &args, &aligned);
     push_ptrs(in, in->ncomp, &args, &aligned);
-    args.i32(static_cast<int32_t>(walk));
-    const int64_t per_block = s->spec.block / 64, grid = (strips * bands + per_block - 1) / per_block;
+    args.i32(static_cast<int32_t>(plan.walk));
+    const int64_t per_block = s->spec.block / 64, grid = (plan.waves + per_block - 1) / per_block;
     ACC_TRY(s->ctx->make_current());
     const acc::Variant &var = s->variants[v];
-    ACC_HIP_TRY(launch_kernel(levels == 4 ? var.fn : var.fn_three, static_cast<unsigned>(grid), 1, 1, static_cast<unsigned>(var.block), 1, 1, 0, st, args.data(), nullptr));
+    ACC_HIP_TRY(launch_kernel(var.fn, static_cast<unsigned>(grid), 1, 1, static_cast<unsigned>(var.block), 1, 1, 0, st, args.data(), nullptr));
     return ACC_OK;
   }();
   return true;
+}
+
+// What a launch of one, two, three and four applications takes, in twentieths of one by itself (entry 0 is not used).  3 x 3, us
+// one / two / three / four: small arrays, where launches count, 500 x 500 Float32 3.2 / 4.8 / 5.8 / 7.2, 768 x 768 Float64 4.3 /
+// 6.4 / 7.7 / 9.1; such that the memory-side cache holds both, where one application by itself writes past it, 3000 x 3000
+// Float32 15.9 / 16.2 / 20.9 / 27.1, Float64 27.1 / 22.3 / 25.9 / 33.2, 4096 x 4096 Float64 45.6 / 35.6 / 42.8 / 54.2; and larger
+// ones, 8192 x 8192 88 / 110 / 111 / 116, Float64 176 / 225 / 217 / 218.  A call of five, as 2 2 1 and as 3 1 1: 12.6 / 12.3,
+// 16.6 / 17.2; 45.8 / 50.8, 68 / 77, 108 / 123; 305 / 272, 620 / 563.  Of six, as 2 2 1 1 and as 3 1 1 1, either side of the
+// lower line: 1500 x 1500 Float32 33.9 / 31.7, 2048 x 2048 37.4 / 39.8; of the upper one: 4096 x 4096 Float64 160 / 176, 6000 x
+// 6000 Float32 219 / 202.
+static const int32_t *stencil_costs(const acc_skel_s *s, const acc_array *out)
+{
+  static const int32_t small[5] = {0, 20, 31, 37, 44}, held[5] = {0, 20, 19, 23, 30}, large[5] = {0, 20, 25, 25, 27};
+  const int64_t bytes = array_size(*out) * (int64_t)s->spec.elt_size;
+  return bytes < ((int64_t)12 << 20) ? small : bytes <= ((int64_t)128 << 20) ? held : large;
+}
+
+// How many launches of four, three and two applications a call of `iters` makes (left[4], left[3] and left[2]; the rest go one by
+// one): as leaves every result where one a launch would, so an even number of fours and twos together -- the arrays then have
+// changed places as often; a three changes them as three single ones do -- and at least one application by itself at the
+// end, whose source is then the result before the last.  Of these splits the one that takes least.  (Strips of two columns a
+// lane are wider for two applications than for three or four: what the rows are too short for is not among them.)
+static void stencil_split(const acc_skel_s *s, const acc_array *out, int32_t iters, int32_t left[5])
+{
+  const int32_t *cost = stencil_costs(s, out);
+  const int64_t many = std::max(iters, 1) - 1;
+  ManyPlan plan;
+  const bool threes = plan_many(s, 3, out, &plan), twos = plan_many(s, 2, out, &plan);
+  const int64_t most = plan_many(s, 4, out, &plan) ? many / 4 : 0;
+  int64_t least = -1;
+  for (int64_t four = most; four >= 0 && four > most - 8; --four)
+    for (int64_t two = four & 1; two <= (twos ? 3 : 0) && 4 * four + 2 * two <= many; two += 2) {
+      const int64_t rest = many - 4 * four - 2 * two, three = threes ? rest / 3 : 0, one = rest - 3 * three;
+      const int64_t all = four * cost[4] + three * cost[3] + two * cost[2] + one * cost[1];
+      if (least >= 0 && all >= least) continue;
+      least = all;
+      left[4] = static_cast<int32_t>(four);
+      left[3] = static_cast<int32_t>(three);
+      left[2] = static_cast<int32_t>(two);
+    }
 }
 
 static int stencil_check(acc_skel s, const acc_array *in, const acc_array *out)
@@ -1555,31 +1612,19 @@ int acc_exec_stencil_iterate(acc_skel s, const acc_array *env, const acc_array *
   ACC_TRY(stencil_check(s, a, b));
   if (iters < 0) return fail(ACC_ERR_INVALID, "stencil: negative iteration count");
   const acc_array *src = a, *dst = b;
-  // Four and three applications a launch as often as leaves every result where one a launch would: an even number of
-  // fours, so that the arrays have changed places as often (a three changes them as three single ones do), and at least
-  // one application by itself at the end, whose source is then the result before the last.  Of these splits the one that
-  // takes least: of large arrays a four takes 1.25 to 1.4 times a single application, a three 1.15 to 1.3.
-  const int32_t many = std::max(iters, 1) - 1;
-  int32_t fours = 0, threes = 0;
-  for (int32_t q = many / 4 / 2 * 2, least = -1; q >= 0 && q > many / 4 - 8; q -= 2) {
-    const int32_t t = (many - 4 * q) / 3, cost = 27 * q + 25 * t + 20 * (many - 4 * q - 3 * t);
-    if (least >= 0 && cost >= least) continue;
-    least = cost;
-    fours = q;
-    threes = t;
-  }
+  int32_t left[5] = {0, 0, 0, 0, 0};
+  stencil_split(s, b, iters, left);
   for (int32_t i = 0; i < iters;) {
-    const int32_t levels = fours > 0 ? 4 : threes > 0 ? 3 : 1;
+    const int32_t levels = left[4] > 0 ? 4 : left[3] > 0 ? 3 : left[2] > 0 ? 2 : 1;
     int rc = ACC_OK;
     if (levels > 1 && !stencil_many(s, levels, env, src, dst, static_cast<hipStream_t>(stream), &rc)) {
-      fours = threes = 0;                // (never after the first: what one launch has taken the others find there)
+      left[4] = left[3] = left[2] = 0;   // (never after the first: what one launch has taken the others find there)
       continue;
     }
     if (levels == 1) rc = stencil_once(s, env, src, nullptr, dst, static_cast<hipStream_t>(stream));
     ACC_TRY(rc);
     i += levels;
-    fours -= levels == 4 ? 1 : 0;
-    threes -= levels == 3 ? 1 : 0;
+    --left[levels];
     std::swap(src, dst);
   }
   if (result_in_b) *result_in_b = (iters & 1);

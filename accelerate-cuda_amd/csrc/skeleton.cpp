@@ -583,6 +583,7 @@ int generate_source(const SkelSpec &sp, bool aligned, std::string *entry, std::s
       o << "#define ACC_TILE_H " << sp.tile_h << "\n#define ACC_PREFETCH " << sp.prefetch << "\n#define ACC_BLOCK " << sp.block << "\n";
       o << "#define ACC_TZ " << sp.tile_z << "\n";
       o << "#define ACC_ZMARCH " << sp.zmarch << "\n";
+      if (sp.stencil_pair) o << "#define ACC_PAIR_LEVELS " << sp.pair_levels << "\n";
       if (sp.stencil_flat) o << "#define ACC_FLAT_PLANES " << sp.flat_planes << "\n#define ACC_FLAT_SPREAD " << flat_spread << "\n";
       tmpl = sp.stencil_pair ? "skel_stencil_pair.h" : sp.stencil_flat ? "skel_stencil_flat.h" : "skel_stencil.h";
       break;
@@ -958,7 +959,7 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
           sp->flat_prefetch = std::max(0, tune("stencil.flat_prefetch", at_once ? sp->flat_planes : (2 * rz + 2) * plane <= 144 ? 1 : 0));
         }
       }
-      // Three or four applications a launch, for calls that make many: of one array of 4- or 8-byte elements whose result is its
+      // Several applications a launch, for calls that make many: of one array of 4- or 8-byte elements whose result is its
       // source the next time, with taps no more than a row and a column away and nothing else to read.
       if (sp->out_rank == 2 && d->kind == ACC_SKEL_STENCIL && sp->stencil_in_comps.size() == 1 && sp->comp_types.empty() &&
           sp->stencil_in_comps[0] == sp->elt_type && sp->env.empty() && type_size(sp->elt_type) >= 4) {
@@ -1042,12 +1043,13 @@ SkelSpec spec_of_variant(const SkelSpec &base, int v)
     spec.svec = std::max(1, spec.svec >> (v / 2));
     spec.tile_w = 64 * spec.svec;
   }
-  // ... 10 and 11: three or four applications a launch; and 8 and 9: lanes over the vectors of a whole plane
+  // ... 10 and 11: four applications a launch (12 and 13 three, 14 and 15 two: built together with those and never by
+  // themselves); and 8 and 9: lanes over the vectors of a whole plane
   if (spec.kind == ACC_SKEL_STENCIL && v >= 10) {
     spec.stencil_pair = true;
+    spec.pair_levels = 4 - (v - 10) / 2;
     spec.stencil_nd = false;
     spec.svec = base.svec;
-    spec.tile_w = 62 * spec.svec;
     spec.tile_h = 1;
   } else if (spec.kind == ACC_SKEL_STENCIL && v >= 8) {
     spec.stencil_flat = true;
@@ -1228,15 +1230,6 @@ int acc_skel_s::load_variant(int v)
       return acc::fail_hip(e, ("hipModuleGetFunction(" + (var.fn_pieces ? lines : pieces) + ")").c_str());
     }
   }
-  if (spec.stencil_pair) {
-    const std::string three = entry_name + "_three";
-    e = hipModuleGetFunction(&var.fn_three, var.module, three.c_str());
-    if (e != hipSuccess) {
-      (void)hipModuleUnload(var.module);
-      var.module = nullptr;
-      return acc::fail_hip(e, ("hipModuleGetFunction(" + three + ")").c_str());
-    }
-  }
   (void)hipFuncGetAttribute(&var.num_regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, var.fn);
   if (this->spec.scan_shape_open && v < 2) {
     // the first build of a scan decides its tile shape: see make_spec
@@ -1268,7 +1261,7 @@ static int variant_count(const acc::SkelSpec &sp)
   return sp.kind == ACC_SKEL_PERMUTE ? (sp.permute_replace ? 2 : 8) : (stencil ? (sp.stencil_nd ? 2 : sp.pair_form ? 12 : sp.flat_planes > 0 ? 10 : 8) : (sp.scan_mid_rows > 0 ? 6 : (sp.scan_small_rows > 0 || sp.chunk_long > 0) ? 4 : 2));
 }
 
-// ... one of which is left out: of a 2-D stencil with two applications a launch (10 and 11) the form that 3-D ones have at 8 and 9
+// ... one of which is left out: of a 2-D stencil with several applications a launch (10 and 11) the form that 3-D ones have at 8 and 9
 static bool variant_exists(const acc::SkelSpec &sp, int v)
 {
   return v >= 0 && v < variant_count(sp) && !(sp.pair_form && (v == 8 || v == 9));
@@ -1320,6 +1313,8 @@ int acc_skel_prefetch(acc_skel s, int variant)
   // (the locked form of a permute is only generated for elements the atomic template does not take, and the other way round)
   if (s->spec.kind == ACC_SKEL_PERMUTE && s->spec.permute_locked && variant >= 2)
     return fail(ACC_ERR_INVALID, "acc_skel_prefetch: a permute under locks has variants 0 and 1");
+  if (s->spec.pair_form && variant >= 10)
+    for (int v = variant + 2; v < 16; v += 2) ACC_TRY(s->start_variant(v));
   return s->start_variant(variant);
 }
 

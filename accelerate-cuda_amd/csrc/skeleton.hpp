@@ -38,7 +38,8 @@ struct SkelSpec {
   int boundary2 = 0;
   std::string boundary2_constant, stencil_in2_type;
   std::vector<int> tap2_dz, tap2_dy, tap2_dx;
-  bool stencil_pair = false;            // a stencil's variants 10 and 11: three or four applications a launch (skel_stencil_pair.h)
+  bool stencil_pair = false;            // a stencil's variants 10 to 15: several applications a launch (skel_stencil_pair.h)
+  int pair_levels = 4;                  // ... how many
   bool pair_form = false;               // ... whether there are any
   bool stencil_flat = false;            // a stencil's variants 8 and 9: lanes over the vectors of a plane (skel_stencil_flat.h)
   int flat_planes = 0, flat_prefetch = 0;   // ... the planes a wave produces, and those it asks for ahead; 0: no such variants
@@ -85,7 +86,6 @@ struct Variant {
   hipFunction_t fn_across_wide = nullptr;   // ... _across_wide, several rows a lane (elements of at most 8 bytes)
   hipFunction_t fn_pieces = nullptr;   // a map in tiles: _pieces, for results whose rows are no whole cache lines
   hipFunction_t fn_lines = nullptr;    // ... _lines, for large ones of elements of 4 and 8 bytes
-  hipFunction_t fn_three = nullptr;    // a stencil's variants 10 and 11: three applications a launch (fn makes four)
   hipFunction_t fn_sweep = nullptr;    // a segmented fold's variants 4-7: _sweep, the segments that were handed over;
                                        // its variants 0-3: _probe, a look at the segment lengths
   int num_regs = 0;
@@ -113,7 +113,7 @@ struct acc_skel_s {
   acc::SkelSpec spec;
   acc::Knobs knobs;           // what the drivers read of the tuning table
   std::string entry;
-  acc::Variant variants[12];  // [0] pointers 16-byte aligned, [1] no assumption; [2], [3]: the same for the
+  acc::Variant variants[16];  // [0] pointers 16-byte aligned, [1] no assumption; [2], [3]: the same for the
                               // table-in-LDS form of a permute whose combination has no atomic instruction;
                               // [4], [5]: for a hinted permute over several LDS windows of targets;
                               // [6], [7]: for integer addition on a table of 16-bit counts in LDS;

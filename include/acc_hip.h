@@ -521,10 +521,10 @@ int acc_exec_stencil2(acc_skel s, const acc_array *env, const acc_array *in1, co
  * repeated run1, computes: Execute.hs:236-244, CUDA.hs:325-333).  The input is
  * a; *result_in_b tells where the last application wrote, the other array then
  * holds what that one read.  (A 2-D stencil of one array of 4- or 8-byte elements
- * with taps next to the element goes three or four applications a launch, but for
- * the last ones; the results are the same.  The variant that does -- 10, or 11 off
- * the 16-byte boundary -- is compiled by the first call of four or more
- * applications, half a second, unless acc_skel_prefetch has.)                 */
+ * with taps next to the element goes two, three or four applications a launch, but
+ * for the last ones; the results are the same.  The variant that does -- 10, or 11
+ * off the 16-byte boundary -- is compiled by the first call of four or more
+ * applications, a third of a second, unless acc_skel_prefetch has.)           */
 int acc_exec_stencil_iterate(acc_skel s, const acc_array *env, const acc_array *a, const acc_array *b,
                              int32_t iters, acc_stream stream, int32_t *result_in_b);
 

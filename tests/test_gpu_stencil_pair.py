@@ -110,6 +110,38 @@ def test_walks_that_go_up(ctx, boundary, ctype, dt, taps):
             assert got[0][0] == got[1][0] and all(np.array_equal(got[0][k], got[1][k]) for k in (1, 2)), (walk, h, iters)
 
 
+@pytest.mark.parametrize("boundary", ["clamp", "mirror", "wrap", "constant"])
+@pytest.mark.parametrize("ctype,dt,taps", [("float", np.float32, BOX), ("double", np.float64, CROSS), ("Int32", np.int32, ROWS), ("Int64", np.int64, BOX)])
+def test_two_a_launch(ctx, boundary, ctype, dt, taps):
+    """arrays of 12 MB and a little more, from which on calls of five and six applications make two a launch: the widths at
+    which the strips of two, of three and of four applications change form, and those that one of them cannot take"""
+    import acchip as A
+    whole = dt in (np.int32, np.int64)
+    fn = " + ".join("(%s)%s * t%d" % (ctype, (3 + 2 * k) if whole else repr(0.07 * (k + 1) - 0.2), k) for k in range(len(taps)))
+    desc = dict(out_rank=2, taps=taps, boundary=boundary, stencil_fn=fn, boundary_constant="(%s)7" % ctype if boundary == "constant" else None)
+    many = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+    with A.tuning("stencil.pair=0", ctx):
+        ones = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
+    vec, esz = 16 // np.dtype(dt).itemsize, np.dtype(dt).itemsize
+    widths = set()
+    for levels in (2, 3, 4):                      # a strip, as the kernel has it: the outermost lanes of either side store nothing
+        outer = -(-levels // vec) if any(dx for _, dx in taps) else 1
+        own = (64 - 2 * outer) * vec
+        widths |= {own, own + 1, own + outer * vec - 1, own + outer * vec, 2 * own + 1}
+    rng = np.random.default_rng(8)
+    for w in sorted(widths):
+        h = (12 << 20) // (w * esz) + 2
+        x = rng.integers(-50, 50, (h, w)).astype(dt)
+        for iters in (5, 6, 8, 10):
+            print(ctype, len(taps), boundary, (h, w), iters, flush=True)
+            got = []
+            for sk in (many, ones):
+                a, b = ctx.array(x), ctx.empty((h, w), dt)
+                res = sk.stencil_iterate(None, a, b, iters)
+                got.append((res is b, a.get(), b.get()))
+            assert got[0][0] == got[1][0] and all(np.array_equal(got[0][k], got[1][k]) for k in (1, 2)), (h, w, iters)
+
+
 @pytest.mark.parametrize("what,rank,shape", [("acc_pair_own", 2, (40, 300)), ("acc_flat_source", 3, (5, 7, 700))])
 def test_a_form_that_cannot_be_built_leaves_the_call_to_another(ctx, what, rank, shape):
     """a preamble that takes a name which only this form's template has: the form does not compile, the others do"""
