@@ -57,8 +57,10 @@ ACC_DEV int acc_flat_boundary(int i, const int sz)
   return acc_max(0, acc_min(i, sz - 1));
 }
 
-/* the neighbouring lane's value; a lane that has no neighbour gets zero (nobody looks) */
-#define ACC_DPP_WAVE_SHL1 0x130
+/* the neighbouring lane's value; a lane that has no neighbour gets that of the wave's other end (what it makes of it is
+ * dropped, but the element function is to see values of the array only) */
+#define ACC_DPP_WAVE_ROL1 0x134
+#define ACC_DPP_WAVE_ROR1 0x13C
 template <int CTRL, typename S>
 ACC_DEV S acc_flat_shift(const S &x)
 {
@@ -166,7 +168,7 @@ struct acc_flat_source {
           first = last ? to_left : first;
           back = next_last ? to_right : back;
         }
-        const S l = acc_flat_shift<ACC_DPP_WAVE_SHR1>(back), t = acc_flat_shift<ACC_DPP_WAVE_SHL1>(first);
+        const S l = acc_flat_shift<ACC_DPP_WAVE_ROR1>(back), t = acc_flat_shift<ACC_DPP_WAVE_ROL1>(first);
         /* (the columns next to the first and the last: with one column a lane, where there are any, the neighbours hold them) */
         const S second = ACC_SVEC > 1 ? v[ACC_SVEC > 1 ? 1 : 0] : (at_right ? v[0] : t), last_but_one = ACC_SVEC > 1 ? v[ACC_SVEC > 1 ? ACC_SVEC - 2 : 0] : (at_left ? v[0] : l);
         const S beyond_l = MODE == ACC_B_CONSTANT ? outside : (MODE == ACC_B_WRAP ? end[ENDS ? i : 0][ENDS ? p : 0] : (MODE == ACC_B_MIRROR ? second : v[0]));

@@ -208,3 +208,31 @@ def test_recorded_before_the_form_is_loaded(ctx, rank, shape):
         assert np.array_equal(got, eager.get()), replay
     hip.hipGraphExecDestroy(graph_exec)
     hip.hipGraphDestroy(graph)
+
+
+@pytest.mark.parametrize("ctype,dt", [("Int32", np.int32), ("double", np.float64)])
+@pytest.mark.parametrize("rank,shape,iters", [(2, (40, 256), 9), (2, (31, 508), 4), (2, (12400, 256), 5), (3, (9, 30, 150), 1)])
+def test_the_element_function_sees_values_of_the_array_only(ctx, ctype, dt, rank, shape, iters):
+    """also where what it makes is dropped, in the lanes at the ends of a wave (2-D: by four, three and two applications a launch):
+    the first zero it sees turns every later result into -1"""
+    import acchip as A
+    taps = BOX if rank == 2 else [(0, 0, 0), (-1, 0, 0), (1, 0, 0), (0, -1, 0), (0, 1, 0), (0, 0, -1), (0, 0, 1)]
+    args = ", ".join("t%d" % k for k in range(len(taps)))
+    pre = """__device__ int zero_seen;
+__device__ __forceinline__ %s look(%s, %s centre) {
+  if (%s) atomicOr(&zero_seen, 1);
+  return __atomic_load_n(&zero_seen, __ATOMIC_RELAXED) ? (%s)-1 : centre;
+}
+""" % (ctype, ", ".join("%s t%d" % (ctype, k) for k in range(len(taps))), ctype, " || ".join("t%d == 0" % k for k in range(len(taps))), ctype)
+    with A.tuning("stencil.flat=2,stencil.thin_3d=0", ctx):
+        sk = ctx.skeleton(A.SKEL_STENCIL, ctype, out_rank=rank, taps=taps, boundary="clamp", preamble=pre,
+                          stencil_fn="look(%s, t%d)" % (args, taps.index((0,) * rank)), wait=True)
+    x = np.random.default_rng(4).integers(1, 50, shape).astype(dt)
+    for _ in range(3):
+        a, b = ctx.array(x), ctx.empty(shape, dt)
+        if rank == 2:
+            res = sk.stencil_iterate(None, a, b, iters)
+        else:
+            sk.stencil(None, a, b)
+            res = b
+        assert np.array_equal(res.get(), x)
