@@ -309,11 +309,18 @@ int acc_exec_map(acc_skel s, const acc_array *env, const acc_array *out, acc_str
     bool whole = (w * esz) % 128 == 0;
     for (int c = 0; c < out->ncomp; ++c) whole = whole && out->ptr[c] % 128 == 0;
     const bool strips = whole && n == w * h && n * esz >= acc::map_strips_from;
-    // Results of no whole lines, or that begin amid one, go out in lines from 28 MB on, where they do not stay in the
-    // memory-side cache (us as they stand / in lines: 5003 x 3001 Float32 33.8 / 28.5, 8191^2 148 / 104, 3891 x 2048 17.9 /
-    // 15.8, 7001 x 2500 Float64 77 / 60, with another operand read along the rows 3001 x 2999 29.4 / 27.6, 5003 x 3001 47 / 43;
-    // but 1001 x 999 4.6 / 5.6, 1500 x 1501 with another operand 8.5 / 10.3, thirty planes of 400 x 501 14.8 / 16.5).
-    const bool in_lines = s->spec.map_lines && !whole && n * esz >= s->knobs.map_lines_from_mb * ((int64_t)1 << 20);
+    // Results of no whole lines, or that begin amid one, go out in lines from 28 MB on, about what the L2s hold together (us as
+    // they stand / in lines, operands that the memory-side cache does not hold: 5003 x 3001 Float32 33.3 / 28.8, 8191^2 148 / 104,
+    // 3891 x 2048 17.9 / 15.8, 7001 x 2500 Float64 77 / 60, with another operand read along the rows 3001 x 2999 29.4 / 27.6, 5003 x
+    // 3001 47 / 43; but 1001 x 999 4.6 / 5.6, 1500 x 1501 with another operand 8.5 / 10.3, thirty planes of 400 x 501 14.8 / 16.5).
+    // Lines have a third of the elements (of 8 bytes a seventh) evaluated twice, which is in the way where they take more than
+    // the memory does.  How much that is is told by the size of the kernel, straight through as it is: up to 16 KB of code, 40
+    // of 8-byte elements.  5003 x 3001 transposed, code of the lines / as it stands / in lines, Float32: e^x 7.7 KB 33.2 / 30.0, a
+    // polynomial of degree 24 14.5 KB 33.8 / 31.6, of 32 17.6 KB 34.1 / 36.1, of 64 29.9 KB 45.1 / 56.3, x^1.7 31.0 KB 50.9 / 68.0;
+    // Float64: degree 32 23.0 KB 67.1 / 58.9, sin 36.3 KB 102 / 92, x^1.7 46.9 KB 95 / 105, degree 64 60.8 KB 94 / 111; Int32: degree 32 13.6 KB 33.8 / 32.7,
+    // 64 21.9 KB 37.9 / 48.8.  (On the wrong side are tanh of Float32, short branches, 11.6 KB 48.5 / 52.5, and a Float64 polynomial of degree 48, 34.9 KB 68.5 / 76.8.)
+    const bool in_lines = s->spec.map_lines && !whole && n * esz >= s->knobs.map_lines_from_mb * ((int64_t)1 << 20) &&
+                          !s->spec.map_loops && s->variants[v].lines_code <= (esz == 8 ? 40 : 16) * (size_t)1024;
     const int64_t down = h <= side || in_lines ? 1 : (strips ? waves : (waves % 2 == 0 && !whole ? 2 : 1));
     const int64_t columns = waves / down * side - (in_lines ? 128 / esz : 0);
     const int64_t groups = ((w + columns - 1) / columns) * ((h + down * side - 1) / (down * side)) * (n / (w * h));

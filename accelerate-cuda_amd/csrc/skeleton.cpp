@@ -9,6 +9,7 @@
 #include <cctype>
 #include <cstdlib>
 #include <cstring>
+#include <elf.h>
 #include <set>
 #include <sstream>
 
@@ -661,6 +662,15 @@ static int segmented_chunk(const SkelSpec &sp, bool long_segments = false)
   return (want + per_load - 1) / per_load * per_load;
 }
 
+// whether `word` stands in a text by itself
+static bool has_word(const std::string &text, const std::string &word)
+{
+  auto part = [&](size_t i) { return i < text.size() && (std::isalnum((unsigned char)text[i]) || text[i] == '_'); };
+  for (size_t at = text.find(word); at != std::string::npos; at = text.find(word, at + 1))
+    if ((at == 0 || !part(at - 1)) && !part(at + word.size())) return true;
+  return false;
+}
+
 int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
 {
   if (!d) return fail(ACC_ERR_INVALID, "NULL skeleton description");
@@ -771,6 +781,7 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
         const int side = 8 * sp->map_tile_block, across = sp->block / 64 * side;
         sp->map_lines = sp->map_tiled && sp->comp_types.empty() && (type_size(sp->elt_type) == 4 || type_size(sp->elt_type) == 8) && across >= 64 &&
                         side * (across + 4) * sp->elt_size <= 65536 && tune("map.tiled_lines", 1) != 0;
+        for (const char *loop : {"for", "while", "do", "goto"}) sp->map_loops = sp->map_loops || has_word(sp->get, loop) || has_word(sp->preamble, loop);
       }
       break;
     case ACC_SKEL_FOLD: case ACC_SKEL_FOLD1:
@@ -1126,6 +1137,34 @@ int acc_skel_s::ensure_variant(int v)
   return other >= 0 ? load_variant(other) : ACC_OK;
 }
 
+// Bytes of machine code of kernel `name` in a code object (a 64-bit ELF file, whose symbols have sizes); 0 if that is not to be
+// found.
+static size_t code_bytes(const void *code, size_t size, const std::string &name)
+{
+  const char *p = static_cast<const char *>(code);
+  Elf64_Ehdr eh;
+  if (!p || size < sizeof(eh)) return 0;
+  std::memcpy(&eh, p, sizeof(eh));
+  if (std::memcmp(eh.e_ident, ELFMAG, SELFMAG) != 0 || eh.e_ident[EI_CLASS] != ELFCLASS64 || eh.e_shentsize != sizeof(Elf64_Shdr)) return 0;
+  auto within = [&](uint64_t at, uint64_t n) { return at <= size && n <= size - at; };
+  auto section = [&](uint64_t i, Elf64_Shdr *sh) {
+    if (i >= eh.e_shnum || !within(eh.e_shoff, (i + 1) * sizeof(*sh))) return false;
+    std::memcpy(sh, p + eh.e_shoff + i * sizeof(*sh), sizeof(*sh));
+    return within(sh->sh_offset, sh->sh_type == SHT_NOBITS ? 0 : sh->sh_size);
+  };
+  for (uint64_t i = 0; i < eh.e_shnum; ++i) {
+    Elf64_Shdr sh, names;
+    if (!section(i, &sh) || (sh.sh_type != SHT_SYMTAB && sh.sh_type != SHT_DYNSYM) || !section(sh.sh_link, &names) || names.sh_type != SHT_STRTAB) continue;
+    for (uint64_t at = 0; at + sizeof(Elf64_Sym) <= sh.sh_size; at += sizeof(Elf64_Sym)) {
+      Elf64_Sym sym;
+      std::memcpy(&sym, p + sh.sh_offset + at, sizeof(sym));
+      if (ELF64_ST_TYPE(sym.st_info) != STT_FUNC || sym.st_name >= names.sh_size || names.sh_size - sym.st_name <= name.size()) continue;
+      if (std::memcmp(p + names.sh_offset + sym.st_name, name.c_str(), name.size() + 1) == 0) return sym.st_size;
+    }
+  }
+  return 0;
+}
+
 int acc_skel_s::load_variant(int v)
 {
   // two threads may meet here on the first launch that needs the unaligned variant
@@ -1229,6 +1268,7 @@ int acc_skel_s::load_variant(int v)
       var.module = nullptr;
       return acc::fail_hip(e, ("hipModuleGetFunction(" + (var.fn_pieces ? lines : pieces) + ")").c_str());
     }
+    if (spec.map_lines) var.lines_code = code_bytes(code, var.job->size, lines);
   }
   (void)hipFuncGetAttribute(&var.num_regs, HIP_FUNC_ATTRIBUTE_NUM_REGS, var.fn);
   if (this->spec.scan_shape_open && v < 2) {

@@ -61,6 +61,7 @@ struct SkelSpec {
   bool map_tiled = false;               // ACC_FLAG_TILED on a map of rank 2 or more: tiles of 32 x 32 elements, a wave each
   int map_tile_block = 4;               // ... a lane's share of a tile: a block of that many elements either way
   bool map_lines = false;               // ... results whose rows are no whole cache lines go out through LDS, in whole lines
+  bool map_loops = false;               // ... the element function's text has loops: what an element takes is not to be told
   bool guarded = false;                 // ACC_FLAG_GUARDED: every kernel takes the address of a loop's guard word last
   bool foldseg_giants = false;          // a segmented fold's variants 4-7: very long segments are handed over to a second launch (skel_foldseg.h)
   bool fold_single = true;              // foldAll in one launch (the last workgroup collects), as generated into the kernel
@@ -86,6 +87,7 @@ struct Variant {
   hipFunction_t fn_across_wide = nullptr;   // ... _across_wide, several rows a lane (elements of at most 8 bytes)
   hipFunction_t fn_pieces = nullptr;   // a map in tiles: _pieces, for results whose rows are no whole cache lines
   hipFunction_t fn_lines = nullptr;    // ... _lines, for large ones of elements of 4 and 8 bytes
+  size_t lines_code = 0;               // ... the bytes of that kernel's code
   hipFunction_t fn_sweep = nullptr;    // a segmented fold's variants 4-7: _sweep, the segments that were handed over;
                                        // its variants 0-3: _probe, a look at the segment lengths
   int num_regs = 0;

@@ -60,3 +60,25 @@ def test_volumes_in_strips_or_by_vectors(ctx, ctype, dt, taps, shape, strips):
         got.append(out.get())
     alike = [np.mean(got[0] == g) for g in got[1:]]            # (a last strip that overlaps its neighbour: either number)
     assert alike[0 if strips else 1] > 0.98 and alike[1 if strips else 0] < 0.5, alike
+
+
+@pytest.mark.parametrize("ctype,dt,degree,loop,lines", [("Int32", np.int32, 4, "", True), ("Int32", np.int32, 20, "", True), ("Int32", np.int32, 64, "", False), ("Int32", np.int32, 0, "for", False),
+                                                        ("Int64", np.int64, 4, "", True), ("Int64", np.int64, 64, "", False), ("Int64", np.int64, 0, "while", False)])
+def test_tiled_maps_in_lines_or_as_they_stand(ctx, ctype, dt, degree, loop, lines):
+    """a result of no whole lines goes out in lines, for which a part of it is evaluated twice, unless its elements are dear"""
+    import acchip as A
+    h, w = 301, 1000
+    loops = {"": "", "for": "for (int i = 0; i < 3; ++i) r = r * q + i; ", "while": "int i = 0; while (i < 3) { r = r * q + i; ++i; } "}[loop]
+    calc = "[&]{ const %s q = arrIn0_0[(ix %% shOut_0) * shOut_1 + ix / shOut_0]; %s r = q; %s%sreturn r * 0 + (%s)blockIdx.x; }()" % (
+        ctype, ctype, loops, "".join("r = (r ^ %d) * q + %d; " % (7 * i + 3, 1 + i) for i in range(degree)), ctype)
+    # (a product by zero that is not seen through: the operands are read, the result says who made it)
+    calc = calc.replace("r * 0", "(r == (%s)0x5a5a5a5b ? 1 : 0)" % ctype)
+    src = ctx.array(np.random.default_rng(3).integers(0, 1000, (w, h)).astype(dt))
+    got = []
+    for knobs in ("map.lines_from_mb=0", "map.lines_from_mb=100000"):
+        with A.tuning(knobs, ctx):
+            sk = ctx.skeleton(A.SKEL_MAP, ctype, env=[(2, ctype)], out_rank=2, flags=A.FLAG_TILED, get=calc, wait=True)
+        out = ctx.empty((h, w), dt)
+        sk.map([src], out)
+        got.append(out.get())
+    assert np.array_equal(got[0], got[1]) != lines
