@@ -966,7 +966,8 @@ int make_spec(const acc_skel_desc *d, const TuningPtr &tuning, SkelSpec *sp)
           }
         const bool at_once = one.size() <= 6 && (int)four.size() * row <= 112;
         if ((2 * rz + 1) * plane <= 192) {
-          sp->flat_planes = std::max(1, std::min(tune("stencil.flat_walk", at_once ? 4 : 8), 16));
+          const int walk = tune("stencil.flat_walk", 0);
+          sp->flat_planes = walk > 0 ? std::min(walk, 16) : at_once ? 4 : 8;
           sp->flat_prefetch = std::max(0, tune("stencil.flat_prefetch", at_once ? sp->flat_planes : (2 * rz + 2) * plane <= 144 ? 1 : 0));
         }
       }

@@ -69,6 +69,37 @@ def test_segments(ctx, right, knobs):
                 assert np.array_equal(outf.get(), chain(y, offs, lambda a, b: a + b, 0.5)), (nseg, mean)
 
 
+@pytest.mark.parametrize("knobs", ["foldseg.giants=0", "foldseg.giants=1"])
+@pytest.mark.parametrize("right", [False, True])
+def test_long_stretches(ctx, right, knobs):
+    """segments of which a staged chunk holds 256 elements or a little less or more, which the whole workgroup then folds, or
+    several chunks, among short ones: such a stretch begins where the workgroup's chunks have it begin, so a sum of Float32
+    has another association for another number of segments a workgroup, and is held to what any association may be off by"""
+    import acchip as A
+    with A.tuning(knobs, ctx):
+        sk = ctx.skeleton(A.SKEL_FOLDSEG, "Word32", env=[(1, "Word32")], get="arrIn0_0[ix]", combine="affine16(x, y)", seed=str(SEED),
+                          preamble=AFFINE, flags=A.FLAG_FOLD_RIGHT if right else 0, wait=True)
+        fl = ctx.skeleton(A.SKEL_FOLDSEG, "float", env=[(1, "float")], get="arrIn0_0[ix]", combine="x + y", seed="0.5f", wait=True)
+    rng = np.random.default_rng(15)
+    for nseg in COUNTS[3:]:
+        print(nseg, flush=True)
+        lens = rng.poisson(20, nseg)
+        at = rng.permutation(nseg)[:6]
+        lens[at] = np.array([255, 256, 257, 511, 3000, 9001])[:len(at)]
+        offs = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+        x = rng.integers(0, 1 << 32, offs[-1] + 5, dtype=np.uint32)
+        out, do = ctx.empty(nseg, np.uint32), ctx.array(offs.astype(np.int32))
+        sk.foldseg([ctx.array(x)], len(x), do, out)
+        assert np.array_equal(out.get(), chain(x, offs, affine, SEED)), nseg
+        if not right:
+            y = rng.standard_normal(len(x)).astype(np.float32)
+            outf = ctx.empty(nseg, np.float32)
+            fl.foldseg([ctx.array(y)], len(y), do, outf)
+            c, m = (np.concatenate([[0], np.cumsum(v)])[offs] for v in (y.astype(np.float64), np.abs(y).astype(np.float64)))
+            # (n additions in any order: n half units in the last place of the sum of the magnitudes)
+            assert np.all(np.abs(outf.get() - (np.diff(c) + 0.5)) <= (lens + 1) * 2.0 ** -24 * (np.diff(m) + 0.5) + 1e-9), nseg
+
+
 @pytest.mark.parametrize("right", [False, True])
 def test_rows(ctx, right):
     import acchip as A

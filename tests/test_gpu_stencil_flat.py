@@ -56,11 +56,11 @@ class _Part(object):
         return self.d
 
 
-@pytest.mark.parametrize("walk", [1, 2, 3, 4, 8, 16, 20])
+@pytest.mark.parametrize("walk", [1, 2, 3, 4, 7, 8, 16])
 @pytest.mark.parametrize("ctype,dt,taps", [("float", np.float32, BOX), ("double", np.float64, STAR), ("Int32", np.int32, ODD)])
 def test_walks_through_several_planes(ctx, ctype, dt, taps, walk):
-    """the ring of planes goes round several times and the last run is cut short: depths round one and two walks, the walk
-    given (left to itself it is the shortest there is at these sizes)"""
+    """the last wave's planes are cut short: depths round one, two and three times the planes a wave makes, their number
+    given"""
     import acchip as A
     fn = " + ".join("(%s)%d * t%d" % (ctype, 3 + k % 5, k) for k in range(len(taps)))
     desc = dict(out_rank=3, taps=taps, stencil_fn=fn)
@@ -83,10 +83,16 @@ def test_walks_through_several_planes(ctx, ctype, dt, taps, walk):
 
 
 @pytest.mark.parametrize("shape", [(83, 84, 300), (160, 150, 150)])
-def test_the_walk_the_driver_chooses(ctx, shape):
-    """volumes for which it is more than the shortest (5 and 8 planes on 256 compute units)"""
+@pytest.mark.parametrize("taps,planes,ahead", [(STAR, 4, 4), (BOX, 8, 1)])
+def test_planes_a_wave_makes_by_itself(ctx, shape, taps, planes, ahead):
+    """four, all asked for at once, where a result reads few rows, else eight with one asked for ahead, whatever the volume; a
+    walk of 0 says the same"""
     import acchip as A
-    desc = dict(out_rank=3, taps=BOX, boundary="mirror", stencil_fn=" + ".join("%d * t%d" % (3 + k % 5, k) for k in range(len(BOX))))
+    desc = dict(out_rank=3, taps=taps, boundary="mirror", stencil_fn=" + ".join("%d * t%d" % (3 + k % 5, k) for k in range(len(taps))))
+    for knobs in ("stencil.flat=1", "stencil.flat_walk=0"):
+        with A.tuning(knobs, ctx):
+            text = A.preview(A.make_desc(A.SKEL_STENCIL, "Int32", **desc), 8)[1]
+        assert "#define ACC_FLAT_PLANES %d\n" % planes in text and "#define ACC_PREFETCH %d\n" % ahead in text
     flat = ctx.skeleton(A.SKEL_STENCIL, "Int32", wait=True, **desc)
     with A.tuning("stencil.nd=1", ctx):
         each = ctx.skeleton(A.SKEL_STENCIL, "Int32", wait=True, **desc)

@@ -1,7 +1,7 @@
-"""Many applications of a 2-D stencil, two a launch (variants 10 and 11), at the sizes where the strips change form: rows of
-one strip exactly, one column and one vector more, two strips; bands cut short, arrays thinner than a band and than what
-two applications reach; operands off the 16-byte boundary; every count of applications up to two pairs of pairs and a
-rest.  One application a launch is the reference: equal in every bit, in the result and in the result before it."""
+"""Many applications of a 2-D stencil, two to four a launch (variants 10 and 11), at the sizes where the strips change form:
+rows of one strip exactly, one column and one vector more, two strips; walks cut short, arrays thinner than a walk and than
+what a launch's applications reach; operands off the 16-byte boundary; counts of applications that split differently.  One
+application a launch is the reference: equal in every bit, in the result and in the result before it."""
 import numpy as np
 import pytest
 
@@ -17,6 +17,13 @@ COLUMNS = [(0, -1), (0, 0), (0, 1)]
 def ctx():
     import acchip as A
     return A.Context(0)
+
+
+def strip(taps, dt, levels=4):
+    """columns of a strip, as the kernel has them: the outermost lanes of either side, as many as go wrong, store nothing"""
+    vec = 16 // np.dtype(dt).itemsize
+    outer = -(-levels // vec) if any(dx for _, dx in taps) else 1
+    return (64 - 2 * outer) * vec
 
 
 class _Part(object):
@@ -40,7 +47,7 @@ def test_pairs_against_single_applications(ctx, boundary, ctype, dt, taps):
     twos = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
     with A.tuning("stencil.pair=0", ctx):
         ones = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
-    own = 62 * (16 // np.dtype(dt).itemsize)
+    own = strip(taps, dt)
     rng = np.random.default_rng(6)
     for shape in ((3, own), (8, own + 1), (9, own + 4), (9, own + 5), (16, 2 * own), (17, 2 * own - 3), (33, 2 * own + 1), (12, 2 * own + 4),
                   (40, 3 * own + 7), (24, 3 * own - 1)):
@@ -68,7 +75,7 @@ def test_walks_and_counts(ctx, boundary, ctype, dt, taps):
     desc = dict(out_rank=2, taps=taps, boundary=boundary, stencil_fn=fn, boundary_constant="(%s)7" % ctype if boundary == "constant" else None)
     with A.tuning("stencil.pair=0", ctx):
         ones = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
-    own = 60 * (16 // np.dtype(dt).itemsize)
+    own = strip(taps, dt)
     rng = np.random.default_rng(7)
     for walk, shape, counts in ((0, (29, 2 * own + 9), range(1, 15)), (28, (90, own + 24), (4, 9)), (5, (37, 2 * own - 8), (4, 9)), (1, (6, own + 16), (5, 9))):
         with A.tuning("stencil.pair_walk=%d" % walk, ctx):
@@ -94,7 +101,7 @@ def test_walks_that_go_up(ctx, boundary, ctype, dt, taps):
     desc = dict(out_rank=2, taps=taps, boundary=boundary, stencil_fn=fn)
     with A.tuning("stencil.pair=0", ctx):
         ones = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
-    own = 60 * (16 // np.dtype(dt).itemsize)
+    own = strip(taps, dt)
     rng = np.random.default_rng(11)
     for walk, h in ((1, 16), (3, 31), (4, 33), (28, 141)):
         with A.tuning("stencil.pair_walk=%d" % walk, ctx):
@@ -124,9 +131,9 @@ def test_two_a_launch(ctx, boundary, ctype, dt, taps):
         ones = ctx.skeleton(A.SKEL_STENCIL, ctype, wait=True, **desc)
     vec, esz = 16 // np.dtype(dt).itemsize, np.dtype(dt).itemsize
     widths = set()
-    for levels in (2, 3, 4):                      # a strip, as the kernel has it: the outermost lanes of either side store nothing
-        outer = -(-levels // vec) if any(dx for _, dx in taps) else 1
-        own = (64 - 2 * outer) * vec
+    for levels in (2, 3, 4):
+        own = strip(taps, dt, levels)
+        outer = (64 - own // vec) // 2
         widths |= {own, own + 1, own + outer * vec - 1, own + outer * vec, 2 * own + 1}
     rng = np.random.default_rng(8)
     for w in sorted(widths):

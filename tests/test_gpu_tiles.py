@@ -80,8 +80,8 @@ def test_large_matrices_of_whole_lines(ctx):
 
 @pytest.mark.parametrize("ctype,dt", [("Int32", np.int32), ("double", np.float64), ("Int16", np.int16)])
 def test_tiles_in_whole_lines(ctx, ctype, dt):
-    """results whose rows are no whole cache lines go out in lines, those whose rows are down strips eight groups tall: widths
-    either side of what a workgroup writes, of whole lines, results that begin anywhere within a line"""
+    """results whose rows are no whole cache lines go out in lines: widths either side of what a workgroup writes, of whole
+    lines, results that begin anywhere within a line"""
     import acchip as A
     get = FORMS["transpose"]
     with A.tuning("map.lines_from_mb=0", ctx):
@@ -101,3 +101,22 @@ def test_tiles_in_whole_lines(ctx, ctype, dt):
                 got = out.get()
                 assert np.array_equal(got[shift:shift + h * w].reshape(h, w), x.T), (h, w, shift)
                 assert np.all(got[:shift] == 77) and np.all(got[shift + h * w:] == 77), (h, w, shift)
+
+
+@pytest.mark.parametrize("ctype,dt", [("Int32", np.int32), ("double", np.float64)])
+def test_in_place(ctx, ctype, dt):
+    """the result is one of the operands, read where it is written: what two workgroups evaluate for the sake of whole lines
+    only the one that writes it counts, and that one has read by then"""
+    import acchip as A
+    with A.tuning("map.lines_from_mb=0", ctx):
+        sk = ctx.skeleton(A.SKEL_MAP, ctype, env=[(2, ctype), (2, ctype)], out_rank=2, flags=A.FLAG_TILED, wait=True,
+                          get="2 * arrIn0_0[ix] + " + FORMS["transpose"].replace("In0", "In1"))
+    rng = np.random.default_rng(14)
+    for h, w in [(33, 97), (65, 193), (1030, 1001), (3001, 999)]:
+        x, y = rng.integers(-1000, 1000, (w, h)).astype(dt), rng.integers(-1000, 1000, (h, w)).astype(dt)
+        src, out, want = ctx.array(x), ctx.array(y), y
+        for _ in range(4):
+            print(ctype, h, w, flush=True)
+            sk.map([out, src], out)
+            want = 2 * want + x.T
+            assert np.array_equal(out.get(), want), (h, w)
