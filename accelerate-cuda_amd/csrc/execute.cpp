@@ -193,6 +193,23 @@ void push_out(const acc_array &out, Args *args, bool *aligned)
   push_ptrs(&out, out.ncomp, args, aligned);
 }
 
+// whether a result shares memory with one of the free array variables
+bool out_in_env(const acc_skel_s *s, const acc_array *env, const acc_array &out)
+{
+  const std::vector<acc::EnvSig> &sig = s->spec.env;
+  const uint64_t n_out = static_cast<uint64_t>(array_size(out));
+  for (size_t k = 0; k < sig.size(); ++k) {
+    const uint64_t n = static_cast<uint64_t>(array_size(env[k]));
+    for (int c = 0; c < env[k].ncomp; ++c)
+      for (int o = 0; o < out.ncomp; ++o) {
+        const uint64_t bytes = n * (uint64_t)acc::type_size(sig[k].type[c]);
+        const uint64_t bytes_out = n_out * (s->spec.comp_types.empty() ? s->spec.elt_size : acc::type_size(s->spec.comp_types[out.ncomp - 1 - o]));
+        if (env[k].ptr[c] < out.ptr[o] + bytes_out && out.ptr[o] < env[k].ptr[c] + bytes) return true;
+      }
+  }
+  return false;
+}
+
 int launch(acc_skel_s *s, int variant, int64_t grid, size_t dyn_lds, hipStream_t stream, Args *args)
 {
   if (grid < 1 || grid > 0x7fffffffLL) return fail(ACC_ERR_INVALID, "%s: grid of %lld blocks", s->entry.c_str(), (long long)grid);
@@ -308,6 +325,12 @@ int acc_exec_map(acc_skel s, const acc_array *env, const acc_array *out, acc_str
     const int64_t waves = s->variants[v].block / 64;
     bool whole = (w * esz) % 128 == 0;
     for (int c = 0; c < out->ncomp; ++c) whole = whole && out->ptr[c] % 128 == 0;
+    // A result in place of an operand takes the form for whole lines whatever its rows are, the one that evaluates every
+    // element once: in the others workgroups evaluate their neighbours' columns too, and lanes beyond the result its last row or
+    // column, which by then may hold what has been written -- no index any more, for instance.  (It is the slower one where
+    // rows are no whole lines: a matrix plus another one transposed, in place, us as pieces or lines / so: 1001 x 999 Float32
+    // 4.6 / 6.3, 12000 x 501 16.2 / 16.9, 5003 x 3001 32.3 / 37.1, 8191^2 161.9 / 161.1, 7001 x 2500 Float64 71 / 91.)
+    whole = whole || out_in_env(s, env, *out);
     const bool strips = whole && n == w * h && n * esz >= acc::map_strips_from;
     // Results of no whole lines, or that begin amid one, go out in lines from 28 MB on, about what the L2s hold together (us as
     // they stand / in lines, operands that the memory-side cache does not hold: 5003 x 3001 Float32 33.3 / 28.8, 8191^2 148 / 104,

@@ -440,7 +440,10 @@ int acc_skel_get_info(acc_skel s, acc_skel_info *out);
  * `stream` and the call returns without waiting.                             */
 
 /* map / generate / transform: executeOp, Execute.hs:264-268.  out has the
- * desc's out_rank; one element is written per index of out.                 */
+ * desc's out_rank; one element is written per index of out.  out may share
+ * storage with an array of env of which an element is read only to make the
+ * element written in its place: every element is then evaluated once.  (Where
+ * they share none, a map in tiles may evaluate elements again.)              */
 int acc_exec_map(acc_skel s, const acc_array *env, const acc_array *out, acc_stream stream);
 
 /* fold / fold1: foldOp / fold1Op / foldCore / foldRec, Execute.hs:282-318.

@@ -103,20 +103,24 @@ def test_tiles_in_whole_lines(ctx, ctype, dt):
                 assert np.all(got[:shift] == 77) and np.all(got[shift + h * w:] == 77), (h, w, shift)
 
 
-@pytest.mark.parametrize("ctype,dt", [("Int32", np.int32), ("double", np.float64)])
-def test_in_place(ctx, ctype, dt):
-    """the result is one of the operands, read where it is written: what two workgroups evaluate for the sake of whole lines
-    only the one that writes it counts, and that one has read by then"""
+@pytest.mark.parametrize("ctype,dt", [("Int32", np.int32), ("double", np.float64), ("Int16", np.int16)])
+@pytest.mark.parametrize("lines_from", [0, 28])
+def test_in_place(ctx, ctype, dt, lines_from):
+    """the result is one of the operands, read where it is written: every element is evaluated once, so that none is made of
+    what has been written already (an index that has been replaced by what it names, for instance)"""
     import acchip as A
-    with A.tuning("map.lines_from_mb=0", ctx):
-        sk = ctx.skeleton(A.SKEL_MAP, ctype, env=[(2, ctype), (2, ctype)], out_rank=2, flags=A.FLAG_TILED, wait=True,
-                          get="2 * arrIn0_0[ix] + " + FORMS["transpose"].replace("In0", "In1"))
+    get = "(atomicAdd((int *)&arrIn2_0[ix], 1), (%s)(2 * arrIn0_0[ix] + %s))" % (ctype, FORMS["transpose"].replace("In0", "In1"))
+    with A.tuning("map.lines_from_mb=%d" % lines_from, ctx):
+        sk = ctx.skeleton(A.SKEL_MAP, ctype, env=[(2, ctype), (2, ctype), (2, "Int32")], out_rank=2, flags=A.FLAG_TILED, wait=True, get=get)
     rng = np.random.default_rng(14)
-    for h, w in [(33, 97), (65, 193), (1030, 1001), (3001, 999)]:
-        x, y = rng.integers(-1000, 1000, (w, h)).astype(dt), rng.integers(-1000, 1000, (h, w)).astype(dt)
-        src, out, want = ctx.array(x), ctx.array(y), y
-        for _ in range(4):
-            print(ctype, h, w, flush=True)
-            sk.map([out, src], out)
-            want = 2 * want + x.T
-            assert np.array_equal(out.get(), want), (h, w)
+    for h, w in [(33, 97), (65, 193), (33, 128), (1030, 1001), (3001, 999), (2, 999)]:
+        x, y = rng.integers(-9, 9, (w, h)).astype(dt), rng.integers(-9, 9, (h, w)).astype(dt)
+        for shift in (0, 1):
+            src, out, want = ctx.array(x), ctx.array(np.concatenate([np.full(shift, 7, dt), y.reshape(-1)])), y
+            here, counts = out.desc(shape=(h, w), offset_elems=shift), ctx.array(np.zeros((h, w), np.int32))
+            for turn in range(1, 4):
+                print(ctype, h, w, shift, flush=True)
+                sk.map([here, src, counts], here)
+                want = 2 * want + x.T
+                assert np.array_equal(out.get()[shift:].reshape(h, w), want) and np.all(out.get()[:shift] == 7), (h, w, shift)
+                assert np.all(counts.get() == turn), (h, w, shift)
